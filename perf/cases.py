@@ -274,6 +274,104 @@ def run(state):
     return (out.detach(),) + torch.autograd.grad(out, params, state["grad"])
 
 
+# ------------------------------------------------------------------------------------------- the results in 64 bits
+
+_FUDGE = 0.001  # the interface's default normalization_term_fudge
+
+
+def _by_images(fn, x, params, grad, want_x=True, step=1):
+    """fn(images, *params) in 64 bits, `step` images at a time; with `grad` (fn's result's) also the gradients, the
+    parameters' summed over the batch.  Few images at a time bound the memory of the term-by-term sums."""
+    params = [p.detach().double() for p in params]
+    outs, gx, gp = [], [], [torch.zeros_like(p) for p in params]
+    for i in range(0, x.shape[0], step):
+        xi = x[i:i + step].detach().double()
+        if grad is None:
+            outs.append(fn(xi, *params))
+            continue
+        leaves = [t.clone().requires_grad_() for t in [xi] * want_x + params]
+        out = fn(*leaves) if want_x else fn(xi, *leaves)
+        g = list(torch.autograd.grad(out, leaves, grad[i:i + step].double()))
+        if want_x:
+            gx.append(g.pop(0))
+        for a, b in zip(gp, g):
+            a += b
+        outs.append(out.detach())
+    out = torch.cat(outs)
+    return out if grad is None else (out,) + ((torch.cat(gx),) if want_x else ()) + tuple(gp)
+
+
+def _exact_similarity(kw):
+    (bh, bw), (sh, sw), (ph, pw) = kw["blocks"], kw["strides"], kw["padding"]
+    norm, nan, l1 = kw.get("normalization_term"), kw.get("ignore_nan_input"), kw.get("similarity_function") == "L1"
+
+    def fn(x, t, w):
+        oh, ow = _out(x.shape[2], ph, bh, sh), _out(x.shape[3], pw, bw, sw)
+        x = torch.nn.functional.pad(x, (pw, pw, ph, ph), value=kw.get("out_of_bounds_value", 0.0))
+        keep = (x == x).double() if nan else torch.ones_like(x)
+        x = torch.where(x == x, x, torch.zeros_like(x)) if nan else x
+        # patch element k = (channel, row, column), output pixel
+        cols = [v.unfold(2, bh, sh).unfold(3, bw, sw).permute(0, 1, 4, 5, 2, 3).reshape(v.shape[0], -1, oh * ow)
+                for v in (x, keep)]
+        t, w = t.reshape(t.shape[0], -1), w.reshape(w.shape[0], -1)
+        if l1:
+            out = torch.cat([-(w[m:m + 8, :, None] * (t[m:m + 8, :, None] - cols[0][:, None]).abs()).sum(2)
+                             for m in range(0, t.shape[0], 8)], 1)
+        else:
+            # NaN inputs are 0 here and their terms weighted 0: products of three matrices give all the sums
+            out = -(w @ (cols[0] * cols[0]) - 2 * (w * t) @ cols[0] + (w * t * t) @ cols[1])
+        if norm:
+            out = 0.5 * (out + (torch.log(w + _FUDGE) - math.log(2 * math.pi)) @ cols[1])
+        return out.reshape(x.shape[0], -1, oh, ow)
+    return fn
+
+
+def _exact_mex(kw, instances):
+    b, s = kw["blocks"][1], kw["strides"][1]
+    p = kw.get("padding", [0, 0, 0])[1]
+
+    def fn(x, off):
+        x = torch.nn.functional.pad(x, (p, p, p, p))  # blocks_out_of_bounds_value is 0
+        cols = x.unfold(2, b, s).unfold(3, b, s)
+        n, c, oh, ow = cols.shape[:4]
+        cols = cols.permute(0, 2, 3, 1, 4, 5).reshape(n, oh, ow, -1)
+        off = torch.log_softmax(off.reshape(off.shape[0], instances, -1), 2)
+        side = math.isqrt(off.shape[0])  # regions interleave: a pixel's is (row, column) modulo the region's side
+        out = x.new_zeros(n, instances, oh, ow)
+        for r in range(off.shape[0]):
+            rh, rw = r // side, r % side
+            part = cols[:, rh::side, rw::side]
+            top, otop = part.amax(-1, keepdim=True).detach(), off[r].amax(-1, keepdim=True).detach()
+            sums = torch.exp(part - top) @ torch.exp(off[r] - otop).T
+            out = out.clone()
+            out[:, :, rh::side, rw::side] = (torch.log(sums) + top + otop[:, 0]).permute(0, 3, 1, 2)
+        return out
+    return fn
+
+
+def exact(case, seed):
+    kind, state = case["kind"], prepare(case, seed)
+    if kind in ("similarity", "similarity_train"):
+        return _by_images(_exact_similarity(state["kw"]), state["x"], (state["t"], state["w"]), state.get("grad"))
+    if kind in ("mex", "mex_train"):
+        return _by_images(_exact_mex(state["kw"], state["n"]), state["x"], (state["off"],), state.get("grad"))
+    if kind == "pair":
+        sim = _by_images(_exact_similarity(state["kw"]), state["x"], (state["t"], state["w"]), None, step=16)
+        return sim, _by_images(_exact_mex(state["mex"], state["n"]), sim, (state["off"],), None, step=16)
+    # the whole network, image by image, from the parameters that the layers and the prepared calls were made of
+    pairs, head = _stack_layers(case)
+    state = prepare(dict(case, kind="stack_train"), seed)
+    kw, opts, instances = state["kw"], state["opts"], state["instances"]
+
+    def network(x, t, w, *offs):
+        cur = _exact_similarity(kw)(x, t, w)
+        for off, n, opt in zip(offs[:-1], instances, opts):
+            cur = 4 * torch.nn.functional.avg_pool2d(_exact_mex(opt, n)(cur, off), 2)
+        return _exact_mex(opts[-1], instances[-1])(cur, offs[-1])
+    grad = state["grad"] if kind == "stack_train" else None
+    return _by_images(network, state["x"], state["params"], grad, want_x=False, step=32)
+
+
 # ------------------------------------------------------------------------------------------- work and tolerances
 
 # Operations of one term of a sum.  Similarity forward: L2 sub, mul, fused multiply-add; L1 sub, |.|-multiply-add; the
