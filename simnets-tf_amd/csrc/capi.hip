@@ -100,6 +100,8 @@ int simnets_hip_similarity_fwd_static(const simnets_similarity_attrs *attrs, con
     const int rc = sim_make_plan(attrs, input_shape, templates_shape, weights_shape, &p);
     if (rc)
         return rc;
+    if (sim_workspace_bytes(p) > SIMNETS_HIP_STATIC_SCRATCH_BYTES)
+        p.split = 0;   // the forms on the vector units need less
     const size_t need = sim_workspace_bytes(p);
     if (need > SIMNETS_HIP_STATIC_SCRATCH_BYTES)
         return SIMNETS_ERR_STATIC_SCRATCH;

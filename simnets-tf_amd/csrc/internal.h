@@ -22,6 +22,7 @@ struct SimPlan {
     int exact_terms;  // the caller named SIMNETS_ALGO_DIRECT: gradients, too, sum the reference's terms one by one
     float fudge, oob;
     int norm_const_every_iteration;
+    int split;        // the library may evaluate the L2 modes on the matrix cores in 16-bit pieces (sim_split.h)
 };
 
 // Validates like SimilarityKernelCommon (ctor + CalculateDimensions) and fills the plan.

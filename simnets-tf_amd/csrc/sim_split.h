@@ -1,0 +1,194 @@
+// Shared by the split matrix-core form of the L2 Similarity modes (similarity_split.hip) and the direct kernels that
+// pack its parameters and recompute the tiles it flags (similarity_direct.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "internal.h"
+
+namespace simnets {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kSplitPixels = 128;   // output pixels of a workgroup, consecutive over the whole batch
+constexpr int kSplitRows = 32;      // templates of one matrix tile
+constexpr int kSplitMaxC = 4096;    // channels whose centres the packing kernel keeps in LDS
+
+// Geometry of one call on the split form.
+struct SplitPlan {
+    bool on;
+    int cg;       // channels of a staged chunk: 16 (a matrix step is one tap) or 8 (a step is two taps)
+    int chunks;   // ceil(C / cg)
+    int steps;    // matrix steps per chunk: taps, or ceil(taps / 2)
+    int pieces;   // 16-bit pieces of the packed parameters per step: 6, with missing values 12
+    int n_mtiles; // ceil(O / 32)
+    int n_ptiles; // ceil(B oh ow / 128)
+    int Wp, Hv;   // columns of a staged row; rows of one image's staged stack
+    size_t packed, ctr, bias, lg, thr, flags, total;   // workspace, from its own start
+};
+
+SplitPlan sim_split_plan(const SimPlan &p);
+
+struct SplitPack {
+    const float *templates, *weights;
+    unsigned short *packed;
+    float *ctr, *bias, *lg, *thr;
+    int O, C, taps, K, cg, chunks, steps, pieces, n_mtiles, mode;
+    float fudge, norm_const;
+    int pack_blocks, thr_blocks;   // pack_blocks = chunks * n_mtiles * ceil(steps / 4)
+};
+
+int sim_split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, float *output, char *ws, hipStream_t s);
+SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float *templates, const float *weights,
+                              char *ws);
+
+// v = p0 + p1 + p2, each the nearest 16-bit value to what is left: 24 bits of mantissa, exact for every v whose pieces
+// are normal numbers.
+__device__ __forceinline__ void split3(float v, __bf16 &p0, __bf16 &p1, __bf16 &p2)
+{
+    p0 = (__bf16)v;
+    const float r = v - (float)p0;
+    p1 = (__bf16)r;
+    p2 = (__bf16)(r - (float)p1);
+}
+
+// What is subtracted from every value of a channel: the mean of up to 32 template elements spread over the channel.  Any
+// value is correct; one near the data keeps the three sums of w (x - t)^2 from cancelling.  Sixteen lanes share a
+// channel; all of them get the result, the same wherever it is computed.
+__device__ __forceinline__ float split_centre_part(const SplitPack &a, int c)
+{
+    const int n = a.O * a.taps, ns = min(32, n), apart = n / ns;
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int q = (threadIdx.x & 15) + 16 * i, e = q * apart, m = e / a.taps;
+        if (q < ns && c < a.C)
+            s += a.templates[((size_t)m * a.C + c) * a.taps + (e - m * a.taps)];
+    }
+    return s;
+}
+
+__device__ __forceinline__ float split_centre(const SplitPack &a, float part)
+{
+    for (int d = 8; d > 0; d >>= 1)
+        part += __shfl_xor(part, d, 16);
+    part /= (float)min(32, a.O * a.taps);
+    return __builtin_fabsf(part) < 1e18f ? part : 0.0f;
+}
+
+// The parameter-only part, run by the first pack_blocks + thr_blocks workgroups (256 threads) of the packing launch;
+// `lds` holds max(C, 16) floats.
+__device__ inline void split_pack_block(const SplitPack &a, int block, float *lds)
+{
+    const int tid = threadIdx.x;
+    const bool masked = a.mode == SIM_MODE_L2_NORM_IGNORE_NAN;
+    auto logterm = [&](float w) {   // as sim_pack_element's
+        return masked ? (float)(0.5 * ((double)logf(w + a.fudge) - 1.8378770664093453 /* log(2 pi) */))
+                      : 0.5f * logf(w + a.fudge);
+    };
+    if (block < a.pack_blocks) {
+        const int parts = (a.steps + 3) / 4;   // of a chunk's steps, four to a workgroup
+        const int mtile = block / (a.chunks * parts), rest = block - mtile * a.chunks * parts;
+        const int chunk = rest / parts, part = rest - chunk * parts;
+        if (tid < a.cg * 16) {
+            const int cl = tid >> 4;
+            const float centre = split_centre(a, split_centre_part(a, chunk * a.cg + cl));
+            if ((tid & 15) == 0) {
+                lds[cl] = centre;
+                if (mtile == 0 && part == 0)
+                    a.ctr[chunk * a.cg + cl] = centre;
+            }
+        }
+        __syncthreads();
+        const int step = 4 * part + (tid >> 6);
+        if (step < a.steps) {
+            const int lane = tid & 63, half = lane >> 5, m = mtile * kSplitRows + (lane & 31);
+            const int tap = a.cg == 16 ? step : 2 * step + half;
+            bf16x8 v[12];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int cl = a.cg == 16 ? 8 * half + j : j, c = chunk * a.cg + cl;
+                float t = 0.0f, w = 0.0f, l = 0.0f;
+                if (m < a.O && c < a.C && tap < a.taps) {
+                    const size_t at = ((size_t)m * a.C + c) * a.taps + tap;
+                    w = a.weights[at];
+                    t = a.templates[at] - lds[cl];
+                    if (masked)
+                        l = logterm(w);
+                }
+                __bf16 p0, p1, p2;
+                auto put = [&](int at, float value) {
+                    split3(value, p0, p1, p2);
+                    v[at][j] = p0;
+                    v[at + 1][j] = p1;
+                    v[at + 2][j] = p2;
+                };
+                put(0, -w);
+                put(3, 2.0f * w * t);
+                if (masked) {
+                    put(6, -(w * t) * t);
+                    put(9, l);
+                }
+            }
+            bf16x8 *dst = reinterpret_cast<bf16x8 *>(a.packed) +
+                          (((size_t)mtile * a.chunks + chunk) * a.steps + step) * a.pieces * 64 + lane;
+#pragma unroll
+            for (int q = 0; q < 12; ++q)
+                if (q < a.pieces)
+                    dst[q * 64] = v[q];
+        }
+        return;
+    }
+    // biases and thresholds, one wave per template
+    for (int c0 = 0; c0 < a.C; c0 += 64) {   // the loads of four channels in flight
+        float part[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            part[i] = split_centre_part(a, c0 + 16 * i + (tid >> 4));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = c0 + 16 * i + (tid >> 4);
+            const float centre = split_centre(a, part[i]);
+            if ((tid & 15) == 0 && c < a.C)
+                lds[c] = centre;
+        }
+    }
+    __syncthreads();
+    const int lane = tid & 63;
+    for (int m = (block - a.pack_blocks) * 4 + (tid >> 6); m < a.n_mtiles * kSplitRows; m += a.thr_blocks * 4) {
+        double tc2 = 0.0, traw = 0.0, lsum = 0.0;
+        bool bad = false;
+        if (m < a.O)
+#pragma unroll 4
+            for (int k = lane; k < a.K; k += 64) {
+                const float t = a.templates[(size_t)m * a.K + k], w = a.weights[(size_t)m * a.K + k];
+                const float tc = t - lds[k / a.taps];
+                tc2 += (double)w * tc * tc;
+                traw += (double)w * t * t;
+                // weights and templates outside this range: the pieces of their products may leave the range of
+                // normal numbers, so such a template is left to the term-by-term kernel
+                bad |= !(w == 0.0f || (w >= 0x1p-60f && w <= 0x1p20f)) || !(__builtin_fabsf(t) <= 0x1p60f);
+                if (a.mode != SIM_MODE_L2) {
+                    const float l = logterm(w);
+                    lsum += l;
+                    bad |= !(__builtin_fabsf(l) <= 1e6f);
+                }
+            }
+        for (int d = 32; d > 0; d >>= 1) {
+            tc2 += __shfl_xor(tc2, d, 64);
+            traw += __shfl_xor(traw, d, 64);
+            lsum += __shfl_xor(lsum, d, 64);
+        }
+        bad = __any(bad);
+        if (lane == 0) {
+            a.bias[m] = masked ? 0.0f : -(float)tc2;
+            a.lg[m] = masked || a.mode == SIM_MODE_L2 ? 0.0f : (float)(lsum + (double)a.norm_const);
+            double thr = 0x1p-60;
+            if (!masked)
+                thr = fmax(thr, fmax(0.25 * tc2, traw / 1024.0));
+            a.thr[m] = bad || !(thr < 1e37) ? INFINITY : (float)thr;
+        }
+    }
+}
+
+}  // namespace simnets

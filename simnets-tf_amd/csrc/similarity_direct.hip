@@ -28,6 +28,7 @@
 #include "internal.h"
 #include "stage.h"
 #include "valu_tile.h"
+#include "sim_split.h"
 #include "sim_step.h"
 
 namespace simnets {
@@ -74,6 +75,9 @@ struct SimKernelArgs {
     const float *thr;  // [O] a partial sum of template m above -thr[m] sends its wave to the recomputing pass
     int *flags;        // [workgroups * kWaves] 1: the wave left its outputs to the recomputing pass
     // self-packing gather kernel only: the parameters as the caller holds them, [O][K] each
+    const int *gate;   // flags [pixel tile of 128][template tile of 32] of the split form's launch in front of this one:
+                       // only workgroups that touch a flagged tile run; null: all do
+    int gate_mtiles;
     const float *raw_t, *raw_w;
     float fudge;
 };
@@ -123,6 +127,17 @@ __device__ __forceinline__ LanePos lane_pos(const SimKernelArgs &a, int wave, in
 
 // Wave-uniform parameter fetch of the gather fallback: the address is the same in every lane, so these
 // become scalar loads (s_load_dwordx8/x16) and the values live in SGPRs.
+// Whether the split form left a tile of these outputs (pixels n0..n1 over the batch, templates m0..m1) to this launch.
+__device__ __forceinline__ bool split_flagged(const SimKernelArgs &a, int n0, int n1, int m0, int m1)
+{
+    const int t0 = n0 / kSplitPixels, nt = n1 / kSplitPixels - t0 + 1;
+    const int r0 = m0 / kSplitRows, nr = m1 / kSplitRows - r0 + 1;
+    int any = 0;
+    for (int i = threadIdx.x; i < nt * nr; i += blockDim.x)
+        any |= a.gate[(size_t)(t0 + i / nr) * a.gate_mtiles + r0 + i % nr];
+    return __syncthreads_or(any) != 0;
+}
+
 template <int MODE, int MT>
 __device__ __forceinline__ void load_params(float (&pa)[2 * MT], float (&pc)[MT], const float SIMNETS_CONST_AS *ppa,
                                             const float SIMNETS_CONST_AS *ppc)
@@ -459,6 +474,13 @@ __global__ __launch_bounds__(kThreads, waves_per_simd(PT, MT)) void sim_direct_k
 {
     extern __shared__ float lds[];
     int wave_bail = 0;
+    if (a.gate != nullptr) {
+        const LanePos lp = lane_pos(a, 0, 0);
+        const int nm = (kWaves >> a.nws_log2) * MT, n0 = lp.b * a.oh * a.ow;
+        if (!split_flagged(a, n0 + lp.row_first * a.ow, n0 + (lp.g_last / a.G + 1) * a.ow - 1, lp.by * nm,
+                           min(a.O, (lp.by + 1) * nm) - 1))
+            return;
+    }
     sim_direct_body<MODE, PT, MT, SWT, false, PLDS, ROW3>(a, lds, wave_bail);
     if constexpr (MODE == SIM_MODE_L2_SQRTW) {
         if (__syncthreads_or(wave_bail)) {
@@ -493,6 +515,11 @@ __global__ __launch_bounds__(64 * WAVES) void sim_small_map_kernel(const SimKern
     }
     const int img_l = lane / a.gpi, g_l = lane - img_l * a.gpi;
     const int b0 = blockIdx.x * a.NI;
+    if (a.gate != nullptr) {
+        const int npix = a.oh * a.ow, m0 = blockIdx.y * MT;
+        if (!split_flagged(a, b0 * npix, min(b0 + a.NI, a.B) * npix - 1, m0, min(m0 + MT, a.O) - 1))
+            return;
+    }
     const bool lane_valid = img_l < a.NI && b0 + img_l < a.B;
     const int img = lane_valid ? img_l : 0, g = lane_valid ? g_l : 0;
     const int b = b0 + img;
@@ -812,12 +839,19 @@ __global__ __launch_bounds__(256) void sim_pack_params_kernel(const float *__res
                                                              float *__restrict__ pc, int *__restrict__ koff, int taps,
                                                              int bw, int CC, int chan_pitch, int TC,
                                                              float *__restrict__ pa2, float *__restrict__ thr,
-                                                             int pack_blocks)
+                                                             int pack_blocks, const SplitPack split)
 {
-    if ((int)blockIdx.x >= pack_blocks) {
+    extern __shared__ float split_lds[];
+    const int split_blocks = split.pack_blocks + split.thr_blocks;
+    if ((int)blockIdx.x < split_blocks) {
+        split_pack_block(split, blockIdx.x, split_lds);
+        return;
+    }
+    const int block = blockIdx.x - split_blocks;
+    if (block >= pack_blocks) {
         const int lane = threadIdx.x & 63;
-        const int nb = gridDim.x - pack_blocks;
-        for (int m = (blockIdx.x - pack_blocks) * 4 + (threadIdx.x >> 6); m < O; m += nb * 4) {
+        const int nb = gridDim.x - split_blocks - pack_blocks;
+        for (int m = (block - pack_blocks) * 4 + (threadIdx.x >> 6); m < O; m += nb * 4) {
             float t2 = 0.0f;
             bool bad = false;
             for (int k = lane; k < K; k += 64) {
@@ -835,7 +869,7 @@ __global__ __launch_bounds__(256) void sim_pack_params_kernel(const float *__res
     }
     const int nthreads = pack_blocks * 256;
     // LDS offset of patch element k inside a staged chunk of CC channels; 0 behind the last k
-    for (int k = blockIdx.x * 256 + threadIdx.x; k < K + 2; k += nthreads) {
+    for (int k = block * 256 + threadIdx.x; k < K + 2; k += nthreads) {
         int off = 0;
         if (k < K) {
             const int c = k / taps, rem = k - c * taps;
@@ -845,7 +879,7 @@ __global__ __launch_bounds__(256) void sim_pack_params_kernel(const float *__res
         koff[k] = off;
     }
     const long long total = (long long)n_mtiles * K * MT;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += nthreads) {
+    for (long long i = (long long)block * 256 + threadIdx.x; i < total; i += nthreads) {
         const int mi = (int)(i % MT);
         const long long r = i / MT;
         const int k = (int)(r % K);
@@ -1043,13 +1077,27 @@ hipError_t launch_mode(const SimKernelArgs &a0, const Tiling &t, bool plds, hipS
     return launch_direct<MODE, kSmallPT, kSmallMT, false>(a, grid, lds_bytes, s);
 }
 
+// The split form, where the tiled kernels can recompute what it flags, and where it is the more precise one: the
+// small-map kernel's sums come in four or eight parts, which for short patches, and with missing values, rounds as
+// little (64 x 24 x 7 x 9, 3 x 3: 5.6e-8 of the output's 2-norm against the split form's 5.9e-8; 64 x 130 x 9 x 10, 5 x 5, a
+// quarter missing: 1.0e-7 against 2.0e-7; from 256 elements on without missing values the split form's is the smaller).
+SplitPlan split_plan(const SimPlan &p, const Tiling &t)
+{
+    if (!t.lds_ok || (t.NI > 0 && (p.K < 256 || p.mode == SIM_MODE_L2_NORM_IGNORE_NAN)))
+        return SplitPlan();
+    const SplitPlan s = sim_split_plan(p);
+    // a small-map grid needs enough workgroups to beat that kernel's split of the patch (8 x 200 x 14 x 14 -> 200, 5 x 5,
+    // 91 tiles: 199 us there, 265 here; 200 x 32 x 7 x 7 -> 64, 154 tiles: 33 and 26)
+    return t.NI > 0 && 1LL * s.n_ptiles * s.n_mtiles < 150 ? SplitPlan() : s;
+}
+
 // The sqrt-weight form runs on the tiled kernels and on the small-map kernel; there only with enough pixels per
 // parameter, or packing the second copy of the parameters costs more than the shorter inner loop saves (512
 // templates over 512 x 7 x 7 inputs: at 32 images 0.425 -> 0.391 ms per self-packing call and 0.413 -> 0.358 ms
 // prepared, at 16 images 0.222 -> 0.223 and 0.212 -> 0.190 ms, at 8 images the same ratios).
 bool use_sqrtw(const SimPlan &p, const Tiling &t)
 {
-    return p.algo == SIMNETS_ALGO_SQRTW && t.lds_ok && (t.NI == 0 || (long long)p.B * p.oh * p.ow >= 512);
+    return p.algo == SIMNETS_ALGO_SQRTW && t.lds_ok && !split_plan(p, t).on && (t.NI == 0 || (long long)p.B * p.oh * p.ow >= 512);
 }
 
 // flags of the guard that live in the workspace: one per workgroup of the small-map kernel (the tiled kernels keep
@@ -1064,10 +1112,10 @@ long long guard_flags(const SimPlan &p, const Tiling &t)
 // the second packed copy and the thresholds (all written by the pack kernel) and, for the small-map kernel, the
 // workgroup flags (written by every main launch, read by the recomputing launch behind it).
 struct Layout {
-    size_t pa, pc, koff, pa2, thr, flags, total;
+    size_t pa, pc, koff, pa2, thr, flags, split, total;
 };
 
-Layout layout(const SimPlan &p, const Tiling &t)
+Layout layout(const SimPlan &p, const Tiling &t, const SplitPlan &split)
 {
     const size_t n_mtiles = (p.O + t.MT - 1) / t.MT;
     // one extra k of slack behind each array: the parameter loads are issued one step ahead
@@ -1085,19 +1133,26 @@ Layout layout(const SimPlan &p, const Tiling &t)
         l.flags = l.thr + align_up((size_t)p.O * sizeof(float), 256);
         l.total = l.flags + align_up((size_t)guard_flags(p, t) * sizeof(int), 256);
     }
+    l.split = l.total;
+    l.total += split.total;
     return l;
 }
 
 }  // namespace
 
-size_t sim_direct_workspace_bytes(const SimPlan &p) { return layout(p, choose_tiling(p)).total; }
+size_t sim_direct_workspace_bytes(const SimPlan &p)
+{
+    const Tiling t = choose_tiling(p);
+    return layout(p, t, split_plan(p, t)).total;
+}
 
 // Writes everything of the workspace that depends on the parameters only (one launch).
 int sim_direct_prepare(const SimPlan &p, const float *templates, const float *weights, void *workspace,
                        size_t workspace_bytes, hipStream_t s)
 {
     const Tiling t = choose_tiling(p);
-    const Layout l = layout(p, t);
+    const SplitPlan split = split_plan(p, t);
+    const Layout l = layout(p, t, split);
     if (workspace_bytes < l.total)
         return SIMNETS_ERR_WORKSPACE;
     char *ws = reinterpret_cast<char *>(workspace);
@@ -1107,11 +1162,14 @@ int sim_direct_prepare(const SimPlan &p, const float *templates, const float *we
     const bool sqrtw = use_sqrtw(p, t);
     const int mode = sqrtw ? (int)SIM_MODE_L2_SQRTW : p.mode;
     const int thr_blocks = sqrtw ? std::min((p.O + 3) / 4, 1024) : 0;
-    hipLaunchKernelGGL(sim_pack_params_kernel, dim3(pack_blocks + thr_blocks), dim3(256), 0, s, templates, weights, p.O,
+    const SplitPack sp = sim_split_pack_args(p, split, templates, weights, ws + l.split);
+    const size_t lds = split.on ? (size_t)std::max(p.C, 16) * sizeof(float) : 0;
+    hipLaunchKernelGGL(sim_pack_params_kernel, dim3(sp.pack_blocks + sp.thr_blocks + pack_blocks + thr_blocks),
+                       dim3(256), lds, s, templates, weights, p.O,
                        p.K, t.MT, n_mtiles, mode, p.fudge, reinterpret_cast<float *>(ws + l.pa),
                        reinterpret_cast<float *>(ws + l.pc), reinterpret_cast<int *>(ws + l.koff), p.bh * p.bw, p.bw, t.CC,
                        t.chan_pitch, t.TC, sqrtw ? reinterpret_cast<float *>(ws + l.pa2) : nullptr,
-                       reinterpret_cast<float *>(ws + l.thr), pack_blocks);
+                       reinterpret_cast<float *>(ws + l.thr), pack_blocks, sp);
     return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
 }
 
@@ -1127,7 +1185,8 @@ static int sim_direct_run_on(const SimPlan &p, const float *input, float *output
                              const float *raw_weights)
 {
     const Tiling t = choose_tiling(p);
-    const Layout l = layout(p, t);
+    const SplitPlan split = split_plan(p, t);
+    const Layout l = layout(p, t, split);
     if (workspace_bytes < l.total)
         return SIMNETS_ERR_WORKSPACE;
     char *ws = reinterpret_cast<char *>(workspace);
@@ -1157,6 +1216,14 @@ static int sim_direct_run_on(const SimPlan &p, const float *input, float *output
     a.pa2 = reinterpret_cast<const float *>(ws + l.pa2);
     a.thr = reinterpret_cast<const float *>(ws + l.thr);
     a.flags = reinterpret_cast<int *>(ws + l.flags);
+    a.gate = nullptr;
+    a.gate_mtiles = split.n_mtiles;
+    if (split.on) {
+        const int rc = sim_split_launch(p, split, input, output, ws + l.split, s);
+        if (rc)
+            return rc;
+        a.gate = reinterpret_cast<const int *>(ws + l.split + split.flags);
+    }
     a.raw_t = raw_templates; a.raw_w = raw_weights; a.fudge = p.fudge;
 
     const bool plds = use_plds(p, t);

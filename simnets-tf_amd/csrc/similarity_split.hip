@@ -1,0 +1,411 @@
+// The L2 Similarity modes as a matrix product on the bf16 matrix cores, at the precision of fp32 (gfx950).
+//
+//   sum_k w (x - t)^2 = sum_k w x'^2 - 2 w t' x' + w t'^2,   x' = x - c, t' = t - c, c one value per channel
+// is a contraction of (w, -2 w t') with (x'^2, x').  Every factor is the exact sum of three 16-bit pieces (split3), and
+// the six products of pieces above 2^-24 of the whole are formed on v_mfma_f32_32x32x16_bf16 (dropped: below 2^-26).  A
+// 32-bit matrix instruction does two terms in 64 cycles where six of these do sixteen in 192 - 2.7 times the rate, and
+// 2.7 times the vector units' two instructions per term.
+//
+// Precision.  The leading product of the squares has accumulators of its own, so an output's sum is rounded K / 16 times
+// at its own size instead of K times in a term-by-term sum; the others, of random sign or 2^-8 of it, share a second
+// set.  Error against 64 bits (2-norm, relative): 256 x 64 x 32 x 32 -> 128, 3 x 3, 0.9e-7 where the term-by-term forms have
+// 3.6e-7; 64 x 250 x 12 x 12 -> 195 1.4e-7 against 7.0e-7.  What cancellation between the three sums costs is bounded by a guard: with T = sum w t'^2,
+// an output of at least T / 4 has sum w (|x'| + |t'|)^2 <= 25 times itself (sqrt(sum w x'^2) <= sqrt(out) + sqrt(T)).
+// A tile with an output below that (or below 1/1024 of the uncentred sum w t^2, the guard of the sqrt-weight form; or
+// not finite; or of a template whose parameters are negative, huge or tiny) is flagged and computed again, term by
+// term, by the direct kernel's launch behind this one, which otherwise returns at once.
+//
+// Missing values (NaN inputs ignored): x' = 0 and a third operand, the 0/1 mask of present values (exact in 16 bits),
+// contracts with -w t'^2 and with the logarithm term, three pieces each.
+//
+// Layout.  A workgroup of four waves computes 128 consecutive output pixels (over the batch: images are a stack of
+// padded rows, so a tile may span images and no lane idles at an image's end) x up to 128 templates.  16 channels (or
+// 8) of the rows it touches are staged in LDS as [piece][channel group of 8][pixel][8 channels], converted once and read
+// by every tap and template; a lane's matrix operand - 8 channels of its pixel - is one ds_read_b128, consecutive
+// lanes' in consecutive 16 bytes.  The parameters are packed in the order the lanes read them and come from L2 straight
+// into registers, one step ahead.  80 KB of LDS and 256 registers: two workgroups per compute unit, so that one stages
+// while the other multiplies.
+//
+// Measured (whole call, vector form before -> this form): 256 x 64 x 32 x 32 -> 128, 3 x 3: 0.80 -> 0.37 ms, 1.3 PFLOP/s of
+// matrix products, what the largest library products reach on this chip: bound by the matrix units' power.  37 x 45 x
+// 29 x 35 -> 75: 172 -> 66 us, where half of the products are padding (96 templates, 48 channels, 37632 pixels).  64
+// images of the first with a quarter missing: 427 -> 159 us.  8 x 64 x 32 x 32 -> 32: 139 -> 39 us.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+
+#include "fast_div.h"
+#include "internal.h"
+#include "sim_split.h"
+
+namespace simnets {
+
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kThreads = 256;
+// staged pixels of a chunk of 16 channels (twice as many of 8): two workgroups' tiles fit the 160 KB of a compute unit
+constexpr int split_lds_pixels(bool masked) { return masked ? 360 : 408; }
+constexpr int split_lds_bytes(bool masked) { return split_lds_pixels(masked) * 32 * (masked ? 7 : 6); }
+
+struct SplitArgs {
+    const float *in;
+    float *out;
+    const bf16x8 *packed;
+    const float *ctr, *bias, *lg, *thr;
+    int *flags;      // [pixel tile][mtile]
+    int C, H, W, O, ow, npix, total;   // npix = oh ow, total = B npix
+    int bw, sh, sw, ph, pw, taps, chunks, steps, n_mtiles, Wp, Hv;
+    int gmax;        // matrix tiles of templates per workgroup: 4, 2 or 1
+    float oob;
+    FastDiv d_npix, d_ow, d_wp, d_hv;
+};
+
+// One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
+template <bool MASKED, int CG, int G>
+__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mtile0, bool norm)
+{
+    constexpr int NI = G, NB = MASKED ? 7 : 6, NA = MASKED ? 12 : 6;
+    constexpr int P = split_lds_pixels(MASKED) * (CG == 16 ? 1 : 2);   // pixels of one plane [channel group][pixel]
+    constexpr int kPlane = split_lds_pixels(MASKED) * 32;
+    constexpr int kItems = (split_lds_pixels(MASKED) * 2 + kThreads - 1) / kThreads;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    const int mtile = mtile0 + wave % G;
+    const int ntile0 = (wave / G) * NI;
+
+    const int n0 = blockIdx.x * kSplitPixels;
+    auto virtual_row = [&](int n, int &img, int &rem, int &c) {   // of the stack of padded images; pixel n's first
+        img = (int)fast_div((unsigned)n, a.d_npix);
+        rem = n - img * a.npix;
+        const int r = (int)fast_div((unsigned)rem, a.d_ow);
+        c = rem - r * a.ow;
+        return img * a.Hv + r * a.sh;
+    };
+    int img0, rem0, c0, i1, i2, i3;
+    const int v0 = virtual_row(n0, img0, rem0, c0);
+    const int rows = virtual_row(min(n0 + kSplitPixels, a.total) - 1, i1, i2, i3) - v0 + a.taps / a.bw;
+    const int staged = min(rows * a.Wp, P);
+
+    // where this thread's staged elements come from (the same for every chunk)
+    unsigned src[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        const int e = tid + i * kThreads;
+        const int g = CG == 16 && e >= staged, q = e - (g ? staged : 0);
+        const int vr = (int)fast_div((unsigned)q, a.d_wp), c = q - vr * a.Wp - a.pw;
+        const int v = v0 + vr, img = (int)fast_div((unsigned)v, a.d_hv), r = v - img * a.Hv - a.ph;
+        const bool in = r >= 0 && r < a.H && c >= 0 && c < a.W;
+        src[i] = in ? (unsigned)(((img * a.C + 8 * g) * a.H + r) * a.W + c) : 0xffffffffu;
+    }
+    // and this lane's operands: the LDS byte address of its pixel's first tap
+    int at[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int n = min(n0 + (ntile0 + i) * 32 + col, a.total - 1);
+        int img, rem, c;
+        const int v = virtual_row(n, img, rem, c);
+        at[i] = ((CG == 16 ? half * P : 0) + (v - v0) * a.Wp + c * a.sw) * 16;
+    }
+
+    f32x16 hi[NI], lo[NI], tm[MASKED ? NI : 1], lg[MASKED ? NI : 1];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        hi[i] = 0.0f;
+        lo[i] = 0.0f;
+        if (MASKED) {
+            tm[i] = 0.0f;
+            lg[i] = 0.0f;
+        }
+    }
+    const bool active = mtile < a.n_mtiles;
+    const bf16x8 *pp = a.packed + (size_t)(active ? mtile : 0) * a.chunks * a.steps * NA * 64 + lane;
+    bf16x8 next[NA];
+#pragma unroll
+    for (int q = 0; q < NA; ++q)
+        next[q] = pp[q * 64];
+
+    const unsigned plane = (unsigned)a.H * a.W;
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            const int e = tid + i * kThreads;
+            if (e < (CG == 16 ? 2 : 1) * staged) {
+                const int g = CG == 16 && e >= staged;
+                const int q = e - (g ? staged : 0);
+                const int cbase = chunk * CG + 8 * g;
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool in = src[i] != 0xffffffffu && cbase + j < a.C;
+                    x[j] = in ? a.in[(size_t)src[i] + (size_t)(chunk * CG + j) * plane] : a.oob;
+                }
+                bf16x8 v[7];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    // channels behind the last have zero parameters: any finite value will do
+                    float d = cbase + j < a.C ? x[j] - a.ctr[cbase + j] : 0.0f;
+                    if (MASKED) {
+                        const bool ok = d == d;
+                        v[6][j] = (__bf16)(ok && cbase + j < a.C ? 1.0f : 0.0f);
+                        d = ok ? d : 0.0f;
+                    }
+                    __bf16 p0, p1, p2;
+                    split3(d * d, p0, p1, p2);
+                    v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
+                    split3(d, p0, p1, p2);
+                    v[3][j] = p0; v[4][j] = p1; v[5][j] = p2;
+                }
+                char *dst = lds + (g * P + q) * 16;
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    *reinterpret_cast<bf16x8 *>(dst + b * kPlane) = v[b];
+            }
+        }
+        __syncthreads();
+        int dh = 0, dw = 0;
+        auto next_tap = [&]() {   // LDS offset of the tap (behind the last: of the first, with zero parameters)
+            const int off = (dh * a.Wp + dw) * 16;
+            if (++dw == a.bw) {
+                dw = 0;
+                ++dh;
+            }
+            return off;
+        };
+        for (int step = 0; step < a.steps; ++step) {
+            bf16x8 A[NA];
+#pragma unroll
+            for (int q = 0; q < NA; ++q)
+                A[q] = next[q];
+            if (chunk + 1 < a.chunks || step + 1 < a.steps)
+                pp += NA * 64;
+#pragma unroll
+            for (int q = 0; q < NA; ++q)
+                next[q] = pp[q * 64];
+            int off = next_tap();
+            if (CG == 8) {
+                const int off2 = 2 * step + 1 < a.taps ? next_tap() : 0;
+                off = half ? off2 : off;
+            }
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                bf16x8 B[NB];
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    B[b] = *reinterpret_cast<const bf16x8 *>(lds + at[i] + off + b * kPlane);
+                auto mul = [](f32x16 &acc, const bf16x8 &x, const bf16x8 &y) {
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc, 0, 0, 0);
+                };
+#pragma unroll
+                for (int f = 0; f < 6; f += 3) {
+                    mul(lo[i], A[f + 2], B[f]);
+                    mul(lo[i], A[f], B[f + 2]);
+                    mul(f == 0 ? hi[i] : lo[i], A[f], B[f]);
+                    mul(lo[i], A[f + 1], B[f + 1]);
+                    mul(lo[i], A[f + 1], B[f]);
+                    mul(lo[i], A[f], B[f + 1]);
+                }
+                if (MASKED)
+#pragma unroll
+                    for (int q = 2; q >= 0; --q) {
+                        mul(tm[i], A[NA - 6 + q], B[NB - 1]);
+                        mul(lg[i], A[NA - 3 + q], B[NB - 1]);
+                    }
+            }
+        }
+    }
+
+    // lane: pixel col of each tile, templates 8 (r / 4) + 4 half + r % 4
+    bool bad = false;
+    if (active) {
+        float bias[16], lgm[16], thr[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4;
+            bias[r] = a.bias[m];
+            lgm[r] = a.lg[m];
+            thr[r] = a.thr[m];
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int n = n0 + (ntile0 + i) * 32 + col;
+            if (n >= a.total)
+                continue;
+            const int img = (int)fast_div((unsigned)n, a.d_npix);
+            float *dst = a.out + ((size_t)img * a.O + mtile * kSplitRows) * a.npix + (n - img * a.npix);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int ml = 8 * (r / 4) + 4 * half + r % 4;
+                if (mtile * kSplitRows + ml >= a.O)
+                    continue;
+                float v;
+                if (MASKED) {
+                    v = (hi[i][r] + tm[i][r]) + lo[i][r];
+                    const float mag = __builtin_fabsf(v);
+                    const bool fine = mag < 1e37f && mag >= -0.25f * tm[i][r] &&
+                                      (mag >= thr[r] || (v == 0.0f && tm[i][r] == 0.0f && thr[r] < 1e37f));
+                    bad |= !fine;
+                    v = 0.5f * v + lg[i][r];
+                } else {
+                    v = (hi[i][r] + bias[r]) + lo[i][r];
+                    const float mag = __builtin_fabsf(v);
+                    bad |= !(mag >= thr[r] && mag < 1e37f);
+                    if (norm)
+                        v = 0.5f * v + lgm[r];
+                }
+                dst[(size_t)ml * a.npix] = v;
+            }
+        }
+    }
+    // one flag per (pixel tile, template tile): the waves of a template tile share it
+    bad = __any(bad);
+    int *shared_flag = reinterpret_cast<int *>(lds);
+    __syncthreads();
+    if (tid < G)
+        shared_flag[tid] = 0;
+    __syncthreads();
+    if (bad && lane == 0)
+        shared_flag[wave % G] = 1;
+    __syncthreads();
+    if (tid < G && mtile0 + tid < a.n_mtiles)
+        a.flags[(size_t)blockIdx.x * a.n_mtiles + mtile0 + tid] = shared_flag[tid];
+}
+
+// The template tiles of a pixel tile are dealt out as groups of gmax and, of the rest, 2 and 1.
+template <bool MASKED, int CG>
+__global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs a, int norm)
+{
+    __shared__ __align__(16) char split_lds[split_lds_bytes(MASKED)];
+    const int full = a.n_mtiles / a.gmax, y = blockIdx.y;
+    int mtile0 = y * a.gmax, g = a.gmax;
+    if (y >= full) {
+        const int rest = a.n_mtiles - full * a.gmax;   // 1..3
+        mtile0 = full * a.gmax;
+        g = rest >= 2 ? 2 : 1;
+        if (y > full) {   // the last one of three
+            mtile0 += 2;
+            g = 1;
+        }
+    }
+    if (!MASKED && g == 4)
+        split_body<MASKED, CG, MASKED ? 2 : 4>(a, split_lds, mtile0, norm);
+    else if (g == 2)
+        split_body<MASKED, CG, 2>(a, split_lds, mtile0, norm);
+    else
+        split_body<MASKED, CG, 1>(a, split_lds, mtile0, norm);
+}
+
+}  // namespace
+
+SplitPlan sim_split_plan(const SimPlan &p)
+{
+    SplitPlan s = {};
+    const bool masked = p.mode == SIM_MODE_L2_NORM_IGNORE_NAN;
+    if (!p.split || p.mode == SIM_MODE_L1 || (p.mode == SIM_MODE_L2_NORM && p.norm_const_every_iteration) || p.B == 0)
+        return s;
+    const int taps = p.bh * p.bw;
+    const long long total = 1LL * p.B * p.oh * p.ow;
+    // few elements per patch: outputs below the guard's line are ordinary there
+    if (p.K < 64 || p.C > kSplitMaxC || 1LL * p.B * p.C * p.H * p.W >= (1LL << 31) || total >= (1LL << 30) ||
+        1LL * p.B * ((p.oh - 1) * p.sh + p.bh) >= (1LL << 30))
+        return s;
+    s.Wp = (p.ow - 1) * p.sw + p.bw;
+    s.Hv = (p.oh - 1) * p.sh + p.bh;
+    // the most rows of the stack that 128 consecutive pixels touch
+    int g = p.ow, h = kSplitPixels;
+    while (h) {
+        const int r = g % h;
+        g = h;
+        h = r;
+    }
+    const int out_rows = (p.ow - g + kSplitPixels - 1) / p.ow + 1;
+    const int crossings = 1LL * p.oh * p.ow % kSplitPixels == 0 ? 0 : (out_rows - 1 + p.oh - 1) / p.oh;
+    const long long staged = 1LL * ((out_rows - 1) * p.sh + p.bh + crossings * std::max(0, p.bh - p.sh)) * s.Wp;
+    const int room = split_lds_pixels(masked);
+    const int c16 = (p.C + 15) / 16 * taps, c8 = (p.C + 7) / 8 * ((taps + 1) / 2);   // matrix steps
+    if (staged > 2 * room)
+        return s;
+    s.cg = staged > room || (c8 < c16 && 8 * c8 < 7 * c16) ? 8 : 16;
+    s.chunks = (p.C + s.cg - 1) / s.cg;
+    s.steps = s.cg == 16 ? taps : (taps + 1) / 2;
+    s.pieces = masked ? 12 : 6;
+    s.n_mtiles = (p.O + kSplitRows - 1) / kSplitRows;
+    s.n_ptiles = (int)((total + kSplitPixels - 1) / kSplitPixels);
+    const double useful = 1.0 * total * p.O * p.K;
+    const double padded = 1.0 * s.n_ptiles * kSplitPixels * s.n_mtiles * kSplitRows * s.chunks * s.steps * 16;
+    // few of the products useful (64 x 17 x 28 x 28 -> 33, 0.33 of them: still 48 -> 35 us; 32 x 3 x 64 x 64 -> 64, 5 x 5, 0.36
+    // in a single chunk: 50 -> 53), or a handful of workgroups: no gain over the vector forms
+    if (useful < (s.chunks > 1 ? 0.3 : 0.4) * padded || 1LL * s.n_ptiles * s.n_mtiles < 32)
+        return s;
+    const int mpad = s.n_mtiles * kSplitRows;
+    s.packed = 0;
+    s.ctr = s.packed + (size_t)s.n_mtiles * s.chunks * s.steps * s.pieces * 1024;
+    s.bias = s.ctr + align_up((size_t)s.chunks * s.cg * sizeof(float), 256);
+    s.lg = s.bias + align_up((size_t)mpad * sizeof(float), 256);
+    s.thr = s.lg + align_up((size_t)mpad * sizeof(float), 256);
+    s.flags = s.thr + align_up((size_t)mpad * sizeof(float), 256);
+    s.total = s.flags + align_up((size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
+    s.on = true;
+    return s;
+}
+
+SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float *templates, const float *weights,
+                              char *ws)
+{
+    SplitPack a;
+    a.templates = templates; a.weights = weights;
+    a.packed = reinterpret_cast<unsigned short *>(ws + sp.packed);
+    a.ctr = reinterpret_cast<float *>(ws + sp.ctr);
+    a.bias = reinterpret_cast<float *>(ws + sp.bias);
+    a.lg = reinterpret_cast<float *>(ws + sp.lg);
+    a.thr = reinterpret_cast<float *>(ws + sp.thr);
+    a.O = p.O; a.C = p.C; a.taps = p.bh * p.bw; a.K = p.K; a.cg = sp.cg; a.chunks = sp.chunks; a.steps = sp.steps;
+    a.pieces = sp.pieces; a.n_mtiles = sp.n_mtiles; a.mode = p.mode; a.fudge = p.fudge;
+    a.norm_const = p.mode == SIM_MODE_L2_NORM ? (float)((double)(-0.5f * (float)p.K) * std::log(2.0 * M_PI)) : 0.0f;
+    a.pack_blocks = sp.on ? sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4) : 0;
+    a.thr_blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows / 4, 256) : 0;
+    return a;
+}
+
+int sim_split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, float *output, char *ws, hipStream_t s)
+{
+    const bool masked = p.mode == SIM_MODE_L2_NORM_IGNORE_NAN;
+    SplitArgs a;
+    a.in = input; a.out = output;
+    a.packed = reinterpret_cast<const bf16x8 *>(ws + sp.packed);
+    a.ctr = reinterpret_cast<const float *>(ws + sp.ctr);
+    a.bias = reinterpret_cast<const float *>(ws + sp.bias);
+    a.lg = reinterpret_cast<const float *>(ws + sp.lg);
+    a.thr = reinterpret_cast<const float *>(ws + sp.thr);
+    a.flags = reinterpret_cast<int *>(ws + sp.flags);
+    a.C = p.C; a.H = p.H; a.W = p.W; a.O = p.O; a.ow = p.ow; a.npix = p.oh * p.ow; a.total = p.B * a.npix;
+    a.bw = p.bw; a.sh = p.sh; a.sw = p.sw; a.ph = p.ph; a.pw = p.pw; a.taps = p.bh * p.bw;
+    a.chunks = sp.chunks; a.steps = sp.steps; a.n_mtiles = sp.n_mtiles; a.Wp = sp.Wp; a.Hv = sp.Hv;
+    a.oob = p.oob;
+    a.d_npix = make_fast_div((unsigned)a.npix);
+    a.d_ow = make_fast_div((unsigned)p.ow);
+    a.d_wp = make_fast_div((unsigned)sp.Wp);
+    a.d_hv = make_fast_div((unsigned)sp.Hv);
+    // as many template tiles per staged pixel tile as leave two workgroups for every compute unit
+    a.gmax = masked ? 2 : 4;
+    while (a.gmax > 1 && (a.gmax / 2 >= sp.n_mtiles || (long long)sp.n_ptiles * ((sp.n_mtiles + a.gmax - 1) / a.gmax) < 256))
+        a.gmax /= 2;
+    const int rest = sp.n_mtiles % a.gmax;
+    const dim3 grid((unsigned)sp.n_ptiles, (unsigned)(sp.n_mtiles / a.gmax + (rest == 0 ? 0 : rest == 3 ? 2 : 1)));
+    const int norm = p.mode == SIM_MODE_L2_NORM;
+    if (masked && sp.cg == 16)
+        hipLaunchKernelGGL((sim_split_kernel<true, 16>), grid, dim3(kThreads), 0, s, a, norm);
+    else if (masked)
+        hipLaunchKernelGGL((sim_split_kernel<true, 8>), grid, dim3(kThreads), 0, s, a, norm);
+    else if (sp.cg == 16)
+        hipLaunchKernelGGL((sim_split_kernel<false, 16>), grid, dim3(kThreads), 0, s, a, norm);
+    else
+        hipLaunchKernelGGL((sim_split_kernel<false, 8>), grid, dim3(kThreads), 0, s, a, norm);
+    return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
+}
+
+}  // namespace simnets

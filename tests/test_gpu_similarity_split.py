@@ -1,0 +1,133 @@
+"""The L2 Similarity modes on the matrix cores in 16-bit pieces (csrc/similarity_split.hip): edges of its tiles, its three
+modes, both chunk sizes, and what its guard hands to the term-by-term kernel.  Reference: torch in 64 bits."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def exact(x, t, w, blocks, strides, padding, mode, oob=0.0, fudge=0.001):
+    x, t, w = x.double(), t.double(), w.double()
+    x = torch.nn.functional.pad(x, (padding[1],) * 2 + (padding[0],) * 2, value=oob)
+    cols = x.unfold(2, blocks[0], strides[0]).unfold(3, blocks[1], strides[1]).permute(0, 1, 4, 5, 2, 3)
+    B, _, _, _, oh, ow = cols.shape
+    cols = cols.reshape(B, -1, oh * ow)
+    t, w = t.reshape(t.shape[0], -1), w.reshape(w.shape[0], -1)
+    out = torch.empty(B, t.shape[0], oh * ow, dtype=torch.float64, device=x.device)
+    for m in range(t.shape[0]):
+        term = -w[m, :, None] * (cols - t[m, :, None]) ** 2
+        if mode != "l2":
+            term = 0.5 * (term + torch.log(w[m] + fudge)[:, None] - math.log(2 * math.pi))
+        if mode == "missing":
+            term = torch.where(cols == cols, term, torch.zeros_like(term))
+        out[:, m] = term.sum(1)
+    return out.reshape(B, -1, oh, ow)
+
+
+def options(mode, g):
+    kw = dict(blocks=g["blocks"], strides=g["strides"], padding=g["padding"])
+    if mode != "l2":
+        kw["normalization_term"] = True
+    if mode == "missing":
+        kw.update(ignore_nan_input=True, out_of_bounds_value=float("nan"))
+    return kw
+
+
+GEOMS = [
+    dict(shape=(5, 16, 40, 40), O=128, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),   # whole tiles, four template tiles
+    dict(shape=(9, 13, 33, 31), O=75, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),    # ragged everywhere, 2 + 1 tiles
+    dict(shape=(7, 45, 29, 35), O=33, blocks=[3, 3], strides=[1, 1], padding=[0, 2]),    # one template in the second tile
+    dict(shape=(40, 40, 12, 11), O=225, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),  # tiles span images, 4 + 4 tiles
+    dict(shape=(37, 32, 7, 7), O=160, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),    # several images to a tile
+    dict(shape=(3, 20, 61, 67), O=34, blocks=[5, 5], strides=[1, 1], padding=[2, 2]),    # wide rows: chunks of 8 channels
+    dict(shape=(9, 24, 62, 65), O=76, blocks=[3, 3], strides=[2, 2], padding=[1, 1]),    # stride 2
+    dict(shape=(6, 100, 45, 20), O=40, blocks=[1, 1], strides=[1, 1], padding=[0, 0]),   # one tap
+    dict(shape=(90, 16, 9, 9), O=32, blocks=[2, 3], strides=[3, 2], padding=[0, 0]),     # strides beyond the block
+    dict(shape=(12, 66, 33, 34), O=31, blocks=[1, 3], strides=[1, 1], padding=[0, 1], out_of_bounds_value=0.5),
+]
+
+
+@pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
+@pytest.mark.parametrize("geom", GEOMS)
+def test_split_form_matches_64_bits(pkg, geom, mode):
+    g = torch.Generator(device="cuda").manual_seed(17)
+    shape, O, blocks = geom["shape"], geom["O"], geom["blocks"]
+    x = torch.randn(shape, generator=g, device="cuda")
+    t = torch.randn((O, shape[1], *blocks), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    kw = options(mode, geom)
+    oob = kw.get("out_of_bounds_value", geom.get("out_of_bounds_value", 0.0))
+    kw["out_of_bounds_value"] = oob
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    got = pkg.similarity(x, t, w, **kw)
+    want = exact(x, t, w, blocks, geom["strides"], geom["padding"], mode, oob)
+    # an output is rounded K / 16 + 4 times at no more than its own size and once more as a sum of three of comparable
+    # size; the logarithms of the normalized modes are summed at about the same size again
+    K = shape[1] * blocks[0] * blocks[1]
+    size = want.abs().clamp_min(float(want.abs().mean()))
+    err = (got.double() - want).abs() / size
+    assert float(err.max()) <= 2 * (K / 16 + 8) * 2.0 ** -24, float(err.max())
+    call = pkg.similarity_prepare(shape, t, w, **kw)
+    assert torch.equal(call(x), got)
+
+
+@pytest.mark.parametrize("kind", ["equal", "offset", "negative", "tiny", "huge", "inf", "nan"])
+@pytest.mark.parametrize("geom", [GEOMS[1], GEOMS[3], GEOMS[4], GEOMS[5]])
+def test_split_form_leaves_what_it_cannot_do_to_the_direct_kernel(pkg, geom, kind):
+    g = torch.Generator(device="cuda").manual_seed(23)
+    shape, O, blocks = geom["shape"], geom["O"], geom["blocks"]
+    kw = options("l2", geom)
+    x = torch.randn(shape, generator=g, device="cuda")
+    t = torch.randn((O, shape[1], *blocks), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    ph, pw = geom["padding"]
+    xp = torch.nn.functional.pad(x, (pw, pw, ph, ph))
+    if kind == "equal":      # templates cut out of the input: outputs of zero, and nearly zero
+        for m in range(0, O, 5):
+            t[m] = xp[m % shape[0], :, m % 5:m % 5 + blocks[0], m % 7:m % 7 + blocks[1]]
+        t[1::10] += 1e-4
+    elif kind == "offset":
+        x += 1000.0
+        t += 1000.0
+        kw["out_of_bounds_value"] = 1000.0
+    elif kind == "negative":
+        w[1::4] *= -1.0
+    elif kind == "tiny":
+        w[2] = 1e-30
+        w[3] = 0.0
+    elif kind == "huge":
+        w[2] = 1e30
+        t[3] = 1e25
+    elif kind == "inf":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.001] = float("inf")
+    elif kind == "nan":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.001] = float("nan")
+    got = pkg.similarity(x, t, w, **kw).cpu().numpy()
+    direct = pkg.similarity(x, t, w, algo="direct", **kw).cpu().numpy()
+    assert np.array_equal(np.isfinite(got), np.isfinite(direct))
+    assert np.array_equal(np.isnan(got), np.isnan(direct))
+    fin = np.isfinite(direct)
+    # K roundings of the term-by-term sum on one side, 25 K / 16 at the guard's line on the other, and what is below it
+    # is the term-by-term sum itself
+    K = shape[1] * blocks[0] * blocks[1]
+    with np.errstate(invalid="ignore", divide="ignore"):
+        err = np.abs(got - direct)[fin] / np.maximum(np.abs(direct[fin]), 1e-37)
+    assert err.max() <= 3 * K * 2.0 ** -24, err.max()
+    if kind == "equal":
+        assert (direct == 0).any() and np.array_equal(got[direct == 0], direct[direct == 0])
+    if kind == "offset":
+        assert np.array_equal(got, direct)
+    if kind == "negative":
+        assert np.array_equal(got[:, 1::4], direct[:, 1::4])
+
+
+def test_split_form_with_everything_missing(pkg):
+    geom = GEOMS[1]
+    x = torch.full(geom["shape"], float("nan"), device="cuda")
+    t = torch.randn((geom["O"], geom["shape"][1], 3, 3), device="cuda")
+    got = pkg.similarity(x, t, t.abs() + 0.1, **options("missing", geom))
+    assert torch.equal(got, torch.zeros_like(got)) and not torch.signbit(got).any()
