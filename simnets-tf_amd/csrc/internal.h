@@ -70,6 +70,11 @@ size_t sim_mfma_grad_input_workspace_bytes(const SimPlan &p);
 int sim_mfma_grad_input_launch(const SimPlan &p, const float *input, const float *templates, const float *weights,
                                const float *output_grad, float *input_grad, void *workspace, size_t workspace_bytes,
                                void *stream);
+// ... in 16-bit pieces (similarity_split.hip); 0 bytes: not on this geometry
+size_t sim_split_grad_input_workspace_bytes(const SimPlan &p);
+int sim_split_grad_input_launch(const SimPlan &p, const float *input, const float *templates, const float *weights,
+                                const float *output_grad, float *input_grad, void *workspace, size_t workspace_bytes,
+                                void *stream);
 size_t sim_grad_input_workspace_bytes(const SimPlan &p);
 size_t sim_grad_params_workspace_bytes(const SimPlan &p);
 int sim_grad_input(const SimPlan &p, const float *input, const float *templates, const float *weights,

@@ -611,6 +611,8 @@ static bool gx_gather(const SimPlan &p) { return !gx_all_phases_fit(p) || p.C <=
 
 size_t sim_grad_input_workspace_bytes(const SimPlan &p)
 {
+    if (const size_t split = sim_split_grad_input_workspace_bytes(p))
+        return split;
     if (sim_mfma_grad_input_supported(p))
         return sim_mfma_grad_input_workspace_bytes(p);
     if (gx_gather(p))
@@ -636,6 +638,9 @@ int sim_grad_input(const SimPlan &p, const float *input, const float *templates,
     const int ignore_nan = p.mode == SIM_MODE_L2_NORM_IGNORE_NAN;
     const long long n_in = (long long)p.B * p.C * p.H * p.W;
 
+    if (sim_split_grad_input_workspace_bytes(p))
+        return sim_split_grad_input_launch(p, input, templates, weights, output_grad, input_grad, workspace,
+                                           workspace_bytes, stream);
     if (sim_mfma_grad_input_supported(p))
         return sim_mfma_grad_input_launch(p, input, templates, weights, output_grad, input_grad, workspace,
                                           workspace_bytes, stream);

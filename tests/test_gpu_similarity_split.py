@@ -131,3 +131,52 @@ def test_split_form_with_everything_missing(pkg):
     t = torch.randn((geom["O"], geom["shape"][1], 3, 3), device="cuda")
     got = pkg.similarity(x, t, t.abs() + 0.1, **options("missing", geom))
     assert torch.equal(got, torch.zeros_like(got)) and not torch.signbit(got).any()
+
+
+@pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
+@pytest.mark.parametrize("geom", GEOMS)
+def test_split_gradients_match_64_bits(pkg, geom, mode):
+    g = torch.Generator(device="cuda").manual_seed(29)
+    shape, O, blocks = geom["shape"], geom["O"], geom["blocks"]
+    x = torch.randn(shape, generator=g, device="cuda") + 0.5
+    t = torch.randn((O, shape[1], *blocks), generator=g, device="cuda") + 0.5
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    kw = options(mode, geom)
+    kw.setdefault("out_of_bounds_value", geom.get("out_of_bounds_value", 0.0))
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    (ph, pw), (sh, sw) = geom["padding"], geom["strides"]
+    # -w (x - t)^2 (halved, with 0.5 log(w + 0.001), in the normalized modes) as three convolutions in 64 bits
+    leaves = [v.double().cpu().requires_grad_() for v in (x, t, w)]
+    xd, td, wd = leaves
+    xp = torch.nn.functional.pad(xd, (pw, pw, ph, ph), value=kw["out_of_bounds_value"])
+    keep = (xp == xp).double()
+    xz = torch.where(xp == xp, xp, torch.zeros_like(xp))
+    conv = lambda a, b: torch.nn.functional.conv2d(a, b, stride=(sh, sw))
+    out = -(conv(xz * xz, wd) - 2 * conv(xz, wd * td) + conv(keep, wd * td * td))
+    if mode != "l2":
+        out = 0.5 * (out + conv(keep, torch.log(wd + 0.001)))
+    go = torch.randn(out.shape, generator=g, device="cuda")
+    want = torch.autograd.grad(out, leaves, go.double().cpu())
+    dx = pkg.similarity_input_grad(x, t, w, go, **kw)
+    # n terms of random sign: their sum's error is 2^-24 of the root of the sum of their squares, some n / 3 times added
+    # at random, and the moments' combination cancels a few of the size of the terms: 4 sqrt(n) 2^-24 of the scale
+    for got, ref, n in ((dx, want[0], O * blocks[0] * blocks[1]),):
+        err = (got.double().cpu() - ref).norm() / ref.norm()
+        assert float(err) <= 4 * math.sqrt(n) * 2.0 ** -24, float(err)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_split_gradients_with_infinite_values(pkg, value):
+    """What is not finite reaches the gradients that read it and no others."""
+    geom = GEOMS[1]
+    g = torch.Generator(device="cuda").manual_seed(31)
+    shape, O = geom["shape"], geom["O"]
+    x, t = torch.randn(shape, generator=g, device="cuda"), torch.randn((O, shape[1], 3, 3), generator=g, device="cuda")
+    kw = options("l2", geom)
+    go = torch.randn((shape[0], O, shape[2], shape[3]), generator=g, device="cuda")
+    go[3, 7, 11, 30] = value
+    dx = pkg.similarity_input_grad(x, t, t.abs() + 0.1, go, **kw)
+    bad = torch.zeros_like(dx, dtype=torch.bool)
+    bad[3, :, 10:13, 29:31] = True
+    assert torch.equal(~torch.isfinite(dx), bad)
