@@ -16,7 +16,8 @@ NATIVE = os.path.join(HERE, "_simnets_native.so")
 BENCH = os.path.join(HERE, "simnets_bench")
 OBJDIR = os.path.join(HERE, "build")
 
-SOURCES = ["host_logic.cpp", "capi.hip", "similarity_direct.hip", "similarity_split.hip", "similarity_mfma.hip", "mex.hip",
+SOURCES = ["host_logic.cpp", "capi.hip", "similarity_direct.hip", "similarity_split.hip",
+           "similarity_split_params.hip", "similarity_mfma.hip", "mex.hip",
            "similarity_grad.hip", "mex_grad.hip", "mex_pool.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

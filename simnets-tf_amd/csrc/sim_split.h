@@ -42,6 +42,17 @@ int sim_split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, 
 SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float *templates, const float *weights,
                               char *ws);
 
+// Parameter gradients (similarity_split_params.hip).
+struct SplitParamsPlan {
+    bool on;
+    int n_mtiles, m_groups, k_groups, TH, TW, rows, cols, pitch, chan, tiles_r, tiles_c, units, S, Opad, Kpad;
+    size_t partial, centres, ctr, packed, total;
+};
+
+SplitParamsPlan sim_split_params_plan(const SimPlan &p);
+int sim_split_params_launch(const SimPlan &p, const SplitParamsPlan &sp, const float *input, const float *templates,
+                            const float *output_grad, char *ws, hipStream_t s);
+
 // v = p0 + p1 + p2, each the nearest 16-bit value to what is left: 24 bits of mantissa, exact for every v whose pieces
 // are normal numbers.
 __device__ __forceinline__ void split3(float v, __bf16 &p0, __bf16 &p1, __bf16 &p2)

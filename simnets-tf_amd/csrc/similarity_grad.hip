@@ -30,6 +30,7 @@
 #include <cmath>
 
 #include "internal.h"
+#include "sim_split.h"
 #include "stage.h"
 #include "valu_tile.h"
 
@@ -1679,10 +1680,34 @@ hipError_t gp_launch(const GradPArgs &a, const GpTiling &t, hipStream_t s)
 
 }  // namespace
 
+// the matrix-core form in 16-bit pieces, unless the kernel for few templates over short patches takes the call
+static SplitParamsPlan split_params_plan(const SimPlan &p)
+{
+    return gp_tiling(p).small ? SplitParamsPlan() : sim_split_params_plan(p);
+}
+
 size_t sim_grad_params_workspace_bytes(const SimPlan &p)
 {
+    const SplitParamsPlan sp = split_params_plan(p);
+    if (sp.on)
+        return sp.total;
     const GpTiling t = gp_tiling(p);
     return align_up(((size_t)t.nacc * t.S + (t.moment ? 1 : 0)) * t.Opad * t.Kpad * sizeof(float), 256);
+}
+
+static int gp_finish(const SimPlan &p, const GpTiling &t, const float *templates, const float *weights,
+                     float *templates_grad, float *weights_grad, const void *workspace, hipStream_t s)
+{
+    const long long total = (long long)p.O * p.K;
+    if (total == 0)
+        return SIMNETS_OK;
+    const int E = total <= 4096 ? 8 : 32;  // few elements: more threads per element
+    if ((total + E - 1) / E > 0x7fffffffLL)
+        return SIMNETS_ERR_TOO_LARGE;
+    const unsigned blocks = (unsigned)((total + E - 1) / E);
+    hipLaunchKernelGGL(sim_grad_params_finish_kernel, dim3(blocks), dim3(256), 0, s, reinterpret_cast<const float *>(workspace), templates, weights,
+                       p.O, p.K, t.Opad, t.Kpad, t.S, p.mode, t.moment ? 1 : 0, p.fudge, E, templates_grad, weights_grad);
+    return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
 }
 
 int sim_grad_params(const SimPlan &p, const float *input, const float *templates, const float *weights,
@@ -1692,7 +1717,15 @@ int sim_grad_params(const SimPlan &p, const float *input, const float *templates
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (workspace_bytes < sim_grad_params_workspace_bytes(p))
         return SIMNETS_ERR_WORKSPACE;
-    const GpTiling t = gp_tiling(p);
+    GpTiling t = gp_tiling(p);
+    const SplitParamsPlan sp = split_params_plan(p);
+    if (sp.on) {
+        const int rc = sim_split_params_launch(p, sp, input, templates, output_grad, reinterpret_cast<char *>(workspace), s);
+        if (rc)
+            return rc;
+        t.S = sp.S; t.Opad = sp.Opad; t.Kpad = sp.Kpad;
+        return gp_finish(p, t, templates, weights, templates_grad, weights_grad, workspace, s);
+    }
     if (p.bh > 0xffff || p.bw > 0xffff || (!t.small && gp_blocks(t) > 0x7fffffffLL))
         return SIMNETS_ERR_TOO_LARGE;
     GradPArgs a;
@@ -1713,16 +1746,7 @@ int sim_grad_params(const SimPlan &p, const float *input, const float *templates
     }
     if (e != hipSuccess)
         return SIMNETS_ERR_HIP;
-    const long long total = (long long)p.O * p.K;
-    if (total == 0)
-        return SIMNETS_OK;
-    const int E = total <= 4096 ? 8 : 32;  // few elements: more threads per element
-    if ((total + E - 1) / E > 0x7fffffffLL)
-        return SIMNETS_ERR_TOO_LARGE;
-    const unsigned blocks = (unsigned)((total + E - 1) / E);
-    hipLaunchKernelGGL(sim_grad_params_finish_kernel, dim3(blocks), dim3(256), 0, s, a.partial, templates, weights,
-                       p.O, p.K, t.Opad, t.Kpad, t.S, p.mode, t.moment ? 1 : 0, p.fudge, E, templates_grad, weights_grad);
-    return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
+    return gp_finish(p, t, templates, weights, templates_grad, weights_grad, workspace, s);
 }
 
 }  // namespace simnets

@@ -159,9 +159,11 @@ def test_split_gradients_match_64_bits(pkg, geom, mode):
     go = torch.randn(out.shape, generator=g, device="cuda")
     want = torch.autograd.grad(out, leaves, go.double().cpu())
     dx = pkg.similarity_input_grad(x, t, w, go, **kw)
+    dt, dw = pkg.similarity_parameters_grad(x, t, w, go, **kw)
     # n terms of random sign: their sum's error is 2^-24 of the root of the sum of their squares, some n / 3 times added
     # at random, and the moments' combination cancels a few of the size of the terms: 4 sqrt(n) 2^-24 of the scale
-    for got, ref, n in ((dx, want[0], O * blocks[0] * blocks[1]),):
+    for got, ref, n in ((dx, want[0], O * blocks[0] * blocks[1]), (dt, want[1], go.numel() // O),
+                        (dw, want[2], go.numel() // O)):
         err = (got.double().cpu() - ref).norm() / ref.norm()
         assert float(err) <= 4 * math.sqrt(n) * 2.0 ** -24, float(err)
 
@@ -180,3 +182,15 @@ def test_split_gradients_with_infinite_values(pkg, value):
     bad = torch.zeros_like(dx, dtype=torch.bool)
     bad[3, :, 10:13, 29:31] = True
     assert torch.equal(~torch.isfinite(dx), bad)
+    dt, dw = pkg.similarity_parameters_grad(x, t, t.abs() + 0.1, go, **kw)
+    for d in (dt, dw):
+        rows = ~torch.isfinite(d.flatten(1))
+        assert rows[7].any() and not rows[:7].any() and not rows[8:].any()
+    go[3, 7, 11, 30] = 0.0
+    x[8, 5, 32, 30] = value      # the last image's last corner: taps 0 and 1 of either axis read it
+    dt, dw = pkg.similarity_parameters_grad(x, t, t.abs() + 0.1, go, **kw)
+    for d in (dt, dw):
+        bad = ~torch.isfinite(d)
+        assert bad[:, 5, 1:, 1:].all()
+        bad[:, 5, 1:, 1:] = False
+        assert not bad.any()
