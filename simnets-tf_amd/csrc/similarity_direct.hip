@@ -69,6 +69,7 @@ struct SimKernelArgs {
     int NI, img_lds;   // small-map kernel: images per workgroup and LDS floats of one image's tile (one channel)
     FastDiv d_chan, d_img, d_tc;   // ... divisions of its staging loop: by NI * img_lds, img_lds, TC
     int plds_off;      // PLDS variants: where the workgroup's parameter copy starts in LDS (floats, multiple of 4)
+    int ksplit;        // tiled kernel: the waves of a workgroup share a template tile and split every chunk's channels
     int xcd_group;     // tiled kernel: number the workgroups so that the template groups of one pixel tile share an XCD
     // sqrt-weight form only (see the guard in sim_direct_kernel)
     const float *pa2;  // [mtile][K][MT][2]  (template, negative weight): what the recomputing pass reads
@@ -110,8 +111,8 @@ __device__ __forceinline__ LanePos lane_pos(const SimKernelArgs &a, int wave, in
     q.b = q.bx / a.tiles;
     q.tile = q.bx - q.b * a.tiles;
     q.ws = wave & (a.nws - 1);                   // which 64 pixel groups of the tile
-    const int wm = wave >> a.nws_log2;           // which MT templates
-    const int nwm = kWaves >> a.nws_log2;
+    const int wm = a.ksplit ? 0 : wave >> a.nws_log2;   // which MT templates
+    const int nwm = a.ksplit ? 1 : kWaves >> a.nws_log2;
     q.mtile = q.by * nwm + wm;
     q.wave_active = q.mtile < a.n_mtiles;
     q.g_first = q.tile * 64 * a.nws;
@@ -176,7 +177,7 @@ constexpr int lds_budget_floats(int pt, int mt) { return pt * mt <= 64 ? kLdsBud
 //        through a table of offsets: a third of the LDS instructions, no per-k address arithmetic.
 // The kernel's body.  wave_bail: sqrt-weight form - out: this wave's guard flag; GATED - in: the flag that selects the
 // waves to recompute.
-template <int MODE, int PT, int MT, int SWT, bool GATED, bool PLDS, bool ROW3>
+template <int MODE, int PT, int MT, int SWT, bool GATED, bool PLDS, bool ROW3, bool KS = false>
 __device__ __forceinline__ void sim_direct_body(const SimKernelArgs &a, float *lds, int &wave_bail)
 {
     const int tid = threadIdx.x;
@@ -285,17 +286,32 @@ __device__ __forceinline__ void sim_direct_body(const SimKernelArgs &a, float *l
         __syncthreads();
         if (PLDS && ch0 == 0)
             fetch_params(pa0, pc0);  // the parameter copy is in place behind the same barrier
+        // KS: this wave's quarter of the chunk's channels
+        int c_lo = 0, c_n = ccn;
+        if (KS) {
+            const int cpw = (ccn + kWaves - 1) / kWaves;
+            c_lo = min(wave * cpw, ccn);
+            c_n = min(c_lo + cpw, ccn) - c_lo;
+            if (c_n == 0)
+                continue;
+            const int k_first = (ch0 + c_lo) * a.bh * a.bw;
+            pa_off = zero_v + k_first * 2 * MT * (unsigned)sizeof(float);
+            pc_off = zero_v + k_first * MT * (unsigned)sizeof(float);
+            fetch_params(pa0, pc0);
+            kt = (const int SIMNETS_CONST_AS *)(a.koff) + k_first;
+        }
         if (PT % 2 == 0 && (MODE == SIM_MODE_L2_SQRTW || MODE == SIM_MODE_L2))
             sim_pin_pairs<PT, MT>(acc);
         if (ROW3 && wave_active) {
             // ---- rows (channel, dh) of the chunk in k order; per row: the next row's values and, per tap, the
             //      next tap's parameters are requested before the arithmetic on the current ones ----
-            const int nrow = ccn * 3;
+            const int nrow = c_n * 3;
+            const int lds_row = lds_base + c_lo * chan_lds;
             int roff = a.TC, rdh = 1;   // LDS offset and dh of the row to request next (row 1 at first)
             float xa[PT + 2], xb[PT + 2];
 #pragma unroll
             for (int j = 0; j < PT + 2; ++j)
-                xa[j] = lds[lds_base + j];
+                xa[j] = lds[lds_row + j];
             auto tap = [&](const float *xr, const float (&pac)[2 * MT], const float (&pcc)[MT], float (&panx)[2 * MT],
                            float (&pcnx)[MT]) {
                 fetch_params(panx, pcnx);  // one k of slack exists behind the arrays
@@ -315,7 +331,7 @@ __device__ __forceinline__ void sim_direct_body(const SimKernelArgs &a, float *l
                 const int off = r + 1 < nrow ? roff : 0;  // behind the chunk's last row: any valid address
 #pragma unroll
                 for (int j = 0; j < PT + 2; ++j)
-                    nxt[j] = lds[lds_base + off + j];
+                    nxt[j] = lds[lds_row + off + j];
                 rdh += 1;
                 roff += a.TC;
                 if (rdh == 3) {
@@ -349,7 +365,7 @@ __device__ __forceinline__ void sim_direct_body(const SimKernelArgs &a, float *l
             // ---- accumulate over the k of these channels, in k order.  Software pipeline: the pixel
             //      values and the parameters of step k+1 are requested before the arithmetic of step k,
             //      ping-ponging between two register sets (no copies) ----
-            const int nk = ccn * a.bh * a.bw;
+            const int nk = c_n * a.bh * a.bw;
             int off_next = kt[1];  // offset of step k+1 (the entries behind the last k are 0)
             auto step = [&](const float (&xc)[PT], const float (&pac)[2 * MT], const float (&pcc)[MT], float (&xnx)[PT],
                             float (&panx)[2 * MT], float (&pcnx)[MT]) {
@@ -412,6 +428,25 @@ __device__ __forceinline__ void sim_direct_body(const SimKernelArgs &a, float *l
         }
     }
 
+    if (KS) {
+        // the waves' sums, (0 + 2) + (1 + 3)
+        float *red = lds + lane;
+#pragma unroll
+        for (int have = 2; have > 0; have >>= 1) {
+            __syncthreads();
+            if (wave >= have && wave < 2 * have)
+#pragma unroll
+                for (int i = 0; i < PT * MT; ++i)
+                    red[((wave - have) * PT * MT + i) * 64] = acc[i / PT][i % PT];
+            __syncthreads();
+            if (wave < have)
+#pragma unroll
+                for (int i = 0; i < PT * MT; ++i)
+                    acc[i / PT][i % PT] += red[(wave * PT * MT + i) * 64];
+        }
+        if (wave != 0)
+            return;
+    }
     if (!wave_active || !lane_valid)
         return;
     // ---- epilogue ----
@@ -469,7 +504,7 @@ __device__ __noinline__ void sim_direct_recompute(lds_float *lds, int wave_bail)
 }
 #endif
 
-template <int MODE, int PT, int MT, int SWT, bool PLDS = false, bool ROW3 = false>
+template <int MODE, int PT, int MT, int SWT, bool PLDS = false, bool ROW3 = false, bool KS = false>
 __global__ __launch_bounds__(kThreads, waves_per_simd(PT, MT)) void sim_direct_kernel(const SimKernelArgs a)
 {
     extern __shared__ float lds[];
@@ -481,7 +516,7 @@ __global__ __launch_bounds__(kThreads, waves_per_simd(PT, MT)) void sim_direct_k
                            min(a.O, (lp.by + 1) * nm) - 1))
             return;
     }
-    sim_direct_body<MODE, PT, MT, SWT, false, PLDS, ROW3>(a, lds, wave_bail);
+    sim_direct_body<MODE, PT, MT, SWT, false, PLDS, ROW3, KS>(a, lds, wave_bail);
     if constexpr (MODE == SIM_MODE_L2_SQRTW) {
         if (__syncthreads_or(wave_bail)) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -902,6 +937,7 @@ struct Tiling {
     int PT, MT, nws, G, gpi, tiles, TC, TRmax, CC;
     int NI;            // > 0: the small-map kernel with NI images per workgroup (CC, chan_pitch are then that kernel's)
     int sm_waves;      // ... and its waves per workgroup
+    bool ksplit;       // tiled kernel: the workgroup's waves split the channels instead of the templates
     int chan_pitch;    // LDS floats of one staged channel
     bool lds_ok;       // the tiled kernels run: the rows of a workgroup's pixel groups fit the LDS tile and the
                        // patches are not too short to be worth staging (else: gather kernel)
@@ -931,6 +967,7 @@ Tiling try_tiling(const SimPlan &p, int PT, int MT, int nws)
         t.CC = (p.C + chunks - 1) / chunks;
     }
     t.NI = 0;
+    t.ksplit = false;
     t.chan_pitch = t.TRmax * t.TC;
     return t;
 }
@@ -972,6 +1009,24 @@ Tiling choose_tiling(const SimPlan &p)
             return big;
     }
     Tiling t = pick(kSmallPT, kSmallMT);
+    // L1 on narrow images or few workgroups: the wide lane tile after all, its four waves a quarter of the channels each,
+    // their sums added through LDS.  A narrow tile's step issues one instruction per 4.5 cycles and SIMD (two waves of 64
+    // arithmetic and some 20 other instructions, a third of the accumulate steps with three sources of one register
+    // parity), the wide one's one per 2.9: 32 x 128 x 28 x 28 -> 128, 3 x 3: 303 -> 208 us; 32 x 64 x 32 x 32 -> 128 168 -> 131;
+    // 178 x 36 x 28 x 27 -> 71 303 -> 260; 46 x 26 x 31 x 31 -> 57, 5 x 5 160 -> 131.  It has to fill its lanes about as well
+    // (184 x 21 x 24 x 21 -> 140, 0.49 of them against 0.66: 259 -> 318), and with few taps a chunk's staging costs more than
+    // the steps gain (86 x 34 x 30 x 30 -> 235, 1 x 1: 84 -> 189).  The shorter sums also round less: 5.2e-7 -> 1.4e-7.
+    if (p.mode == SIM_MODE_L1 && p.C >= 2 * kWaves && p.bh * p.bw >= 9) {
+        Tiling big = try_tiling(p, kBigPT, kBigMT, 1);
+        auto useful = [&](const Tiling &c) { return (double)c.gpi / (c.tiles * 64 * c.nws) * p.ow / (c.G * c.PT); };
+        const long long big_waves = 1LL * p.B * big.tiles * ((p.O + kBigMT - 1) / kBigMT) * kWaves;
+        if (big.lds_ok && big.fast_stage && big_waves >= 1024 && 1.3 * useful(big) >= useful(t)) {
+            big.ksplit = true;
+            if (big.CC > kWaves)
+                big.CC = big.CC / kWaves * kWaves;
+            return big;
+        }
+    }
     // Short patches (the 2x2 first layer of the missing-data network, 1x1 and 3x3 patches of one channel): a pixel's
     // whole patch is a handful of loads, and staging rows through LDS behind a barrier only adds dependent phases -
     // one pixel per lane straight from global memory, four template tiles per pixel group of 256 (1x28x28 -> 32, 2x2
@@ -1010,6 +1065,20 @@ hipError_t launch_direct(const SimKernelArgs &a, dim3 grid, size_t lds_bytes, hi
     // (the normalized modes keep the table-driven loop: with their extra operands the row form does not fit the
     // register file)
     constexpr bool kRow3 = PT == kBigPT && !PLDS && (MODE == SIM_MODE_L1 || MODE == SIM_MODE_L2 || MODE == SIM_MODE_L2_SQRTW);
+    if constexpr (MODE == SIM_MODE_L1 && PT == kBigPT) {
+        if (a.ksplit) {
+            if (a.sw == 1 && a.bh == 3 && a.bw == 3)
+                hipLaunchKernelGGL((sim_direct_kernel<MODE, PT, MT, 1, false, true, true>), grid, dim3(kThreads), lds_bytes, s,
+                                   a);
+            else if (a.sw == 1)
+                hipLaunchKernelGGL((sim_direct_kernel<MODE, PT, MT, 1, false, false, true>), grid, dim3(kThreads), lds_bytes,
+                                   s, a);
+            else
+                hipLaunchKernelGGL((sim_direct_kernel<MODE, PT, MT, 0, false, false, true>), grid, dim3(kThreads), lds_bytes,
+                                   s, a);
+            return hipGetLastError();
+        }
+    }
     if (kRow3 && a.sw == 1 && a.bh == 3 && a.bw == 3) {
         hipLaunchKernelGGL((sim_direct_kernel<MODE, PT, MT, 1, false, kRow3>), grid, dim3(kThreads), lds_bytes, s,
                            a);
@@ -1062,9 +1131,11 @@ hipError_t launch_mode(const SimKernelArgs &a0, const Tiling &t, bool plds, hipS
                                floats * sizeof(float), s, a);
         return hipGetLastError();
     }
-    const int nwm = kWaves / a.nws;
+    const int nwm = a.ksplit ? 1 : kWaves / a.nws;
     dim3 grid((unsigned)(a.B * a.tiles), (unsigned)((a.n_mtiles + nwm - 1) / nwm));
     size_t lds_bytes = (size_t)a.CC * a.TRmax * a.TC * sizeof(float);
+    if (a.ksplit)   // two waves' sums
+        lds_bytes = std::max(lds_bytes, (size_t)2 * kBigPT * kBigMT * 64 * sizeof(float));
     if (GATED)
         return hipSuccess;   // the tiled kernels recompute flagged waves inside the main launch
     a.xcd_group = grid.y > 1 && grid.x % 8 == 0;
@@ -1206,6 +1277,7 @@ static int sim_direct_run_on(const SimPlan &p, const float *input, float *output
     a.TC = t.TC; a.TRmax = t.TRmax; a.CC = t.CC; a.fast_stage = t.fast_stage;
     a.plds_off = (int)align_up((size_t)t.CC * t.chan_pitch, 4);
     a.xcd_group = 0;
+    a.ksplit = t.ksplit;
     a.NI = t.NI; a.img_lds = t.TRmax * t.TC;
     a.d_chan = make_fast_div((unsigned)std::max(1, t.chan_pitch)); a.d_img = make_fast_div((unsigned)std::max(1, a.img_lds));
     a.d_tc = make_fast_div((unsigned)std::max(1, t.TC));
