@@ -118,8 +118,9 @@ __device__ __forceinline__ void gx_step(float (&acc)[MT][PT], const float (&xv)[
 constexpr int gx_waves_per_simd(int pt, int mt) { return pt * mt <= 32 ? 3 : 2; }
 constexpr int gx_lds_budget(int pt, int mt) { return pt * mt <= 32 ? kLdsBudgetFloats / 2 : kLdsBudgetFloats; }
 
-// MULTI: small phase grids, a wave covers a.NI images.
-template <int MODE, int PT, int MT, bool MULTI = false>
+// MULTI: small phase grids, a wave covers a.NI images.  KS: the four waves of a workgroup share one channel tile and split
+// the templates of every chunk.
+template <int MODE, int PT, int MT, bool MULTI = false, bool KS = MULTI>
 __global__ __launch_bounds__(kThreads, gx_waves_per_simd(PT, MT)) void sim_grad_input_kernel(const GradXPhases phases)
 {
     const GradXArgs &a = phases.p[blockIdx.z];
@@ -133,10 +134,9 @@ __global__ __launch_bounds__(kThreads, gx_waves_per_simd(PT, MT)) void sim_grad_
     constexpr bool multi = MULTI;
     const int b0 = multi ? blockIdx.x * a.NI : blockIdx.x / a.tiles;
     const int tile = multi ? 0 : blockIdx.x - b0 * a.tiles;
-    // (MULTI: the four waves of a workgroup share one channel tile and split the steps of every chunk)
-    const int ws = multi ? 0 : wave & (a.nws - 1);
-    const int wm = multi ? 0 : wave >> a.nws_log2;
-    const int nwm = multi ? 1 : kWaves >> a.nws_log2;
+    const int ws = KS ? 0 : wave & (a.nws - 1);
+    const int wm = KS ? 0 : wave >> a.nws_log2;
+    const int nwm = KS ? 1 : kWaves >> a.nws_log2;
     const int ctile = blockIdx.y * nwm + wm;
     const bool wave_active = ctile < a.n_ctiles;
 
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(kThreads, gx_waves_per_simd(PT, MT)) void sim_grad_
         // software pipeline over the (o, tap) steps of this chunk: the g values and the parameters of
         // the next step are requested before the arithmetic of the current one
         int nk = ccn * a.nI * a.nJ;
-        if constexpr (multi) {
+        if constexpr (KS) {
             // this wave's quarter of the chunk's templates
             const int taps = a.nI * a.nJ;
             const int cpw = (ccn + kWaves - 1) / kWaves;
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kThreads, gx_waves_per_simd(PT, MT)) void sim_grad_
         }
     }
 
-    if constexpr (multi) {
+    if constexpr (KS) {
         // partial sums of waves 1..3 -> wave 0, in wave order; the tile's LDS is reused
         constexpr int kPart = MT * PT * 64;
         __syncthreads();
@@ -468,7 +468,7 @@ struct GxTiling {
     bool lds_ok, fast_stage;
 };
 
-GxTiling gx_try(const SimPlan &p, const Phase &f, int PT, int nws, int MT = 8)
+GxTiling gx_try(const SimPlan &p, const Phase &f, int PT, int nws, int MT = 8, bool wide_ksplit = false)
 {
     GxTiling t;
     t.PT = PT; t.MT = MT; t.nws = nws;
@@ -495,6 +495,10 @@ GxTiling gx_try(const SimPlan &p, const Phase &f, int PT, int nws, int MT = 8)
         t.NI = 1;   // (the small-grid variant has the 4 x 8 lane tile)
     t.ksplit = MT != 8 ? false : t.NI > 1 || (nws == 1 && t.tiles == 1 && t.gpi <= 64 && plain_waves <= 1024 && p.O >= kWaves &&
                             1LL * t.TRmax * t.TC <= kStagePos * kThreads);
+    if (wide_ksplit) {
+        t.NI = 1;
+        t.ksplit = true;
+    }
     const long long per_chan = 1LL * t.NI * t.TRmax * t.TC;
     t.lds_ok = per_chan <= budget;
     t.fast_stage = per_chan <= kStagePos * kThreads;
@@ -552,7 +556,25 @@ GxTiling gx_tiling(const SimPlan &p, const Phase &f)
         if (big.lds_ok && waves >= 1536)
             return big;
     }
-    return pick(4);
+    const GxTiling t = pick(4);
+    // L1: the 8 x 8 lane tile with the four waves of a workgroup a quarter of the templates each, where that takes fewer
+    // issue slots.  A step costs 121 instructions on the 4 x 8 tile; a quarter of one on the 8 x 8 tile 55, with its share
+    // of staging and of adding up the sums about 80; a SIMD issues one per 4 cycles from one wave, per 2 from more.
+    // 32 x 64 x 32 x 32, 128 templates, 3 x 3 (1024 waves -> 2048): 362 -> 265 us; 22 x 17 x 56 x 55, 137: 432 -> 254; 24 x 21 x 27 x
+    // 26, 88: 233 -> 133; 178 x 36 x 28 x 27, 71: 503 -> 452; not 32 x 128 x 28 x 28, 128 (2048 waves -> 4096): 465 -> 480.  The
+    // shorter sums round less: error against 64 bits 6.0e-7 -> 3.1e-7.
+    if (p.mode == SIM_MODE_L1 && !t.ksplit && p.C >= 8 && p.O >= 2 * kWaves && f.nI * f.nJ >= 4) {
+        const GxTiling big = gx_try(p, f, 8, 1, 8, true);
+        const int n_ctiles = (p.C + 7) / 8, nwm = kWaves / t.nws;
+        auto time = [&](double instructions, long long waves) {   // the stride phases run together
+            return instructions * std::max(4.0, 2.0 * p.sh * p.sw * waves / 1024);
+        };
+        if (big.lds_ok && big.fast_stage &&
+            time(80, 1LL * p.B * big.tiles * n_ctiles * kWaves) <
+                0.95 * time(121, 1LL * p.B * t.tiles * ((n_ctiles + nwm - 1) / nwm) * kWaves))
+            return big;
+    }
+    return t;
 }
 
 size_t gx_phase_param_bytes(const SimPlan &p, const Phase &f)
@@ -589,12 +611,15 @@ hipError_t gx_launch_phases(const GradXPhases &ph, int n, int PT, int MT, bool k
         gy = std::max(gy, (unsigned)a.grid_y);
         size_t floats = (size_t)a.CC * std::max(a.NI, 1) * a.TRmax * a.TC;
         if (ksplit)  // the LDS also holds three waves' partial sums at the end
-            floats = std::max<size_t>(floats, (size_t)(kWaves - 1) * 8 * 4 * 64);
+            floats = std::max<size_t>(floats, (size_t)(kWaves - 1) * MT * PT * 64);
         lds_floats = std::max(lds_floats, floats);
     }
     dim3 grid(gx, gy, (unsigned)n);
     const size_t lds_bytes = lds_floats * sizeof(float);
-    if (ksplit)
+    if (ksplit && PT == 8) {
+        if constexpr (MODE == GX_L1)
+            hipLaunchKernelGGL((sim_grad_input_kernel<MODE, 8, 8, false, true>), grid, dim3(kThreads), lds_bytes, s, ph);
+    } else if (ksplit)
         hipLaunchKernelGGL((sim_grad_input_kernel<MODE, 4, 8, true>), grid, dim3(kThreads), lds_bytes, s, ph);
     else if (MT == 4)
         hipLaunchKernelGGL((sim_grad_input_kernel<MODE, 8, 4>), grid, dim3(kThreads), lds_bytes, s, ph);
@@ -708,7 +733,7 @@ int sim_grad_input(const SimPlan &p, const float *input, const float *templates,
             a.row_limit = p.oh - 1 + f.nI - 1 - f.a0;
             a.col_limit = p.ow - 1 + f.nJ - 1 - f.b0;
             const int nwm = kWaves / t.nws;
-            a.grid_x = t.ksplit ? (p.B + t.NI - 1) / t.NI : p.B * t.tiles;
+            a.grid_x = t.ksplit && t.PT == 4 ? (p.B + t.NI - 1) / t.NI : p.B * t.tiles;
             a.grid_y = t.ksplit ? n_ctiles : (n_ctiles + nwm - 1) / nwm;
             jobs.push_back(j);
         }
