@@ -88,7 +88,7 @@ __device__ __forceinline__ float split_centre(const SplitPack &a, float part)
 }
 
 // The parameter-only part, run by the first pack_blocks + thr_blocks workgroups (256 threads) of the packing launch;
-// `lds` holds max(C, 16) floats.
+// `lds` holds max(C, 16) floats and then 12 doubles.
 __device__ inline void split_pack_block(const SplitPack &a, int block, float *lds)
 {
     const int tid = threadIdx.x;
@@ -150,7 +150,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
         }
         return;
     }
-    // biases and thresholds, one wave per template
+    // biases and thresholds, one template per workgroup (at a time)
     for (int c0 = 0; c0 < a.C; c0 += 64) {   // the loads of four channels in flight
         float part[4];
 #pragma unroll
@@ -165,13 +165,13 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
         }
     }
     __syncthreads();
-    const int lane = tid & 63;
-    for (int m = (block - a.pack_blocks) * 4 + (tid >> 6); m < a.n_mtiles * kSplitRows; m += a.thr_blocks * 4) {
+    double *sums = reinterpret_cast<double *>(lds + ((a.C + 15) / 16 * 16));   // [4 waves][3]
+    for (int m = block - a.pack_blocks; m < a.n_mtiles * kSplitRows; m += a.thr_blocks) {
         double tc2 = 0.0, traw = 0.0, lsum = 0.0;
         bool bad = false;
         if (m < a.O)
 #pragma unroll 4
-            for (int k = lane; k < a.K; k += 64) {
+            for (int k = tid; k < a.K; k += 256) {
                 const float t = a.templates[(size_t)m * a.K + k], w = a.weights[(size_t)m * a.K + k];
                 const float tc = t - lds[k / a.taps];
                 tc2 += (double)w * tc * tc;
@@ -190,8 +190,15 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
             traw += __shfl_xor(traw, d, 64);
             lsum += __shfl_xor(lsum, d, 64);
         }
-        bad = __any(bad);
-        if (lane == 0) {
+        if ((tid & 63) == 0) {
+            double *mine = sums + 3 * (tid >> 6);
+            mine[0] = tc2; mine[1] = traw; mine[2] = lsum;
+        }
+        bad = __syncthreads_or(bad);
+        if (tid == 0) {
+            tc2 = (sums[0] + sums[3]) + (sums[6] + sums[9]);
+            traw = (sums[1] + sums[4]) + (sums[7] + sums[10]);
+            lsum = (sums[2] + sums[5]) + (sums[8] + sums[11]);
             a.bias[m] = masked ? 0.0f : -(float)tc2;
             a.lg[m] = masked || a.mode == SIM_MODE_L2 ? 0.0f : (float)(lsum + (double)a.norm_const);
             double thr = 0x1p-60;
@@ -199,6 +206,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
                 thr = fmax(thr, fmax(0.25 * tc2, traw / 1024.0));
             a.thr[m] = bad || !(thr < 1e37) ? INFINITY : (float)thr;
         }
+        __syncthreads();
     }
 }
 

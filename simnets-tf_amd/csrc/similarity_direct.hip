@@ -914,23 +914,31 @@ __global__ __launch_bounds__(256) void sim_pack_params_kernel(const float *__res
         koff[k] = off;
     }
     const long long total = (long long)n_mtiles * K * MT;
-    for (long long i = (long long)block * 256 + threadIdx.x; i < total; i += nthreads) {
-        const int mi = (int)(i % MT);
-        const long long r = i / MT;
-        const int k = (int)(r % K);
-        const int mtile = (int)(r / K);
-        const int m = mtile * MT + mi;
-        float t = 0.0f, w = 0.0f;
-        if (m < O) {
-            t = templates[(size_t)m * K + k];
-            w = weights[(size_t)m * K + k];
+    auto pack = [&](auto first, auto end) {   // 32-bit indices where they suffice: a 64-bit division costs ten times one
+        for (auto i = first; i < end; i += nthreads) {
+            const int mi = (int)(i % MT);
+            const auto r = i / MT;
+            const int k = (int)(r % K);
+            const int mtile = (int)(r / K);
+            const int m = mtile * MT + mi;
+            float t = 0.0f, w = 0.0f;
+            if (m < O) {
+                t = templates[(size_t)m * K + k];
+                w = weights[(size_t)m * K + k];
+            }
+            const size_t at = i;
+            sim_pack_element(mode, m < O, t, w, fudge, pa[2 * at], pa[2 * at + 1], pc[at]);
+            if (pa2 != nullptr) {
+                float unused;
+                sim_pack_element(SIM_MODE_L2, m < O, t, w, fudge, pa2[2 * at], pa2[2 * at + 1], unused);
+            }
         }
-        sim_pack_element(mode, m < O, t, w, fudge, pa[2 * i], pa[2 * i + 1], pc[i]);
-        if (pa2 != nullptr) {
-            float unused;
-            sim_pack_element(SIM_MODE_L2, m < O, t, w, fudge, pa2[2 * i], pa2[2 * i + 1], unused);
-        }
-    }
+    };
+    const unsigned first = (unsigned)block * 256 + threadIdx.x;
+    if (total < (1ll << 31))
+        pack(first, (unsigned)total);
+    else
+        pack((long long)first, total);
 }
 
 struct Tiling {
@@ -1234,7 +1242,7 @@ int sim_direct_prepare(const SimPlan &p, const float *templates, const float *we
     const int mode = sqrtw ? (int)SIM_MODE_L2_SQRTW : p.mode;
     const int thr_blocks = sqrtw ? std::min((p.O + 3) / 4, 1024) : 0;
     const SplitPack sp = sim_split_pack_args(p, split, templates, weights, ws + l.split);
-    const size_t lds = split.on ? (size_t)std::max(p.C, 16) * sizeof(float) : 0;
+    const size_t lds = split.on ? align_up(p.C, 16) * sizeof(float) + 12 * sizeof(double) : 0;
     hipLaunchKernelGGL(sim_pack_params_kernel, dim3(sp.pack_blocks + sp.thr_blocks + pack_blocks + thr_blocks),
                        dim3(256), lds, s, templates, weights, p.O,
                        p.K, t.MT, n_mtiles, mode, p.fudge, reinterpret_cast<float *>(ws + l.pa),

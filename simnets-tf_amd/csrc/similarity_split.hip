@@ -487,7 +487,7 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     a.pieces = sp.pieces; a.n_mtiles = sp.n_mtiles; a.mode = p.mode; a.fudge = p.fudge;
     a.norm_const = p.mode == SIM_MODE_L2_NORM ? (float)((double)(-0.5f * (float)p.K) * std::log(2.0 * M_PI)) : 0.0f;
     a.pack_blocks = sp.on ? sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4) : 0;
-    a.thr_blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows / 4, 256) : 0;
+    a.thr_blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows, 512) : 0;
     return a;
 }
 
