@@ -1701,6 +1701,64 @@ __global__ __launch_bounds__(256) void mex_grad_offsets_finish_rows_kernel(const
         gr[k] -= expf(nr[k]) * sum;   // reads back what this lane stored above
 }
 
+// The same for few rows of many chunks: one workgroup of 1024 per row, 128 threads on each of the eight interleaved sums,
+// eight chunks of two elements requested at a time.  With a wave per row the chunks are one chain of round trips to
+// memory (32 rows of 144 elements, 200 chunks: eight workgroups, 25 round trips, 21.7 us; here four, 6.2 us); with
+// many rows the waves of others hide it, and with few chunks there is no chain.  Same values: the additions, the row
+// sum's included, keep their order.
+__global__ __launch_bounds__(1024) void mex_grad_offsets_finish_tall_rows_kernel(const float *__restrict__ partial,
+                                                                                long long n, int chunks, int K,
+                                                                                const float *__restrict__ normalized,
+                                                                                float *__restrict__ doff)
+{
+    __shared__ float sm[8 * kFinishRowsMaxK];
+    const long long row = blockIdx.x;
+    const float *pr = partial + (size_t)row * K;
+    float *gr = doff + (size_t)row * K;
+    const int tid = threadIdx.x, j = tid >> 7;
+    for (int k0 = tid & 127; k0 < K; k0 += 256) {
+        float s2[2] = {0.0f, 0.0f};
+        for (int c0 = j; c0 < chunks; c0 += 64) {
+            float v[8][2];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    v[u][e] = pr[(size_t)min(c0 + 8 * u, chunks - 1) * n + min(k0 + 128 * e, K - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    s2[e] = c0 + 8 * u < chunks ? s2[e] + v[u][e] : s2[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            if (k0 + 128 * e < K)
+                sm[j * K + k0 + 128 * e] = s2[e];
+    }
+    __syncthreads();
+    float t = 0.0f;
+    if (tid < K) {   // K <= kFinishRowsMaxK = the workgroup's threads
+        t = sm[tid];
+#pragma unroll
+        for (int i = 1; i < 8; ++i)
+            t += sm[i * K + tid];
+        sm[tid] = t;
+        if (normalized == nullptr)
+            gr[tid] = t;
+    }
+    if (normalized == nullptr)
+        return;
+    __syncthreads();
+    float sum = 0.0f;
+    for (int k = tid & 63; k < K; k += 64)
+        sum += sm[k];
+    for (int d = 32; d > 0; d >>= 1)
+        sum += __shfl_xor(sum, d, 64);
+    if (tid < K)
+        gr[tid] = t - expf(normalized[(size_t)row * K + tid]) * sum;
+}
+
 // The same for few long rows (a classifier head: 10 rows of 512): one workgroup per row, the four waves split its
 // elements (thread t takes t, t + 256, ...), the row sum of the chain rule goes through LDS.
 __global__ __launch_bounds__(256) void mex_grad_offsets_finish_wide_rows_kernel(const float *__restrict__ partial,
@@ -2294,6 +2352,12 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
         if (rows <= 64 && d.K >= 256 && d.K <= kFinishRowsMaxK) {
             // few long rows: a workgroup per row
             hipLaunchKernelGGL(mex_grad_offsets_finish_wide_rows_kernel, dim3((unsigned)rows), dim3(256), 0, s, go.partial,
+                               n_off, go.cpr, d.K, p.normalize_offsets ? go.off : nullptr, offsets_grad);
+            return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
+        }
+        // (33 elements and more: shorter rows have several lanes to an element in the kernel below)
+        if (d.K > 32 && d.K <= kFinishRowsMaxK && rows <= 512 && go.cpr >= 64) {
+            hipLaunchKernelGGL(mex_grad_offsets_finish_tall_rows_kernel, dim3((unsigned)rows), dim3(1024), 0, s, go.partial,
                                n_off, go.cpr, d.K, p.normalize_offsets ? go.off : nullptr, offsets_grad);
             return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
         }

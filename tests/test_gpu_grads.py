@@ -915,3 +915,29 @@ def test_similarity_grads_random_geometries(pkg):
         print("case", case, (B, C, H, W), O, kw, flush=True)
         # L1: the gradient is a sum of signs, which an input equal to a template value would flip: not with random data
         check_sim_grads(pkg, x, t, w, seed=case, **kw)
+
+
+@pytest.mark.parametrize("C,M,blocks", [(11, 5, 3), (16, 33, 3), (41, 30, 5), (5, 17, 3)])   # K = 99, 144, 1025, 45
+def test_mex_offsets_grad_few_rows_of_many_chunks(pkg, C, M, blocks):
+    """One region over many pixels: few rows of partial sums, the chunks of a row split over a workgroup (K of 33 to 1024;
+    one case beyond, one of the shortest).  Without and with the normalisation's chain rule, against torch in 64 bits."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((24, C, 17, 19), generator=g, device="cuda")
+    pad = blocks // 2
+    kw = dict(softmax_mode=True, blocks=[C, blocks, blocks], strides=[C, 1, 1], padding=[0, pad, pad],
+              use_unshared_regions=False, shared_offset_region=[-1])
+    off = torch.randn(pkg.mex_output_shape(tuple(x.shape), M, **kw)[1], generator=g, device="cuda") * 0.3
+    cols = torch.nn.functional.unfold(x.double(), blocks, padding=pad)          # [B, K, pixels], zero padding
+    K = cols.shape[1]
+    for normalize in (False, True):
+        y = pkg.mex(x, off, M, normalize_offsets=normalize, **kw)
+        go = torch.randn(y.shape, generator=g, device="cuda")
+        got = pkg.mex_offsets_grad(x, off, y, go, M, normalize_offsets=normalize, **kw)
+        o64 = off.double().reshape(M, K).requires_grad_()
+        o = o64 - torch.logsumexp(o64, 1, keepdim=True) if normalize else o64
+        want = torch.stack([torch.logsumexp(cols + o[m][None, :, None], 1) for m in range(M)], 1)
+        ref = torch.autograd.grad(want, o64, go.double().reshape(want.shape))[0]
+        n = go.numel() // M
+        # n products of probabilities and gradients of random sign, each within a few units of its last place
+        err = float((got.double().reshape(M, K) - ref).norm() / ref.norm())
+        assert err <= 4 * math.sqrt(n) * 2.0 ** -24, err
