@@ -36,7 +36,8 @@ struct MexGradArgs {
     float *dx;             // input gradient
     float *partial;        // offsets gradient partial sums [chunk][R][M][K]
     int overlap;           // patches overlap: the per-patch gradients go to `col`, mex_col2im_kernel adds them up
-    float *col;            // [B][Co*Ho*Wo][K] gradient of every patch element (overlapping patches only)
+    float *col;            // [B][K][Co*Ho*Wo] gradient of every patch element (overlapping patches only): lanes hold
+                           // consecutive output pixels both where it is written and where it is added up
     int cpr;               // pixel chunks per region
     int msplit;            // input gradient: the instances are split over gridDim.z workgroups (1: no split) ...
     int mg_per_split;      // ... of this many packed groups (GM_TM instances) each, which write their partial
@@ -141,13 +142,13 @@ __device__ __forceinline__ void mex_grad_input_wave(const MexGradArgs &ga, int r
     if (!valid)
         return;
     float *dimg = dx + (size_t)px.b * a.C * a.H * a.W;
-    float *dcol = ga.col + ((size_t)px.b * plane + px.out_off) * a.K + k0;
+    float *dcol = ga.col + ((size_t)px.b * a.K + k0) * plane + px.out_off;
 #pragma unroll
     for (int j = 0; j < GX_KT; ++j) {
         if (io[j] < 0)
             continue;
         if (ga.overlap)
-            dcol[j] = acc[j];
+            dcol[j * plane] = acc[j];
         else
             dimg[io[j]] = acc[j];
     }
@@ -483,7 +484,7 @@ __global__ __launch_bounds__(256) void mex_grad_input_mfma_kernel(const MexGradA
             const float val = acc[t][v] * (buffered ? xin[v][t]
                                                     : __builtin_amdgcn_exp2f(__builtin_fmaf(xin[v][t], a.c1, -ap[p])));
             if (ga.overlap)
-                ga.col[((size_t)pb[p] * plane + pout[p]) * a.K + k] = val;
+                ga.col[((size_t)pb[p] * a.K + k) * plane + pout[p]] = val;
             else
                 dxo[at[v][t]] = val;
         }
@@ -556,7 +557,8 @@ __global__ __launch_bounds__(256) void mex_col2im_kernel(const MexKernelArgs a, 
     const int co_lo = first(c, a.pc, a.bc, a.sc), co_hi = min(a.Co - 1, (c + a.pc) / a.sc);
     const int ho_lo = first(h, a.ph, a.bh, a.sh), ho_hi = min(a.Ho - 1, (h + a.ph) / a.sh);
     const int wo_lo = first(w, a.pw, a.bw, a.sw), wo_hi = min(a.Wo - 1, (w + a.pw) / a.sw);
-    const float *cb = col + (size_t)b * a.Co * a.Ho * a.Wo * a.K;
+    const size_t plane = (size_t)a.Co * a.Ho * a.Wo;
+    const float *cb = col + (size_t)b * plane * a.K;
     float acc = 0.0f;
     for (int co = co_lo; co <= co_hi; ++co) {
         const int dc = c + a.pc - co * a.sc;
@@ -564,7 +566,7 @@ __global__ __launch_bounds__(256) void mex_col2im_kernel(const MexKernelArgs a, 
             const int dh = h + a.ph - ho * a.sh;
             for (int wo = wo_lo; wo <= wo_hi; ++wo) {
                 const int dw = w + a.pw - wo * a.sw;
-                acc += cb[(((size_t)co * a.Ho + ho) * a.Wo + wo) * a.K + (dc * a.bh + dh) * a.bw + dw];
+                acc += cb[((dc * a.bh + dh) * a.bw + dw) * plane + ((size_t)co * a.Ho + ho) * a.Wo + wo];
             }
         }
     }
@@ -1840,7 +1842,7 @@ __global__ __launch_bounds__(1024) void mex_grad_head_kernel(const MexGradArgs g
             const float *src = (lane & 16) ? ga.out + ((size_t)px.b * a.M + ml) * plane + oo
                                            : ga.g + ((size_t)px.b * a.M + ml) * gplane + pooled_g_offset(ga, oo);
             go[p] = *src;
-            col[p] = ((size_t)px.b * plane + oo) * a.K;
+            col[p] = (size_t)px.b * a.K * plane + oo;
         }
         // Straight-line arithmetic: instances past the last one repeat it with a zero gradient (their sums are never
         // stored), threads past the last patch element compute on the out-of-bounds value (nothing of theirs is
@@ -1861,7 +1863,7 @@ __global__ __launch_bounds__(1024) void mex_grad_head_kernel(const MexGradArgs g
             }
             if (want_input && io[p] >= 0) {
                 if (ga.overlap)
-                    ga.col[col[p] + k] = dxa;
+                    ga.col[col[p] + k * plane] = dxa;
                 else
                     ga.dx[img[p] + io[p]] = dxa;
             }
@@ -1889,7 +1891,7 @@ struct MexGradTiling {
     bool mfma;           // finite epsilon: the matrix-core kernels, fed by the forward pass's packed offsets
     size_t norm_bytes, partial_bytes, packed_bytes;
     bool overlap;        // input gradient: patches overlap
-    size_t col_bytes;    // ... and their per-patch gradients pass through a [B][Co*Ho*Wo][K] buffer
+    size_t col_bytes;    // ... and their per-patch gradients pass through a [B][K][Co*Ho*Wo] buffer
     bool tiles_input;    // patches tile the input exactly: every element is written by exactly one patch
     int msplit, mg_per_split;  // input gradient, matrix form: instance groups split over gridDim.z workgroups
     size_t split_bytes;  // ... whose partial gradients [split][input] are added by mex_sum_splits_kernel
