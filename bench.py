@@ -30,7 +30,12 @@ EXP_RATE_MEASURED = 19.66e12  # v_exp_f32 at a quarter of the 128 lanes/clk/CU V
 
 # HBM bytes per launch of the dominant kernel of the headline workload, from rocprofv3 FETCH_SIZE / WRITE_SIZE runs
 # scaled by a copy kernel of known size; not measured inside this run: "traffic_source" names the committed summary.
+PEAK_BF16_TFLOPS = 2500.0  # dense bf16 matrix peak
+# The default form of the L2 modes multiplies 16-bit pieces on the bf16 matrix cores: six products for each of two
+# operands per term, a third operand (three products for each of two sums) where NaN inputs are ignored
+PIECES_FLOP, PIECES_MASKED_FLOP = 24, 36
 MEASURED_TRAFFIC = {
+    "pieces": (197.0e6, "profiles/similarity_split_l2.md"),
     "sqrtw": (231.8e6, "profiles/sim_direct_l2_config3.md"),
     "direct": (None, "no counter run of the current three-instruction kernel"),
     "mfma": (223.3e6, "profiles/sim_direct_l2_config3_other_forms.md"),
@@ -216,9 +221,9 @@ def main():
         torch.cuda.synchronize()
     wall_ms, ev_ms = timed(sim3("L2", args.algo), args.steps, args.warmup)
     gmacs = gmac3 / (ev_ms * 1e-3)
-    flop_per_gmac = 4
+    path = args.algo or "pieces"
+    flop_per_gmac, peak = (PIECES_FLOP, PEAK_BF16_TFLOPS) if path == "pieces" else (4, PEAK_FP32_TFLOPS)
     achieved_tflops = gmacs * flop_per_gmac / 1e12
-    path = args.algo or "sqrtw"
     traffic, traffic_source = MEASURED_TRAFFIC[path]
     result = {
         "metric": "Similarity L2 fwd generalized-GMAC/s (config 3), 1 MI355X",
@@ -230,19 +235,19 @@ def main():
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": "config3: Similarity L2 fwd 256x64x32x32, 128 templates 64x3x3, s1 p1 "
                                "-> 256x128x32x32 (M=262144 N=128 K=576)",
-                   "algo": args.algo or "auto (sqrt-weight form; waves with a partial sum near zero are recomputed "
-                                        "term by term)",
+                   "algo": args.algo or "auto (16-bit pieces on the bf16 matrix cores, fp32 sums; tiles with an output "
+                                        "near zero are recomputed term by term)",
                    "entry_point": "simnets_hip_similarity_fwd (packs the parameters in every step)",
                    "gmac_per_step": gmac3},
-        # compute bound: the FP32 vector ALU ("valu") unless the matrix-core path is asked for; the two peaks are
-        # the same 157.3 TFLOP/s
-        "roofline": {"bound": "mfma" if args.algo == "mfma" else "valu",
-                     "achieved": round(achieved_tflops, 2), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(achieved_tflops / PEAK_FP32_TFLOPS, 4),
+        # compute bound: by default the products of pieces at the bf16 matrix peak; "direct" and "sqrtw" run on the
+        # FP32 vector ALU ("valu"), "mfma" on the FP32 matrix instructions, whose peaks are the same 157.3 TFLOP/s
+        "roofline": {"bound": "mfma" if path in ("pieces", "mfma") else "valu",
+                     "achieved": round(achieved_tflops, 2), "peak": peak, "unit": "TFLOP/s",
+                     "frac": round(achieved_tflops / peak, 4),
                      "traffic": traffic, "traffic_source": traffic_source,
                      "kernel_ms": round(ev_ms, 4), "flop_per_gmac": flop_per_gmac,
                      "cold_start": {"kernel_ms": round(cold_ev_ms, 4), "ms_per_step": round(cold_wall_ms, 4),
-                                    "frac": round(gmac3 * flop_per_gmac / (cold_ev_ms * 1e-3) / 1e12 / PEAK_FP32_TFLOPS, 4),
+                                    "frac": round(gmac3 * flop_per_gmac / (cold_ev_ms * 1e-3) / 1e12 / peak, 4),
                                     "what": "the same %d steps timed right after the %d warm-up steps, before the "
                                             "%.1f s of untimed load that precede the headline's steps"
                                             % (args.steps, args.warmup, args.settle)},
@@ -256,14 +261,17 @@ def main():
     oracle = None
 
     def entry(ms, gmac, nbytes, bound, flop=None, mex=False):
-        """bound: which roofline prices this shape ("valu", "mfma", "hbm"); frac is taken against it.
+        """bound: which roofline prices this shape ("valu", "mfma", "pieces", "hbm"); frac is taken against it.
+        "pieces": the products of 16-bit pieces (`flop` counts them) at the bf16 matrix peak.
         MEX rows (mex=True) are priced on HBM: the product form runs one exponential per patch element and one fused
         multiply-add per term on the matrix cores, so neither the exponential rate nor the vector ALU bounds them."""
         rate = gmac / (ms * 1e-3)
         e = {"kernel_ms": round(ms, 4), "gmac_per_s_G": round(rate / 1e9, 1), "bound": bound,
              "algorithmic_bytes": int(nbytes),
              "hbm_frac": round(nbytes / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4)}
-        if flop and not mex:
+        if bound == "pieces":
+            e["bf16_matrix_frac"] = round(rate * flop / 1e12 / PEAK_BF16_TFLOPS, 4)
+        elif flop and not mex:
             e["valu_frac"] = round(rate * flop / 1e12 / PEAK_FP32_TFLOPS, 4)
         if mex:
             e["reference_formulation_not_executed"] = {
@@ -273,7 +281,8 @@ def main():
                 "exp_frac_measured_rate": round(rate / EXP_RATE_MEASURED, 4),
                 "valu_frac": round(rate * (flop or 5) / 1e12 / PEAK_FP32_TFLOPS, 4)}
             e["matrix_pipe_frac"] = round(rate * 2 / 1e12 / PEAK_FP32_TFLOPS, 4)
-        e["frac"] = {"valu": e.get("valu_frac"), "mfma": e.get("valu_frac"), "hbm": e["hbm_frac"]}[bound]
+        e["frac"] = {"valu": e.get("valu_frac"), "mfma": e.get("valu_frac"), "hbm": e["hbm_frac"],
+                     "pieces": e.get("bf16_matrix_frac")}[bound]
         return e
 
     def cpu_leg(sample, run_single, run_all, gmac_single, gmac_all, err):
@@ -314,7 +323,8 @@ def main():
         others["config3_L1_direct"] = entry(ms, gmac3, bytes3, "valu", flop=3)
         prep3 = pkg.similarity_prepare(x3.shape, T3, W3, similarity_function="L2", algo=args.algo, **kw3)
         _, ms = timed(lambda: prep3(X3, out=out3), args.steps, args.warmup)
-        others["config3_L2_prepared"] = entry(ms, gmac3, bytes3, "mfma" if args.algo == "mfma" else "valu", flop=4)
+        others["config3_L2_prepared"] = entry(ms, gmac3, bytes3, {"pieces": "pieces", "mfma": "mfma"}.get(path, "valu"),
+                                              flop=flop_per_gmac)
         others["config3_L2_prepared"]["entry_point"] = "simnets_hip_similarity_fwd_prepared (parameters packed once)"
         del prep3
         for algo in ("direct", "sqrtw", "mfma"):
@@ -325,8 +335,7 @@ def main():
                 others["config3_L2_" + algo] = entry(ms, gmac3, bytes3, "mfma" if algo == "mfma" else "valu", flop=4)
             except pkg.SimnetsError as e:
                 others["config3_L2_" + algo] = {"error": str(e)}
-        # worst case of the sqrt-weight form's guard: every wave stops after the first channel chunk and is
-        # recomputed term by term (inputs and templates 1000 +- 3: all outputs far below the thresholds)
+        # worst case of the default form's guard: every tile is flagged and recomputed term by term (inputs and templates 1000 +- 3: all outputs far below the thresholds)
         g = np.random.default_rng(77)
         XA = to_dev((g.normal(size=x3.shape) + 1000).astype(np.float32))
         TA = to_dev((g.normal(size=t3.shape) + 1000).astype(np.float32))
@@ -336,13 +345,13 @@ def main():
         others["config3_L2_guard_worst_case"] = {
             "kernel_ms": round(ms_w, 4), "direct_same_data_ms": round(ms_d, 4), "ratio": round(ms_w / ms_d, 3),
             "bit_identical_to_direct": bool(torch.equal(got_w, out3)),
-            "data": "inputs and templates ~ N(1000, 1): every wave is flagged"}
+            "data": "inputs and templates ~ N(1000, 1): every tile is flagged"}
         del XA, TA, got_w
 
         # the reference's other L2 modes at this scale (include/utils/similarity_utils.hpp:38-80): the normalisation
         # term (half the log-weight per element, and with NaN inputs ignored only for the elements present), 25 % of the
-        # input missing, NaN beyond the border.  Priced at the functor's 6 flop per term (subtract, square, weight,
-        # halve, add the log term, accumulate); the kernels spend 4 instructions on them.
+        # input missing, NaN beyond the border.  Priced at the products of 16-bit pieces that
+        # the default form executes.
         def sim3_mode(X, mode):
             return lambda: pkg.similarity(X, T3, W3, similarity_function="L2", out=out3, **dict(kw3, **mode))
 
@@ -356,8 +365,9 @@ def main():
         }
         for name, (_, Xm, mode) in modes3.items():
             _, ms = timed(sim3_mode(Xm, mode), args.steps, args.warmup)
-            others[name] = entry(ms, gmac3, bytes3, "valu", flop=6)
-            others[name]["flop_per_gmac"] = 6
+            flop = PIECES_MASKED_FLOP if "ignore_nan_input" in mode else PIECES_FLOP
+            others[name] = entry(ms, gmac3, bytes3, "pieces", flop=flop)
+            others[name]["flop_per_gmac"] = flop
             others[name]["attrs"] = {k: (str(v) if isinstance(v, float) else v) for k, v in mode.items()}
             if "ignore_nan_input" in mode:
                 others[name]["data"] = "25 % of the input elements are NaN"
@@ -606,10 +616,12 @@ def main():
         G3 = to_dev(np.random.default_rng(6789).normal(size=(256, 128, 32, 32)).astype(np.float32))
         _, ms = timed(lambda: pkg.similarity_input_grad(X3, T3, W3, G3, similarity_function="L2", **kw3), args.steps,
                       args.warmup)
-        others["config5_similarity_input_grad_L2"] = entry(ms, gmac3, 2 * 67108864 + 589824 + 134217728, "mfma", flop=4)
+        others["config5_similarity_input_grad_L2"] = entry(ms, gmac3, 2 * 67108864 + 589824 + 134217728, "pieces",
+                                                           flop=PIECES_FLOP)
         _, ms = timed(lambda: pkg.similarity_parameters_grad(X3, T3, W3, G3, similarity_function="L2", **kw3),
                       args.steps, args.warmup)
-        others["config5_similarity_params_grad_L2"] = entry(ms, gmac3, 67108864 + 3 * 589824 + 134217728, "mfma", flop=5)
+        others["config5_similarity_params_grad_L2"] = entry(ms, gmac3, 67108864 + 3 * 589824 + 134217728, "pieces",
+                                                            flop=PIECES_FLOP)
         Y2 = pkg.mex(X2, O2, n2, normalize_offsets=True, **kw2)
         G2 = to_dev(np.random.default_rng(6789).normal(size=(64, 64, 16, 16)).astype(np.float32))
         _, ms = timed(lambda: pkg.mex_input_grad(X2, O2, Y2, G2, n2, normalize_offsets=True, **kw2), args.steps,
