@@ -63,6 +63,22 @@ __device__ __forceinline__ void split3(float v, __bf16 &p0, __bf16 &p1, __bf16 &
     p2 = (__bf16)(r - (float)p1);
 }
 
+// The same for values that may be infinite or NaN, which stay in one piece.
+__device__ __forceinline__ void split3_any(float v, __bf16 &p0, __bf16 &p1, __bf16 &p2)
+{
+    split3(v, p0, p1, p2);
+    const bool finite = __builtin_fabsf(v) < INFINITY;
+    p1 = finite ? p1 : (__bf16)0.0f;
+    p2 = finite ? p2 : (__bf16)0.0f;
+}
+
+// A sum of products of such pieces, hi the leading one's and lo the lesser ones'.  An infinite factor meets the other's
+// lesser pieces, zeros and either sign among them, so lo says nothing there; hi holds the infinity with the sign it has.
+__device__ __forceinline__ float split_sum(float hi, float lo)
+{
+    return __builtin_isfinite(hi) ? hi + lo : hi;
+}
+
 // What is subtracted from every value of a channel: the mean of up to 32 template elements spread over the channel.  Any
 // value is correct; one near the data keeps the three sums of w (x - t)^2 from cancelling.  Sixteen lanes share a
 // channel; all of them get the result, the same wherever it is computed.

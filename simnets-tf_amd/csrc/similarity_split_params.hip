@@ -65,14 +65,6 @@ __device__ __forceinline__ Unit unit_of(const ParamsArgs &a, int u)
 
 __device__ __forceinline__ int first_unit(const ParamsArgs &a, int s) { return (int)((long long)s * a.units / a.S); }
 
-__device__ __forceinline__ void split3_any(float v, __bf16 &p0, __bf16 &p1, __bf16 &p2)
-{
-    split3(v, p0, p1, p2);
-    const bool finite = __builtin_fabsf(v) < INFINITY;   // else one piece, as it is
-    p1 = finite ? p1 : (__bf16)0.0f;
-    p2 = finite ? p2 : (__bf16)0.0f;
-}
-
 // Blocks 0 .. S n_mtiles - 1: g of one share of the pixels and one template tile, a thread one template's pairs of pixels
 // (eight neighbouring threads read 64 contiguous bytes), and the share's sums G.  The blocks behind: the centres of 16
 // channels each.
@@ -276,8 +268,8 @@ __device__ __forceinline__ void params_body(const ParamsArgs &a, char *lds, int 
                 continue;
             const size_t slab = (size_t)a.Opad * a.Kpad;
             float *dst = a.partial + (size_t)s * slab + (size_t)o * a.Kpad + k;
-            dst[0] = hi[1][i][r] + lo[1][i][r];
-            dst[(size_t)a.S * slab] = hi[0][i][r] + lo[0][i][r];
+            dst[0] = split_sum(hi[1][i][r], lo[1][i][r]);
+            dst[(size_t)a.S * slab] = split_sum(hi[0][i][r], lo[0][i][r]);
         }
     }
 }

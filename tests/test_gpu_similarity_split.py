@@ -194,3 +194,40 @@ def test_split_gradients_with_infinite_values(pkg, value):
         assert bad[:, 5, 1:, 1:].all()
         bad[:, 5, 1:, 1:] = False
         assert not bad.any()
+
+
+def terms_64(x, t, w, go):
+    """Parameter gradients of plain L2, 3 x 3, stride 1, padding 1, sum by sum in the order of values (x - t) in 32 bits, as
+    the operator defines them, added in 64 bits: infinities and NaN appear where an fp32 evaluation of the terms has them."""
+    O, C = t.shape[:2]
+    cols = torch.nn.functional.unfold(x, 3, padding=1).permute(1, 0, 2).reshape(C * 9, -1)
+    g = go.permute(1, 0, 2, 3).reshape(O, -1)
+    dt, dw = (torch.empty((O, C * 9), dtype=torch.float64, device=x.device) for _ in range(2))
+    for o in range(O):
+        d = cols - t[o].reshape(-1, 1)
+        dt[o] = (2 * w[o].reshape(-1, 1) * (g[o] * d)).double().sum(1)
+        dw[o] = -((g[o] * d) * d).double().sum(1)
+    return dt.reshape(t.shape), dw.reshape(t.shape)
+
+
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), 3e19])
+@pytest.mark.parametrize("ones", [True, False])
+def test_split_parameter_gradients_keep_infinities(pkg, value, ones):
+    """An infinite input, or one whose square overflows, gives the gradients the infinities that the terms have - where the
+    output gradient's lesser pieces are zero (g = 1) and where they have signs of their own."""
+    geom = GEOMS[1]
+    g = torch.Generator(device="cuda").manual_seed(37)
+    shape, O = geom["shape"], geom["O"]
+    x, t = torch.randn(shape, generator=g, device="cuda"), torch.randn((O, shape[1], 3, 3), generator=g, device="cuda")
+    w = t.abs() + 0.1
+    go = torch.rand((shape[0], O, shape[2], shape[3]), generator=g, device="cuda") + 0.5
+    if ones:
+        go = torch.ones_like(go)
+    x[8, 5, 20, 30] = value
+    want = terms_64(x, t, w, go)
+    assert want[1][:, 5].isinf().any() and not want[0].isnan().any() and not want[1].isnan().any()
+    for got, ref in zip(pkg.similarity_parameters_grad(x, t, w, go, **options("l2", geom)), want):
+        inf = ref.isinf()
+        assert torch.equal(got[inf].double(), ref[inf])
+        err = (got.double() - ref)[~inf].norm() / ref[~inf].norm()
+        assert float(err) <= 4 * math.sqrt(go.numel() // O) * 2.0 ** -24, float(err)
