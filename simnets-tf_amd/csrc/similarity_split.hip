@@ -64,9 +64,35 @@ struct SplitArgs {
     int bw, sh, sw, ph, pw, taps, chunks, steps, n_mtiles, Wp, Hv;
     int gmax;        // matrix tiles of templates per workgroup: 4, 2 or 1
     float oob;
-    const float *x;  // input gradient: the forward's input, of the output's shape
+    const float *x;  // input gradient: the forward's input, of the output's shape; templates and weights [C][O][taps]
+    const float *templates, *weights;
+    float scale;
     FastDiv d_npix, d_ow, d_wp, d_hv;
 };
+
+// Input gradient of one element (input channel ch, pixel rem of its image) term by term: where the sums A and (x - c) B are
+// infinite with one sign, only the terms tell which way their difference goes.  Not inlined, and with the kernel's
+// arguments read again from its argument segment (they end where the implicit arguments begin; the kernel's other
+// argument is an int): the main loop's registers stay as they are.
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __noinline__ float split_grad_terms(int img, int ch, int rem, float x)
+{
+    const SplitArgs &a = *reinterpret_cast<const SplitArgs *>(
+        reinterpret_cast<const char *>(__builtin_amdgcn_implicitarg_ptr()) - (sizeof(SplitArgs) + 8));
+    const int y = rem / a.ow, xo = rem - y * a.ow;
+    float sum = 0.0f;
+    for (int o = 0; o < a.C; ++o)
+        for (int tap = 0; tap < a.taps; ++tap) {
+            const int dh = tap / a.bw, r = y + dh - a.ph, c = xo + tap - dh * a.bw - a.pw;
+            if (r < 0 || r >= a.H || c < 0 || c >= a.W)
+                continue;
+            const size_t at = ((size_t)o * a.O + ch) * a.taps + (a.taps - 1 - tap);
+            sum += a.in[(((size_t)img * a.C + o) * a.H + r) * a.W + c] * (a.scale * a.weights[at]) * (a.templates[at] - x);
+        }
+    return sum;
+}
+static_assert(sizeof(SplitArgs) % 8 == 0, "the explicit arguments end 8 bytes behind the block");
+#endif
 
 // One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
 template <int KIND, int CG, int G>
@@ -164,11 +190,8 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mt
                     }
                     __bf16 p0, p1, p2;
                     if (GRAD) {
-                        split3(d, p0, p1, p2);
-                        const bool finite = __builtin_fabsf(d) < INFINITY;   // else one piece, as it is
-                        v[0][j] = p0;
-                        v[1][j] = finite ? p1 : (__bf16)0.0f;
-                        v[2][j] = finite ? p2 : (__bf16)0.0f;
+                        split3_any(d, p0, p1, p2);
+                        v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
                         continue;
                     }
                     split3(d * d, p0, p1, p2);
@@ -269,14 +292,31 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mt
                 const int ml = min(8 * (r / 4) + 4 * half + r % 4, a.O - 1 - mtile * kSplitRows);
                 x[r] = a.x[base + (size_t)ml * a.npix];
             }
+            float v[16], any = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                v[r] = __builtin_fmaf(-(x[r] - ctr[r]), tm[i][r] + lg[i][r], hi[i][r] + lo[i][r]);
+                any = __builtin_fmaf(v[r], 0.0f, any);   // NaN once a value is not finite
+            }
+            if (any != any) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float A = split_sum(hi[i][r], lo[i][r]);
+                    v[r] = __builtin_fmaf(-(x[r] - ctr[r]), split_sum(tm[i][r], lg[i][r]), A);
+#if defined(__HIP_DEVICE_COMPILE__)
+                    if (v[r] != v[r] && __builtin_isinf(A))
+                        v[r] = split_grad_terms(img, min(mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4, a.O - 1),
+                                                n - img * a.npix, x[r]);
+#endif
+                    if (flag && x[r] != x[r])
+                        v[r] = 0.0f;
+                }
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int ml = 8 * (r / 4) + 4 * half + r % 4;
-                float v = __builtin_fmaf(-(x[r] - ctr[r]), tm[i][r] + lg[i][r], hi[i][r] + lo[i][r]);
-                if (flag && x[r] != x[r])
-                    v = 0.0f;
                 if (mtile * kSplitRows + ml < a.O)
-                    a.out[base + (size_t)ml * a.npix] = v;
+                    a.out[base + (size_t)ml * a.npix] = v[r];
             }
         }
         return;
@@ -400,9 +440,9 @@ __global__ __launch_bounds__(kThreads) void sim_split_grad_pack_kernel(const Spl
             t = a.templates[at] - centre[row];
         }
         __bf16 p0, p1, p2;
-        split3(w * t, p0, p1, p2);
+        split3_any(w * t, p0, p1, p2);
         v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
-        split3(w, p0, p1, p2);
+        split3_any(w, p0, p1, p2);
         v[3][j] = p0; v[4][j] = p1; v[5][j] = p2;
     }
     bf16x8 *dst = reinterpret_cast<bf16x8 *>(a.packed) +
@@ -492,11 +532,10 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
 }
 
 template <int KIND>
-static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, const float *x, float *output, char *ws,
-                        int flag, hipStream_t s)
+static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, float *output, char *ws, int flag,
+                        hipStream_t s, SplitArgs a = {})
 {
-    SplitArgs a;
-    a.in = input; a.x = x; a.out = output;
+    a.in = input; a.out = output;
     a.packed = reinterpret_cast<const bf16x8 *>(ws + sp.packed);
     a.ctr = reinterpret_cast<const float *>(ws + sp.ctr);
     a.bias = reinterpret_cast<const float *>(ws + sp.bias);
@@ -527,8 +566,8 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
 int sim_split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, float *output, char *ws, hipStream_t s)
 {
     if (p.mode == SIM_MODE_L2_NORM_IGNORE_NAN)
-        return split_launch<SPLIT_MASKED>(p, sp, input, nullptr, output, ws, 0, s);
-    return split_launch<SPLIT_FWD>(p, sp, input, nullptr, output, ws, p.mode == SIM_MODE_L2_NORM, s);
+        return split_launch<SPLIT_MASKED>(p, sp, input, output, ws, 0, s);
+    return split_launch<SPLIT_FWD>(p, sp, input, output, ws, p.mode == SIM_MODE_L2_NORM, s);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -573,11 +612,13 @@ int sim_split_grad_input_launch(const SimPlan &p, const float *input, const floa
     char *ws = reinterpret_cast<char *>(workspace);
     SplitPack a = sim_split_pack_args(q, sp, templates, weights, ws);
     a.O = p.O; a.C = p.C;   // of the templates' layout
-    const bool norm = p.mode != SIM_MODE_L2;   // the normalized functor halves the plain one
-    hipLaunchKernelGGL(sim_split_grad_pack_kernel, dim3(a.pack_blocks), dim3(kThreads), 0, s, a, norm ? 1.0f : 2.0f);
+    SplitArgs g = {};
+    g.x = input; g.templates = templates; g.weights = weights;
+    g.scale = p.mode != SIM_MODE_L2 ? 1.0f : 2.0f;   // the normalized functor halves the plain one
+    hipLaunchKernelGGL(sim_split_grad_pack_kernel, dim3(a.pack_blocks), dim3(kThreads), 0, s, a, g.scale);
     if (hipGetLastError() != hipSuccess)
         return SIMNETS_ERR_HIP;
-    return split_launch<SPLIT_GRAD>(q, sp, output_grad, input, input_grad, ws, p.mode == SIM_MODE_L2_NORM_IGNORE_NAN, s);
+    return split_launch<SPLIT_GRAD>(q, sp, output_grad, input_grad, ws, p.mode == SIM_MODE_L2_NORM_IGNORE_NAN, s, g);
 }
 
 }  // namespace simnets

@@ -231,3 +231,29 @@ def test_split_parameter_gradients_keep_infinities(pkg, value, ones):
         assert torch.equal(got[inf].double(), ref[inf])
         err = (got.double() - ref)[~inf].norm() / ref[~inf].norm()
         assert float(err) <= 4 * math.sqrt(go.numel() // O) * 2.0 ** -24, float(err)
+
+
+@pytest.mark.parametrize("geom, where", [(GEOMS[1], "g"), (GEOMS[2], "g"), (GEOMS[1], "w")])
+def test_split_input_gradient_keeps_infinities(pkg, geom, where):
+    """One infinite output gradient, or weight: the input gradients that it reaches are infinite with the sign of their
+    term g w (t - x), whichever way the channel's centre lies."""
+    g = torch.Generator(device="cuda").manual_seed(41)
+    shape, O = geom["shape"], geom["O"]
+    x, t = torch.randn(shape, generator=g, device="cuda"), torch.randn((O, shape[1], 3, 3), generator=g, device="cuda")
+    w = t.abs() + 0.1
+    kw = options("l2", geom)
+    out = pkg.similarity(x, t, w, **kw).shape
+    go = torch.rand(tuple(out), generator=g, device="cuda") + 0.5
+    want = torch.zeros_like(x)
+    ph, pw = geom["padding"]
+    if where == "g":
+        go[3, 7, 11, 20] = float("inf")
+        r, c = 11 - ph, 20 - pw
+        want[3, :, r:r + 3, c:c + 3] = t[7] - x[3, :, r:r + 3, c:c + 3]
+    else:
+        w[7, 3, 1, 1] = float("inf")
+        want[:, 3] = t[7, 3, 1, 1] - x[:, 3]    # the padding lets the middle tap read every input pixel
+    dx = pkg.similarity_input_grad(x, t, w, go, **kw)
+    reached = want != 0
+    assert torch.equal(torch.isfinite(dx), ~reached)
+    assert torch.equal(dx[reached], torch.sign(want[reached]) * float("inf"))
