@@ -491,9 +491,10 @@ GxTiling gx_try(const SimPlan &p, const Phase &f, int PT, int nws, int MT = 8, b
     }
     // ... and so does a grid that would give the SIMDs at most one wave each (one image per wave then)
     const long long plain_waves = (long long)p.B * (((p.C + t.MT - 1) / t.MT + kWaves - 1) / kWaves) * kWaves;
-    if (MT != 8)
-        t.NI = 1;   // (the small-grid variant has the 4 x 8 lane tile)
-    t.ksplit = MT != 8 ? false : t.NI > 1 || (nws == 1 && t.tiles == 1 && t.gpi <= 64 && plain_waves <= 1024 && p.O >= kWaves &&
+    const bool small_tile = PT == 4 && MT == 8;   // the lane tile of the small-grid variant
+    if (!small_tile)
+        t.NI = 1;
+    t.ksplit = !small_tile ? false : t.NI > 1 || (nws == 1 && t.tiles == 1 && t.gpi <= 64 && plain_waves <= 1024 && p.O >= kWaves &&
                             1LL * t.TRmax * t.TC <= kStagePos * kThreads);
     if (wide_ksplit) {
         t.NI = 1;
@@ -548,12 +549,13 @@ GxTiling gx_tiling(const SimPlan &p, const Phase &f)
         if (t.lds_ok && !pick(4).ksplit)
             return t;
     }
-    // 8 x 8 lane tile for wide phase grids with many channels, if the grid then still gives every SIMD two waves
+    // 8 x 8 lane tile for wide phase grids with many channels, if the grid then still gives every SIMD two waves; not
+    // where it leaves half of a wave's lanes idle, which the 4 x 8 tile fills with the next images' pixels
     if (f.nb >= 32 && p.C >= 32) {
         const GxTiling big = pick(8);
         const int n_ctiles = (p.C + 7) / 8, nwm = kWaves / big.nws;
         const long long waves = (long long)p.B * big.tiles * ((n_ctiles + nwm - 1) / nwm) * kWaves;
-        if (big.lds_ok && waves >= 1536)
+        if (big.lds_ok && waves >= 1536 && 2 * big.gpi > 64)
             return big;
     }
     const GxTiling t = pick(4);
@@ -619,6 +621,8 @@ hipError_t gx_launch_phases(const GradXPhases &ph, int n, int PT, int MT, bool k
     if (ksplit && PT == 8) {
         if constexpr (MODE == GX_L1)
             hipLaunchKernelGGL((sim_grad_input_kernel<MODE, 8, 8, false, true>), grid, dim3(kThreads), lds_bytes, s, ph);
+        else
+            return hipErrorInvalidValue;   // gx_tiling gives the wide split form to L1 only
     } else if (ksplit)
         hipLaunchKernelGGL((sim_grad_input_kernel<MODE, 4, 8, true>), grid, dim3(kThreads), lds_bytes, s, ph);
     else if (MT == 4)

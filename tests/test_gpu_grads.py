@@ -79,6 +79,31 @@ def check_sim_grads(pkg, x, t, w, seed=99, strict=True, **kw):
     assert_grad_close(dw, want_dw, true_dw, "weights grad", strict)
 
 
+@pytest.mark.parametrize("func, algo", [("L1", None), ("L2", None), ("L2", "direct")])
+@pytest.mark.parametrize("shape, O", [((64, 256, 4, 32), 8), ((512, 32, 4, 32), 8), ((220, 40, 3, 33), 9), ((100, 128, 5, 61), 6)])
+def test_similarity_input_grad_wide_images_of_few_rows(pkg, shape, O, func, algo):
+    """Few rows of 32 columns and more, many channels, large batch: the wide lane tile would leave half of its lanes
+    without pixels (first three shapes: at most 32 groups of eight pixels an image; last: 40)."""
+    g = torch.Generator(device="cuda").manual_seed(43)
+    x = torch.randn(shape, generator=g, device="cuda")
+    t = torch.randn((O, shape[1], 3, 3), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") + 0.1
+    go = torch.randn((shape[0], O, *shape[2:]), generator=g, device="cuda")
+    dx = pkg.similarity_input_grad(x, t, w, go, similarity_function=func, blocks=[3, 3], strides=[1, 1], padding=[1, 1],
+                                   algo=algo)
+    xd = x.double().requires_grad_()
+    cols = torch.nn.functional.unfold(xd, 3, padding=1)
+    total = 0
+    for o in range(O):
+        d = cols - t[o].double().reshape(1, -1, 1)
+        term = d.abs() if func == "L1" else d * d
+        total = total - (go[:, o].double().flatten(1) * (w[o].double().reshape(1, -1, 1) * term).sum(1)).sum()
+    want, = torch.autograd.grad(total, xd)
+    # 9 O terms of random sign in 32 bits, the products form adding two sums of their size
+    err = (dx.double() - want).norm() / want.norm()
+    assert float(err) <= 2 * math.sqrt(9 * O) * 2.0 ** -24, float(err)
+
+
 # ---- the reference's own gradient test matrix (python/simnets/test/__init__.py:55-103, :143-154) ------------
 @pytest.mark.parametrize("strides", [[1, 1], [2, 2]])
 @pytest.mark.parametrize("blocks", [[1, 1], [3, 3]])
