@@ -257,3 +257,19 @@ def test_split_input_gradient_keeps_infinities(pkg, geom, where):
     reached = want != 0
     assert torch.equal(torch.isfinite(dx), ~reached)
     assert torch.equal(dx[reached], torch.sign(want[reached]) * float("inf"))
+
+
+@pytest.mark.parametrize("shape, O, depth", [((256, 16, 32, 32), 32, 48), ((32, 128, 28, 28), 128, 26)])
+def test_split_parameter_gradients_sum_of_the_output_gradient(pkg, shape, O, depth):
+    """x = 0 and t = +-1: the template gradients are +-2 G, and their error is that of G = sum g alone.  Its longest chain of
+    additions: 4 within sixteen values, 12 (7) of those per thread, 3 across threads, 21 + 8 (4 + 8) of the partial sums.
+    Each rounds by 0.3 ulp (root mean square; an ulp is on average 1.4 * 2^-24 of a value), of partial sums that grow like a
+    random walk: 0.4 * 2^-24 sqrt(depth / 2) of the total."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    t = torch.randn((O, shape[1], 3, 3), generator=g, device="cuda").sign()
+    go = torch.randn((shape[0], O, *shape[2:]), generator=g, device="cuda")
+    dt, _ = pkg.similarity_parameters_grad(torch.zeros(shape, device="cuda"), t, torch.ones_like(t), go, padding=[1, 1],
+                                           strides=[1, 1])
+    want = -2 * t.double() * go.double().sum((0, 2, 3))[:, None, None, None]
+    err = float((dt - want).norm() / want.norm())
+    assert err <= 2 * 0.4 * 2.0 ** -24 * math.sqrt(depth / 2), err
