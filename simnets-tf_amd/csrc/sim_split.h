@@ -46,7 +46,7 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
 struct SplitParamsPlan {
     bool on;
     int n_mtiles, m_groups, k_groups, TH, TW, rows, cols, pitch, chan, tiles_r, tiles_c, units, S, Opad, Kpad;
-    size_t partial, centres, ctr, packed, total;
+    size_t partial, centres, ctr, ctr64, spread, packed, total;
 };
 
 SplitParamsPlan sim_split_params_plan(const SimPlan &p);

@@ -1,6 +1,6 @@
 // Parameter gradients of the L2 Similarity modes on the bf16 matrix cores, at the precision of fp32 (gfx950): the moments
 //   S1[o, k] = sum_px g[px, o] x'[px, k],   S2[o, k] = sum_px g[px, o] x'[px, k]^2,   x' = x - c, c one value per channel
-// (and G[o] = sum_px g) that the finish kernel of similarity_grad.hip combines, every factor as three 16-bit pieces and
+// or, where templates share a pattern, per patch element (and G[o] = sum_px g) that the finish kernel of similarity_grad.hip combines, every factor as three 16-bit pieces and
 // the six products of pieces that matter, as in similarity_split.hip; the leading one has accumulators of its own.
 //
 // The contraction runs over images and output pixels.  A lane's eight values of a matrix operand are eight images at one
@@ -38,7 +38,9 @@ constexpr int kImages = 8;           // images of a matrix operand
 struct ParamsArgs {
     const float *g, *x, *templates;
     bf16x8 *packed;      // g: [mtile][unit][pixel pair][piece][64 lanes]
-    float *partial, *centres, *ctr;   // [2 S1, S2; 2: G][S][Opad][Kpad]; [Opad][Kpad]; [C]
+    float *partial, *centres;   // [2 S1, S2; 2: G][S][Opad][Kpad]; [Opad][Kpad] what was subtracted, for the finish kernel
+    float *ctr, *ctr64;         // centres: [C], and [64 templates][Kpad]
+    float2 *spread;             // [Kpad] sum of the squares of t about the channel's centre and about the 64 templates' own
     int B, C, H, W, O, K, oh, ow, bh, bw, sh, sw, ph, pw, taps;
     int Opad, Kpad, S, n_mtiles;
     int TH, TW, pairs;   // output tile; TH * TW / 2 pixel pairs
@@ -65,26 +67,65 @@ __device__ __forceinline__ Unit unit_of(const ParamsArgs &a, int u)
 
 __device__ __forceinline__ int first_unit(const ParamsArgs &a, int s) { return (int)((long long)s * a.units / a.S); }
 
-// Blocks 0 .. S n_mtiles - 1: g of one share of the pixels and one template tile, a thread one template's pairs of pixels
-// (eight neighbouring threads read 64 contiguous bytes), and the share's sums G.  The blocks behind: the centres of 16
-// channels each.
-__global__ __launch_bounds__(kThreads) void sim_split_params_pack_kernel(const ParamsArgs a, const SplitPack pk)
+// One channel's centre, the mean of its template elements (any value is correct); its patch elements' centres, the mean
+// over each 64 templates, and how far the templates lie from the two.
+__device__ __forceinline__ void params_channel_block(const ParamsArgs &a, int c)
 {
-    const int tid = threadIdx.x;
-    int block = blockIdx.x;
-    if (block >= a.S * a.n_mtiles) {
-        const int c = (block - a.S * a.n_mtiles) * 16 + (tid >> 4);
-        const float centre = split_centre(pk, split_centre_part(pk, c));
-        if (c >= a.C)
-            return;
-        if ((tid & 15) == 0)
-            a.ctr[c] = centre;
-        for (int i = tid & 15; i < a.O * a.taps; i += 16) {
-            const int o = (int)fast_div((unsigned)i, a.d_taps);
-            a.centres[(size_t)o * a.Kpad + c * a.taps + (i - o * a.taps)] = centre;
+    __shared__ float wave_sum[kThreads / 64];
+    const int tid = threadIdx.x, n = a.O * a.taps, l8 = tid & 7;
+    float sum = 0.0f;
+#pragma unroll 4
+    for (int i = tid; i < n; i += kThreads) {
+        const int o = (int)fast_div((unsigned)i, a.d_taps);
+        sum += a.templates[((size_t)o * a.C + c) * a.taps + (i - o * a.taps)];
+    }
+    for (int d = 32; d > 0; d >>= 1)
+        sum += __shfl_xor(sum, d, 64);
+    if ((tid & 63) == 0)
+        wave_sum[tid >> 6] = sum;
+    __syncthreads();
+    sum = ((wave_sum[0] + wave_sum[1]) + (wave_sum[2] + wave_sum[3])) / (float)n;
+    const float centre = __builtin_fabsf(sum) < 1e18f ? sum : 0.0f;
+    if (tid == 0)
+        a.ctr[c] = centre;
+    for (int tap = tid >> 3; tap < a.taps; tap += kThreads / 8) {   // eight lanes to a patch element
+        const int k = c * a.taps + tap;
+        float2 spread = make_float2(0.0f, 0.0f);
+        for (int o0 = 0; o0 < a.O; o0 += 64) {
+            float t[8], s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                t[i] = a.templates[((size_t)min(o0 + 8 * i + l8, a.O - 1) * a.C + c) * a.taps + tap] - centre;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                t[i] = o0 + 8 * i + l8 < a.O ? t[i] : 0.0f;
+                s1 += t[i];
+                s2 += t[i] * t[i];
+            }
+            for (int d = 4; d > 0; d >>= 1) {
+                s1 += __shfl_xor(s1, d, 8);
+                s2 += __shfl_xor(s2, d, 8);
+            }
+            const float mean = s1 / (float)min(64, a.O - o0);
+            if (l8 == 0)
+                a.ctr64[(size_t)(o0 / 64) * a.Kpad + k] = __builtin_fabsf(centre + mean) < 1e18f ? centre + mean : 0.0f;
+            spread.x += s2;
+            spread.y += s2 - s1 * mean;
         }
+        if (l8 == 0)
+            a.spread[k] = spread;
+    }
+}
+
+// The first C blocks: params_channel_block.  The S n_mtiles behind: g of one share of the pixels and one template tile, a
+// thread one template's pairs of pixels (eight neighbouring threads read 64 contiguous bytes), and the share's sums G.
+__global__ __launch_bounds__(kThreads) void sim_split_params_pack_kernel(const ParamsArgs a)
+{
+    if ((int)blockIdx.x < a.C) {
+        params_channel_block(a, blockIdx.x);
         return;
     }
+    const int tid = threadIdx.x, block = blockIdx.x - a.C;
     const int mtile = block / a.S, s = block - mtile * a.S;
     const int row = tid >> 3, o = mtile * kSplitRows + row;
     const int q0 = first_unit(a, s) * a.pairs, q1 = first_unit(a, s + 1) * a.pairs;
@@ -128,6 +169,25 @@ __global__ __launch_bounds__(kThreads) void sim_split_params_pack_kernel(const P
         sum += __shfl_xor(sum, d, 8);
     if ((tid & 7) == 0 && o < a.O)
         a.partial[((size_t)2 * a.S + s) * a.Opad * a.Kpad + (size_t)o * a.Kpad] = sum;
+}
+
+// This share's sums of one patch element k and a lane's sixteen templates; with the first share what was subtracted.
+__device__ __forceinline__ void params_store(const ParamsArgs &a, int mtile, int k, int s, int half, float centre,
+                                             const f32x16 &hi2, const f32x16 &lo2, const f32x16 &hi1, const f32x16 &lo1)
+{
+    const size_t slab = (size_t)a.Opad * a.Kpad;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int o = mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4;
+        if (o >= a.O)
+            continue;
+        const size_t at = (size_t)o * a.Kpad + k;
+        float *dst = a.partial + (size_t)s * slab + at;
+        dst[0] = split_sum(hi1[r], lo1[r]);
+        dst[(size_t)a.S * slab] = split_sum(hi2[r], lo2[r]);
+        if (s == 0)
+            a.centres[at] = centre;
+    }
 }
 
 // G template tiles from mtile0 x 64 patch elements; a wave holds one template tile x NI column tiles.
@@ -267,17 +327,126 @@ __device__ __forceinline__ void params_body(const ParamsArgs &a, char *lds, int 
         const int k = k0 + ((wave / G) * NI + i) * 32 + col;
         if (k >= a.K)
             continue;
+        params_store(a, mtile, k, s, half, a.ctr[(int)fast_div((unsigned)k, a.d_taps)], hi[0][i], lo[0][i], hi[1][i], lo[1][i]);
+    }
+}
+
+// The same for 64 patch elements whose templates lie far from their channel's centre and near one another (whole-image
+// patches, templates that began as one prototype): there S2 - 2 t' S1 + t'^2 G, t' = t - c, cancels, by 3e-4 of the
+// gradient where what the templates share is 30 times what they differ by.  Centred element by element, over the 64
+// templates of two tiles, t' is that difference.  A pixel that several taps read then needs a value for each, so a slot
+// of LDS holds one patch element at one pixel: ten pixels at a time, staged for every 64 templates.  The gradients of
+// 64 x 16 x 32 x 32, 64 templates, 4 x 4 at stride 4 take 21 us (one centre to a channel: 22, the fp32 form: 33) and have
+// 1.0e-7 of error whatever is shared (fp32 form: 1.4e-7); 32 x 128 x 28 x 28, 128 templates, 3 x 3: 188 us (111, 212).
+constexpr int kElemPairs = 5, kElemPitch = 2 * kElemPairs + 1;   // odd: see the note on pitches
+
+__device__ __forceinline__ void params_elements_body(const ParamsArgs &a, char *lds, int mtile0)
+{
+    constexpr int kPlane = kSlots * 16;
+    constexpr int kUsed = kColumns * kElemPitch, kItems = (kUsed + kThreads - 1) / kThreads;
+    static_assert(kUsed <= kSlots, "a slot for every element and pixel");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    const int mtile = mtile0 + (wave & 1), kcol = (wave >> 1) * 32 + col;
+    const bool active = mtile < a.n_mtiles;
+    const int k0 = blockIdx.y * kColumns, s = blockIdx.x;
+    const int u0 = first_unit(a, s), u1 = first_unit(a, s + 1);
+    const float *centres = a.ctr64 + (size_t)(mtile0 / 2) * a.Kpad;
+
+    // this thread's slots: patch element (tap and channel) and pixel of the ten (-1: none)
+    int src[kItems], tap[kItems], pos[kItems];
+    float ctr[kItems];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int o = mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4;
-            if (o >= a.O)
-                continue;
-            const size_t slab = (size_t)a.Opad * a.Kpad;
-            float *dst = a.partial + (size_t)s * slab + (size_t)o * a.Kpad + k;
-            dst[0] = split_sum(hi[1][i][r], lo[1][i][r]);
-            dst[(size_t)a.S * slab] = split_sum(hi[0][i][r], lo[0][i][r]);
+    for (int i = 0; i < kItems; ++i) {
+        const int e = tid + i * kThreads, kl = e / kElemPitch, k = min(k0 + kl, a.K - 1);
+        const int c = (int)fast_div((unsigned)k, a.d_taps), t = k - c * a.taps, dh = t / a.bw;
+        pos[i] = e < kUsed && e - kl * kElemPitch < 2 * kElemPairs ? e - kl * kElemPitch : -1;
+        tap[i] = dh << 16 | (t - dh * a.bw);
+        src[i] = c * a.H * a.W;
+        ctr[i] = centres[k];
+    }
+    f32x16 hi[2], lo[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        hi[f] = 0.0f;
+        lo[f] = 0.0f;
+    }
+    const bf16x8 *pp = a.packed + ((size_t)(active ? mtile : 0) * a.units + u0) * a.pairs * 192 + lane;
+    const size_t image = (size_t)a.C * a.H * a.W;
+    for (int u = u0; u < u1; ++u) {
+        const Unit un = unit_of(a, u);
+        for (int q0 = 0; q0 < a.pairs; q0 += kElemPairs) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kItems; ++i) {
+                if (pos[i] < 0)
+                    continue;
+                const int q = q0 + (pos[i] >> 1), py = (int)fast_div((unsigned)q, a.d_tw2);
+                const int ro = un.r0 + py, co = un.c0 + 2 * (q - py * (a.TW / 2)) + (pos[i] & 1);
+                const int r = ro * a.sh - a.ph + (tap[i] >> 16), c = co * a.sw - a.pw + (tap[i] & 0xffff);
+                const bool in = r >= 0 && r < a.H && c >= 0 && c < a.W, there = q < a.pairs && ro < a.oh && co < a.ow;
+                const float *p = a.x + (size_t)un.img * image + src[i] + (ptrdiff_t)r * a.W + c;
+                float x[kImages];
+#pragma unroll
+                for (int j = 0; j < kImages; ++j)
+                    x[j] = in && there && un.img + j < a.B ? p[j * image] : a.oob;
+                bf16x8 v[6];
+#pragma unroll
+                for (int j = 0; j < kImages; ++j) {
+                    const float d = there && un.img + j < a.B ? x[j] - ctr[i] : 0.0f;
+                    __bf16 p0, p1, p2;
+                    split3_any(d * d, p0, p1, p2);
+                    v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
+                    split3_any(d, p0, p1, p2);
+                    v[3][j] = p0; v[4][j] = p1; v[5][j] = p2;
+                }
+#pragma unroll
+                for (int b = 0; b < 6; ++b)
+                    *reinterpret_cast<bf16x8 *>(lds + b * kPlane + (tid + i * kThreads) * 16) = v[b];
+            }
+            __syncthreads();
+            const int n = min(kElemPairs, a.pairs - q0);
+            for (int j = 0; j < n; ++j, pp += 192) {
+                bf16x8 A[3], B[6];
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    A[i] = pp[i * 64];
+#pragma unroll
+                for (int b = 0; b < 6; ++b)
+                    B[b] = *reinterpret_cast<const bf16x8 *>(lds + b * kPlane + (kcol * kElemPitch + 2 * j + half) * 16);
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    auto mul = [&](f32x16 &acc, int x, int y) {
+                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[x], B[3 * f + y], acc, 0, 0, 0);
+                    };
+                    mul(lo[f], 2, 0);
+                    mul(lo[f], 0, 2);
+                    mul(hi[f], 0, 0);
+                    mul(lo[f], 1, 1);
+                    mul(lo[f], 1, 0);
+                    mul(lo[f], 0, 1);
+                }
+            }
         }
     }
+    if (active && k0 + kcol < a.K)
+        params_store(a, mtile, k0 + kcol, s, half, centres[k0 + kcol], hi[0], lo[0], hi[1], lo[1]);
+}
+
+// Whether these 64 patch elements' templates lie further from their channels' centres than the fp32 form, which centres
+// each 64 templates element by element, would leave them: by a tenth of the sum of squares.  There the two forms' errors
+// are equal (64 x 16 x 32 x 32, 64 templates, 4 x 4 at stride 4: 1.3e-7 and 1.4e-7; at twice the sum 4.1e-7 and 1.4e-7);
+// templates without a common part stay below (1 + 1/24 on average with 24 of them, fewer do not come here).
+__device__ __forceinline__ bool params_elements(const ParamsArgs &a)
+{
+    const int k = blockIdx.y * kColumns + (threadIdx.x & 63);
+    float2 v = k < a.K ? a.spread[k] : make_float2(0.0f, 0.0f);
+    for (int d = 32; d > 0; d >>= 1) {
+        v.x += __shfl_xor(v.x, d, 64);
+        v.y += __shfl_xor(v.y, d, 64);
+    }
+    return __builtin_amdgcn_readfirstlane(!(v.x <= 1.1f * v.y));
 }
 
 // blockIdx: (share of the pixels, 64 patch elements, template tiles dealt out as groups of 4, the rest as one of 4, 2 or 1)
@@ -285,6 +454,11 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_params_kernel(const Par
 {
     __shared__ __align__(16) char lds[kSlots * 16 * 6];
     const int mtile0 = blockIdx.z * 4, rest = a.n_mtiles - mtile0;
+    if (params_elements(a)) {
+        for (int two = 0; two < min(rest, 4); two += 2)
+            params_elements_body(a, lds, mtile0 + two);
+        return;
+    }
     const int g = rest >= 3 ? 4 : rest;
     if (g == 4)
         params_body<4>(a, lds, mtile0);
@@ -356,7 +530,9 @@ SplitParamsPlan sim_split_params_plan(const SimPlan &p)
     s.partial = 0;
     s.centres = 3 * (size_t)s.S * slab;    // where the finish kernel reads them
     s.ctr = s.centres + slab;
-    s.packed = s.ctr + align_up((size_t)p.C * sizeof(float), 256);
+    s.ctr64 = s.ctr + align_up((size_t)p.C * sizeof(float), 256);
+    s.spread = s.ctr64 + (size_t)(s.n_mtiles + 1) / 2 * s.Kpad * sizeof(float);
+    s.packed = s.spread + (size_t)s.Kpad * sizeof(float2);
     s.total = s.packed + (size_t)packed;
     s.on = true;
     return s;
@@ -371,6 +547,8 @@ int sim_split_params_launch(const SimPlan &p, const SplitParamsPlan &sp, const f
     a.partial = reinterpret_cast<float *>(ws + sp.partial);
     a.centres = reinterpret_cast<float *>(ws + sp.centres);
     a.ctr = reinterpret_cast<float *>(ws + sp.ctr);
+    a.ctr64 = reinterpret_cast<float *>(ws + sp.ctr64);
+    a.spread = reinterpret_cast<float2 *>(ws + sp.spread);
     a.B = p.B; a.C = p.C; a.H = p.H; a.W = p.W; a.O = p.O; a.K = p.K; a.oh = p.oh; a.ow = p.ow;
     a.bh = p.bh; a.bw = p.bw; a.sh = p.sh; a.sw = p.sw; a.ph = p.ph; a.pw = p.pw; a.taps = p.bh * p.bw;
     a.Opad = sp.Opad; a.Kpad = sp.Kpad; a.S = sp.S; a.n_mtiles = sp.n_mtiles;
@@ -385,9 +563,7 @@ int sim_split_params_launch(const SimPlan &p, const SplitParamsPlan &sp, const f
     a.d_chan = make_fast_div((unsigned)sp.chan);
     a.d_pitch = make_fast_div((unsigned)sp.pitch);
     a.d_taps = make_fast_div((unsigned)a.taps);
-    SplitPack pk = {};
-    pk.templates = templates; pk.O = p.O; pk.C = p.C; pk.taps = a.taps;
-    hipLaunchKernelGGL(sim_split_params_pack_kernel, dim3(sp.S * sp.n_mtiles + (p.C + 15) / 16), dim3(kThreads), 0, s, a, pk);
+    hipLaunchKernelGGL(sim_split_params_pack_kernel, dim3(p.C + sp.S * sp.n_mtiles), dim3(kThreads), 0, s, a);
     hipLaunchKernelGGL(sim_split_params_kernel, dim3(sp.S, sp.k_groups, sp.m_groups), dim3(kThreads), 0, s, a);
     return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
 }

@@ -1,5 +1,6 @@
 """The L2 Similarity modes on the matrix cores in 16-bit pieces (csrc/similarity_split.hip): edges of its tiles, its three
 modes, both chunk sizes, and what its guard hands to the term-by-term kernel.  Reference: torch in 64 bits."""
+import ctypes
 import math
 
 import numpy as np
@@ -34,6 +35,27 @@ def options(mode, g):
     if mode == "missing":
         kw.update(ignore_nan_input=True, out_of_bounds_value=float("nan"))
     return kw
+
+
+def pieces_used(pkg, shape, O, mode="l2", **kw):
+    """Which of the operator's calls take the form in 16-bit pieces on this geometry, from their workspaces: those of the
+    forms that can be asked for by name are of another size."""
+    def sizes(algo, **options):
+        attrs, i4 = pkg.ops.similarity_attrs(algo=algo, **options), ctypes.c_int * 4
+        x, t = i4(*shape), i4(O, shape[1], *options["blocks"])
+        n = [ctypes.c_size_t() for _ in range(3)]
+        assert lib.simnets_hip_similarity_workspace_bytes(ctypes.byref(attrs), x, t, ctypes.byref(n[0])) == 0
+        assert lib.simnets_hip_similarity_grad_workspace_bytes(ctypes.byref(attrs), x, t, ctypes.byref(n[1]),
+                                                               ctypes.byref(n[2])) == 0
+        return [v.value for v in n]
+    lib = pkg._lib.lib()
+    kw = {k: v for k, v in kw.items() if k in ("blocks", "strides", "padding")}
+    norm = dict(normalization_term=mode != "l2", ignore_nan_input=mode == "missing")
+    named = [sizes(algo, **kw, **norm) for algo in (["direct", "sqrtw"] if mode == "l2" else ["direct"])]
+    # (the gradients' geometry rules are the same for all L2 modes)
+    grads, fp32 = sizes(None, **kw), sizes("sqrtw", **kw)
+    return dict(forward=all(sizes(None, **kw, **norm)[0] != n[0] for n in named), input=grads[1] != fp32[1],
+                params=grads[2] != fp32[2] and mode != "missing")
 
 
 GEOMS = [
@@ -273,3 +295,39 @@ def test_split_parameter_gradients_sum_of_the_output_gradient(pkg, shape, O, dep
     want = -2 * t.double() * go.double().sum((0, 2, 3))[:, None, None, None]
     err = float((dt - want).norm() / want.norm())
     assert err <= 2 * 0.4 * 2.0 ** -24 * math.sqrt(depth / 2), err
+
+
+@pytest.mark.parametrize("spread", [0.3, 0.1, 0.01])
+@pytest.mark.parametrize("shape, O, blocks, strides, padding", [
+    ((64, 16, 32, 32), 64, [4, 4], [4, 4], [0, 0]),
+    ((70, 5, 24, 37), 200, [4, 4], [4, 4], [0, 0]),     # ragged everywhere; 4 + 3 tiles, one and a quarter groups of 64
+    ((233, 40, 22, 21), 33, [2, 2], [2, 2], [0, 0]),    # one template in the second tile
+    ((64, 12, 37, 38), 129, [3, 3], [3, 3], [3, 0]),    # out-of-bounds rows, 4 + 1 tiles
+    ((500, 70, 3, 4), 64, [3, 3], [1, 1], [0, 0]),      # nearly whole images
+])
+def test_split_parameter_gradients_of_templates_that_share_a_pattern(pkg, shape, O, blocks, strides, padding, spread):
+    """Templates, and patches, that are one pattern of size 1 plus differences of size `spread`: the gradients come from the
+    differences, and are as exact as those of templates without a pattern (the bound of test_split_gradients_match_64_bits)."""
+    g = torch.Generator(device="cuda").manual_seed(47)
+    B, C, H, W = shape
+    bh, bw = blocks
+    pattern = torch.randn((1, C, bh, bw), generator=g, device="cuda")
+    t = pattern + spread * torch.randn((O, C, bh, bw), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    tiled = pattern.repeat(1, 1, H // bh + 2, W // bw + 2)
+    at = [padding[0] % bh, padding[1] % bw]    # where the first pixel lies in its block
+    x = tiled[:, :, at[0]:at[0] + H, at[1]:at[1] + W] + spread * torch.randn(shape, generator=g, device="cuda")
+    kw = dict(blocks=blocks, strides=strides, padding=padding)
+    assert pieces_used(pkg, shape, O, **kw)["params"]
+    xp = torch.nn.functional.pad(x.double(), (padding[1],) * 2 + (padding[0],) * 2)
+    cols = xp.unfold(2, bh, strides[0]).unfold(3, bw, strides[1])
+    oh, ow = cols.shape[2:4]
+    cols = cols.permute(0, 2, 3, 1, 4, 5).reshape(B * oh * ow, -1) - pattern.double().flatten()
+    td = t.double().flatten(1) - pattern.double().flatten()
+    go = torch.randn((B, O, oh, ow), generator=g, device="cuda")
+    gd = go.double().permute(1, 0, 2, 3).reshape(O, -1)
+    s1, s2, s0 = gd @ cols, gd @ (cols * cols), gd.sum(1, keepdim=True)
+    want = (2 * w.double().flatten(1) * (s1 - td * s0), -(s2 - 2 * td * s1 + td * td * s0))
+    for got, ref in zip(pkg.similarity_parameters_grad(x, t, w, go, **kw), want):
+        err = (got.double().flatten(1) - ref).norm() / ref.norm()
+        assert float(err) <= 4 * math.sqrt(B * oh * ow) * 2.0 ** -24, float(err)
