@@ -12,6 +12,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kSplitPixels = 128;   // output pixels of a workgroup, consecutive over the whole batch
 constexpr int kSplitRows = 32;      // templates of one matrix tile
+constexpr float kSplitLead = 0.125f;   // of sum w t'^2, added to an output's sum in advance and taken off at its end
 constexpr int kSplitMaxC = 4096;    // channels whose centres the packing kernel keeps in LDS
 
 // Geometry of one call on the split form.
@@ -35,6 +36,7 @@ struct SplitPack {
     float *ctr, *bias, *lg, *thr;
     int O, C, taps, K, cg, chunks, steps, pieces, n_mtiles, mode;
     float fudge, norm_const;
+    float line;   // outputs below `line` times sum w t'^2 are left to the term-by-term kernel
     int pack_blocks, thr_blocks;   // pack_blocks = chunks * n_mtiles * ceil(steps / 4)
 };
 
@@ -215,11 +217,11 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
             tc2 = (sums[0] + sums[3]) + (sums[6] + sums[9]);
             traw = (sums[1] + sums[4]) + (sums[7] + sums[10]);
             lsum = (sums[2] + sums[5]) + (sums[8] + sums[11]);
-            a.bias[m] = masked ? 0.0f : -(float)tc2;
+            a.bias[m] = masked ? 0.0f : (float)(-(1.0 + kSplitLead) * tc2);
             a.lg[m] = masked || a.mode == SIM_MODE_L2 ? 0.0f : (float)(lsum + (double)a.norm_const);
             double thr = 0x1p-60;
             if (!masked)
-                thr = fmax(thr, fmax(0.25 * tc2, traw / 1024.0));
+                thr = fmax(thr, fmax((double)a.line * tc2, traw / 1024.0));
             a.thr[m] = bad || !(thr < 1e37) ? INFINITY : (float)thr;
         }
         __syncthreads();

@@ -6,17 +6,22 @@
 // 32-bit matrix instruction does two terms in 64 cycles where six of these do sixteen in 192 - 2.7 times the rate, and
 // 2.7 times the vector units' two instructions per term.
 //
-// Precision.  The leading product of the squares has accumulators of its own, so an output's sum is rounded K / 16 times
-// at its own size instead of K times in a term-by-term sum; the others, of random sign or 2^-8 of it, share a second
-// set.  Error against 64 bits (2-norm, relative): 256 x 64 x 32 x 32 -> 128, 3 x 3, 0.9e-7 where the term-by-term forms have
-// 3.6e-7; 64 x 250 x 12 x 12 -> 195 1.4e-7 against 7.0e-7.  What cancellation between the three sums costs is bounded by a guard: with T = sum w t'^2,
-// an output of at least T / 4 has sum w (|x'| + |t'|)^2 <= 25 times itself (sqrt(sum w x'^2) <= sqrt(out) + sqrt(T)).
-// A tile with an output below that (or below 1/1024 of the uncentred sum w t^2, the guard of the sqrt-weight form; or
+// Precision.  The two leading products (squares, cross terms) have accumulators of their own, so that an output's sum is
+// rounded K / 8 times at its own size; the lesser ones, 2^-8 of that, share a second set.  The sum begins with an eighth
+// of T = sum w t'^2, against which an unrelated input's sum - w x'^2 runs, and ends with the rest of T taken off; what the
+// last addition rounds is carried.  Inputs unrelated to the templates (error against 64 bits, 2-norm, relative): 256 x 64 x 32 x
+// 32 -> 128, 3 x 3, 0.8e-7 where the term-by-term forms have 3.6e-7; 32 x 128 x 28 x 28 -> 128 1.0e-7 against 5.1e-7.  Inputs near
+// a template lose to cancellation: the sum passes through T - out, and its error grows as T / out.  A patch at out / T = 2, 1
+// and 0.5 from its template, 576 elements: 0.8e-7, 0.6e-7 and 3.3e-7 (root mean square; term by term 3.6e-7), 2304: 1.4e-7,
+// 0.9e-7, 5.5e-7 (7.7e-7), 72: 0.5e-7, 0.6e-7, 1.3e-7 (1.3e-7).  The guard's line lies where the two are equal, at 0.43 T (half
+// for the shortest patches, split_line); with the cross terms' leading product among the lesser ones, eleven roundings of
+// it to a step, it was 1.6e-6 at 0.5 and 576 elements, and 4.4e-7 at 2.
+// A tile with an output below the line (or below 1/1024 of the uncentred sum w t^2, the guard of the sqrt-weight form; or
 // not finite; or of a template whose parameters are negative, huge or tiny) is flagged and computed again, term by
 // term, by the direct kernel's launch behind this one, which otherwise returns at once.
 //
 // Missing values (NaN inputs ignored): x' = 0 and a third operand, the 0/1 mask of present values (exact in 16 bits),
-// contracts with -w t'^2 and with the logarithm term, three pieces each.
+// contracts with -w t'^2 and with the logarithm term, three pieces each; T is that of the present values.
 //
 // Layout.  A workgroup of four waves computes 128 consecutive output pixels (over the batch: images are a stack of
 // padded rows, so a tile may span images and no lane idles at an image's end) x up to 128 templates.  16 channels (or
@@ -64,6 +69,7 @@ struct SplitArgs {
     int bw, sh, sw, ph, pw, taps, chunks, steps, n_mtiles, Wp, Hv;
     int gmax;        // matrix tiles of templates per workgroup: 4, 2 or 1
     float oob;
+    float line;      // missing values: an output has to reach this times its present sum w t'^2
     const float *x;  // input gradient: the forward's input, of the output's shape; templates and weights [C][O][taps]
     const float *templates, *weights;
     float scale;
@@ -94,11 +100,18 @@ __device__ __noinline__ float split_grad_terms(int img, int ch, int rem, float x
 static_assert(sizeof(SplitArgs) % 8 == 0, "the explicit arguments end 8 bytes behind the block");
 #endif
 
+// a + b + c, |c| the smallest, rounded about once: what the rounding of a + b loses is added to c.
+__device__ __forceinline__ float split_three(float a, float b, float c)
+{
+    const float sum = a + b, of_b = sum - a;
+    return sum + (c + ((a - (sum - of_b)) + (b - of_b)));
+}
+
 // One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
 template <int KIND, int CG, int G>
 __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mtile0, int flag)
 {
-    constexpr bool MASKED = KIND == SPLIT_MASKED, GRAD = KIND == SPLIT_GRAD;
+    constexpr bool MASKED = KIND == SPLIT_MASKED, GRAD = KIND == SPLIT_GRAD, WHOLE = KIND == SPLIT_FWD;
     constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND);
     constexpr int P = split_lds_pixels(KIND) * (CG == 16 ? 1 : 2);   // pixels of one plane [channel group][pixel]
     constexpr int kPlane = split_lds_pixels(KIND) * 32;
@@ -206,6 +219,16 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mt
             }
         }
         __syncthreads();
+        if (WHOLE && chunk == 0) {   // the sums begin with kSplitLead sum w t'^2
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float lead = a.bias[(active ? mtile : 0) * kSplitRows + 8 * (r / 4) + 4 * half + r % 4] *
+                                   -(kSplitLead / (1.0f + kSplitLead));
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    hi[i][r] = lead;
+            }
+        }
         int dh = 0, dw = 0;
         auto next_tap = [&]() {   // LDS offset of the tap (behind the last: of the first, with zero parameters)
             const int off = (dh * a.Wp + dw) * 16;
@@ -256,7 +279,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mt
                 for (int f = 0; f < 6; f += 3) {
                     mul(lo[i], A[f + 2], B[f]);
                     mul(lo[i], A[f], B[f + 2]);
-                    mul(f == 0 ? hi[i] : lo[i], A[f], B[f]);
+                    mul(hi[i], A[f], B[f]);
                     mul(lo[i], A[f + 1], B[f + 1]);
                     mul(lo[i], A[f + 1], B[f]);
                     mul(lo[i], A[f], B[f + 1]);
@@ -346,14 +369,14 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mt
                     continue;
                 float v;
                 if (MASKED) {
-                    v = (hi[i][r] + tm[i][r]) + lo[i][r];
+                    v = split_three(hi[i][r], tm[i][r], lo[i][r]);
                     const float mag = __builtin_fabsf(v);
-                    const bool fine = mag < 1e37f && mag >= -0.25f * tm[i][r] &&
+                    const bool fine = mag < 1e37f && mag >= a.line * -tm[i][r] &&
                                       (mag >= thr[r] || (v == 0.0f && tm[i][r] == 0.0f && thr[r] < 1e37f));
                     bad |= !fine;
                     v = 0.5f * v + lg[i][r];
                 } else {
-                    v = (hi[i][r] + bias[r]) + lo[i][r];
+                    v = split_three(hi[i][r], bias[r], lo[i][r]);
                     const float mag = __builtin_fabsf(v);
                     bad |= !(mag >= thr[r] && mag < 1e37f);
                     if (norm)
@@ -454,6 +477,10 @@ __global__ __launch_bounds__(kThreads) void sim_split_grad_pack_kernel(const Spl
 
 }  // namespace
 
+// The guard's line as a share of sum w t'^2: where this form's error (see the head of the file) is that of the sum it
+// stands for, term by term or with square roots of the weights.  Its last roundings weigh more in a short sum.
+static float split_line(int K) { return K < 128 ? 0.5f : 0.43f; }
+
 // Chunks, tiles and workspace of the contraction that `p` describes, with `kind`'s operands; .on if it fits and is worth
 // while.
 static SplitPlan split_geometry(const SimPlan &p, int kind)
@@ -525,6 +552,7 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     a.thr = reinterpret_cast<float *>(ws + sp.thr);
     a.O = p.O; a.C = p.C; a.taps = p.bh * p.bw; a.K = p.K; a.cg = sp.cg; a.chunks = sp.chunks; a.steps = sp.steps;
     a.pieces = sp.pieces; a.n_mtiles = sp.n_mtiles; a.mode = p.mode; a.fudge = p.fudge;
+    a.line = split_line(p.K);
     a.norm_const = p.mode == SIM_MODE_L2_NORM ? (float)((double)(-0.5f * (float)p.K) * std::log(2.0 * M_PI)) : 0.0f;
     a.pack_blocks = sp.on ? sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4) : 0;
     a.thr_blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows, 512) : 0;
@@ -546,6 +574,7 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     a.bw = p.bw; a.sh = p.sh; a.sw = p.sw; a.ph = p.ph; a.pw = p.pw; a.taps = p.bh * p.bw;
     a.chunks = sp.chunks; a.steps = sp.steps; a.n_mtiles = sp.n_mtiles; a.Wp = sp.Wp; a.Hv = sp.Hv;
     a.oob = p.oob;
+    a.line = split_line(p.K);
     a.d_npix = make_fast_div((unsigned)a.npix);
     a.d_ow = make_fast_div((unsigned)p.ow);
     a.d_wp = make_fast_div((unsigned)sp.Wp);

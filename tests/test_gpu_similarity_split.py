@@ -331,3 +331,35 @@ def test_split_parameter_gradients_of_templates_that_share_a_pattern(pkg, shape,
     for got, ref in zip(pkg.similarity_parameters_grad(x, t, w, go, **kw), want):
         err = (got.double().flatten(1) - ref).norm() / ref.norm()
         assert float(err) <= 4 * math.sqrt(B * oh * ow) * 2.0 ** -24, float(err)
+
+
+@pytest.mark.parametrize("mode", ["l2", "missing"])
+@pytest.mark.parametrize("ratio", [2.0, 1.0, 0.5, 0.3])
+@pytest.mark.parametrize("C, block", [(64, 3), (20, 3), (64, 1)])
+def test_split_form_near_a_template(pkg, C, block, ratio, mode):
+    """Outputs at a given share of sum w t^2, on either side of the guard's line: no further from the 64-bit value than the
+    term-by-term sum, K additions of which each rounds by 0.4 * 2^-24 of a partial sum (root mean square, as in
+    test_split_parameter_gradients_sum_of_the_output_gradient): 0.4 * 2^-24 sqrt(K / 3) for terms of one sign."""
+    g = torch.Generator(device="cuda").manual_seed(53)
+    K, O, n = C * block * block, 64, 28 // block
+    shape = (16, C, n * block, n * block)
+    t = torch.randn((O, C, block, block), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    which = torch.randint(0, O, (shape[0], n, n), generator=g, device="cuda")
+    x = t[which].permute(0, 3, 1, 4, 2, 5).reshape(shape)
+    x = x + math.sqrt(ratio) * torch.randn(shape, generator=g, device="cuda")
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    kw = options(mode, dict(blocks=[block, block], strides=[1, 1], padding=[0, 0]))
+    assert pieces_used(pkg, shape, O, mode, **kw)["forward"]
+    if mode == "missing":   # weights at which the logarithm terms vanish: the distance alone
+        w = torch.full_like(w, 2 * math.pi - 0.001)
+    got = pkg.similarity(x, t, w, **kw)[:, :, ::block, ::block].gather(1, which[:, None])[:, 0].double()
+    cols = x.double().unfold(2, block, block).unfold(3, block, block).permute(0, 2, 3, 1, 4, 5)
+    d = torch.nan_to_num(cols - t.double()[which])
+    want = -(w.double()[which] * d * d).flatten(3).sum(-1) * (0.5 if mode == "missing" else 1.0)
+    if mode == "missing":
+        log = 0.5 * (torch.log(w.flatten()[:1].double() + 0.001) - math.log(2 * math.pi))
+        want = want + log * (cols == cols).flatten(3).sum(-1)
+    err = float((((got - want) / want) ** 2).mean().sqrt())
+    assert err <= 1.5 * 0.4 * 2.0 ** -24 * math.sqrt(K / 3), err
