@@ -67,10 +67,11 @@ enum { SIMNETS_SIM_L1 = 0, SIMNETS_SIM_L2 = 1 };
 /* How the weighted distance is evaluated.  All choices implement the same operator. */
 enum {
     SIMNETS_ALGO_AUTO = 0,   /* the L2 modes over patches of 64 elements and more: products of 16-bit pieces on the
-                                matrix cores, 24 bits of every factor, fp32 sums; tiles with an output below 0.43 (short
-                                patches: 0.5) of sum_k w (t - c)^2 (c: a centre per channel) or 1/1024 of sum_k w t^2,
-                                or not finite, are recomputed with DIRECT's arithmetic.  Elsewhere SQRTW for plain L2
-                                (no normalization term), DIRECT for every other mode */
+                                matrix cores, 24 bits of every factor, fp32 sums; outputs below 0.43 (short patches: 0.5)
+                                of sum_k w (t - c)^2 (c: a centre per channel) or 1/1024 of sum_k w t^2, or not finite, are
+                                summed again term by term (where there are many together, by DIRECT's kernel, whose sums
+                                of their neighbours are then taken, too).  Elsewhere SQRTW for plain L2 (no
+                                normalization term), DIRECT for every other mode */
     SIMNETS_ALGO_DIRECT = 1, /* d = t - x; acc += (-w*d)*d   (L1: acc += -w*|d|), NaN-capable, every mode */
     SIMNETS_ALGO_SQRTW = 2,  /* plain L2 only: d = sqrt(w)*t - sqrt(w)*x in one fma; acc += -d*d.  The rounding of d
                                 could exceed 4e-6 relative only for outputs closer to zero than sum_k w t^2 / 1024.

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "internal.h"
+#include "sim_step.h"
 
 namespace simnets {
 
@@ -25,7 +26,7 @@ struct SplitPlan {
     int n_mtiles; // ceil(O / 32)
     int n_ptiles; // ceil(B oh ow / 128)
     int Wp, Hv;   // columns of a staged row; rows of one image's staged stack
-    size_t packed, ctr, bias, lg, thr, flags, total;   // workspace, from its own start
+    size_t packed, ctr, bias, lg, thr, flags, exact, logs, total;   // workspace, from its own start
 };
 
 SplitPlan sim_split_plan(const SimPlan &p);
@@ -34,9 +35,11 @@ struct SplitPack {
     const float *templates, *weights;
     unsigned short *packed;
     float *ctr, *bias, *lg, *thr;
+    float2 *exact;   // [O][K] template and negative weight as the term-by-term kernels take them ...
+    float *logs;     // ... and the normalized modes' logarithm terms
     int O, C, taps, K, cg, chunks, steps, pieces, n_mtiles, mode;
     float fudge, norm_const;
-    float line;   // outputs below `line` times sum w t'^2 are left to the term-by-term kernel
+    float line;   // outputs below `line` times sum w t'^2 are recomputed term by term
     int pack_blocks, thr_blocks;   // pack_blocks = chunks * n_mtiles * ceil(steps / 4)
 };
 
@@ -111,10 +114,6 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
 {
     const int tid = threadIdx.x;
     const bool masked = a.mode == SIM_MODE_L2_NORM_IGNORE_NAN;
-    auto logterm = [&](float w) {   // as sim_pack_element's
-        return masked ? (float)(0.5 * ((double)logf(w + a.fudge) - 1.8378770664093453 /* log(2 pi) */))
-                      : 0.5f * logf(w + a.fudge);
-    };
     if (block < a.pack_blocks) {
         const int parts = (a.steps + 3) / 4;   // of a chunk's steps, four to a workgroup
         const int mtile = block / (a.chunks * parts), rest = block - mtile * a.chunks * parts;
@@ -142,8 +141,9 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
                     const size_t at = ((size_t)m * a.C + c) * a.taps + tap;
                     w = a.weights[at];
                     t = a.templates[at] - lds[cl];
+                    float unused0, unused1;
                     if (masked)
-                        l = logterm(w);
+                        sim_pack_element(a.mode, true, t, w, a.fudge, unused0, unused1, l);
                 }
                 __bf16 p0, p1, p2;
                 auto put = [&](int at, float value) {
@@ -186,19 +186,24 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
     double *sums = reinterpret_cast<double *>(lds + ((a.C + 15) / 16 * 16));   // [4 waves][3]
     for (int m = block - a.pack_blocks; m < a.n_mtiles * kSplitRows; m += a.thr_blocks) {
         double tc2 = 0.0, traw = 0.0, lsum = 0.0;
-        bool bad = false;
+        bool bad = false, weighted = false;
         if (m < a.O)
 #pragma unroll 4
             for (int k = tid; k < a.K; k += 256) {
                 const float t = a.templates[(size_t)m * a.K + k], w = a.weights[(size_t)m * a.K + k];
                 const float tc = t - lds[k / a.taps];
+                float2 tw;
+                float l;
+                sim_pack_element(a.mode, true, t, w, a.fudge, tw.x, tw.y, l);
+                a.exact[(size_t)m * a.K + k] = tw;
+                weighted |= w != 0.0f;
                 tc2 += (double)w * tc * tc;
                 traw += (double)w * t * t;
                 // weights and templates outside this range: the pieces of their products may leave the range of
                 // normal numbers, so such a template is left to the term-by-term kernel
                 bad |= !(w == 0.0f || (w >= 0x1p-60f && w <= 0x1p20f)) || !(__builtin_fabsf(t) <= 0x1p60f);
                 if (a.mode != SIM_MODE_L2) {
-                    const float l = logterm(w);
+                    a.logs[(size_t)m * a.K + k] = l;
                     lsum += l;
                     bad |= !(__builtin_fabsf(l) <= 1e6f);
                 }
@@ -213,13 +218,14 @@ __device__ inline void split_pack_block(const SplitPack &a, int block, float *ld
             mine[0] = tc2; mine[1] = traw; mine[2] = lsum;
         }
         bad = __syncthreads_or(bad);
+        weighted = __syncthreads_or(weighted);
         if (tid == 0) {
             tc2 = (sums[0] + sums[3]) + (sums[6] + sums[9]);
             traw = (sums[1] + sums[4]) + (sums[7] + sums[10]);
             lsum = (sums[2] + sums[5]) + (sums[8] + sums[11]);
             a.bias[m] = masked ? 0.0f : (float)(-(1.0 + kSplitLead) * tc2);
             a.lg[m] = masked || a.mode == SIM_MODE_L2 ? 0.0f : (float)(lsum + (double)a.norm_const);
-            double thr = 0x1p-60;
+            double thr = weighted ? 0x1p-60 : 0.0;   // without weights zero is the exact sum
             if (!masked)
                 thr = fmax(thr, fmax((double)a.line * tc2, traw / 1024.0));
             a.thr[m] = bad || !(thr < 1e37) ? INFINITY : (float)thr;

@@ -16,9 +16,15 @@
 // 0.9e-7, 5.5e-7 (7.7e-7), 72: 0.5e-7, 0.6e-7, 1.3e-7 (1.3e-7).  The guard's line lies where the two are equal, at 0.43 T (half
 // for the shortest patches, split_line); with the cross terms' leading product among the lesser ones, eleven roundings of
 // it to a step, it was 1.6e-6 at 0.5 and 576 elements, and 4.4e-7 at 2.
-// A tile with an output below the line (or below 1/1024 of the uncentred sum w t^2, the guard of the sqrt-weight form; or
-// not finite; or of a template whose parameters are negative, huge or tiny) is flagged and computed again, term by
-// term, by the direct kernel's launch behind this one, which otherwise returns at once.
+// An output below the line (or below 1/1024 of the uncentred sum w t^2, the guard of the sqrt-weight form; or not finite) is
+// computed again term by term by its workgroup (split_recompute): the others keep their value, so it does not matter
+// what shares a tile.  A tile with more of them than that is worth, or with a template whose parameters are negative,
+// huge or tiny, is flagged and left whole to the direct kernel's launch behind this one, which otherwise returns at once.
+// Templates fitted to the inputs (k-means of 1/f images with three factors over the channels, 256 x 64 x 32 x 32 -> 128, 3 x 3):
+// 0.15 % of the outputs in 84 % of the tiles, 0.46 ms; with every such tile left to the direct kernel 1.39, the sqrt-weight
+// form 0.81.  64 x 16 x 32 x 32 -> 64: 46 us, 83 and 55; 64 x 8 x 32 x 32 -> 32, 72 elements, 0.9 % of the outputs: 31, 47 and 30,
+// and with 1.3 %, where some tiles have too many: 53.  Several templates near every output are the worst that can be: 256
+// x 576 x 14 x 14 -> 128, 1 x 1, 6 % of the outputs, 643 us where the sqrt-weight form takes 420.
 //
 // Missing values (NaN inputs ignored): x' = 0 and a third operand, the 0/1 mask of present values (exact in 16 bits),
 // contracts with -w t'^2 and with the logarithm term, three pieces each; T is that of the present values.
@@ -49,6 +55,10 @@ namespace simnets {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(1))) float global_float;
+typedef __attribute__((address_space(1))) float2_t global_float2;
 
 constexpr int kThreads = 256;
 enum SplitKind { SPLIT_FWD, SPLIT_MASKED /* forward, NaN inputs ignored */, SPLIT_GRAD /* input gradient */ };
@@ -57,6 +67,8 @@ enum SplitKind { SPLIT_FWD, SPLIT_MASKED /* forward, NaN inputs ignored */, SPLI
 constexpr int split_lds_pixels(int kind) { return kind == SPLIT_MASKED ? 360 : kind == SPLIT_FWD ? 408 : 816; }
 constexpr int split_operands(int kind) { return kind == SPLIT_MASKED ? 7 : kind == SPLIT_FWD ? 6 : 3; }
 constexpr int split_lds_bytes(int kind) { return split_lds_pixels(kind) * 32 * split_operands(kind); }
+// pixels of one staged plane [channel group][pixel]
+constexpr int split_plane_pixels(int kind, int cg) { return split_lds_pixels(kind) * (cg == 16 ? 1 : 2); }
 constexpr int split_pieces(int kind) { return kind == SPLIT_MASKED ? 12 : 6; }
 
 struct SplitArgs {
@@ -64,6 +76,8 @@ struct SplitArgs {
     float *out;
     const bf16x8 *packed;
     const float *ctr, *bias, *lg, *thr;
+    const float2 *exact;   // see SplitPack
+    const float *logs;
     int *flags;      // [pixel tile][mtile]
     int C, H, W, O, ow, npix, total;   // npix = oh ow, total = B npix
     int bw, sh, sw, ph, pw, taps, chunks, steps, n_mtiles, Wp, Hv;
@@ -73,18 +87,27 @@ struct SplitArgs {
     const float *x;  // input gradient: the forward's input, of the output's shape; templates and weights [C][O][taps]
     const float *templates, *weights;
     float scale;
-    FastDiv d_npix, d_ow, d_wp, d_hv;
+    float norm_const;
+    int K;
+    FastDiv d_npix, d_ow, d_wp, d_hv, d_taps, d_bw;
 };
 
-// Input gradient of one element (input channel ch, pixel rem of its image) term by term: where the sums A and (x - c) B are
-// infinite with one sign, only the terms tell which way their difference goes.  Not inlined, and with the kernel's
-// arguments read again from its argument segment (they end where the implicit arguments begin; the kernel's other
-// argument is an int): the main loop's registers stay as they are.
+// Cold paths read the kernel's arguments again from its argument segment (they end where the implicit arguments begin; the
+// kernel's other argument is an int), instead of keeping them in registers past the main loop.
 #if defined(__HIP_DEVICE_COMPILE__)
+static_assert(sizeof(SplitArgs) % 8 == 0, "the explicit arguments end 8 bytes behind the block");
+__device__ __forceinline__ const SplitArgs &split_kernel_args()
+{
+    return *reinterpret_cast<const SplitArgs *>(reinterpret_cast<const char *>(__builtin_amdgcn_implicitarg_ptr()) -
+                                                (sizeof(SplitArgs) + 8));
+}
+
+// Input gradient of one element (input channel ch, pixel rem of its image) term by term: where the sums A and (x - c) B are
+// infinite with one sign, only the terms tell which way their difference goes.  Not inlined: the main loop's registers and
+// schedule stay as they are.
 __device__ __noinline__ float split_grad_terms(int img, int ch, int rem, float x)
 {
-    const SplitArgs &a = *reinterpret_cast<const SplitArgs *>(
-        reinterpret_cast<const char *>(__builtin_amdgcn_implicitarg_ptr()) - (sizeof(SplitArgs) + 8));
+    const SplitArgs &a = split_kernel_args();
     const int y = rem / a.ow, xo = rem - y * a.ow;
     float sum = 0.0f;
     for (int o = 0; o < a.C; ++o)
@@ -97,7 +120,171 @@ __device__ __noinline__ float split_grad_terms(int img, int ch, int rem, float x
         }
     return sum;
 }
-static_assert(sizeof(SplitArgs) % 8 == 0, "the explicit arguments end 8 bytes behind the block");
+
+// Outputs of a tile (of 4096) that a workgroup recomputes by itself.  One at a time 2.5 % of them (256 x 576 x 14 x 14 -> 128, 1 x
+// 1: 17.9 ms for all, the direct kernel 0.45) to 3.3 % (64 x 144 x 32 x 32 -> 64: 2.3 ms, 0.08) take as long as the tile does
+// on the direct kernel.
+constexpr int kSplitListed = 192;   // (fitted templates have a few tiles with five times the mean)
+
+// LDS of a workgroup whose products are done and that has outputs to recompute.
+template <int KIND, int CG>
+struct NearOutputs {
+    static constexpr int kPlane = split_plane_pixels(KIND, CG);
+    int count[4], total;                            // of each template tile, and of the list
+    float sum[4 * kSplitListed];
+    float x[CG * kPlane];                           // a chunk's channels of the rows that the pixels read
+    unsigned short list[4 * kSplitListed];          // pixel << 7 | template
+    unsigned short element[CG * kPlane];            // where a patch element of the chunk lies in x
+};
+
+// Outputs below the guard's line, term by term with the direct kernels' arithmetic, eight lanes to an output and twelve
+// terms of a lane in flight; their patches from memory where they are few, else from the rows, staged again in fp32, chunk
+// by chunk.  near[i]: this lane's, bit r.  A tile with more of them than kSplitListed, or with a template whose
+// parameters are out of range, is flagged for the direct kernel instead.  G: the workgroup's template tiles, 4, 2 or 1.
+// LOGS: the mode has logarithm terms.  Inlined once, at the kernel's end: a call, or a copy in each split_body, spills SGPRs of
+// the bodies (37 x 45 x 29 x 35 -> 75 62 -> 65 to 72 us).
+template <int KIND, int CG, bool LOGS>
+__device__ __forceinline__ void split_recompute(lds_char *lds, int mtile0, int G, u32x4 near)
+{
+    constexpr int kLanes = 8, kTerms = 12, kOutputs = kThreads / kLanes;
+    typedef NearOutputs<KIND, CG> Near;
+    static_assert(sizeof(Near) <= split_lds_bytes(KIND), "in the memory of the staged pieces");
+    const SplitArgs a = split_kernel_args();
+    __attribute__((address_space(3))) Near &q = *(__attribute__((address_space(3))) Near *)lds;
+    const int tid = threadIdx.x, wave = tid >> 6, n0 = blockIdx.x * kSplitPixels;
+    if (tid < 4)
+        q.count[tid] = 0;
+    if (tid == 4)
+        q.total = 0;
+    __syncthreads();
+    int bits = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        bits += __builtin_popcount(near[i]);
+    if (bits)
+        atomicAdd((int *)&q.count[wave % G], bits);
+    if (tid < G * kSplitRows && mtile0 + tid / kSplitRows < a.n_mtiles && a.thr[mtile0 * kSplitRows + tid] == INFINITY)
+        atomicAdd((int *)&q.count[tid / kSplitRows], kSplitPixels * kSplitRows);
+    __syncthreads();
+    for (int g = 0; g < G && mtile0 + g < a.n_mtiles; ++g) {
+        const int outputs = min(kSplitPixels, a.total - n0) * min(kSplitRows, a.O - (mtile0 + g) * kSplitRows);
+        const bool leave = q.count[g] > min(kSplitListed, outputs / 2);
+        if (tid == 0)
+            a.flags[(size_t)blockIdx.x * a.n_mtiles + mtile0 + g] = leave;
+        if (wave % G != g || leave || !bits)
+            continue;
+        int slot = atomicAdd((int *)&q.total, bits);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            for (unsigned rest = near[i]; rest; rest &= rest - 1, ++slot) {
+                const int r = __builtin_ctz(rest), ml = g * kSplitRows + 8 * (r / 4) + 4 * (tid >> 5 & 1) + r % 4;
+                q.list[slot] = (unsigned short)((((wave / G) * G + i) * 32 + (tid & 31)) << 7 | ml);
+            }
+    }
+    __syncthreads();
+    const int listed = q.total, lane = tid % kLanes;
+    const global_float *in = (const global_float *)a.in, *logs = (const global_float *)a.logs;
+    const global_float2 *exact = (const global_float2 *)a.exact;
+    auto pixel = [&](int e, int &img, int &rem, int &r, int &c) {   // its image, place in it, output row and column
+        const int n = n0 + (q.list[e] >> 7);
+        img = (int)fast_div((unsigned)n, a.d_npix);
+        rem = n - img * a.npix;
+        r = (int)fast_div((unsigned)rem, a.d_ow);
+        c = rem - r * a.ow;
+    };
+    auto store = [&](int e, float sum) {
+        int img, rem, r, c;
+        pixel(e, img, rem, r, c);
+        const int m = mtile0 * kSplitRows + (q.list[e] & 127);
+        ((global_float *)a.out)[((size_t)img * a.O + m) * a.npix + rem] = LOGS ? sum + a.norm_const : sum;
+    };
+    // n terms of list entry e, from patch element k on, summed over its lanes; value(j): the input under the j-th
+    auto terms = [&](int e, int k, int n, auto value) {
+        const size_t at = (size_t)(mtile0 * kSplitRows + (q.list[e] & 127)) * a.K + k;
+        float sum = 0.0f;
+        for (int j0 = lane; j0 < n; j0 += kLanes * kTerms) {
+            float x[kTerms], l[kTerms];
+            float2_t tw[kTerms];
+#pragma unroll
+            for (int i = 0; i < kTerms; ++i) {   // behind the last: the last
+                const int j = min(j0 + kLanes * i, n - 1);
+                tw[i] = exact[at + j];
+                l[i] = LOGS ? logs[at + j] : 0.0f;
+                x[i] = value(j);
+            }
+#pragma unroll
+            for (int i = 0; i < kTerms; ++i) {
+                const float d = tw[i].x - x[i], term = __builtin_fmaf(tw[i].y * d, d, l[i]);
+                sum += j0 + kLanes * i >= n || (KIND == SPLIT_MASKED && x[i] != x[i]) ? 0.0f : term;
+            }
+        }
+        for (int d = kLanes / 2; d > 0; d >>= 1)
+            sum += __shfl_xor(sum, d, kLanes);
+        return sum;
+    };
+    if (listed <= kOutputs) {
+        const int e = tid / kLanes;
+        if (e >= listed)
+            return;
+        int img, rem, r, c;
+        pixel(e, img, rem, r, c);
+        const int r0 = r * a.sh - a.ph, c0 = c * a.sw - a.pw, first = (img * a.C * a.H + r0) * a.W + c0;
+        const float sum = terms(e, 0, a.K, [&](int k) {
+            const int ch = (int)fast_div((unsigned)k, a.d_taps), tap = k - ch * a.taps;
+            const int dh = (int)fast_div((unsigned)tap, a.d_bw), dw = tap - dh * a.bw, h = r0 + dh, w = c0 + dw;
+            const bool inside = (h >= 0) & (h < a.H) & (w >= 0) & (w < a.W);
+            const float x = in[inside ? first + (ch * a.H + dh) * a.W + dw : 0];
+            return inside ? x : a.oob;
+        });
+        if (lane == 0)
+            store(e, sum);
+        return;
+    }
+    auto virtual_row = [&](int n) {   // of the stack of padded images, as in split_body
+        const int img = (int)fast_div((unsigned)n, a.d_npix);
+        return img * a.Hv + (int)fast_div((unsigned)(n - img * a.npix), a.d_ow) * a.sh;
+    };
+    const int v0 = virtual_row(n0);
+    const int rows = virtual_row(min(n0 + kSplitPixels, a.total) - 1) - v0 + a.taps / a.bw;
+    const int staged = min(rows * a.Wp, Near::kPlane);
+    for (int k = tid; k < CG * a.taps; k += kThreads) {
+        const int ch = (int)fast_div((unsigned)k, a.d_taps), tap = k - ch * a.taps;
+        const int dh = (int)fast_div((unsigned)tap, a.d_bw);
+        q.element[k] = (unsigned short)(ch * Near::kPlane + dh * a.Wp + tap - dh * a.bw);
+    }
+    const size_t plane = (size_t)a.H * a.W;
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+        const int channels = min(CG, a.C - chunk * CG);
+        for (int p = tid; p < staged; p += kThreads) {
+            const int vr = (int)fast_div((unsigned)p, a.d_wp), c = p - vr * a.Wp - a.pw;
+            const int img = (int)fast_div((unsigned)(v0 + vr), a.d_hv), r = v0 + vr - img * a.Hv - a.ph;
+            const bool inside = (r >= 0) & (r < a.H) & (c >= 0) & (c < a.W);
+            const size_t at = inside ? ((size_t)(img * a.C + chunk * CG) * a.H + r) * a.W + c : 0;
+            float x[CG];
+#pragma unroll
+            for (int j = 0; j < CG; ++j)
+                x[j] = in[inside ? at + min(j, channels - 1) * plane : 0];
+#pragma unroll
+            for (int j = 0; j < CG; ++j)
+                q.x[j * Near::kPlane + p] = inside ? x[j] : a.oob;
+        }
+        __syncthreads();
+        for (int e = tid / kLanes; e < listed; e += kOutputs) {
+            int img, rem, r, c;
+            pixel(e, img, rem, r, c);
+            const int base = (img * a.Hv + r * a.sh - v0) * a.Wp + c * a.sw;
+            float sum = terms(e, chunk * CG * a.taps, channels * a.taps, [&](int j) { return q.x[base + q.element[j]]; });
+            if (lane == 0) {
+                sum += chunk == 0 ? 0.0f : q.sum[e];
+                if (chunk + 1 < a.chunks)
+                    q.sum[e] = sum;
+                else
+                    store(e, sum);
+            }
+        }
+        __syncthreads();
+    }
+}
 #endif
 
 // a + b + c, |c| the smallest, rounded about once: what the rounding of a + b loses is added to c.
@@ -109,11 +296,11 @@ __device__ __forceinline__ float split_three(float a, float b, float c)
 
 // One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
 template <int KIND, int CG, int G>
-__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mtile0, int flag)
+__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 &near, int mtile0, int flag)
 {
     constexpr bool MASKED = KIND == SPLIT_MASKED, GRAD = KIND == SPLIT_GRAD, WHOLE = KIND == SPLIT_FWD;
     constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND);
-    constexpr int P = split_lds_pixels(KIND) * (CG == 16 ? 1 : 2);   // pixels of one plane [channel group][pixel]
+    constexpr int P = split_plane_pixels(KIND, CG);
     constexpr int kPlane = split_lds_pixels(KIND) * 32;
     constexpr int kItems = (split_lds_pixels(KIND) * 2 + kThreads - 1) / kThreads;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -345,7 +532,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mt
         return;
     }
     const bool norm = flag;
-    bool bad = false;
     if (active) {
         float bias[16], lgm[16], thr[16];
 #pragma unroll
@@ -368,36 +554,25 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, int mt
                 if (mtile * kSplitRows + ml >= a.O)
                     continue;
                 float v;
+                bool fine;
                 if (MASKED) {
                     v = split_three(hi[i][r], tm[i][r], lo[i][r]);
                     const float mag = __builtin_fabsf(v);
-                    const bool fine = mag < 1e37f && mag >= a.line * -tm[i][r] &&
-                                      (mag >= thr[r] || (v == 0.0f && tm[i][r] == 0.0f && thr[r] < 1e37f));
-                    bad |= !fine;
+                    fine = mag < 1e37f && mag >= a.line * -tm[i][r] &&
+                           (mag >= thr[r] || (v == 0.0f && tm[i][r] == 0.0f && thr[r] < 1e37f));
                     v = 0.5f * v + lg[i][r];
                 } else {
                     v = split_three(hi[i][r], bias[r], lo[i][r]);
                     const float mag = __builtin_fabsf(v);
-                    bad |= !(mag >= thr[r] && mag < 1e37f);
+                    fine = mag >= thr[r] && mag < 1e37f;
                     if (norm)
                         v = 0.5f * v + lgm[r];
                 }
+                near[i] |= fine ? 0u : 1u << r;
                 dst[(size_t)ml * a.npix] = v;
             }
         }
     }
-    // one flag per (pixel tile, template tile): the waves of a template tile share it
-    bad = __any(bad);
-    int *shared_flag = reinterpret_cast<int *>(lds);
-    __syncthreads();
-    if (tid < G)
-        shared_flag[tid] = 0;
-    __syncthreads();
-    if (bad && lane == 0)
-        shared_flag[wave % G] = 1;
-    __syncthreads();
-    if (tid < G && mtile0 + tid < a.n_mtiles)
-        a.flags[(size_t)blockIdx.x * a.n_mtiles + mtile0 + tid] = shared_flag[tid];
 }
 
 // The template tiles of a pixel tile are dealt out as groups of gmax and, of the rest, 2 and 1.  flag: forward, the
@@ -406,6 +581,10 @@ template <int KIND, int CG>
 __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs a, int flag)
 {
     __shared__ __align__(16) char split_lds[split_lds_bytes(KIND)];
+    __shared__ int any_near;   // of the workgroup's outputs, one below the guard's line
+    if (KIND != SPLIT_GRAD && threadIdx.x == 0)
+        any_near = 0;
+    u32x4 near = 0;   // [i] bit r: output r of this lane's pixel tile i is
     const int full = a.n_mtiles / a.gmax, y = blockIdx.y;
     int mtile0 = y * a.gmax, g = a.gmax;
     if (y >= full) {
@@ -418,11 +597,26 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
         }
     }
     if (KIND == SPLIT_FWD && g == 4)
-        split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, mtile0, flag);
+        split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, near, mtile0, flag);
     else if (g == 2)
-        split_body<KIND, CG, 2>(a, split_lds, mtile0, flag);
+        split_body<KIND, CG, 2>(a, split_lds, near, mtile0, flag);
     else
-        split_body<KIND, CG, 1>(a, split_lds, mtile0, flag);
+        split_body<KIND, CG, 1>(a, split_lds, near, mtile0, flag);
+    if constexpr (KIND != SPLIT_GRAD) {
+        if (near[0] | near[1] | near[2] | near[3])
+            any_near = 1;
+        __syncthreads();
+        // (unlikely: the code behind everything else; between the bodies it costs 37 x 45 x 29 x 35 -> 75 4 us of 62)
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(any_near), 0)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+            if (KIND == SPLIT_MASKED || flag)
+                split_recompute<KIND, CG, true>((lds_char *)split_lds, mtile0, g, near);
+            else
+                split_recompute<KIND, CG, KIND == SPLIT_MASKED>((lds_char *)split_lds, mtile0, g, near);
+#endif
+        } else if ((int)threadIdx.x < g && mtile0 + (int)threadIdx.x < a.n_mtiles)
+            a.flags[(size_t)blockIdx.x * a.n_mtiles + mtile0 + threadIdx.x] = 0;
+    }
 }
 
 // Packs the input gradient's coefficients, rows = input channels, contraction = (template, flipped tap): three pieces
@@ -526,7 +720,9 @@ static SplitPlan split_geometry(const SimPlan &p, int kind)
     s.lg = s.bias + align_up((size_t)mpad * sizeof(float), 256);
     s.thr = s.lg + align_up((size_t)mpad * sizeof(float), 256);
     s.flags = s.thr + align_up((size_t)mpad * sizeof(float), 256);
-    s.total = s.flags + align_up((size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
+    s.exact = s.flags + align_up((size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
+    s.logs = s.exact + (kind == SPLIT_GRAD ? 0 : align_up((size_t)p.O * p.K * sizeof(float2), 256));
+    s.total = s.logs + (kind == SPLIT_GRAD || p.mode == SIM_MODE_L2 ? 0 : align_up((size_t)p.O * p.K * sizeof(float), 256));
     s.on = true;
     return s;
 }
@@ -540,6 +736,8 @@ SplitPlan sim_split_plan(const SimPlan &p)
     return split_geometry(p, p.mode == SIM_MODE_L2_NORM_IGNORE_NAN ? SPLIT_MASKED : SPLIT_FWD);
 }
 
+static float split_norm_const(int K) { return (float)((double)(-0.5f * (float)K) * std::log(2.0 * M_PI)); }
+
 SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float *templates, const float *weights,
                               char *ws)
 {
@@ -550,10 +748,12 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     a.bias = reinterpret_cast<float *>(ws + sp.bias);
     a.lg = reinterpret_cast<float *>(ws + sp.lg);
     a.thr = reinterpret_cast<float *>(ws + sp.thr);
+    a.exact = reinterpret_cast<float2 *>(ws + sp.exact);
+    a.logs = reinterpret_cast<float *>(ws + sp.logs);
     a.O = p.O; a.C = p.C; a.taps = p.bh * p.bw; a.K = p.K; a.cg = sp.cg; a.chunks = sp.chunks; a.steps = sp.steps;
     a.pieces = sp.pieces; a.n_mtiles = sp.n_mtiles; a.mode = p.mode; a.fudge = p.fudge;
     a.line = split_line(p.K);
-    a.norm_const = p.mode == SIM_MODE_L2_NORM ? (float)((double)(-0.5f * (float)p.K) * std::log(2.0 * M_PI)) : 0.0f;
+    a.norm_const = p.mode == SIM_MODE_L2_NORM ? split_norm_const(p.K) : 0.0f;
     a.pack_blocks = sp.on ? sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4) : 0;
     a.thr_blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows, 512) : 0;
     return a;
@@ -570,6 +770,10 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     a.lg = reinterpret_cast<const float *>(ws + sp.lg);
     a.thr = reinterpret_cast<const float *>(ws + sp.thr);
     a.flags = reinterpret_cast<int *>(ws + sp.flags);
+    a.exact = reinterpret_cast<const float2 *>(ws + sp.exact);
+    a.logs = reinterpret_cast<const float *>(ws + sp.logs);
+    a.norm_const = p.mode == SIM_MODE_L2_NORM ? split_norm_const(p.K) : 0.0f;
+    a.K = p.K;
     a.C = p.C; a.H = p.H; a.W = p.W; a.O = p.O; a.ow = p.ow; a.npix = p.oh * p.ow; a.total = p.B * a.npix;
     a.bw = p.bw; a.sh = p.sh; a.sw = p.sw; a.ph = p.ph; a.pw = p.pw; a.taps = p.bh * p.bw;
     a.chunks = sp.chunks; a.steps = sp.steps; a.n_mtiles = sp.n_mtiles; a.Wp = sp.Wp; a.Hv = sp.Hv;
@@ -579,6 +783,8 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     a.d_ow = make_fast_div((unsigned)p.ow);
     a.d_wp = make_fast_div((unsigned)sp.Wp);
     a.d_hv = make_fast_div((unsigned)sp.Hv);
+    a.d_taps = make_fast_div((unsigned)a.taps);
+    a.d_bw = make_fast_div((unsigned)p.bw);
     // as many template tiles per staged pixel tile as leave a workgroup for every compute unit
     a.gmax = KIND == SPLIT_FWD ? 4 : 2;
     while (a.gmax > 1 && (a.gmax / 2 >= sp.n_mtiles || (long long)sp.n_ptiles * ((sp.n_mtiles + a.gmax - 1) / a.gmax) < 256))

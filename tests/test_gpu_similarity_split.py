@@ -363,3 +363,39 @@ def test_split_form_near_a_template(pkg, C, block, ratio, mode):
         want = want + log * (cols == cols).flatten(3).sum(-1)
     err = float((((got - want) / want) ** 2).mean().sqrt())
     assert err <= 1.5 * 0.4 * 2.0 ** -24 * math.sqrt(K / 3), err
+
+
+@pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
+@pytest.mark.parametrize("near", [1, 3, 8])
+@pytest.mark.parametrize("shape, O, block", [
+    ((20, 40, 22, 21), 225, 3),    # chunks of 16 channels, the last of 8
+    ((20, 20, 34, 37), 34, 5),     # chunks of 8, the last of 4
+    ((20, 65, 24, 25), 33, 1),     # a single tap
+])
+def test_split_form_recomputes_outputs_near_a_template_alone(pkg, shape, O, block, near, mode):
+    """The first image's last row of patches lies close to `near` templates, 19 to 264 outputs: they have the error of a sum
+    of their terms, K roundings of at most its size; and the images that share their tiles have the values that they have
+    in other company, unless there are more than 128 in a tile."""
+    g = torch.Generator(device="cuda").manual_seed(59)
+    C, K = shape[1], shape[1] * block * block
+    kw = options(mode, dict(blocks=[block, block], strides=[1, 1], padding=[0, 0]))
+    x = torch.randn(shape, generator=g, device="cuda")
+    t = torch.randn((O, C, block, block), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    value = 2 * torch.randn((C, 1, 1), generator=g, device="cuda")
+    t[:near] = value + 0.1 * torch.randn((near, C, block, block), generator=g, device="cuda")
+    t[near:2 * near] = -value    # the channels' centres stay away from it
+    other = x.clone()
+    x[0, :, -block:] = value
+    assert pieces_used(pkg, shape, O, mode, **kw)["forward"]
+    got = pkg.similarity(x, t, w, **kw)
+    want = exact(x[:1], t, w, [block, block], [1, 1], [0, 0], mode, kw.get("out_of_bounds_value", 0.0))
+    size = want[0, :near, -1].abs()
+    if mode != "l2":    # the terms' and the logarithms' sums have either sign
+        size = size + 0.5 * (K * math.log(2 * math.pi) + torch.log(w[:near].double() + 0.001).abs().flatten(1).sum(1))[:, None]
+    err = ((got[0, :near, -1].double() - want[0, :near, -1]).abs() / size).max()
+    assert float(err) <= K * 2.0 ** -24, float(err)
+    if near * got.shape[3] * (block + 1) // 2 <= 128:    # patches that reach half way into those rows are near, too
+        assert torch.equal(pkg.similarity(other, t, w, **kw)[1:], got[1:])
