@@ -69,7 +69,22 @@ GEOMS = [
     dict(shape=(6, 100, 45, 20), O=40, blocks=[1, 1], strides=[1, 1], padding=[0, 0]),   # one tap
     dict(shape=(90, 16, 9, 9), O=32, blocks=[2, 3], strides=[3, 2], padding=[0, 0]),     # strides beyond the block
     dict(shape=(12, 66, 33, 34), O=31, blocks=[1, 3], strides=[1, 1], padding=[0, 1], out_of_bounds_value=0.5),
+    dict(shape=(80, 32, 7, 7), O=160, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),    # several images to a tile
+    dict(shape=(20, 20, 34, 37), O=34, blocks=[5, 5], strides=[1, 1], padding=[2, 2]),   # chunks of 8 in every mode
+    dict(shape=(20, 40, 41, 31), O=60, blocks=[1, 3], strides=[2, 2], padding=[0, 0]),   # a stride beyond the block
+    dict(shape=(20, 40, 41, 20), O=60, blocks=[2, 2], strides=[1, 3], padding=[0, 0]),   # ... the other way
 ]
+
+
+def test_geometries_reach_the_form(pkg):
+    """The tests below would pass on any form: which of them run on this one."""
+    runs = {mode: [pieces_used(pkg, mode=mode, **g) for g in GEOMS] for mode in ("l2", "norm", "missing")}
+    used = lambda mode, what: [i for i, r in enumerate(runs[mode]) if r[what]]
+    for mode in ("l2", "norm"):
+        assert used(mode, "forward") == [0, 1, 2, 3, 5, 6, 7, 9, 10, 11, 12, 13]
+        assert used(mode, "params") == [0, 1, 2, 3, 4, 6, 9, 10, 11, 12, 13]
+    assert used("missing", "forward") == [0, 1, 2, 3, 7, 9, 11, 12, 13]
+    assert used("l2", "input") == [0, 1, 2, 3, 5, 7, 9, 11]
 
 
 @pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
