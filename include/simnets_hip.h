@@ -132,8 +132,9 @@ int simnets_hip_similarity_fwd(const simnets_similarity_attrs *attrs, const int 
  * caller-owned buffer of simnets_hip_similarity_workspace_bytes bytes (256-byte aligned), and
  * simnets_hip_similarity_fwd_prepared runs only the forward kernels on it.  attrs, input_shape (batch size
  * included: the tiling depends on it) and templates_shape must be the ones the buffer was prepared with; results
- * are those of simnets_hip_similarity_fwd bit for bit.  The buffer may also hold a few bytes of per-call scratch (the
- * workgroup flags of the sqrt-weight form on small maps), so calls that share one prepared buffer must not overlap. */
+ * are those of simnets_hip_similarity_fwd bit for bit.  The buffer also holds per-call scratch (AUTO's flags of the tiles
+ * that its matrix-core form leaves to DIRECT's kernel, the workgroup flags of the sqrt-weight form on small maps), so
+ * calls that share one prepared buffer must not overlap. */
 int simnets_hip_similarity_prepare(const simnets_similarity_attrs *attrs, const int input_shape[4],
                                    const int templates_shape[4], const int weights_shape[4], const float *templates,
                                    const float *weights, void *prepared, size_t prepared_bytes, void *stream);
@@ -145,8 +146,10 @@ int simnets_hip_similarity_fwd_prepared(const simnets_similarity_attrs *attrs, c
  * serving loops, harnesses that forbid hipMalloc) and so have no workspace to pass.  It has no counterpart in the
  * reference.  Same arguments minus the workspace, same kernels, same results bit for bit; the scratch is a fixed
  * device array of SIMNETS_HIP_STATIC_SCRATCH_BYTES inside the library (one copy per GPU, held until the process
- * ends) and the call allocates nothing.  Calls whose simnets_hip_similarity_workspace_bytes exceeds that size
- * return SIMNETS_ERR_STATIC_SCRATCH before anything is launched.  All calls on one GPU share that GPU's array:
+ * ends) and the call allocates nothing.  With SIMNETS_ALGO_AUTO, where the packed pieces of its matrix-core form exceed that
+ * size, the call runs the form that AUTO takes elsewhere (SQRTW for plain L2, DIRECT for the normalized modes), bit for
+ * bit as if that had been asked for.  Calls for whose form, by simnets_hip_similarity_workspace_bytes, the size does not
+ * suffice return SIMNETS_ERR_STATIC_SCRATCH before anything is launched.  All calls on one GPU share that GPU's array:
  * calls that may overlap on one GPU (different streams, different threads) race; order them on one stream.  The
  * first call on a device looks up the array's address (hipGetSymbolAddress): make it outside graph capture. */
 #define SIMNETS_HIP_STATIC_SCRATCH_BYTES (4u << 20)

@@ -133,3 +133,31 @@ def test_static_scratch_rejects_what_does_not_fit(pkg):
     assert nbytes.value > _lib.STATIC_SCRATCH_BYTES
     rc = l.simnets_hip_similarity_fwd_static(C.byref(a), xs, ts, ts, None, None, None, None, None)
     assert rc == -21 and "scratch" in _lib.strerror(rc)
+
+
+@pytest.mark.parametrize("normalize, named", [(False, "sqrtw"), (True, "direct")])
+def test_static_scratch_smaller_than_the_packed_pieces(pkg, normalize, named):
+    """The default form's packed pieces do not fit, those of the form it takes elsewhere do: the call is that form's."""
+    from simnets_tf_amd import _lib, ops
+    l = _lib.lib()
+    x, t, w = _inputs(11, (33, 64, 24, 25), 320, (3, 3))
+    kw = dict(blocks=[3, 3], strides=[1, 1], padding=[1, 1], normalization_term=normalize)
+    I4 = C.c_int * 4
+    xs, ts = I4(*x.shape), I4(*t.shape)
+    sizes = []
+    for algo in (None, named):
+        nbytes = C.c_size_t()
+        assert l.simnets_hip_similarity_workspace_bytes(C.byref(ops.similarity_attrs(algo=algo, **kw)), xs, ts,
+                                                        C.byref(nbytes)) == 0
+        sizes.append(nbytes.value)
+    assert sizes[0] > _lib.STATIC_SCRATCH_BYTES >= sizes[1]
+    X, T, W = (torch.from_numpy(v).cuda() for v in (x, t, w))
+    want = pkg.similarity(X, T, W, algo=named, **kw)
+    got = torch.empty_like(want)
+    rc = l.simnets_hip_similarity_fwd_static(C.byref(ops.similarity_attrs(**kw)), xs, ts, ts, X.data_ptr(), T.data_ptr(),
+                                             W.data_ptr(), got.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.strerror(rc)
+    assert torch.equal(got, want)
+    # K additions of terms of one size on the one side, K / 16 on the other (and the logarithms)
+    default = pkg.similarity(X, T, W, **kw)
+    assert float((got - default).norm() / default.norm()) <= 576 * 2.0 ** -24
