@@ -28,12 +28,12 @@ PEAK_HBM_GBS = 8000.0
 EXP_RATE_STATED = 9.83e12  # exponentials per second the work table of the baseline document prices MEX against
 EXP_RATE_MEASURED = 19.66e12  # v_exp_f32 at a quarter of the 128 lanes/clk/CU VALU rate (17.6e12 measured on the box)
 
-# HBM bytes per launch of the dominant kernel of the headline workload, from rocprofv3 FETCH_SIZE / WRITE_SIZE runs
-# scaled by a copy kernel of known size; not measured inside this run: "traffic_source" names the committed summary.
 PEAK_BF16_TFLOPS = 2500.0  # dense bf16 matrix peak
 # The default form of the L2 modes multiplies 16-bit pieces on the bf16 matrix cores: six products for each of two
 # operands per term, a third operand (three products for each of two sums) where NaN inputs are ignored
 PIECES_FLOP, PIECES_MASKED_FLOP = 24, 36
+# HBM bytes per launch of the dominant kernel of the headline workload, from rocprofv3 FETCH_SIZE / WRITE_SIZE runs
+# scaled by a copy kernel of known size; not measured inside this run: "traffic_source" names the committed summary.
 MEASURED_TRAFFIC = {
     "pieces": (197.0e6, "profiles/similarity_split_l2.md"),
     "sqrtw": (231.8e6, "profiles/sim_direct_l2_config3.md"),

@@ -75,10 +75,10 @@ struct SimKernelArgs {
     const float *pa2;  // [mtile][K][MT][2]  (template, negative weight): what the recomputing pass reads
     const float *thr;  // [O] a partial sum of template m above -thr[m] sends its wave to the recomputing pass
     int *flags;        // [workgroups * kWaves] 1: the wave left its outputs to the recomputing pass
-    // self-packing gather kernel only: the parameters as the caller holds them, [O][K] each
     const int *gate;   // flags [pixel tile of 128][template tile of 32] of the split form's launch in front of this one:
                        // only workgroups that touch a flagged tile run; null: all do
     int gate_mtiles;
+    // self-packing gather kernel only: the parameters as the caller holds them, [O][K] each
     const float *raw_t, *raw_w;
     float fudge;
 };
@@ -126,8 +126,6 @@ __device__ __forceinline__ LanePos lane_pos(const SimKernelArgs &a, int wave, in
     return q;
 }
 
-// Wave-uniform parameter fetch of the gather fallback: the address is the same in every lane, so these
-// become scalar loads (s_load_dwordx8/x16) and the values live in SGPRs.
 // Whether the split form left a tile of these outputs (pixels n0..n1 over the batch, templates m0..m1) to this launch.
 __device__ __forceinline__ bool split_flagged(const SimKernelArgs &a, int n0, int n1, int m0, int m1)
 {
@@ -139,6 +137,8 @@ __device__ __forceinline__ bool split_flagged(const SimKernelArgs &a, int n0, in
     return __syncthreads_or(any) != 0;
 }
 
+// Wave-uniform parameter fetch of the gather fallback: the address is the same in every lane, so these
+// become scalar loads (s_load_dwordx8/x16) and the values live in SGPRs.
 template <int MODE, int MT>
 __device__ __forceinline__ void load_params(float (&pa)[2 * MT], float (&pc)[MT], const float SIMNETS_CONST_AS *ppa,
                                             const float SIMNETS_CONST_AS *ppc)
