@@ -826,7 +826,15 @@ static SplitPlan split_grad_plan(const SimPlan &p)
 {
     if (!p.split || p.mode == SIM_MODE_L1 || p.B == 0 || p.sh != 1 || p.sw != 1 || p.ph > p.bh - 1 || p.pw > p.bw - 1)
         return SplitPlan();
-    return split_geometry(grad_as_forward(p), SPLIT_GRAD);
+    const SimPlan q = grad_as_forward(p);
+    const SplitPlan s = split_geometry(q, SPLIT_GRAD);
+    // Fewer tiles than fill the chip twice: a workgroup walks the whole contraction, 1.6 us to stage a chunk and 0.49 a step,
+    // where the fp32 form splits it over workgroups and takes some 45 us + 1 per tap + 38 per 10^9 terms.  Short
+    // contractions are the faster ones here (8 x 128 x 16 x 16, 128 templates, 3 x 3, 64 tiles: 53 us, fp32 form 62; 64 templates 30
+    // and 58; 8 x 64 x 28 x 28, 64, 5 x 5, 59 and 98), long ones there (1 x 32 x 64 x 64, 256 templates, 32 tiles: 98 and 57; 4 x 256 x
+    // 14 x 14, 256: 106 and 76; 6 x 64 x 28 x 28, 1024, 1 x 1: 138 and 55); 6 x 128 x 32 x 32, 256, 192 tiles: 100 and 95.
+    const double here = 6 + s.chunks * (1.6 + 0.49 * s.steps), there = 45 + p.bh * p.bw + 38e-9 * p.B * p.H * p.W * p.C * q.K;
+    return s.on && 1LL * s.n_ptiles * s.n_mtiles < 512 && here > there ? SplitPlan() : s;
 }
 
 size_t sim_split_grad_input_workspace_bytes(const SimPlan &p)

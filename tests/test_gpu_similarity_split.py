@@ -84,7 +84,7 @@ def test_geometries_reach_the_form(pkg):
         assert used(mode, "forward") == [0, 1, 2, 3, 5, 6, 7, 9, 10, 11, 12, 13]
         assert used(mode, "params") == [0, 1, 2, 3, 4, 6, 9, 10, 11, 12, 13]
     assert used("missing", "forward") == [0, 1, 2, 3, 7, 9, 11, 12, 13]
-    assert used("l2", "input") == [0, 1, 2, 3, 5, 7, 9, 11]
+    assert used("l2", "input") == [0, 1, 2, 5, 7, 9, 11]    # (3: few tiles of a long contraction)
 
 
 @pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
