@@ -1166,8 +1166,11 @@ SplitPlan split_plan(const SimPlan &p, const Tiling &t)
         return SplitPlan();
     const SplitPlan s = sim_split_plan(p);
     // a small-map grid needs enough workgroups to beat that kernel's split of the patch (8 x 200 x 14 x 14 -> 200, 5 x 5,
-    // 91 tiles: 199 us there, 265 here; 200 x 32 x 7 x 7 -> 64, 154 tiles: 33 and 26)
-    return t.NI > 0 && 1LL * s.n_ptiles * s.n_mtiles < 150 ? SplitPlan() : s;
+    // 91 tiles: 199 us there, 265 here; 200 x 32 x 7 x 7 -> 64, 154 tiles: 33 and 26); more of them where a staged chunk is read by
+    // one tap only, and by 32 pixels that straddle images (1 x 1, 512 channels: 7 x 7, 154 tiles 97 and 126, 230 tiles 125 and
+    // 125; 14 x 14, 186 tiles 92 and 126; but 8 x 8, 180 tiles 112 and 87)
+    const int enough = p.bh * p.bw == 1 && p.oh * p.ow % 32 != 0 ? 230 : 150;
+    return t.NI > 0 && 1LL * s.n_ptiles * s.n_mtiles < enough ? SplitPlan() : s;
 }
 
 // The sqrt-weight form runs on the tiled kernels and on the small-map kernel; there only with enough pixels per
