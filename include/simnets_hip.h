@@ -157,7 +157,8 @@ int simnets_hip_similarity_fwd_static(const simnets_similarity_attrs *attrs, con
                                       const int templates_shape[4], const int weights_shape[4], const float *input,
                                       const float *templates, const float *weights, float *output, void *stream);
 
-/* Backward.  Scratch sizes of the two gradient calls (either pointer may be NULL). */
+/* Backward.  Scratch sizes of the two gradient calls (either pointer may be NULL).  The parameter gradients' holds a packed
+ * copy of the output gradient, 1.5 times its size and at most 1 GiB, where AUTO takes its matrix-core form. */
 int simnets_hip_similarity_grad_workspace_bytes(const simnets_similarity_attrs *attrs, const int input_shape[4],
                                                 const int templates_shape[4], size_t *input_grad_bytes,
                                                 size_t *params_grad_bytes);
