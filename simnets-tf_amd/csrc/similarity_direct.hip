@@ -877,7 +877,7 @@ __global__ __launch_bounds__(256) void sim_pack_params_kernel(const float *__res
                                                              int pack_blocks, const SplitPack split)
 {
     extern __shared__ float split_lds[];
-    const int split_blocks = split.pack_blocks + split.thr_blocks;
+    const int split_blocks = split.blocks;
     if ((int)blockIdx.x < split_blocks) {
         split_pack_block(split, blockIdx.x, split_lds);
         return;
@@ -1245,8 +1245,8 @@ int sim_direct_prepare(const SimPlan &p, const float *templates, const float *we
     const int mode = sqrtw ? (int)SIM_MODE_L2_SQRTW : p.mode;
     const int thr_blocks = sqrtw ? std::min((p.O + 3) / 4, 1024) : 0;
     const SplitPack sp = sim_split_pack_args(p, split, templates, weights, ws + l.split);
-    const size_t lds = split.on ? align_up(p.C, 16) * sizeof(float) + 12 * sizeof(double) : 0;
-    hipLaunchKernelGGL(sim_pack_params_kernel, dim3(sp.pack_blocks + sp.thr_blocks + pack_blocks + thr_blocks),
+    const size_t lds = split.on ? split_pack_lds_bytes(p.C, p.K) : 0;
+    hipLaunchKernelGGL(sim_pack_params_kernel, dim3(sp.blocks + pack_blocks + thr_blocks),
                        dim3(256), lds, s, templates, weights, p.O,
                        p.K, t.MT, n_mtiles, mode, p.fudge, reinterpret_cast<float *>(ws + l.pa),
                        reinterpret_cast<float *>(ws + l.pc), reinterpret_cast<int *>(ws + l.koff), p.bh * p.bw, p.bw, t.CC,

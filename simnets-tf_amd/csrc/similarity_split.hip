@@ -1,21 +1,23 @@
-// The L2 Similarity modes as a matrix product on the bf16 matrix cores, at the precision of fp32 (gfx950).
+// The L2 Similarity modes as a matrix product on the 16-bit matrix cores, at the precision of fp32 (gfx950).
 //
 //   sum_k w (x - t)^2 = sum_k w x'^2 - 2 w t' x' + w t'^2,   x' = x - c, t' = t - c, c one value per channel
-// is a contraction of (w, -2 w t') with (x'^2, x').  Every factor is the exact sum of three 16-bit pieces (split3), and
-// the six products of pieces above 2^-24 of the whole are formed on v_mfma_f32_32x32x16_bf16 (dropped: below 2^-26).  A
-// 32-bit matrix instruction does two terms in 64 cycles where six of these do sixteen in 192 - 2.7 times the rate, and
-// 2.7 times the vector units' two instructions per term.
+// is a contraction of (w, -2 w t') with (x'^2, x').  Forward: every factor is the sum of two half-precision pieces of 11
+// bits, hi + lo (split2), and three products of pieces are formed on v_mfma_f32_32x32x16_f16; the one left out, lo lo, is
+// below 2^-22 of the whole with either sign.  Half precision has a narrow exponent: the packing kernel scales channels and
+// templates by powers of two (split_pack_block), the lesser piece of a value is kept times 2048 and meets a copy of hi
+// divided by as much, and a value that overflows makes its outputs NaN, which the guard below hands on.  Input gradient:
+// three bf16 pieces and six products (see the end of the file).
 //
-// Precision.  The two leading products (squares, cross terms) have accumulators of their own, so that an output's sum is
-// rounded K / 8 times at its own size; the lesser ones, 2^-8 of that, share a second set.  The sum begins with an eighth
-// of T = sum w t'^2, against which an unrelated input's sum - w x'^2 runs, and ends with the rest of T taken off; what the
-// last addition rounds is carried.  Inputs unrelated to the templates (error against 64 bits, 2-norm, relative): 256 x 64 x 32 x
-// 32 -> 128, 3 x 3, 0.8e-7 where the term-by-term forms have 3.6e-7; 32 x 128 x 28 x 28 -> 128 1.0e-7 against 5.1e-7.  Inputs near
-// a template lose to cancellation: the sum passes through T - out, and its error grows as T / out.  A patch at out / T = 2, 1
-// and 0.5 from its template, 576 elements: 0.8e-7, 0.6e-7 and 3.3e-7 (root mean square; term by term 3.6e-7), 2304: 1.4e-7,
-// 0.9e-7, 5.5e-7 (7.7e-7), 72: 0.5e-7, 0.6e-7, 1.3e-7 (1.3e-7).  The guard's line lies where the two are equal, at 0.43 T (half
-// for the shortest patches, split_line); with the cross terms' leading product among the lesser ones, eleven roundings of
-// it to a step, it was 1.6e-6 at 0.5 and 576 elements, and 4.4e-7 at 2.
+// Precision.  The matrix unit cuts what lies below 2^-26 of a sum off each of its products, and these have 22 bits: of
+// terms of one sign that is a bias (4.4e-7 at 576 elements).  So the squares are those about their channel's sampled mean,
+// x'^2 - m, whose sums stay small and have no bias, and a chunk's products (144 elements of 3 x 3) have a sum of their own
+// that is added in fp32.  Error against 64 bits (2-norm, relative): 256 x 64 x 32 x 32 -> 128, 3 x 3, inputs unrelated to the
+// templates 0.4e-7 (three bf16 pieces: 0.8e-7, term by term 3.6e-7), 256 channels 0.4e-7 (1.3e-7); inputs all zero
+// 1.0e-7 (0.6e-7), without their negative values 0.4e-7, ten times as large 0.8e-7 (1.7e-7).
+// Inputs near a template lose to cancellation, as T / out, T = sum w t'^2.  A patch at out / T = 2, 1 and 0.5 from its
+// template, 576 elements: 0.5e-7, 0.9e-7 and 2.3e-7 (root mean square; term by term 3.6e-7), 2304: 0.4e-7, 0.8e-7, 2.1e-7
+// (7.7e-7), 64: 0.6e-7, 0.9e-7, 1.0e-7 (1.3e-7).  The guard's line lies at 0.43 T (half for the shortest patches,
+// split_line).
 // An output below the line (or below 1/1024 of the uncentred sum w t^2, the guard of the sqrt-weight form; or not finite) is
 // computed again term by term by its workgroup (split_recompute): the others keep their value, so it does not matter
 // what shares a tile.  A tile with more of them than that is worth, or with a template whose parameters are negative,
@@ -26,21 +28,24 @@
 // and with 1.3 %, where some tiles have too many: 53.  Several templates near every output are the worst that can be: 256
 // x 576 x 14 x 14 -> 128, 1 x 1, 6 % of the outputs, 643 us where the sqrt-weight form takes 420.
 //
-// Missing values (NaN inputs ignored): x' = 0 and a third operand, the 0/1 mask of present values (exact in 16 bits),
-// contracts with -w t'^2 and with the logarithm term, three pieces each; T is that of the present values.
+// Missing values (NaN inputs ignored): both operands 0 and a third, the 0/1 mask of present values, which contracts with
+// -w (t'^2 + m) and with the logarithm term, two pieces each; T is that of the present values.
 //
 // Layout.  A workgroup of four waves computes 128 consecutive output pixels (over the batch: images are a stack of
 // padded rows, so a tile may span images and no lane idles at an image's end) x up to 128 templates.  16 channels (or
 // 8) of the rows it touches are staged in LDS as [piece][channel group of 8][pixel][8 channels], converted once and read
 // by every tap and template; a lane's matrix operand - 8 channels of its pixel - is one ds_read_b128, consecutive
 // lanes' in consecutive 16 bytes.  The parameters are packed in the order the lanes read them and come from L2 straight
-// into registers, one step ahead.  80 KB of LDS and 256 registers: two workgroups per compute unit, so that one stages
-// while the other multiplies.
+// into registers, one step ahead; the next chunk's input is requested during a chunk's last step, by buffer loads (an
+// offset per pixel, one per channel, zeros outside of the image: no 64-bit address per value).  256 registers: two
+// workgroups per compute unit, so that one stages while the other multiplies.
 //
-// Measured (whole call, vector form before -> this form): 256 x 64 x 32 x 32 -> 128, 3 x 3: 0.80 -> 0.37 ms, 1.3 PFLOP/s of
-// matrix products, what the largest library products reach on this chip: bound by the matrix units' power.  37 x 45 x
-// 29 x 35 -> 75: 172 -> 66 us, where half of the products are padding (96 templates, 48 channels, 37632 pixels).  64
-// images of the first with a quarter missing: 427 -> 159 us.  8 x 64 x 32 x 32 -> 32: 139 -> 39 us.
+// Measured (whole call, vector form, three bf16 pieces, this form): 256 x 64 x 32 x 32 -> 128, 3 x 3: 0.80, 0.372, 0.228 ms.
+// The kernel's 210 us are 1.1 PFLOP/s of matrix products at 1.55 GHz: the clock sinks with them (products of random
+// numbers alone run at 1.57 PFLOP/s and 1.65 GHz, of zeros at 2.35), 155 us would be that rate.  37 x 45 x 29 x 35 -> 75: 172, 66,
+// 50 us, where half of the products are padding (96 templates, 48 channels, 37632 pixels).  64 images of the first with a
+// quarter missing: 427, 160, 108 us.
+// Tried: 2 x 2 tiles a wave (half of the LDS reads, twice the parameter loads): 250 us for 228.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -55,6 +60,7 @@ namespace simnets {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(1))) float global_float;
@@ -65,25 +71,26 @@ enum SplitKind { SPLIT_FWD, SPLIT_MASKED /* forward, NaN inputs ignored */, SPLI
 
 // staged pixels of a chunk of 16 channels (twice as many of 8): two workgroups' tiles fit the 160 KB of a compute unit
 constexpr int split_lds_pixels(int kind) { return kind == SPLIT_MASKED ? 360 : kind == SPLIT_FWD ? 408 : 816; }
-constexpr int split_operands(int kind) { return kind == SPLIT_MASKED ? 7 : kind == SPLIT_FWD ? 6 : 3; }
+constexpr int split_operands(int kind) { return kind == SPLIT_MASKED ? 5 : kind == SPLIT_FWD ? 4 : 3; }
 constexpr int split_lds_bytes(int kind) { return split_lds_pixels(kind) * 32 * split_operands(kind); }
 // pixels of one staged plane [channel group][pixel]
 constexpr int split_plane_pixels(int kind, int cg) { return split_lds_pixels(kind) * (cg == 16 ? 1 : 2); }
-constexpr int split_pieces(int kind) { return kind == SPLIT_MASKED ? 12 : 6; }
+constexpr int split_pieces(int kind) { return kind == SPLIT_MASKED ? 8 : kind == SPLIT_FWD ? 4 : 6; }
 
 struct SplitArgs {
     const float *in;
     float *out;
-    const bf16x8 *packed;
-    const float *ctr, *bias, *lg, *thr;
+    const void *packed;
+    const float *chan, *rows;   // see SplitPack
+    const float *ctr;           // input gradient: centres of the rows
     const float2 *exact;   // see SplitPack
     const float *logs;
     int *flags;      // [pixel tile][mtile]
     int C, H, W, O, ow, npix, total;   // npix = oh ow, total = B npix
     int bw, sh, sw, ph, pw, taps, chunks, steps, n_mtiles, Wp, Hv;
     int gmax;        // matrix tiles of templates per workgroup: 4, 2 or 1
+    int per_sum;     // chunks whose products share accumulators
     float oob;
-    float line;      // missing values: an output has to reach this times its present sum w t'^2
     const float *x;  // input gradient: the forward's input, of the output's shape; templates and weights [C][O][taps]
     const float *templates, *weights;
     float scale;
@@ -144,14 +151,14 @@ struct NearOutputs {
 // LOGS: the mode has logarithm terms.  Inlined once, at the kernel's end: a call, or a copy in each split_body, spills SGPRs of
 // the bodies (37 x 45 x 29 x 35 -> 75 62 -> 65 to 72 us).
 template <int KIND, int CG, bool LOGS>
-__device__ __forceinline__ void split_recompute(lds_char *lds, int mtile0, int G, u32x4 near)
+__device__ __forceinline__ void split_recompute(lds_char *lds, int ptile, int mtile0, int G, u32x4 near)
 {
     constexpr int kLanes = 8, kTerms = 12, kOutputs = kThreads / kLanes;
     typedef NearOutputs<KIND, CG> Near;
     static_assert(sizeof(Near) <= split_lds_bytes(KIND), "in the memory of the staged pieces");
     const SplitArgs a = split_kernel_args();
     __attribute__((address_space(3))) Near &q = *(__attribute__((address_space(3))) Near *)lds;
-    const int tid = threadIdx.x, wave = tid >> 6, n0 = blockIdx.x * kSplitPixels;
+    const int tid = threadIdx.x, wave = tid >> 6, n0 = ptile * kSplitPixels;
     if (tid < 4)
         q.count[tid] = 0;
     if (tid == 4)
@@ -163,14 +170,14 @@ __device__ __forceinline__ void split_recompute(lds_char *lds, int mtile0, int G
         bits += __builtin_popcount(near[i]);
     if (bits)
         atomicAdd((int *)&q.count[wave % G], bits);
-    if (tid < G * kSplitRows && mtile0 + tid / kSplitRows < a.n_mtiles && a.thr[mtile0 * kSplitRows + tid] == INFINITY)
+    if (tid < G * kSplitRows && mtile0 + tid / kSplitRows < a.n_mtiles && a.rows[4 * (mtile0 * kSplitRows + tid) + SPLIT_THR] == INFINITY)
         atomicAdd((int *)&q.count[tid / kSplitRows], kSplitPixels * kSplitRows);
     __syncthreads();
     for (int g = 0; g < G && mtile0 + g < a.n_mtiles; ++g) {
         const int outputs = min(kSplitPixels, a.total - n0) * min(kSplitRows, a.O - (mtile0 + g) * kSplitRows);
         const bool leave = q.count[g] > min(kSplitListed, outputs / 2);
         if (tid == 0)
-            a.flags[(size_t)blockIdx.x * a.n_mtiles + mtile0 + g] = leave;
+            a.flags[(size_t)ptile * a.n_mtiles + mtile0 + g] = leave;
         if (wave % G != g || leave || !bits)
             continue;
         int slot = atomicAdd((int *)&q.total, bits);
@@ -287,18 +294,11 @@ __device__ __forceinline__ void split_recompute(lds_char *lds, int mtile0, int G
 }
 #endif
 
-// a + b + c, |c| the smallest, rounded about once: what the rounding of a + b loses is added to c.
-__device__ __forceinline__ float split_three(float a, float b, float c)
+// Input gradient.  One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
+template <int CG, int G>
+__device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, int mtile0, int flag)
 {
-    const float sum = a + b, of_b = sum - a;
-    return sum + (c + ((a - (sum - of_b)) + (b - of_b)));
-}
-
-// One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
-template <int KIND, int CG, int G>
-__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 &near, int mtile0, int flag)
-{
-    constexpr bool MASKED = KIND == SPLIT_MASKED, GRAD = KIND == SPLIT_GRAD, WHOLE = KIND == SPLIT_FWD;
+    constexpr int KIND = SPLIT_GRAD;
     constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND);
     constexpr int P = split_plane_pixels(KIND, CG);
     constexpr int kPlane = split_lds_pixels(KIND) * 32;
@@ -344,19 +344,16 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
     }
 
     // (input gradient: hi + lo = A, tm + lg = B)
-    constexpr bool FOUR = MASKED || GRAD;
-    f32x16 hi[NI], lo[NI], tm[FOUR ? NI : 1], lg[FOUR ? NI : 1];
+    f32x16 hi[NI], lo[NI], tm[NI], lg[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         hi[i] = 0.0f;
         lo[i] = 0.0f;
-        if (FOUR) {
-            tm[i] = 0.0f;
-            lg[i] = 0.0f;
-        }
+        tm[i] = 0.0f;
+        lg[i] = 0.0f;
     }
     const bool active = mtile < a.n_mtiles;
-    const bf16x8 *pp = a.packed + (size_t)(active ? mtile : 0) * a.chunks * a.steps * NA * 64 + lane;
+    const bf16x8 *pp = (const bf16x8 *)a.packed + (size_t)(active ? mtile : 0) * a.chunks * a.steps * NA * 64 + lane;
     bf16x8 next[NA];
 #pragma unroll
     for (int q = 0; q < NA; ++q)
@@ -378,26 +375,12 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                     const bool in = src[i] != 0xffffffffu && cbase + j < a.C;
                     x[j] = in ? a.in[(size_t)src[i] + (size_t)(chunk * CG + j) * plane] : a.oob;
                 }
-                bf16x8 v[7];
+                bf16x8 v[3];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    // channels behind the last have zero parameters: any finite value will do
-                    float d = cbase + j >= a.C ? 0.0f : GRAD ? x[j] : x[j] - a.ctr[cbase + j];
-                    if (MASKED) {
-                        const bool ok = d == d;
-                        v[6][j] = (__bf16)(ok && cbase + j < a.C ? 1.0f : 0.0f);
-                        d = ok ? d : 0.0f;
-                    }
-                    __bf16 p0, p1, p2;
-                    if (GRAD) {
-                        split3_any(d, p0, p1, p2);
-                        v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
-                        continue;
-                    }
-                    split3(d * d, p0, p1, p2);
+                    __bf16 p0, p1, p2;   // (channels behind the last have zero parameters: any finite value will do)
+                    split3_any(cbase + j >= a.C ? 0.0f : x[j], p0, p1, p2);
                     v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
-                    split3(d, p0, p1, p2);
-                    v[3][j] = p0; v[4][j] = p1; v[5][j] = p2;
                 }
                 char *dst = lds + (g * P + q) * 16;
 #pragma unroll
@@ -406,16 +389,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
             }
         }
         __syncthreads();
-        if (WHOLE && chunk == 0) {   // the sums begin with kSplitLead sum w t'^2
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float lead = a.bias[(active ? mtile : 0) * kSplitRows + 8 * (r / 4) + 4 * half + r % 4] *
-                                   -(kSplitLead / (1.0f + kSplitLead));
-#pragma unroll
-                for (int i = 0; i < NI; ++i)
-                    hi[i][r] = lead;
-            }
-        }
         int dh = 0, dw = 0;
         auto next_tap = [&]() {   // LDS offset of the tap (behind the last: of the first, with zero parameters)
             const int off = (dh * a.Wp + dw) * 16;
@@ -449,137 +422,410 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                 auto mul = [](f32x16 &acc, const bf16x8 &x, const bf16x8 &y) {
                     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc, 0, 0, 0);
                 };
-                if (GRAD) {
-#pragma unroll
-                    for (int f = 0; f < 6; f += 3) {
-                        f32x16 &h = f == 0 ? hi[i] : tm[i], &l = f == 0 ? lo[i] : lg[i];
-                        mul(l, A[f + 2], B[0]);
-                        mul(l, A[f], B[2]);
-                        mul(h, A[f], B[0]);
-                        mul(l, A[f + 1], B[1]);
-                        mul(l, A[f + 1], B[0]);
-                        mul(l, A[f], B[1]);
-                    }
-                    continue;
-                }
 #pragma unroll
                 for (int f = 0; f < 6; f += 3) {
-                    mul(lo[i], A[f + 2], B[f]);
-                    mul(lo[i], A[f], B[f + 2]);
-                    mul(hi[i], A[f], B[f]);
-                    mul(lo[i], A[f + 1], B[f + 1]);
-                    mul(lo[i], A[f + 1], B[f]);
-                    mul(lo[i], A[f], B[f + 1]);
+                    f32x16 &h = f == 0 ? hi[i] : tm[i], &l = f == 0 ? lo[i] : lg[i];
+                    mul(l, A[f + 2], B[0]);
+                    mul(l, A[f], B[2]);
+                    mul(h, A[f], B[0]);
+                    mul(l, A[f + 1], B[1]);
+                    mul(l, A[f + 1], B[0]);
+                    mul(l, A[f], B[1]);
                 }
-                if (MASKED)
-#pragma unroll
-                    for (int q = 2; q >= 0; --q) {
-                        mul(tm[i], A[NA - 6 + q], B[NB - 1]);
-                        mul(lg[i], A[NA - 3 + q], B[NB - 1]);
-                    }
             }
         }
     }
 
     // lane: pixel col of each tile, templates (input gradient: channels) 8 (r / 4) + 4 half + r % 4
-    if (GRAD) {
-        if (!active)
-            return;
-        float ctr[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            ctr[r] = a.ctr[mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4];
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int n = n0 + (ntile0 + i) * 32 + col;
-            if (n >= a.total)
-                continue;
-            const int img = (int)fast_div((unsigned)n, a.d_npix);
-            const size_t base = ((size_t)img * a.O + mtile * kSplitRows) * a.npix + (n - img * a.npix);
-            float x[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int ml = min(8 * (r / 4) + 4 * half + r % 4, a.O - 1 - mtile * kSplitRows);
-                x[r] = a.x[base + (size_t)ml * a.npix];
-            }
-            float v[16], any = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                v[r] = __builtin_fmaf(-(x[r] - ctr[r]), tm[i][r] + lg[i][r], hi[i][r] + lo[i][r]);
-                any = __builtin_fmaf(v[r], 0.0f, any);   // NaN once a value is not finite
-            }
-            if (any != any) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float A = split_sum(hi[i][r], lo[i][r]);
-                    v[r] = __builtin_fmaf(-(x[r] - ctr[r]), split_sum(tm[i][r], lg[i][r]), A);
-#if defined(__HIP_DEVICE_COMPILE__)
-                    if (v[r] != v[r] && __builtin_isinf(A))
-                        v[r] = split_grad_terms(img, min(mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4, a.O - 1),
-                                                n - img * a.npix, x[r]);
-#endif
-                    if (flag && x[r] != x[r])
-                        v[r] = 0.0f;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int ml = 8 * (r / 4) + 4 * half + r % 4;
-                if (mtile * kSplitRows + ml < a.O)
-                    a.out[base + (size_t)ml * a.npix] = v[r];
-            }
-        }
+    if (!active)
         return;
-    }
-    const bool norm = flag;
-    if (active) {
-        float bias[16], lgm[16], thr[16];
+    float ctr[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        ctr[r] = a.ctr[mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int n = n0 + (ntile0 + i) * 32 + col;
+        if (n >= a.total)
+            continue;
+        const int img = (int)fast_div((unsigned)n, a.d_npix);
+        const size_t base = ((size_t)img * a.O + mtile * kSplitRows) * a.npix + (n - img * a.npix);
+        float x[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int m = mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4;
-            bias[r] = a.bias[m];
-            lgm[r] = a.lg[m];
-            thr[r] = a.thr[m];
+            const int ml = min(8 * (r / 4) + 4 * half + r % 4, a.O - 1 - mtile * kSplitRows);
+            x[r] = a.x[base + (size_t)ml * a.npix];
         }
+        float v[16], any = 0.0f;
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int n = n0 + (ntile0 + i) * 32 + col;
-            if (n >= a.total)
-                continue;
-            const int img = (int)fast_div((unsigned)n, a.d_npix);
-            float *dst = a.out + ((size_t)img * a.O + mtile * kSplitRows) * a.npix + (n - img * a.npix);
+        for (int r = 0; r < 16; ++r) {
+            v[r] = __builtin_fmaf(-(x[r] - ctr[r]), tm[i][r] + lg[i][r], hi[i][r] + lo[i][r]);
+            any = __builtin_fmaf(v[r], 0.0f, any);   // NaN once a value is not finite
+        }
+        if (any != any) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int ml = 8 * (r / 4) + 4 * half + r % 4;
-                if (mtile * kSplitRows + ml >= a.O)
-                    continue;
-                float v;
-                bool fine;
-                if (MASKED) {
-                    v = split_three(hi[i][r], tm[i][r], lo[i][r]);
-                    const float mag = __builtin_fabsf(v);
-                    fine = mag < 1e37f && mag >= a.line * -tm[i][r] &&
-                           (mag >= thr[r] || (v == 0.0f && tm[i][r] == 0.0f && thr[r] < 1e37f));
-                    v = 0.5f * v + lg[i][r];
-                } else {
-                    v = split_three(hi[i][r], bias[r], lo[i][r]);
-                    const float mag = __builtin_fabsf(v);
-                    fine = mag >= thr[r] && mag < 1e37f;
-                    if (norm)
-                        v = 0.5f * v + lgm[r];
-                }
-                near[i] |= fine ? 0u : 1u << r;
-                dst[(size_t)ml * a.npix] = v;
+                const float A = split_sum(hi[i][r], lo[i][r]);
+                v[r] = __builtin_fmaf(-(x[r] - ctr[r]), split_sum(tm[i][r], lg[i][r]), A);
+#if defined(__HIP_DEVICE_COMPILE__)
+                if (v[r] != v[r] && __builtin_isinf(A))
+                    v[r] = split_grad_terms(img, min(mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4, a.O - 1),
+                                            n - img * a.npix, x[r]);
+#endif
+                if (flag && x[r] != x[r])
+                    v[r] = 0.0f;
             }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int ml = 8 * (r / 4) + 4 * half + r % 4;
+            if (mtile * kSplitRows + ml < a.O)
+                a.out[base + (size_t)ml * a.npix] = v[r];
         }
     }
 }
 
-// The template tiles of a pixel tile are dealt out as groups of gmax and, of the rest, 2 and 1.  flag: forward, the
-// normalized mode; input gradient, NaN inputs ignored.
+// How a workgroup's pixels, 128 from n0 on, lie in the stack of padded images: the virtual row of the first, and what is
+// staged for them.
+__device__ __forceinline__ int split_virtual_row(const SplitArgs &a, int n, int &img, int &c)
+{
+    img = (int)fast_div((unsigned)n, a.d_npix);
+    const int rem = n - img * a.npix, r = (int)fast_div((unsigned)rem, a.d_ow);
+    c = rem - r * a.ow;
+    return img * a.Hv + r * a.sh;
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef const __attribute__((address_space(4))) float uniform_float;
+
+// Forward.  One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel
+// tiles.
+template <int KIND, int CG, int G>
+__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 &near, int ptile, int mtile0, int norm)
+{
+    constexpr bool MASKED = KIND == SPLIT_MASKED;
+    constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND), kWaves = kThreads / 64;
+    constexpr int P = split_plane_pixels(KIND, CG);
+    constexpr int kPlane = split_lds_pixels(KIND) * 32;
+    constexpr int kHalves = CG / 8;                               // groups of eight channels
+    constexpr int kItems = (kHalves * ((P + 63) / 64) + kWaves - 1) / kWaves;   // of 64 pixels and eight channels
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    const int mtile = mtile0 + wave % G;
+    const int ntile0 = wave / G * NI;
+
+    const int n0 = ptile * kSplitPixels;
+    int img0, img1, c0, c1;
+    const int v0 = split_virtual_row(a, n0, img0, c0);
+    const int rows = split_virtual_row(a, min(n0 + kSplitPixels, a.total) - 1, img1, c1) - v0 + a.taps / a.bw;
+    const int staged = min(rows * a.Wp, P), per_half = (staged + 63) / 64;
+
+    // The images from this tile's first on, for loads that give zero outside of them (and wherever voffset is kOutside).
+    const unsigned plane = (unsigned)a.H * a.W * 4u;
+    constexpr unsigned kOutside = 0x80000000u;
+    const float *base = a.in + (size_t)img0 * a.C * a.H * a.W;
+    const size_t behind = (size_t)(a.total / a.npix - img0) * a.C * plane;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)(behind < 0x7ffffffcu ? behind : 0x7ffffffcu), 0x00020000);
+    // where this lane's staged elements come from (the same for every chunk)
+    unsigned src[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        const int item = wave + kWaves * i, g = CG == 16 && item >= per_half, q = (item - (g ? per_half : 0)) * 64 + lane;
+        const int vr = (int)fast_div((unsigned)q, a.d_wp), c = q - vr * a.Wp - a.pw;
+        const int v = v0 + vr, img = (int)fast_div((unsigned)v, a.d_hv), r = v - img * a.Hv - a.ph;
+        const bool in = q < staged && r >= 0 && r < a.H && c >= 0 && c < a.W;
+        src[i] = in ? (unsigned)((((img - img0) * a.C + 8 * g) * a.H + r) * a.W + c) * 4u : kOutside;
+    }
+    // and this lane's operands: the LDS byte address of its pixel's first tap
+    int at[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        int img, c;
+        const int v = split_virtual_row(a, min(n0 + (ntile0 + i) * 32 + col, a.total - 1), img, c);
+        at[i] = ((CG == 16 ? half * P : 0) + (v - v0) * a.Wp + c * a.sw) * 16;
+    }
+
+    // sum: of the chunks before this one, whose own is acc; with missing values tm, the present -w (t'^2 + m / s^2), and lg
+    constexpr bool TWO = !MASKED && NI <= 2;   // the two products' chunk sums apart: room for them
+    f32x16 sum[NI], acc[NI], ac2[TWO ? NI : 1], tm[MASKED ? NI : 1], lg[MASKED ? NI : 1];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        sum[i] = 0.0f;
+        acc[i] = 0.0f;
+        if (TWO)
+            ac2[i] = 0.0f;
+        if (MASKED) {
+            tm[i] = 0.0f;
+            lg[i] = 0.0f;
+        }
+    }
+    const bool active = mtile < a.n_mtiles;
+    const int taps_h = a.taps / a.bw;
+    const f16x8 *pp = (const f16x8 *)a.packed + (size_t)(active ? mtile : 0) * a.chunks * a.steps * NA * 64;
+    f16x8 next[NA];   // the packed parameters of the next step
+#pragma unroll
+    for (int q = 0; q < NA; ++q)
+        next[q] = pp[q * 64 + lane];
+
+    float x[kItems][8];
+    auto request = [&](int chunk) {   // a chunk's values of this lane's pixels, channels behind the last as the last
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            const int item = wave + kWaves * i;
+            if (item >= kHalves * per_half)
+                continue;
+            const int g = CG == 16 && item >= per_half, there = a.C - 1 - (chunk * CG + 8 * g);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                x[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                    rsrc, src[i], (chunk * CG + max(-8 * g, min(j, there))) * plane, 0));
+        }
+    };
+    request(0);
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            const int item = wave + kWaves * i;
+            if (item >= kHalves * per_half)
+                continue;
+            const int g = CG == 16 && item >= per_half, q = (item - (g ? per_half : 0)) * 64 + lane;
+            const int c0 = chunk * CG + 8 * g;
+            uniform_float *chan = (uniform_float *)(a.chan + c0);
+            if (a.oob != 0.0f)   // (a NaN too)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    x[i][j] = src[i] == kOutside ? a.oob : x[i][j];
+            if (c0 + 8 > a.C)    // channels behind the last have zero parameters: any finite value will do
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    x[i][j] = c0 + j < a.C ? x[i][j] : 0.0f;
+            f16x8 v[5];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float s = chan[SPLIT_S * a.chunks * CG + j], ncs = chan[SPLIT_NCS * a.chunks * CG + j];
+                float d = __builtin_fmaf(x[i][j], s, ncs);
+                float d2 = __builtin_fmaf(d, d, -chan[SPLIT_M * a.chunks * CG + j]);
+                if (MASKED) {
+                    const bool ok = x[i][j] == x[i][j];
+                    d = ok ? d : 0.0f;
+                    d2 = ok ? d2 : 0.0f;
+                    v[4][j] = ok ? (_Float16)1.0f : (_Float16)0.0f;
+                }
+                _Float16 hi, lo;
+                split2(d2, hi, lo);
+                v[0][j] = hi; v[1][j] = lo;
+                split2(d, hi, lo);
+                v[2][j] = hi; v[3][j] = lo;
+            }
+            if (q < staged) {
+                char *dst = lds + (g * P + q) * 16;
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    *reinterpret_cast<f16x8 *>(dst + b * kPlane) = v[b];
+            }
+        }
+        __syncthreads();
+        int dh = 0, dw = 0;
+        auto next_tap = [&]() {   // LDS offset of the next tap (behind the last: of the first, with zero parameters)
+            const int off = dh < taps_h ? (dh * a.Wp + dw) * 16 : 0;
+            if (++dw == a.bw) {
+                dw = 0;
+                ++dh;
+            }
+            return off;
+        };
+        auto next_offset = [&]() {   // of a step's operands
+            const int off = next_tap();
+            if (CG == 16)
+                return off;
+            const int off2 = next_tap();
+            return half ? off2 : off;
+        };
+        auto fetch = [&](f16x8 &to, int from, int b) { to = *reinterpret_cast<const f16x8 *>(lds + from + b * kPlane); };
+        auto mul = [](f32x16 &to, const f16x8 &p, const f16x8 &v) {
+            to = __builtin_amdgcn_mfma_f32_32x32x16_f16(p, v, to, 0, 0, 0);
+        };
+        const f16x8 low = (_Float16)(1.0f / kSplitLow);
+        f16x8 A[NA];
+        auto advance = [&](int step) {   // this step's parameters from those ahead, and the request of the next ones
+#pragma unroll
+            for (int q = 0; q < NA; ++q)
+                A[q] = next[q];
+            if (chunk + 1 < a.chunks || step + 1 < a.steps)
+                pp += NA * 64;
+#pragma unroll
+            for (int q = 0; q < NA; ++q)
+                next[q] = pp[q * 64 + lane];
+            if (step + 1 == a.steps && chunk + 1 < a.chunks)
+                request(chunk + 1);
+        };
+        int off = next_offset();
+        if (!active) {
+            if (chunk + 1 < a.chunks)
+                request(chunk + 1);
+        } else if constexpr (NI == 4) {
+            // An accumulator's products follow one another at 48 cycles, two accumulators' in turn at 32: two pixel tiles at
+            // a time, their squares while their cross terms' operands are requested, then the other way round.
+            f16x8 Bq[2][2], Be[2][2];
+            auto fetch_pair = [&](f16x8 (&to)[2][2], int pair, int from, int b) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    fetch(to[i][1], at[2 * pair + i] + from, b + 1);
+                    fetch(to[i][0], at[2 * pair + i] + from, b);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto products = [&](int pair, const f16x8 &hi, const f16x8 &lo, const f16x8 (&b)[2][2]) {
+                const f16x8 lower = hi * low;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    mul(acc[2 * pair + i], lower, b[i][1]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    mul(acc[2 * pair + i], lo, b[i][0]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    mul(acc[2 * pair + i], hi, b[i][0]);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            fetch_pair(Bq, 0, off, 0);
+            for (int step = 0; step < a.steps; ++step) {
+                advance(step);
+                const int off_next = next_offset();
+#pragma unroll
+                for (int pair = 0; pair < 2; ++pair) {
+                    fetch_pair(Be, pair, off, 2);
+                    products(pair, A[0], A[1], Bq);
+                    fetch_pair(Bq, 1 - pair, pair == 0 ? off : off_next, 0);
+                    products(pair, A[2], A[3], Be);
+                }
+                off = off_next;
+            }
+        } else {
+            constexpr int kAhead = MASKED ? 0 : 1;   // (missing values: no registers left for it)
+            f16x8 B[1 + kAhead][NB];
+            auto fetch_all = [&](f16x8 (&to)[NB], int from) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    fetch(to[b], from, b);
+            };
+            if (kAhead)
+                fetch_all(B[0], at[0] + off);
+            for (int step = 0; step < a.steps; ++step) {
+                advance(step);
+                const int off_next = next_offset();
+                const f16x8 A0 = A[0] * low, A2 = A[2] * low;
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    if (kAhead) {
+                        fetch_all(B[(i + 1) & kAhead], i + 1 < NI ? at[(i + 1) % NI] + off : at[0] + off_next);
+                        __builtin_amdgcn_sched_barrier(0);
+                    } else
+                        fetch_all(B[0], at[i] + off);
+                    const f16x8 (&b)[NB] = B[i & kAhead];
+                    f32x16 &cross = TWO ? ac2[TWO ? i : 0] : acc[i];
+                    mul(acc[i], A0, b[1]);
+                    if (MASKED)
+                        mul(lg[MASKED ? i : 0], A[NA - 1], b[NB - 1]);
+                    mul(cross, A2, b[3]);
+                    if (MASKED)
+                        mul(tm[MASKED ? i : 0], A[NA - 4], b[NB - 1]);
+                    mul(acc[i], A[1], b[0]);
+                    if (MASKED)
+                        mul(lg[MASKED ? i : 0], A[NA - 2], b[NB - 1]);
+                    mul(cross, A[3], b[2]);
+                    if (MASKED)   // (the lesser piece of what tm sums, where small sums are kept)
+                        mul(acc[i], A[NA - 3], b[NB - 1]);
+                    mul(acc[i], A[0], b[0]);
+                    mul(cross, A[2], b[2]);
+                    if (kAhead)
+                        __builtin_amdgcn_sched_barrier(0);
+                }
+                if (kAhead && (NI & 1))
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+                        B[0][b] = B[kAhead][b];
+                off = off_next;
+            }
+        }
+        // a sum of its own for every so many products: see the head of the file
+        if ((chunk + 1) % a.per_sum == 0 || chunk + 1 == a.chunks)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                sum[i] += TWO ? acc[i] + ac2[TWO ? i : 0] : acc[i];
+                acc[i] = 0.0f;
+                if (TWO)
+                    ac2[i] = 0.0f;
+            }
+    }
+
+    // lane: pixel col of each tile, templates 8 (r / 4) + 4 half + r % 4
+    if (!active)
+        return;
+    const f32x4 *rows4 = reinterpret_cast<const f32x4 *>(a.rows) + mtile * kSplitRows + 4 * half;
+    const float *lgs = a.rows + (size_t)4 * a.n_mtiles * kSplitRows + mtile * kSplitRows + 4 * half;
+    f32x4 row[16];
+    float lgm[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        row[r] = rows4[8 * (r / 4) + r % 4];
+        lgm[r] = !MASKED && norm ? lgs[8 * (r / 4) + r % 4] : 0.0f;
+    }
+    // stores by a pixel's offset and a row's; rows behind the last template go outside of the buffer
+    const int left = a.O - mtile * kSplitRows;
+    const unsigned image = (unsigned)a.npix * 4u;
+    float *tile = a.out + ((size_t)img0 * a.O + mtile * kSplitRows) * a.npix;
+    const size_t room = ((size_t)(a.total / a.npix - img0) * a.O - mtile * kSplitRows) * image;
+    const __amdgpu_buffer_rsrc_t to =
+        __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)(room < 0x7ffffffcu ? room : 0x7ffffffcu), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int n = n0 + (ntile0 + i) * 32 + col;
+        const int img = (int)fast_div((unsigned)n, a.d_npix);
+        const unsigned pixel = n < a.total ? ((unsigned)((img - img0) * a.O + 4 * half) * a.npix + (n - img * a.npix)) * 4u : kOutside;
+        unsigned flagged = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int ml = 8 * (r / 4) + r % 4;
+            float v;
+            bool fine;
+            if (MASKED) {
+                v = (sum[i][r] + tm[i][r]) * row[r][SPLIT_UNSCALE];
+                const float mag = __builtin_fabsf(v);
+                fine = mag < 1e37f && mag >= row[r][SPLIT_GUARD] * -(tm[i][r] * row[r][SPLIT_UNSCALE]) &&
+                       (mag >= row[r][SPLIT_THR] || (v == 0.0f && tm[i][r] == 0.0f && row[r][SPLIT_THR] < 1e37f));
+                v = __builtin_fmaf(0.5f, v, lg[i][r] * (1.0f / kSplitLogScale));
+            } else {
+                v = __builtin_fmaf(sum[i][r], row[r][SPLIT_UNSCALE], row[r][SPLIT_BIAS]) + row[r][SPLIT_BIAS_LESSER];
+                const float mag = __builtin_fabsf(v);
+                fine = mag >= row[r][SPLIT_THR] && mag < 1e37f;
+                if (norm)
+                    v = __builtin_fmaf(0.5f, v, lgm[r]);
+            }
+            flagged |= fine ? 0u : 1u << r;
+            unsigned at = pixel;
+            if (left < kSplitRows)
+                at = ml + 4 * half < left ? at : kOutside;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), to, at, ml * image, 0);
+        }
+        if (left < kSplitRows)   // of the rows that are templates
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                flagged &= 8 * (r / 4) + r % 4 + 4 * half < left ? ~0u : ~(1u << r);
+        near[i] = n < a.total ? flagged : 0u;
+    }
+}
+#endif
+
+// The template tiles of a pixel tile are dealt out as groups of gmax and, of the rest, 2 and 1 (forward, of four: the rest
+// as one).  flag: forward, the normalized mode; input gradient, NaN inputs ignored.
 template <int KIND, int CG>
 __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs a, int flag)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __align__(16) char split_lds[split_lds_bytes(KIND)];
     __shared__ int any_near;   // of the workgroup's outputs, one below the guard's line
     if (KIND != SPLIT_GRAD && threadIdx.x == 0)
@@ -590,33 +836,53 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
     if (y >= full) {
         const int rest = a.n_mtiles - full * a.gmax;   // 1..3
         mtile0 = full * a.gmax;
-        g = rest >= 2 ? 2 : 1;
+        g = rest == 3 && KIND == SPLIT_FWD ? 4 : rest >= 2 ? 2 : 1;
         if (y > full) {   // the last one of three
             mtile0 += 2;
             g = 1;
         }
     }
-    if (KIND == SPLIT_FWD && g == 4)
-        split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, near, mtile0, flag);
-    else if (g == 2)
-        split_body<KIND, CG, 2>(a, split_lds, near, mtile0, flag);
-    else
-        split_body<KIND, CG, 1>(a, split_lds, near, mtile0, flag);
-    if constexpr (KIND != SPLIT_GRAD) {
+    // consecutive workgroups go to the eight XCDs in turn: a run of neighbouring pixel tiles, which share rows, to each
+    const int run = gridDim.x / 8, x = blockIdx.x;
+    const int ptile = x < run * 8 ? x % 8 * run + x / 8 : x;
+    if constexpr (KIND == SPLIT_GRAD) {
+        if (g == 2)
+            split_grad_body<CG, 2>(a, split_lds, mtile0, flag);
+        else
+            split_grad_body<CG, 1>(a, split_lds, mtile0, flag);
+    } else {
+        if (KIND == SPLIT_FWD && g == 4)
+            split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, near, ptile, mtile0, flag);
+        else if (g == 2)
+            split_body<KIND, CG, 2>(a, split_lds, near, ptile, mtile0, flag);
+        else
+            split_body<KIND, CG, 1>(a, split_lds, near, ptile, mtile0, flag);
         if (near[0] | near[1] | near[2] | near[3])
             any_near = 1;
         __syncthreads();
         // (unlikely: the code behind everything else; between the bodies it costs 37 x 45 x 29 x 35 -> 75 4 us of 62)
         if (__builtin_expect(__builtin_amdgcn_readfirstlane(any_near), 0)) {
-#if defined(__HIP_DEVICE_COMPILE__)
             if (KIND == SPLIT_MASKED || flag)
-                split_recompute<KIND, CG, true>((lds_char *)split_lds, mtile0, g, near);
+                split_recompute<KIND, CG, true>((lds_char *)split_lds, ptile, mtile0, g, near);
             else
-                split_recompute<KIND, CG, KIND == SPLIT_MASKED>((lds_char *)split_lds, mtile0, g, near);
-#endif
+                split_recompute<KIND, CG, KIND == SPLIT_MASKED>((lds_char *)split_lds, ptile, mtile0, g, near);
         } else if ((int)threadIdx.x < g && mtile0 + (int)threadIdx.x < a.n_mtiles)
-            a.flags[(size_t)blockIdx.x * a.n_mtiles + mtile0 + threadIdx.x] = 0;
+            a.flags[(size_t)ptile * a.n_mtiles + mtile0 + threadIdx.x] = 0;
     }
+#endif
+}
+
+// The sum of a channel's sampled template elements, and their mean.
+__device__ __forceinline__ float split_grad_centre_part(const SplitPack &a, int c)
+{
+    const SplitSample s = split_sample(a, c);
+    return (s.there[0] ? s.t[0] : 0.0f) + (s.there[1] ? s.t[1] : 0.0f);
+}
+
+__device__ __forceinline__ float split_grad_centre(const SplitPack &a, float part)
+{
+    part = split_sample_sum(part) / (float)min(32, a.O * a.taps);
+    return __builtin_fabsf(part) < 1e18f ? part : 0.0f;
 }
 
 // Packs the input gradient's coefficients, rows = input channels, contraction = (template, flipped tap): three pieces
@@ -630,10 +896,10 @@ __global__ __launch_bounds__(kThreads) void sim_split_grad_pack_kernel(const Spl
     float sum[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-        sum[i] = split_centre_part(a, mtile * kSplitRows + 16 * i + (tid >> 4));
+        sum[i] = split_grad_centre_part(a, mtile * kSplitRows + 16 * i + (tid >> 4));
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const float c = split_centre(a, sum[i]);
+        const float c = split_grad_centre(a, sum[i]);
         if ((tid & 15) == 0) {
             centre[16 * i + (tid >> 4)] = c;
             if (chunk == 0 && part == 0)
@@ -685,6 +951,10 @@ static SplitPlan split_geometry(const SimPlan &p, int kind)
     if (p.C > kSplitMaxC || 1LL * p.B * p.C * p.H * p.W >= (1LL << 31) || total >= (1LL << 30) ||
         1LL * p.B * ((p.oh - 1) * p.sh + p.bh) >= (1LL << 30))
         return s;
+    // a workgroup addresses the images it touches by 31 bits
+    const long long touched = (kSplitPixels - 1) / (1LL * p.oh * p.ow) + 2;
+    if (kind != SPLIT_GRAD && 4 * touched * std::max(1LL * p.C * p.H * p.W, 1LL * p.O * p.oh * p.ow) >= (1LL << 31))
+        return s;
     s.Wp = (p.ow - 1) * p.sw + p.bw;
     s.Hv = (p.oh - 1) * p.sh + p.bh;
     // the most rows of the stack that 128 consecutive pixels touch
@@ -715,11 +985,9 @@ static SplitPlan split_geometry(const SimPlan &p, int kind)
         return s;
     const int mpad = s.n_mtiles * kSplitRows;
     s.packed = 0;
-    s.ctr = s.packed + (size_t)s.n_mtiles * s.chunks * s.steps * s.pieces * 1024;
-    s.bias = s.ctr + align_up((size_t)std::max(s.chunks * s.cg, mpad) * sizeof(float), 256);
-    s.lg = s.bias + align_up((size_t)mpad * sizeof(float), 256);
-    s.thr = s.lg + align_up((size_t)mpad * sizeof(float), 256);
-    s.flags = s.thr + align_up((size_t)mpad * sizeof(float), 256);
+    s.chan = s.packed + (size_t)s.n_mtiles * s.chunks * s.steps * s.pieces * 1024;
+    s.rows = s.chan + align_up((size_t)std::max(SPLIT_CHANNEL_FIELDS * s.chunks * s.cg, mpad) * sizeof(float), 256);
+    s.flags = s.rows + align_up((size_t)5 * mpad * sizeof(float), 256);
     s.exact = s.flags + align_up((size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
     s.logs = s.exact + (kind == SPLIT_GRAD ? 0 : align_up((size_t)p.O * p.K * sizeof(float2), 256));
     s.total = s.logs + (kind == SPLIT_GRAD || p.mode == SIM_MODE_L2 ? 0 : align_up((size_t)p.O * p.K * sizeof(float), 256));
@@ -744,18 +1012,18 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     SplitPack a;
     a.templates = templates; a.weights = weights;
     a.packed = reinterpret_cast<unsigned short *>(ws + sp.packed);
-    a.ctr = reinterpret_cast<float *>(ws + sp.ctr);
-    a.bias = reinterpret_cast<float *>(ws + sp.bias);
-    a.lg = reinterpret_cast<float *>(ws + sp.lg);
-    a.thr = reinterpret_cast<float *>(ws + sp.thr);
+    a.chan = a.ctr = reinterpret_cast<float *>(ws + sp.chan);
+    a.rows = reinterpret_cast<float *>(ws + sp.rows);
     a.exact = reinterpret_cast<float2 *>(ws + sp.exact);
     a.logs = reinterpret_cast<float *>(ws + sp.logs);
     a.O = p.O; a.C = p.C; a.taps = p.bh * p.bw; a.K = p.K; a.cg = sp.cg; a.chunks = sp.chunks; a.steps = sp.steps;
     a.pieces = sp.pieces; a.n_mtiles = sp.n_mtiles; a.mode = p.mode; a.fudge = p.fudge;
     a.line = split_line(p.K);
+    a.d_taps = make_fast_div((unsigned)a.taps);
+    a.d_steps = make_fast_div((unsigned)std::max(1, sp.steps));
     a.norm_const = p.mode == SIM_MODE_L2_NORM ? split_norm_const(p.K) : 0.0f;
     a.pack_blocks = sp.on ? sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4) : 0;
-    a.thr_blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows, 512) : 0;
+    a.blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows, 512) : 0;
     return a;
 }
 
@@ -764,11 +1032,9 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
                         hipStream_t s, SplitArgs a = {})
 {
     a.in = input; a.out = output;
-    a.packed = reinterpret_cast<const bf16x8 *>(ws + sp.packed);
-    a.ctr = reinterpret_cast<const float *>(ws + sp.ctr);
-    a.bias = reinterpret_cast<const float *>(ws + sp.bias);
-    a.lg = reinterpret_cast<const float *>(ws + sp.lg);
-    a.thr = reinterpret_cast<const float *>(ws + sp.thr);
+    a.packed = ws + sp.packed;
+    a.chan = a.ctr = reinterpret_cast<const float *>(ws + sp.chan);
+    a.rows = reinterpret_cast<const float *>(ws + sp.rows);
     a.flags = reinterpret_cast<int *>(ws + sp.flags);
     a.exact = reinterpret_cast<const float2 *>(ws + sp.exact);
     a.logs = reinterpret_cast<const float *>(ws + sp.logs);
@@ -778,7 +1044,7 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     a.bw = p.bw; a.sh = p.sh; a.sw = p.sw; a.ph = p.ph; a.pw = p.pw; a.taps = p.bh * p.bw;
     a.chunks = sp.chunks; a.steps = sp.steps; a.n_mtiles = sp.n_mtiles; a.Wp = sp.Wp; a.Hv = sp.Hv;
     a.oob = p.oob;
-    a.line = split_line(p.K);
+    a.per_sum = std::max(1, 2 / sp.steps);
     a.d_npix = make_fast_div((unsigned)a.npix);
     a.d_ow = make_fast_div((unsigned)p.ow);
     a.d_wp = make_fast_div((unsigned)sp.Wp);
@@ -790,7 +1056,7 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     while (a.gmax > 1 && (a.gmax / 2 >= sp.n_mtiles || (long long)sp.n_ptiles * ((sp.n_mtiles + a.gmax - 1) / a.gmax) < 256))
         a.gmax /= 2;
     const int rest = sp.n_mtiles % a.gmax;
-    const dim3 grid((unsigned)sp.n_ptiles, (unsigned)(sp.n_mtiles / a.gmax + (rest == 0 ? 0 : rest == 3 ? 2 : 1)));
+    const dim3 grid((unsigned)sp.n_ptiles, (unsigned)(sp.n_mtiles / a.gmax + (rest == 0 ? 0 : rest == 3 && KIND != SPLIT_FWD ? 2 : 1)));
     if (sp.cg == 16)
         hipLaunchKernelGGL((sim_split_kernel<KIND, 16>), grid, dim3(kThreads), 0, s, a, flag);
     else
