@@ -414,3 +414,67 @@ def test_split_form_recomputes_outputs_near_a_template_alone(pkg, shape, O, bloc
     assert float(err) <= K * 2.0 ** -24, float(err)
     if near * got.shape[3] * (block + 1) // 2 <= 128:    # patches that reach half way into those rows are near, too
         assert torch.equal(pkg.similarity(other, t, w, **kw)[1:], got[1:])
+
+
+@pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
+@pytest.mark.parametrize("kind", ["channels", "templates", "far", "small", "sparse", "equal"])
+@pytest.mark.parametrize("geom", [GEOMS[1], GEOMS[11], GEOMS[7]])   # chunks of 16 and 8 channels, a single tap
+def test_split_form_scales(pkg, geom, kind, mode):
+    """Half-precision pieces of values of any size: channels and templates of very different scales, inputs far from the
+    templates and close to zero, weights mostly zero, templates that tell no scale.  Bound: test_split_form_matches_64_bits;
+    the size of an output is that of its logarithms' sum where that is the larger."""
+    g = torch.Generator(device="cuda").manual_seed(61)
+    shape, O, blocks = geom["shape"], geom["O"], geom["blocks"]
+    x = torch.randn(shape, generator=g, device="cuda")
+    t = torch.randn((O, shape[1], *blocks), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    if kind == "channels":
+        f = 10.0 ** (torch.rand((shape[1], 1, 1), generator=g, device="cuda") * 6 - 3)
+        x, t, w = x * f, t * f, w / f ** 2
+    elif kind == "templates":
+        w *= 10.0 ** (torch.rand((O, 1, 1, 1), generator=g, device="cuda") * 8 - 5)
+    elif kind == "far":
+        x *= 300.0
+    elif kind == "small":
+        x *= 1e-3
+    elif kind == "sparse":
+        w *= torch.rand(t.shape, generator=g, device="cuda") < 0.05
+    elif kind == "equal":
+        t.fill_(0.25)
+    kw = options(mode, geom)
+    oob = kw.setdefault("out_of_bounds_value", geom.get("out_of_bounds_value", 0.0))
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    got = pkg.similarity(x, t, w, **kw).double()
+    want = exact(x, t, w, blocks, geom["strides"], geom["padding"], mode, oob)
+    K = shape[1] * blocks[0] * blocks[1]
+    size = want.abs()
+    if mode != "l2":
+        logs = 0.5 * (K * math.log(2 * math.pi) + torch.log(w.double() + 0.001).abs().flatten(1).sum(1))
+        size = torch.maximum(size, logs[None, :, None, None])
+    size = size.clamp_min(1e-30)
+    assert float(((got - want).abs() / size).max()) <= 2 * (K / 16 + 8) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("O, block", [(64, 3), (63, 3), (23, 5), (24, 5), (144, 2)])    # 576, 567, 575, 600, 576 terms
+def test_split_input_gradient_scales(pkg, O, block):
+    """Either side of the line between two and three pieces, images whose output gradients differ by 10^35, channels whose
+    weights and templates do: each image and channel by itself has the error of its own sums."""
+    g = torch.Generator(device="cuda").manual_seed(67)
+    B, C, H, W = 36, 37, 23, 30
+    f = 10.0 ** (torch.rand((C, 1, 1), generator=g, device="cuda") * 6 - 3)
+    x = torch.randn((B, C, H, W), generator=g, device="cuda") * f
+    t = torch.randn((O, C, block, block), generator=g, device="cuda") * f
+    w = (torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1) / f ** 2
+    go = torch.randn((B, O, H - block + 1, W - block + 1), generator=g, device="cuda")
+    go *= 10.0 ** torch.linspace(-20, 15, B, device="cuda")[:, None, None, None]
+    go[5] = 0.0
+    kw = dict(blocks=[block, block], strides=[1, 1], padding=[0, 0])
+    assert pieces_used(pkg, (B, C, H, W), O, **kw)["input"]
+    got = pkg.similarity_input_grad(x, t, w, go, **kw).double().cpu()
+    xd, td, wd, gd = (v.double().cpu() for v in (x, t, w, go))
+    up = lambda k: torch.nn.functional.conv_transpose2d(gd, k)
+    want = 2 * (up(wd * td) - xd * up(wd))
+    assert not got[5].any()
+    err = (got - want).flatten(2).norm(dim=2) / want.flatten(2).norm(dim=2).clamp_min(1e-300)
+    assert float(err.max()) <= 4 * math.sqrt(O * block * block) * 2.0 ** -24, float(err.max())
