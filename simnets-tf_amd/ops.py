@@ -50,15 +50,6 @@ def _current_stream(device):
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def _freeze(v):
-    """Hashable form of an attribute value (floats by repr: NaN out-of-bounds values must compare equal)."""
-    if isinstance(v, (list, tuple)):
-        return tuple(_freeze(e) for e in v)
-    if isinstance(v, dict):
-        return tuple(sorted((k, _freeze(e)) for k, e in v.items()))
-    return repr(v) if isinstance(v, float) else v
-
-
 def similarity_attrs(templates_shape=None, similarity_function=None, blocks=None, strides=None, padding=None,
                      normalization_term=None, normalization_term_fudge=None, ignore_nan_input=None,
                      out_of_bounds_value=None, algo=None, norm_const_every_iteration=False):
