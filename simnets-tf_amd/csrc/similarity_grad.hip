@@ -18,7 +18,7 @@
 // Parameter gradients
 //   dT[o,k], dW[o,k] = sum over all B*oh*ow output pixels of W(g[px,o], patch(px)[k], t[o,k], w[o,k]).
 //   A lane owns 8 templates x 4 patch elements (its t values and the running sums in VGPRs), a wave
-//   64 x 32, a workgroup 128 x 64 (or 64 x 128); pixels stream through LDS in chunks of 64, g as
+//   64 x 32, a workgroup 128 x 64 (or 64 x 128); pixels stream through LDS in chunks of 32, g as
 //   [o/4][pixel][4] and the gathered patch elements as [k/4][pixel][4], so that every lane reads its
 //   operands with three 16-byte LDS reads per pixel.  The pixel range is split over workgroups; the
 //   partial sums are written out and added up in a fixed order by a second kernel, which also
@@ -39,6 +39,15 @@ namespace simnets {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+
+// The halves of a pair in an even register and the odd one behind it.  A vector instruction whose three sources lie in
+// registers of one parity does not issue beside another wave's; left to the compiler, half of the L1 gradients'
+// three-source instructions were such.
+__device__ __forceinline__ void pin_pair(const floatx2 &v)
+{
+    asm volatile("" : : "v"(v));
+}
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
@@ -96,12 +105,17 @@ __device__ __forceinline__ void gx_step(float (&acc)[MT][PT], const float (&xv)[
             // median with -|w| and |w| is w * sign(t - x) (exactly 0 for t == x).  NaN inputs never get here:
             // the tile holds 0 in their place and their gradient is stored as 0, which is what sign(NaN) = 0
             // gives in the reference.
-            const float nbig = -__builtin_copysignf(0x1p100f, p1);
+            floatx2 big;
+            big.y = __builtin_copysignf(0x1p100f, p1);
+            // p0 is in an even register, p1 in an odd one; with the sums' pairs below, 176 -> 52 instructions of 384 with
+            // sources of one parity and 16 sign changes fewer: 32 x 64 x 32 x 32, 128 templates, 3 x 3: 237 -> 222 us.  The
+            // differences in even registers too (none of one parity) cost 58 copies to two steps.
+            pin_pair(big);
             const float lim = __builtin_fabsf(p1);
             float d[PT];
 #pragma unroll
             for (int p = 0; p < PT; ++p)
-                d[p] = __builtin_fmaf(nbig, xv[m][p], p0);
+                d[p] = __builtin_fmaf(-big.y, xv[m][p], p0);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int p = 0; p < PT; ++p)
@@ -111,6 +125,12 @@ __device__ __forceinline__ void gx_step(float (&acc)[MT][PT], const float (&xv)[
 #pragma unroll
         for (int p = 0; p < PT; ++p)
             acc[m][p] = __builtin_fmaf(gv[p], u[p], acc[m][p]);
+        if (MODE == GX_L1)   // (gv of even pixels is in an even register)
+#pragma unroll
+            for (int p = 0; p < PT; p += 2) {
+                const floatx2 pair = {acc[m][p + 1], acc[m][p]};
+                pin_pair(pair);
+            }
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -791,6 +811,7 @@ struct GradPArgs {
     int nchunks, cps;  // pixel chunks in total, and per split
     int S;
     float oob;
+    FastDiv d_ow, d_ohow;
 };
 
 // MODE: SimMode of the forward op.  WO: waves along the templates (1 or 2).
@@ -802,10 +823,12 @@ struct GradPArgs {
 // instructions; the finish kernel combines the moments in double precision.  The centre keeps tc of the order
 // of the spread of the templates, which bounds the cancellation: the error is eps sqrt(N) |g| (xc^2 + tc^2),
 // the same order as that of the term-by-term sums unless every template and every patch sit in one point.
-// MOM (L1): scaled-sign form.  With dB = 2^64 (x - t) (one fma against the pre-scaled template; exact scaling),
-// sign(x - t) = med3(dB, -1, 1) and |x - t| = 2^-64 |dB|: four instructions per term (fma, med3, fma, fma against
-// g and 2^-64 g) instead of seven with compares and selects, bit-identical to them unless 0 < |x - t| < 2^-64,
-// |g| < 2^-62 or a value beyond 2^63.  A pixel chunk with a NaN input (found while staging, uniform for the
+// MOM (L1): scaled-sign form.  With d = x - t, 2^-64 sign(d) = med3(d, -2^-64, 2^-64): four instructions per term (sub,
+// med3, fma, fma) instead of seven with compares and selects; the sum of g sign(d) is scaled back where it leaves,
+// bit-identical to them unless 0 < |x - t| < 2^-64 or |g| < 2^-62.  32 x 64 x 32 x 32, 128 templates, 3 x 3: 267 -> 241 us
+// with two-source differences, stages of eight, the pairs (d, sign) and (sum, sum) across the parities, and staging
+// without branches (1030 -> 340 instructions a chunk); two waves to a SIMD issue one instruction per 3.3 cycles (instruction
+// streams of this kind without memory: 2.7).  A pixel chunk with a NaN input (found while staging, uniform for the
 // workgroup) takes the compare-and-select arithmetic, which has the reference's NaN rules.
 // MF (with MOM, L2 modes): the moments on the fp32 matrix cores.  S1 = g^T xc, S2 = g^T xc^2 (and, with ignore-NaN,
 // G = g^T keep) are contractions over the pixels: a wave's 64 templates x 32 patch elements are two
@@ -891,13 +914,19 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
         for (int kk = 0; kk < LK; ++kk) {
             const bool ok = !MF && lane_o(oo) < a.O && k0 + kk < a.K;
             t[oo][kk] = ok ? t[oo][kk] : 0.0f;
-            if constexpr (SGN)
-                t[oo][kk] *= 0x1p64f;
             at[oo][kk] = 0.0f;
             aw[oo][kk] = 0.0f;
             if constexpr (NORM)
                 an[oo][kk] = 0.0f;
         }
+    // scaled-sign form: 2^-64 in a vector register (a constant of the instruction, or a scalar one, halves its rate)
+    floatx2 unit = {0.0f, 0x1p-64f};
+    if constexpr (SGN) {
+        float v;
+        asm volatile("v_mov_b32 %0, 0x1f800000" : "=v"(v));
+        unit.y = v;
+        pin_pair(unit);
+    }
     // moment form: centre per patch element of this lane
     float ctr[LK] = {0.0f, 0.0f, 0.0f, 0.0f};
     // matrix-core form: this lane's column (patch element) and pixel parity, the centre of the column, accumulators
@@ -948,44 +977,66 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
     const int g_row = (wo * 16 + lo) * PCP, x_row = (wk * 8 + lk) * PCP;
 
     // global -> registers: the g values and the patch elements (im2col_3d rule: outside the image -> oob) of
-    // pixel sp of a chunk, four templates / four patch elements per float4
-    auto load_chunk = [&](int chunk, float4 (&gv)[GR], float4 (&xv)[XR]) {
-        const long long q = (long long)chunk * PC + sp;
-        const bool qok = q < a.npix;
-        const long long qq = qok ? q : 0;
-        const int b = (int)(qq / ohow);
-        const int pix = (int)(qq - (long long)b * ohow);
-        const int yo = pix / a.ow, xo = pix - yo * a.ow;
-        const float *gb = a.g + ((size_t)b * a.O) * ohow + pix;
+    // pixel sp of the next chunk, four templates / four patch elements per float4.  The chunks come in order, so the
+    // pixel's image and place are carried along; every load is made, on an address inside the array, and what does not
+    // count is replaced behind it (a load inside a condition costs some ten scalar instructions and a branch).
+    const int chunk_begin = split * a.cps;
+    const int chunk_end = min((split + 1) * a.cps, a.nchunks);
+    const long long q_first = (long long)chunk_begin * PC + sp;
+    int load_b = (int)(q_first / ohow), load_pix = (int)(q_first - (long long)load_b * ohow);
+    auto load_chunk = [&](float4 (&gv)[GR], float4 (&xv)[XR]) {
+        const bool qok = load_b < a.B;
+        const int b = min(load_b, a.B - 1), pix = load_pix;
+        const int yo = (int)fast_div((unsigned)pix, a.d_ow), xo = pix - yo * a.ow;
+        const int on = (int)fast_div((unsigned)(pix + PC), a.d_ohow);
+        load_b += on;
+        load_pix = pix + PC - on * ohow;
+        const int o0 = o_wg + sg * 4;
+        const float *gb = a.g + ((size_t)b * a.O + min(o0, a.O - 1)) * ohow + pix;
+        if (o_wg + OWG <= a.O) {
 #pragma unroll
-        for (int r = 0; r < GR; ++r) {
-            const int o = o_wg + (sg + NSG * r) * 4;
-            float e[4];
+            for (int r = 0; r < GR; ++r) {
+                gv[r].x = gb[(size_t)(4 * NSG * r + 0) * ohow];
+                gv[r].y = gb[(size_t)(4 * NSG * r + 1) * ohow];
+                gv[r].z = gb[(size_t)(4 * NSG * r + 2) * ohow];
+                gv[r].w = gb[(size_t)(4 * NSG * r + 3) * ohow];
+            }
+        } else {
+            const int last = max(a.O - 1 - o0, 0);
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                e[u] = (qok && o + u < a.O) ? gb[(size_t)(o + u) * ohow] : 0.0f;
-            gv[r] = make_float4(e[0], e[1], e[2], e[3]);
+            for (int r = 0; r < GR; ++r) {
+                float e[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    e[u] = gb[(size_t)min(4 * NSG * r + u, last) * ohow];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    e[u] = o0 + 4 * NSG * r + u < a.O ? e[u] : 0.0f;
+                gv[r] = make_float4(e[0], e[1], e[2], e[3]);
+            }
         }
         const int iy0 = yo * a.sh - a.ph, ix0 = xo * a.sw - a.pw;
-        const float *xb = a.x + (size_t)b * a.C * a.H * a.W + (ptrdiff_t)iy0 * a.W + ix0;
+        const float *xb = a.x + (size_t)b * a.C * a.H * a.W;
+        const int at0 = iy0 * a.W + ix0;
+        float e[XR][4];
 #pragma unroll
-        for (int r = 0; r < XR; ++r) {
-            const int kk = (sg + NSG * r) * 4;
-            float e[4];
+        for (int r = 0; r < XR; ++r)
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int kofs = ktab[2 * (kk + u)], ij = ktab[2 * (kk + u) + 1];
+                const int kk = (sg + NSG * r) * 4 + u;
+                const int kofs = ktab[2 * kk], ij = ktab[2 * kk + 1];
                 const int iy = iy0 + (ij >> 16), ix = ix0 + (ij & 0xffff);
-                float val = 0.0f;
-                if (qok && kofs >= 0) {
-                    val = a.oob;
-                    if (iy >= 0 && iy < a.H && ix >= 0 && ix < a.W)
-                        val = xb[kofs];
-                }
-                e[u] = val;
+                const bool used = kofs >= 0, in = ((unsigned)iy < (unsigned)a.H) & ((unsigned)ix < (unsigned)a.W) & used;
+                const float v = xb[in ? kofs + at0 : 0];
+                e[r][u] = (qok & used) ? (in ? v : a.oob) : 0.0f;
             }
-            xv[r] = make_float4(e[0], e[1], e[2], e[3]);
-        }
+#pragma unroll
+        for (int r = 0; r < XR; ++r)
+            xv[r] = make_float4(e[r][0], e[r][1], e[r][2], e[r][3]);
+        if (!qok)
+#pragma unroll
+            for (int r = 0; r < GR; ++r)
+                gv[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     };
     // registers -> LDS buffer `buf`: g as [o/4][pixel][4], patch elements as [k/4][pixel][4]
     // moment form without ignore-NaN: sum of g per template.  Every chunk passes through store_chunk once, so the
@@ -1007,8 +1058,6 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
             reinterpret_cast<float4 *>(xs[buf])[(sg + NSG * r) * PCP + sp] = xv[r];
     };
 
-    const int chunk_begin = split * a.cps;
-    const int chunk_end = min((split + 1) * a.cps, a.nchunks);
     // matrix-core form, one chunk: two pixels per step, rows = templates (g at ga, second tile a1_off further),
     // columns = patch elements (xc, xc^2, keep from xb); `ps` floats from pixel to pixel; the reads of the next step
     // are issued before this step's matrix instructions
@@ -1139,7 +1188,7 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
     };
     bool nan_chunk = false;  // scaled-sign form: the chunk in use holds a NaN input (uniform for the workgroup)
     if (chunk_begin < chunk_end && !ROW) {
-        load_chunk(chunk_begin, gv, xv);
+        load_chunk(gv, xv);
         store_chunk(0, gv, xv);
         if constexpr (SGN)
             nan_chunk = has_nan(xv);
@@ -1152,38 +1201,50 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
         const int buf = (chunk - chunk_begin) & 1;
         const bool more = chunk + 1 < chunk_end;
         if (more)
-            load_chunk(chunk + 1, gv, xv);   // in flight while this chunk is used
+            load_chunk(gv, xv);   // in flight while this chunk is used
         const float4 *g4 = reinterpret_cast<const float4 *>(gs[buf]) + g_row;
         const float4 *x4 = reinterpret_cast<const float4 *>(xs[buf]) + x_row;
 
-        // scaled-sign form of a pixel (chunks without NaN inputs)
+        // scaled-sign form of a pixel (chunks without NaN inputs): eight pairs at a time and stage by stage, so that no
+        // instruction directly follows its producer
         auto compute_sgn = [&](const float4 &ga, const float4 &gb2, const float4 &xq) {
             const float gl[LO] = {ga.x, ga.y, ga.z, ga.w, gb2.x, gb2.y, gb2.z, gb2.w};
             const float xl[LK] = {xq.x, xq.y, xq.z, xq.w};
-            float gsc[LO];
 #pragma unroll
-            for (int oo = 0; oo < LO; ++oo)
-                gsc[oo] = gl[oo] * 0x1p-64f;
+            for (int o2 = 0; o2 < LO; o2 += 2) {
+                floatx2 d[2 * LK];   // the difference and its sign
 #pragma unroll
-            for (int oo = 0; oo < LO; ++oo)
+                for (int i = 0; i < 2 * LK; ++i)
+                    d[i].x = xl[i % LK] - t[o2 + i / LK][i % LK];
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int kk = 0; kk < LK; ++kk) {
-                    const float db = __builtin_fmaf(xl[kk], 0x1p64f, -t[oo][kk]);
-                    const float sg = __builtin_amdgcn_fmed3f(db, -1.0f, 1.0f);
-                    at[oo][kk] = __builtin_fmaf(sg, gl[oo], at[oo][kk]);
-                    aw[oo][kk] = __builtin_fmaf(gsc[oo], __builtin_fabsf(db), aw[oo][kk]);
+                for (int i = 0; i < 2 * LK; ++i)
+                    d[i].y = __builtin_amdgcn_fmed3f(d[i].x, -unit.y, unit.y);
+#pragma unroll
+                for (int i = 0; i < 2 * LK; ++i)
+                    pin_pair(d[i]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 2 * LK; ++i) {
+                    const int oo = o2 + i / LK, kk = i % LK;
+                    aw[oo][kk] = __builtin_fmaf(gl[oo], __builtin_fabsf(d[i].x), aw[oo][kk]);
                 }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 2 * LK; ++i) {
+                    const int oo = o2 + i / LK, kk = i % LK;
+                    at[oo][kk] = __builtin_fmaf(d[i].y, gl[oo], at[oo][kk]);
+                    const floatx2 sums = {at[oo][kk], aw[oo][kk]};
+                    pin_pair(sums);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         };
-        // scaled-sign form, chunk with a NaN input: the compare-and-select arithmetic below on the templates scaled
-        // back.  The factor is opaque to the compiler (set per pixel) so that the 32 products are formed where they
-        // are used and not kept in registers.
+        // scaled-sign form, chunk with a NaN input: the compare-and-select arithmetic below
         auto compute = [&](const float4 &ga, const float4 &gb2, const float4 &xq) {
             const float gl[LO] = {ga.x, ga.y, ga.z, ga.w, gb2.x, gb2.y, gb2.z, gb2.w};
             float xl[LK] = {xq.x, xq.y, xq.z, xq.w};
             float keep[LK];
-            float unscale = 1.0f;
-            if constexpr (SGN)
-                asm volatile("v_mov_b32 %0, 0x1f800000" : "=v"(unscale));  // 2^-64
             if constexpr (MOM2) {
                 float xc[LK], x2[LK];
 #pragma unroll
@@ -1217,7 +1278,7 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
                 float d[LK], e[LK], gg[LK];
 #pragma unroll
                 for (int kk = 0; kk < LK; ++kk) {
-                    d[kk] = xl[kk] - (SGN ? t[oo][kk] * unscale : t[oo][kk]);
+                    d[kk] = xl[kk] - t[oo][kk];
                     gg[kk] = IGN ? gl[oo] * keep[kk] : gl[oo];
                 }
                 if (L1) {
@@ -1225,7 +1286,7 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
                     for (int kk = 0; kk < LK; ++kk) {
                         float sgn = d[kk] < 0.0f ? -gg[kk] : gg[kk];
                         sgn = __builtin_islessgreater(d[kk], 0.0f) ? sgn : 0.0f;
-                        at[oo][kk] += sgn;
+                        at[oo][kk] = SGN ? __builtin_fmaf(sgn, unit.y, at[oo][kk]) : at[oo][kk] + sgn;
                         aw[oo][kk] = __builtin_fmaf(gg[kk], __builtin_fabsf(d[kk]), aw[oo][kk]);
                     }
                 } else {
@@ -1302,7 +1363,8 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
 #pragma unroll
     for (int oo = 0; oo < LO && !MF; ++oo) {
         const size_t o = (size_t)lane_o(oo) * a.Kpad + k0;
-        *reinterpret_cast<float4 *>(pt + o) = make_float4(at[oo][0], at[oo][1], at[oo][2], at[oo][3]);
+        constexpr float kBack = SGN ? 0x1p64f : 1.0f;
+        *reinterpret_cast<float4 *>(pt + o) = make_float4(at[oo][0] * kBack, at[oo][1] * kBack, at[oo][2] * kBack, at[oo][3] * kBack);
         *reinterpret_cast<float4 *>(pw + o) = make_float4(aw[oo][0], aw[oo][1], aw[oo][2], aw[oo][3]);
         if constexpr (IGN || (NORM && !MOM))
             *reinterpret_cast<float4 *>(pn + o) = make_float4(an[oo][0], an[oo][1], an[oo][2], an[oo][3]);
@@ -1766,6 +1828,8 @@ int sim_grad_params(const SimPlan &p, const float *input, const float *templates
     a.npix = (long long)p.B * p.oh * p.ow;
     a.nchunks = t.nchunks; a.cps = t.cps; a.S = t.S;
     a.oob = p.oob;
+    a.d_ow = make_fast_div((unsigned)p.ow);
+    a.d_ohow = make_fast_div((unsigned)(p.oh * p.ow));
     hipError_t e;
     switch (p.mode) {
     case SIM_MODE_L1: e = gp_launch<SIM_MODE_L1>(a, t, s); break;

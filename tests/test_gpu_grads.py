@@ -550,6 +550,27 @@ def test_similarity_l1_params_grad_scaled_sign_form_equals_the_term_by_term_form
     assert_grad_close(np.where(ok, fast[1], 0), np.where(ok, want_dw, 0), np.where(ok, true_dw, 0), "weights grad")
 
 
+@pytest.mark.parametrize("shape,O,block,stride", [
+    ((5, 8, 5, 6), 128, 3, 1),     # a whole template tile; a chunk of 32 pixels holds parts of two images, the last is short
+    ((70, 16, 3, 3), 129, 3, 2),   # images of 4 pixels, one template past the tile
+    ((37, 20, 1, 1), 64, 1, 1),    # images of one pixel, the tile of 64 templates
+    ((3, 3, 40, 33), 7, 5, 1),     # few templates
+])
+def test_similarity_l1_params_grad_staging(pkg, shape, O, block, stride):
+    """The chunks of 32 output pixels that the L1 parameter gradients stage: maps smaller than a chunk, a short last chunk,
+    whole and ragged template tiles; both forms, negative weights among the templates."""
+    x, t, w = sim_inputs(23, shape, O, (block, block))
+    w[::3] *= -1.0
+    kw = dict(similarity_function="L1", blocks=[block, block], strides=[stride, stride], padding=[block // 2, block // 2],
+              out_of_bounds_value=0.5)
+    check_sim_grads(pkg, x, t, w, **kw)
+    og = np.random.default_rng(9).normal(size=orc.similarity_fwd(x, t, w, **kw).shape).astype(np.float32)
+    fast = pkg.similarity_parameters_grad(dev(x), dev(t), dev(w), dev(og), **kw)
+    exact = pkg.similarity_parameters_grad(dev(x), dev(t), dev(w), dev(og), algo="direct", **kw)
+    for a, b in zip(fast, exact):
+        assert np.array_equal(a.cpu().numpy(), b.cpu().numpy())
+
+
 @pytest.mark.parametrize("func,norm,ign", [("L2", False, False), ("L2", True, False), ("L2", True, True)])
 @pytest.mark.parametrize("case", [
     dict(shape=(3, 5, 9, 32), O=70, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),     # ow = 32, ragged O and K
