@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256, PX == 2 ? 4 : 1) void mex_fwd_kernel(const Mex
                 bool ok = true;
                 if (CHECK) {
                     const int ci = gp.ci0 + ke.y, hi_ = gp.hi0 + ke.z, wi = gp.wi0 + ke.w;
-                    ok = ci >= 0 && ci < a.C && hi_ >= 0 && hi_ < a.H && wi >= 0 && wi < a.W;
+                    ok = mex_inside(a, ci, hi_, wi);
                 }
                 const float raw = *(ok ? gp.base + ke.x : a.in);   // (always a valid address)
                 const float v = (ok ? raw : a.oob) * a.scale;
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256, PX == 2 ? 4 : 1) void mex_fwd_kernel(const Mex
                     bool ok = true;
                     if (CHECK) {
                         const int ci = pref_c[3 * p] + dc, hi = pref_c[3 * p + 1] + dh, wi = pref_c[3 * p + 2] + dw;
-                        ok = ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
+                        ok = mex_inside(a, ci, hi, wi);
                     }
                     g[i] = ok ? a.in[pref_off[p] + o] : a.oob;
                 }
@@ -200,20 +200,32 @@ __global__ __launch_bounds__(256, PX == 2 ? 4 : 1) void mex_fwd_kernel(const Mex
             }
         } else {
             // patch elements: xs[kk][sp] = patch(sp)[k0 + kk], kk = sk, sk + KSTEP, ...: all gathers of the chunk
-            // in flight before the first LDS store
+            // in flight before the first LDS store.  Outside the input a lane loads the first element instead and
+            // drops it: a load inside the condition is a branch per element, whose table entry is waited for alone
+            // (32 x 16 x 20 x 20, 3 x 3 blocks, 32 instances: 25 -> 14 us).  Of the last chunk only the
+            // blocks of eight that hold any of its elements are fetched.
+            // The table entries of a wave's U elements (sk is the same for a whole wave, TP being a multiple of 64) come
+            // with one vector load, element u's in lane u.
+            constexpr int UB = U < 8 ? U : 8;
+            static_assert(U <= 64, "one lane per patch element");
+            const int4 kl = a.ktab[k0 + min(sk_u + (lane & (U - 1)) * KSTEP, kc - 1)];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                // sk is the same for a whole wave (TP is a multiple of 64): the table entry comes through a scalar load
-                const int kk = sk_u + u * KSTEP;
-                const int4 ke = a.ktab[k0 + (full ? kk : min(kk, kc - 1))];
-                const int o = ke.x;
-                if (CHECK) {
-                    const int dc = ke.y, dh = ke.z, dw = ke.w;
-                    const int ci = gp.ci0 + dc, hi = gp.hi0 + dh, wi = gp.wi0 + dw;
-                    const bool ok = ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
-                    v[u] = ok ? gp.base[o] : a.oob;
-                } else {
-                    v[u] = gp.base[o];
+            for (int u0 = 0; u0 < U; u0 += UB) {
+                if (!full && u0 * KSTEP >= kc)
+                    break;
+#pragma unroll
+                for (int u = u0; u < u0 + UB; ++u) {
+                    const int kx = __builtin_amdgcn_readlane(kl.x, u);
+                    if (CHECK) {
+                        const int ci = gp.ci0 + __builtin_amdgcn_readlane(kl.y, u);
+                        const int hi = gp.hi0 + __builtin_amdgcn_readlane(kl.z, u);
+                        const int wi = gp.wi0 + __builtin_amdgcn_readlane(kl.w, u);
+                        const bool ok = mex_inside(a, ci, hi, wi);
+                        const float raw = *(ok ? gp.base + kx : a.in);
+                        v[u] = ok ? raw : a.oob;
+                    } else {
+                        v[u] = gp.base[kx];
+                    }
                 }
             }
         }
@@ -816,7 +828,7 @@ __global__ __launch_bounds__(256) void mex_small_kernel(const MexKernelArgs a)
         const int rem = kk - dc * bhw;
         const int dh = rem / a.bw, dw = rem - dh * a.bw;
         const int ci = px.ci0 + dc, hi = px.hi0 + dh, wi = px.wi0 + dw;
-        const bool ok = ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
+        const bool ok = mex_inside(a, ci, hi, wi);
         x[j] = ok ? px.base[((ptrdiff_t)dc * a.H + dh) * a.W + dw] : a.oob;
     }
     // Wave reductions through the data-parallel-primitive lane patterns (neighbour, pair, half-row mirror, row mirror:

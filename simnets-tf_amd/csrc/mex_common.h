@@ -91,6 +91,13 @@ __device__ __forceinline__ PixelRef locate(const MexKernelArgs &a, int r, int sl
     return p;
 }
 
+// Whether input element (ci, hi, wi) exists.  Three comparisons and no branch: written with && the compiler turns a
+// gather's elements into nested branches, whose table entries and loads are then waited for one by one.
+__device__ __forceinline__ bool mex_inside(const MexKernelArgs &a, int ci, int hi, int wi)
+{
+    return ((unsigned)ci < (unsigned)a.C) & ((unsigned)hi < (unsigned)a.H) & ((unsigned)wi < (unsigned)a.W);
+}
+
 // Everything of the argument block that follows from the plan alone (pointers and tiling are the
 // caller's).
 inline MexKernelArgs mex_kernel_args(const MexPlan &p)

@@ -75,7 +75,7 @@ __device__ __forceinline__ float patch_element(const MexKernelArgs &a, const Pix
     const int dh = rem / a.bw;
     const int dw = rem - dh * a.bw;
     const int ci = px.ci0 + dc, hi = px.hi0 + dh, wi = px.wi0 + dw;
-    const bool ok = ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
+    const bool ok = mex_inside(a, ci, hi, wi);
     const ptrdiff_t o = ((ptrdiff_t)ci * a.H + hi) * a.W + wi;
     *img_off = ok ? o : -1;
     // (the load on an address that is always valid, the choice afterwards: loads inside conditions are waited for one
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void mex_grad_factors_kernel(const MexGradArgs
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int ci = px.ci0 + ke[i].y, hi = px.hi0 + ke[i].z, wi = px.wi0 + ke[i].w;
-            const bool ok = ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
+            const bool ok = mex_inside(a, ci, hi, wi);
             inside |= ok ? 1u << i : 0u;
             const float *src = ok ? px.base + ke[i].x : a.in;
             xg[i] = *src;
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(256) void mex_grad_input_mfma_kernel(const MexGradA
             const int p = t * 16 + lr;
             const int b = pb[p];
             const int ci = pc0[p] + dc, hi = ph0[p] + dh, wi = pw0[p] + dw;
-            ok[v][t] = k < a.K && b >= 0 && ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
+            ok[v][t] = (k < a.K) & (b >= 0) & mex_inside(a, ci, hi, wi);
             at[v][t] = ok[v][t] ? (size_t)b * chw + ((size_t)ci * a.H + hi) * a.W + wi : 0;
             if (buffered)
                 xin[v][t] = ga.exbuf[ok[v][t] ? (row0 + p) * ga.Kp + k : 0];
@@ -671,12 +671,19 @@ __global__ __launch_bounds__(256) void mex_grad_offsets_kernel(const MexGradArgs
 // grid.x: (region, pixel chunk of 64*pxl slots); grid.y: tile of 64 instances; grid.z: tile of 64 patch elements
 constexpr int GOM_MT = 64, GOM_KT = 64;
 
-__global__ __launch_bounds__(256) void mex_grad_offsets_mfma_kernel(const MexGradArgs ga)
+//
+// PIPE: the next group's values are requested in front of the current group's arithmetic (two sets of 48 registers:
+// one workgroup per compute unit's share of registers less); a launch of one group per workgroup has no next one and
+// fits three workgroups to a compute unit (32 x 16 x 20 x 20, 3 x 3 blocks, 32 instances: 28.8 us with one resident
+// workgroup and a branch per gathered element, 13.8 now).
+template <bool PIPE>
+__global__ __launch_bounds__(256, PIPE ? 2 : 3) void mex_grad_offsets_mfma_kernel(const MexGradArgs ga)
 {
     const MexKernelArgs &a = ga.k;
     __shared__ float wt[64 * 65];   // [pixel][instance], padded rows
     __shared__ float ex[64 * 65];   // [pixel][k], padded rows
     __shared__ float pmn[4 * 64];
+    __shared__ __attribute__((aligned(16))) float cst[2 * GOM_MT];   // per instance: bound term, exponent term
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -685,6 +692,17 @@ __global__ __launch_bounds__(256) void mex_grad_offsets_mfma_kernel(const MexGra
     const int m0 = blockIdx.y * GOM_MT, k0 = blockIdx.z * GOM_KT;
     const int n_mg = a.n_mgroups;
     const float *omax_r = a.omax + (size_t)r * n_mg * GM_TM, *orng_r = a.orng + (size_t)r * n_mg * GM_TM;
+    // this thread's instances when staging (16 of the tile, the same for the whole wave)
+    const int ms0 = m0 + wave * 16;
+    const bool wave_active = ms0 < a.M;
+    // the records of the wave's 16 patch elements: one vector load (lane i holds element i), read back lane by lane
+    // where they are used - as 16 wave-uniform loads in front of the 16 gathers each was waited for on its own
+    const int4 kl = a.ktab[min(k0 + wave * 16 + (lane & 15), a.K - 1)];
+    if (tid < GOM_MT) {
+        const int m = min(m0 + tid, a.M - 1);
+        cst[tid] = a.c0 + (omax_r[m] - orng_r[m]);
+        cst[GOM_MT + tid] = omax_r[m] + a.c0;
+    }
     {
         int wide = 0;
         for (int m = tid; m < a.M; m += 256)
@@ -705,11 +723,6 @@ __global__ __launch_bounds__(256) void mex_grad_offsets_mfma_kernel(const MexGra
 #pragma unroll
     for (int t = 0; t < 4; ++t)
         acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    // this thread's instances when staging (16 of the tile, the same for the whole wave) and their constants
-    const int ms0 = m0 + wave * 16;
-    // the records of the wave's 16 patch elements: one vector load (lane i holds element i), read back lane by lane
-    // where they are used - as 16 wave-uniform loads in front of the 16 gathers each was waited for on its own
-    const int4 kl = a.ktab[min(k0 + wave * 16 + (lane & 15), a.K - 1)];
     const bool buffered = ga.wbuf != nullptr;   // W and 2^(xs - a) come from mex_grad_factors_kernel
     // global loads of a group of 64 pixel slots: this thread's pixel, its 16 instances' output and gradient values
     // and 16 of the tile's patch elements; the loads of group s + 1 are issued before group s is processed
@@ -722,28 +735,24 @@ __global__ __launch_bounds__(256) void mex_grad_offsets_mfma_kernel(const MexGra
         q.valid = px.out_off >= 0;
         const float *gp = ga.g + (size_t)px.b * a.M * gplane + (q.valid ? pooled_g_offset(ga, px.out_off) : 0);
         const float *op = ga.out + (size_t)px.b * a.M * plane + (q.valid ? px.out_off : 0);
+        // Every load on a valid address and no branches: inside a condition each would be waited for in front of the
+        // next.  Instances and patch elements past the last one repeat it; their rows and columns are not stored.
+        if (wave_active) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int m = ms0 + i;
-            q.ov[i] = 0.0f;
-            q.gv[i] = 0.0f;
-            if (m < a.M) {
+            for (int i = 0; i < 16; ++i) {
+                const int m = min(ms0 + i, a.M - 1);
                 q.ov[i] = op[(size_t)m * plane];
-                q.gv[i] = q.valid ? gp[(size_t)m * gplane] : 0.0f;
+                q.gv[i] = gp[(size_t)m * gplane];
             }
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const int k = k0 + wave * 16 + i;
-            q.xr[i] = 0.0f;
-            if (q.valid && k < a.K) {
-                // {offset inside an image, dc, dh, dw} of element i
-                const int kx = __builtin_amdgcn_readlane(kl.x, i), ky = __builtin_amdgcn_readlane(kl.y, i);
-                const int kz = __builtin_amdgcn_readlane(kl.z, i), kw = __builtin_amdgcn_readlane(kl.w, i);
-                const int ci = px.ci0 + ky, hi = px.hi0 + kz, wi = px.wi0 + kw;
-                const bool ok = ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
-                q.xr[i] = ok ? px.base[kx] : a.oob;
-            }
+            // {offset inside an image, dc, dh, dw} of element i
+            const int kx = __builtin_amdgcn_readlane(kl.x, i), ky = __builtin_amdgcn_readlane(kl.y, i);
+            const int kz = __builtin_amdgcn_readlane(kl.z, i), kw = __builtin_amdgcn_readlane(kl.w, i);
+            const bool ok = mex_inside(a, px.ci0 + ky, px.hi0 + kz, px.wi0 + kw);
+            const float raw = *(ok ? px.base + kx : a.in);
+            q.xr[i] = ok ? raw : a.oob;
         }
     };
     Group cur;
@@ -785,52 +794,50 @@ __global__ __launch_bounds__(256) void mex_grad_offsets_mfma_kernel(const MexGra
             }
             continue;
         }
-        if (s == 0)
-            load_group(0, cur);
+        if (s == 0 || !PIPE)
+            load_group(s, cur);
         Group nxt;
-        if (s + 1 < ga.pxl)
+        if (PIPE && s + 1 < ga.pxl)
             load_group(s + 1, nxt);   // in flight while this group is processed
         float amin = INFINITY;
+        if (wave_active)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int m = ms0 + i;
-            if (m < a.M)
-                amin = fminf(amin, __builtin_fmaf(cur.ov[i], a.c1, -(a.c0 + (omax_r[m] - orng_r[m]))));
-        }
-        __syncthreads();  // the previous group's matrix instructions are done with wt / ex / ap
+            for (int i = 0; i < 16; ++i)
+                amin = fminf(amin, __builtin_fmaf(cur.ov[i], a.c1, -cst[wave * 16 + i]));
+        __syncthreads();  // the previous group's matrix instructions are done with wt / ex / pmn
         pmn[wave * 64 + lane] = amin;
         __syncthreads();
         const float a_p = cur.valid ? fminf(fminf(pmn[lane], pmn[64 + lane]), fminf(pmn[128 + lane], pmn[192 + lane])) : 0.0f;
+        if (wave_active) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int m = ms0 + i;
-            // (an empty slot holds the values of another region's pixel: its exponent can be anything, and zero times
-            // an overflowed factor would put NaN into the sums)
-            float w = 0.0f;
-            if (cur.valid && m < a.M)
-                w = cur.gv[i] * __builtin_amdgcn_exp2f(__builtin_fmaf(-cur.ov[i], a.c1, a_p) + (omax_r[m] + a.c0));
-            wt[lane * 65 + wave * 16 + i] = w;
+            for (int i = 0; i < 16; ++i) {
+                // (an empty slot holds the values of another region's pixel: its exponent can be anything, and zero times
+                // an overflowed factor would put NaN into the sums)
+                const float w = cur.gv[i] * __builtin_amdgcn_exp2f(__builtin_fmaf(-cur.ov[i], a.c1, a_p) + cst[GOM_MT + wave * 16 + i]);
+                wt[lane * 65 + wave * 16 + i] = cur.valid ? w : 0.0f;
+            }
         }
         // patch exponentials: this thread's pixel, 16 of the tile's patch elements
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const int kk = wave * 16 + i, k = k0 + kk;
-            float e = 0.0f;
-            if (cur.valid && k < a.K)
-                e = __builtin_amdgcn_exp2f(__builtin_fmaf(cur.xr[i], a.c1, -a_p));
-            ex[lane * 65 + kk] = e;
+            const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(cur.xr[i], a.c1, -a_p));
+            ex[lane * 65 + wave * 16 + i] = cur.valid ? e : 0.0f;
         }
         __syncthreads();
+        if (wave_active) {
 #pragma unroll 4
-        for (int ps = 0; ps < 64; ps += 4) {
-            const float av = wt[(ps + lq) * 65 + wave * 16 + lr];
+            for (int ps = 0; ps < 64; ps += 4) {
+                const float av = wt[(ps + lq) * 65 + wave * 16 + lr];
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, ex[(ps + lq) * 65 + t * 16 + lr], acc[t], 0, 0, 0);
+                for (int t = 0; t < 4; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, ex[(ps + lq) * 65 + t * 16 + lr], acc[t], 0, 0, 0);
+            }
         }
-        if (s + 1 < ga.pxl)
+        if (PIPE && s + 1 < ga.pxl)
             cur = nxt;
     }
+    if (!wave_active)
+        return;
     // ---- partial sums of this pixel chunk: acc * 2^(os_mk - mo_m) ----
     float *dst = ga.partial + ((size_t)chunk * a.R + r) * a.M * a.K;
     // (the 16 offset exponentials first, on clamped indices, then the products and stores)
@@ -1829,7 +1836,7 @@ __global__ __launch_bounds__(1024) void mex_grad_head_kernel(const MexGradArgs g
             const PixelRef px = locate(a, r, min(slot, a.slots - 1));   // (the same pixel for the whole workgroup)
             valid[p] = slot < a.slots && px.out_off >= 0;
             const int ci = px.ci0 + dc, hi = px.hi0 + dh, wi = px.wi0 + dw;
-            const bool ok = kv && ci >= 0 && ci < a.C && hi >= 0 && hi < a.H && wi >= 0 && wi < a.W;
+            const bool ok = kv && mex_inside(a, ci, hi, wi);
             io[p] = ok ? (ci * a.H + hi) * a.W + wi : -1;
             img[p] = (size_t)px.b * a.C * a.H * a.W;
             // (loads on addresses that are always valid, the choice made afterwards: a load inside a condition is
@@ -2338,8 +2345,11 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
             const int gy = (d.M + GOM_MT - 1) / GOM_MT, gz = (d.K + GOM_KT - 1) / GOM_KT;
             if (gx > 0x7fffffffLL || gy > 65535 || gz > 65535)
                 return SIMNETS_ERR_TOO_LARGE;
-            hipLaunchKernelGGL(mex_grad_offsets_mfma_kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)gz), dim3(256),
-                               0, s, go);
+            const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
+            if (go.pxl > 1)
+                hipLaunchKernelGGL(mex_grad_offsets_mfma_kernel<true>, grid, dim3(256), 0, s, go);
+            else
+                hipLaunchKernelGGL(mex_grad_offsets_mfma_kernel<false>, grid, dim3(256), 0, s, go);
         } else {
             const int gy = (d.M + 4 * GO_MT - 1) / (4 * GO_MT);
             const int gz = (d.K + GO_KT - 1) / GO_KT;

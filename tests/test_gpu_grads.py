@@ -987,3 +987,34 @@ def test_mex_offsets_grad_few_rows_of_many_chunks(pkg, C, M, blocks):
         # n products of probabilities and gradients of random sign, each within a few units of its last place
         err = float((got.double().reshape(M, K) - ref).norm() / ref.norm())
         assert err <= 4 * math.sqrt(n) * 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("B,C,H,W,M,blocks", [
+    (24, 7, 17, 19, 33, 3),    # one group of 64 pixels a workgroup; instances and patch elements behind the last tile's
+    (64, 4, 32, 33, 40, 3),    # several groups, the next one requested ahead; a last group with empty slots
+    (24, 15, 17, 19, 16, 3),   # K = 135: the forward's second chunk holds seven elements
+    (24, 29, 9, 11, 5, 3),     # K = 261: three chunks
+])
+def test_mex_overlapping_blocks_chunk_and_tile_remainders(pkg, B, C, H, W, M, blocks):
+    """Gathers without branches: forward and offsets gradient of padded overlapping blocks with a border value other than
+    zero, where chunks, instance tiles and pixel groups do not come out even; against torch in 64 bits."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn((B, C, H, W), generator=g, device="cuda")
+    pad = blocks // 2
+    kw = dict(softmax_mode=True, blocks=[C, blocks, blocks], strides=[C, 1, 1], padding=[0, pad, pad],
+              blocks_out_of_bounds_value=0.75, use_unshared_regions=False, shared_offset_region=[-1])
+    off = torch.randn(pkg.mex_output_shape(tuple(x.shape), M, **kw)[1], generator=g, device="cuda") * 0.3
+    y = pkg.mex(x, off, M, **kw)
+    go = torch.randn(y.shape, generator=g, device="cuda")
+    got = pkg.mex_offsets_grad(x, off, y, go, M, **kw)
+    cols = torch.nn.functional.unfold(torch.nn.functional.pad(x.double(), (pad,) * 4, value=0.75), blocks)
+    K = cols.shape[1]
+    o = off.double().reshape(M, K).requires_grad_()
+    want = torch.stack([torch.logsumexp(cols + o[m][None, :, None], 1) for m in range(M)], 1)
+    ref = torch.autograd.grad(want, o, go.double().reshape(want.shape))[0]
+    # a sum of K positive terms, each and its exponent within a few units of the last place
+    err = float((y.double().reshape(want.shape) - want).abs().max() / want.abs().max())
+    assert err <= 8 * 2.0 ** -24, err
+    n = go.numel() // M
+    err = float((got.double().reshape(M, K) - ref).norm() / ref.norm())
+    assert err <= 4 * math.sqrt(n) * 2.0 ** -24, err
