@@ -159,6 +159,7 @@ __device__ __forceinline__ void load_params(float (&pa)[2 * MT], float (&pc)[MT]
 #define SIMNETS_BIG_MT 8
 #endif
 constexpr int kBigPT = SIMNETS_BIG_PT, kBigMT = SIMNETS_BIG_MT;
+constexpr int kMidPT = 14, kLowPT = 12;    // L1: the wide variant on images whose width these fill better (choose_tiling)
 constexpr int kSmallPT = 4, kSmallMT = 8;
 constexpr int kGatherMaxK = 12;            // patch lengths up to which the gather kernel replaces the tiled ones
 constexpr int kSmStageGroups = 2;   // small-map kernel: channel groups whose loads are in flight at once while staging
@@ -474,6 +475,11 @@ __device__ __forceinline__ void sim_direct_body(const SimKernelArgs &a, float *l
             for (int q = 0; q < PT / 4; ++q)
                 if (w0 + 4 * q < a.ow)
                     *reinterpret_cast<float4 *>(o + 4 * q) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        } else if (a.vec_store && PT % 2 == 0) {
+#pragma unroll
+            for (int q = 0; q < PT / 2; ++q)
+                if (w0 + 2 * q < a.ow)
+                    *reinterpret_cast<float2 *>(o + 2 * q) = make_float2(v[2 * q], v[2 * q + 1]);
         } else {
 #pragma unroll
             for (int p = 0; p < PT; ++p)
@@ -1007,6 +1013,25 @@ Tiling choose_tiling(const SimPlan &p)
         const int n_mtiles = (p.O + t.MT - 1) / t.MT, nwm = kWaves / t.nws;
         return (long long)p.B * t.tiles * ((n_mtiles + nwm - 1) / nwm) * kWaves;
     };
+    // L1, the wide lane tile's columns: 16, 14 or 12, whichever leaves fewer of them, and of the lanes, empty (28 columns
+    // are two of 14 without a rest, 36 three of 12).  Estimated by the workgroups each compute unit takes one behind
+    // the other, two of them side by side, times the instructions of a step (0.8 columns' worth of them are loads and
+    // addresses).  3 x 3 unless stated: 32 x 128 x 28 x 28 -> 128 209 -> 193 us; 32 x 64 x 56 x 56 -> 64 235 -> 203; 32 x 32 x 36 x 36 ->
+    // 128, 5 x 5 297 -> 219; 64 x 64 x 24 x 24 -> 64, the 4 x 8 tile's before, 150 -> 93; 200 x 17 x 53 x 55 -> 33 470 -> 360.  Not for
+    // patches of fewer taps, whose time is the staging (64 x 64 x 56 x 56 -> 64, 1 x 1: 87 -> 93).
+    auto narrower = [&](Tiling best, auto make) {
+        auto cost = [&](const Tiling &c) {
+            const int n_mtiles = (p.O + kBigMT - 1) / kBigMT, nwm = c.ksplit ? 1 : kWaves / c.nws;
+            const double w = (double)p.B * c.tiles * ((n_mtiles + nwm - 1) / nwm) / 512;
+            return (w <= 0.5 ? 0.6 : w <= 1 ? 1 : (w + std::ceil(w)) / 2) * (c.PT + 0.8);
+        };
+        for (int PT : {kMidPT, kLowPT}) {
+            const Tiling c = make(PT);
+            if (c.lds_ok && c.fast_stage && cost(c) < 0.97 * cost(best))
+                best = c;
+        }
+        return best;
+    };
     // Wide rows and many templates: 16 pixels x 8 templates per lane (128 accumulators, two waves per SIMD; 8x8
     // and 16x4 tiles measured slower on the 256x64x32x32 / 128-template case) - provided the grid then still
     // gives the SIMDs about two waves each (1.5 on average): a SIMD with a single wave issues at half rate.  Otherwise 4 x 8, which
@@ -1014,7 +1039,7 @@ Tiling choose_tiling(const SimPlan &p)
     if (p.ow >= 32 && p.O >= 32) {
         const Tiling big = pick(kBigPT, kBigMT);
         if (big.lds_ok && waves(big) >= 1536)
-            return big;
+            return p.mode == SIM_MODE_L1 && p.bh * p.bw >= 9 ? narrower(big, [&](int PT) { return pick(PT, kBigMT); }) : big;
     }
     Tiling t = pick(kSmallPT, kSmallMT);
     // L1 on narrow images or few workgroups: the wide lane tile after all, its four waves a quarter of the channels each,
@@ -1025,11 +1050,20 @@ Tiling choose_tiling(const SimPlan &p)
     // (184 x 21 x 24 x 21 -> 140, 0.49 of them against 0.66: 259 -> 318), and with few taps a chunk's staging costs more than
     // the steps gain (86 x 34 x 30 x 30 -> 235, 1 x 1: 84 -> 189).  The shorter sums also round less: 5.2e-7 -> 1.4e-7.
     if (p.mode == SIM_MODE_L1 && p.C >= 2 * kWaves && p.bh * p.bw >= 9) {
-        Tiling big = try_tiling(p, kBigPT, kBigMT, 1);
         auto useful = [&](const Tiling &c) { return (double)c.gpi / (c.tiles * 64 * c.nws) * p.ow / (c.G * c.PT); };
-        const long long big_waves = 1LL * p.B * big.tiles * ((p.O + kBigMT - 1) / kBigMT) * kWaves;
-        if (big.lds_ok && big.fast_stage && big_waves >= 1024 && 1.3 * useful(big) >= useful(t)) {
-            big.ksplit = true;
+        auto make = [&](int PT) {
+            Tiling c = try_tiling(p, PT, kBigMT, 1);
+            const long long c_waves = 1LL * p.B * c.tiles * ((p.O + kBigMT - 1) / kBigMT) * kWaves;
+            c.ksplit = true;
+            c.lds_ok = c.lds_ok && c.fast_stage && c_waves >= 1024 && 1.3 * useful(c) >= useful(t);
+            return c;
+        };
+        Tiling big = make(kBigPT);
+        for (int PT : {kMidPT, kLowPT})   // (the first that qualifies)
+            if (!big.lds_ok)
+                big = make(PT);
+        if (big.lds_ok) {
+            big = narrower(big, make);
             if (big.CC > kWaves)
                 big.CC = big.CC / kWaves * kWaves;
             return big;
@@ -1072,8 +1106,8 @@ hipError_t launch_direct(const SimKernelArgs &a, dim3 grid, size_t lds_bytes, hi
 {
     // (the normalized modes keep the table-driven loop: with their extra operands the row form does not fit the
     // register file)
-    constexpr bool kRow3 = PT == kBigPT && !PLDS && (MODE == SIM_MODE_L1 || MODE == SIM_MODE_L2 || MODE == SIM_MODE_L2_SQRTW);
-    if constexpr (MODE == SIM_MODE_L1 && PT == kBigPT) {
+    constexpr bool kRow3 = PT > kSmallPT && !PLDS && (MODE == SIM_MODE_L1 || MODE == SIM_MODE_L2 || MODE == SIM_MODE_L2_SQRTW);
+    if constexpr (MODE == SIM_MODE_L1 && PT > kSmallPT) {
         if (a.ksplit) {
             if (a.sw == 1 && a.bh == 3 && a.bw == 3)
                 hipLaunchKernelGGL((sim_direct_kernel<MODE, PT, MT, 1, false, true, true>), grid, dim3(kThreads), lds_bytes, s,
@@ -1149,6 +1183,12 @@ hipError_t launch_mode(const SimKernelArgs &a0, const Tiling &t, bool plds, hipS
     a.xcd_group = grid.y > 1 && grid.x % 8 == 0;
     if (t.PT == kBigPT && t.MT == kBigMT)
         return launch_direct<MODE, kBigPT, kBigMT, false>(a, grid, lds_bytes, s);
+    if constexpr (MODE == SIM_MODE_L1) {
+        if (t.PT == kMidPT)
+            return launch_direct<MODE, kMidPT, kBigMT, false>(a, grid, lds_bytes, s);
+        if (t.PT == kLowPT)
+            return launch_direct<MODE, kLowPT, kBigMT, false>(a, grid, lds_bytes, s);
+    }
     if (plds) {
         lds_bytes = ((size_t)a.plds_off + (size_t)nwm * (a.K + 1) * kSmallMT * 3) * sizeof(float);
         return launch_direct<MODE, kSmallPT, kSmallMT, true>(a, grid, lds_bytes, s);

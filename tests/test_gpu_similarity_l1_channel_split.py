@@ -47,3 +47,15 @@ def test_l1_with_the_contraction_split_over_waves(pkg, geom):
         err = float((dx[b:b + 1].double() - ref).norm() / ref.norm())
         assert err <= 4 * math.sqrt(n) * 2.0 ** -24, err
     assert torch.equal(pkg.similarity_prepare(shape, t, w, **kw)(x), got)
+
+
+@pytest.mark.parametrize("geom", [
+    dict(shape=(33, 13, 28, 28), O=60, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),     # 2 x 14 columns, split channels
+    dict(shape=(40, 9, 24, 23), O=64, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),      # 2 x 12, the last column empty
+    dict(shape=(64, 17, 36, 36), O=40, blocks=[5, 5], strides=[1, 1], padding=[2, 2]),     # 3 x 12, the table-driven loop
+    dict(shape=(200, 5, 53, 55), O=33, blocks=[3, 3], strides=[1, 1], padding=[1, 1]),     # 4 x 14, whole channels
+    dict(shape=(150, 9, 83, 84), O=40, blocks=[3, 3], strides=[2, 2], padding=[1, 1]),     # 3 x 14 at stride 2
+    dict(shape=(220, 4, 38, 36), O=70, blocks=[3, 4], strides=[1, 1], padding=[1, 2]),     # 37 columns, the table-driven loop
+])
+def test_l1_on_lane_tiles_of_14_and_12_columns(pkg, geom):
+    test_l1_with_the_contraction_split_over_waves(pkg, geom)
