@@ -651,8 +651,14 @@ __device__ __forceinline__ void pack_row32(const float (&x)[32], int normalize, 
 // a small layer is this one launch.
 // INF (plain call only): infinite epsilon - the extreme value of patch + offset through max_chunk, from the panel and
 // the scaled offsets; nothing of the product form (column maxima, packed exponentials, row ranges) is touched.
+// Two halves and one chunk, not pooled: three workgroups on a compute unit instead of two, whose load, exponential and
+// store phases overlap.  For their LDS the partial maxima use the panel tile's place (a barrier more), for their registers
+// the offsets tiles go to LDS as they arrive.  1024 x 32 x 16 x 16 -> 64 instances: 33.2 -> 31.4 us (3.2 TB/s of input and
+// output); 256 x 32 x 16 x 16 -> 200 31.4 -> 29.0.  Holding the offsets in registers spills and loses 20 %.
+constexpr bool panel_three(int nh, int nch, bool pool, bool inf) { return nh == 2 && nch == 1 && !pool && !inf; }
+
 template <int NH, int NCH, bool POOL, bool SELFPACK = false, bool INF = false>
-__global__ __launch_bounds__(256 * NH) void mex_pool_panel_kernel(const MexKernelArgs a, const PoolArgs q,
+__global__ __launch_bounds__(256 * NH, panel_three(NH, NCH, POOL, INF) ? 6 : 1) void mex_pool_panel_kernel(const MexKernelArgs a, const PoolArgs q,
                                                                   const PanelArgs g)
 {
     static_assert(!SELFPACK || (NH == 1 && NCH == 1 && !POOL), "in-kernel packing: one row per thread, one chunk");
@@ -663,7 +669,9 @@ __global__ __launch_bounds__(256 * NH) void mex_pool_panel_kernel(const MexKerne
     constexpr int NV = 2 * NCH;   // float4 of the panel per thread: rows kslot + 16 u
     __shared__ __attribute__((aligned(16))) float xs[KC * XP];       // [k][column ^ swizzle]
     __shared__ __attribute__((aligned(16))) float os[R * KC * TM];   // [region][k][instance ^ swizzle]
-    __shared__ __attribute__((aligned(16))) float pmx[16 * XP];      // [kslot][column]: partial column maxima
+    constexpr bool kThree = panel_three(NH, NCH, POOL, INF);
+    __shared__ __attribute__((aligned(16))) float pmx_own[kThree ? 4 : 16 * XP];
+    float *pmx = kThree ? xs : pmx_own;                              // [kslot][column]: partial column maxima
     __shared__ float msh[XP];                                        // column maxima
     __shared__ float omax_sh[SELFPACK ? R * TM : 1];                 // SELFPACK: row maxima of the scaled offsets
     // per slot: where instance 0 goes in the pooled tensor (POOL = false: where the window's first pixel goes in the
@@ -835,6 +843,11 @@ __global__ __launch_bounds__(256 * NH) void mex_pool_panel_kernel(const MexKerne
         const int cg = (part << g.lgF) | pg;   // 0 .. XP / 4 - 1
         reinterpret_cast<float4 *>(pmx)[kslot * (XP / 4) + cg] = pm;
     }
+#define SIMNETS_PANEL_PUT(i) dst[((i) / NO) * TILE4 + ((i) % NO) * kThreads] = on##i;
+    if constexpr (kThree) {   // (held until the chunk loop they would not fit the registers of three workgroups)
+        float4 *dst = reinterpret_cast<float4 *>(os) + ((tid & ~15) | ((tid & 15) ^ (((tid >> 4) & 3) << 2)));
+        SIMNETS_PANEL_PUT(0) SIMNETS_PANEL_PUT(1) SIMNETS_PANEL_PUT(2) SIMNETS_PANEL_PUT(3)
+    }
     float rx[SELFPACK ? KC : 1];   // SELFPACK: the row, its logsumexp (0 without normalisation) and its scaled maximum
     float row_lse = 0.0f, row_hi = 0.0f, row_xh = 0.0f;
     if constexpr (SELFPACK) {
@@ -893,6 +906,8 @@ __global__ __launch_bounds__(256 * NH) void mex_pool_panel_kernel(const MexKerne
         // nothing finite in the column: the terms are exp2(-inf) = 0
         msub[0] = m.x == -INFINITY ? 0.0f : m.x; msub[1] = m.y == -INFINITY ? 0.0f : m.y;
         msub[2] = m.z == -INFINITY ? 0.0f : m.z; msub[3] = m.w == -INFINITY ? 0.0f : m.w;
+        if (kThree)
+            __syncthreads();   // the maxima have been read, their place becomes the panel's tile
     }
 
     const int lr = lane & 15, lq = lane >> 4;
@@ -923,14 +938,12 @@ __global__ __launch_bounds__(256 * NH) void mex_pool_panel_kernel(const MexKerne
                 for (int k = 0; k < KC; ++k)
                     orow[k * TM + (mi ^ ((k & 3) << 4))] =
                         row_valid ? __builtin_amdgcn_exp2f(mex_offset_exponent(rx[k], row_xh, row_lse, a.scale)) : 0.0f;
-            } else {
+            } else if constexpr (!kThree) {
                 float4 *dst = reinterpret_cast<float4 *>(os) + ((tid & ~15) | ((tid & 15) ^ (((tid >> 4) & 3) << 2)));
-#define SIMNETS_PANEL_PUT(i) dst[((i) / NO) * TILE4 + ((i) % NO) * kThreads] = on##i;
                 SIMNETS_PANEL_PUT(0) SIMNETS_PANEL_PUT(1) SIMNETS_PANEL_PUT(2) SIMNETS_PANEL_PUT(3)
                 if constexpr (NO == 2) {
                     SIMNETS_PANEL_PUT(4) SIMNETS_PANEL_PUT(5) SIMNETS_PANEL_PUT(6) SIMNETS_PANEL_PUT(7)
                 }
-#undef SIMNETS_PANEL_PUT
             }
             // (columns of parts past the batch stay unwritten: a column only reaches its own, unstored, outputs)
             if (pvalid) {
@@ -997,6 +1010,7 @@ __global__ __launch_bounds__(256 * NH) void mex_pool_panel_kernel(const MexKerne
 #undef SIMNETS_PANEL_STEP
 #undef SIMNETS_PANEL_LAST
 #undef SIMNETS_PANEL_NEXT
+#undef SIMNETS_PANEL_PUT
             if (c + 1 < NCH)
                 __syncthreads();  // everyone is done with this chunk's tiles
         }

@@ -967,3 +967,26 @@ def test_similarity_forward_random_geometries(pkg):
             continue
         print("case", case, (B, C, H, W), O, kw, flush=True)
         assert rel_err(run_similarity(pkg, x, t, w, **kw), want) <= SIM_TOL
+
+
+@pytest.mark.parametrize("im,n", [((131, 32, 16, 16), 70), ((521, 32, 8, 8), 20)])
+@pytest.mark.parametrize("spread,eps", [("narrow", 1.0), ("narrow", -2.0), ("mixed", 3.0), ("wide", 1.0)])
+def test_mex_panel_form_of_two_halves_and_one_chunk(pkg, im, n, spread, eps):
+    """Grids large enough for the 32-channel panel of two halves, whose partial maxima share the panel tile's place; the
+    last workgroup is part empty.  A column without a finite element and one with an infinity beside ordinary ones."""
+    test_mex_panel_form_of_the_plain_call(pkg, im, n, spread, eps)
+    if spread != "narrow":
+        return
+    g = np.random.default_rng(48)
+    kw = dict(softmax_mode=True, blocks=[im[1], 1, 1], strides=[im[1], 1, 1], use_unshared_regions=True,
+              unshared_offset_region=[1, 2, 2])
+    x = g.normal(size=im).astype(np.float32)
+    off = (g.normal(size=(4, n, im[1], 1, 1)) * 0.3).astype(np.float32)
+    want = run_mex(pkg, x, off, n, **kw)
+    x[1, :, 3, 2] = -np.inf
+    x[2, 5, 1, 1] = np.inf
+    got = run_mex(pkg, x, off, n, **kw)
+    keep = np.ones(want.shape, bool)
+    keep[1, :, 3, 2] = keep[2, :, 1, 1] = False
+    assert np.array_equal(got[keep], want[keep])
+    assert not np.isfinite(got[~keep]).any()
