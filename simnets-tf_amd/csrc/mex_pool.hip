@@ -157,14 +157,17 @@ __device__ __forceinline__ void max_chunk(float (&best)[4][4], const float *xs, 
 
 // NH = column halves of a workgroup (64 pixel columns = 4 tiles of 16 each), 4 instance waves per half: two halves
 // share the offsets tiles and double the waves per SIMD the LDS budget allows, which is what hides the latencies of
-// the short dependent phases; one half only when there are no slots for a second one.
+// the short dependent phases; one half only when there are no slots for a second one.  With the Similarity inside two such
+// workgroups fit a compute unit's registers, and their phases overlap: against one of four halves (a copy of the offsets
+// tiles and a fetch of taps and parameters per 256 columns) the missing-data network takes 185 us instead of 191 at 2048
+// images, 221 instead of 232 at 700 with 64 templates and 96 instances, 68.0 instead of 68.6 at 512.
 // SIMF: the input of the MEX layer is a Similarity layer's output whose channels are exactly the MEX patch (blocks
 // [O, 1, 1], no padding): the staging evaluates Similarity channel k of its pixel from the layer's input (the patch
 // taps of the pixel sit in LDS, the packed parameters of channel k come through scalar loads) with the Similarity
 // kernel's own combine step in the same order, so the value is the one that kernel would have stored, and neither
 // that tensor nor its launches exist.
 template <int R, int NH, bool CHECK, bool SIMF>
-__global__ __launch_bounds__(256 * NH) void mex_pool_kernel(const MexKernelArgs a, const PoolArgs q)
+__global__ __launch_bounds__(256 * NH, NH == 2 && SIMF ? 4 : 1) void mex_pool_kernel(const MexKernelArgs a, const PoolArgs q)
 {
     constexpr int XP = 64 * NH;         // pixel columns of a workgroup
     constexpr int kThreads = 256 * NH;
@@ -1254,14 +1257,7 @@ int pool_launch(const MexPlan &p, int ph, int pw, const float *input, const floa
     q.Wp = d.width_out / pw;
     // two column halves per workgroup whenever there are slots for both: the extra waves per compute unit pay even
     // when the launch then has fewer workgroups than compute units (measured on 512 images of 2x2 pixels)
-    // ... and four halves (16 waves) when there are many slots and the patches are short: the offsets tiles are
-    // then copied once per 256 pixel columns
     int nh = a.slots > 64 / (ph * pw) ? 2 : 1;
-    // ... only with the Similarity inside (its patch taps and parameters are then fetched once per 256 columns:
-    // 512 images of the first layer 24.2 -> 18.3 us); without it two halves are as fast or faster (15.6 against
-    // 16.0 us, 104.7 against 111.0 us at 4096 images)
-    if (sp && ph * pw == 4 && d.K <= 2 * KC && a.slots >= 64 * 128)
-        nh = 4;
     // a single chunk on a grid that two halves would leave below one workgroup per compute unit: one half (64 images
     // of 32 x 16 x 16: 6.7 -> 6.1 us)
     const int spw2 = 2 * 64 / (ph * pw);   // slots of a workgroup of two halves
@@ -1285,8 +1281,7 @@ int pool_launch(const MexPlan &p, int ph, int pw, const float *input, const floa
     if (panel)
         e = nh == 1 ? launch_panel<1, true>(a, q, pg, grid, s) : launch_panel<2, true>(a, q, pg, grid, s);
     else if (ph * pw == 4)
-        e = nh == 4 ? launch_pool<4, 4>(a, q, grid, inside, s)
-                    : (nh == 2 ? launch_pool<4, 2>(a, q, grid, inside, s) : launch_pool<4, 1>(a, q, grid, inside, s));
+        e = nh == 2 ? launch_pool<4, 2>(a, q, grid, inside, s) : launch_pool<4, 1>(a, q, grid, inside, s);
     else
         e = nh == 2 ? launch_pool<2, 2>(a, q, grid, inside, s) : launch_pool<2, 1>(a, q, grid, inside, s);
     return e == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
