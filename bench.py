@@ -29,9 +29,10 @@ EXP_RATE_STATED = 9.83e12  # exponentials per second the work table of the basel
 EXP_RATE_MEASURED = 19.66e12  # v_exp_f32 at a quarter of the 128 lanes/clk/CU VALU rate (17.6e12 measured on the box)
 
 PEAK_BF16_TFLOPS = 2500.0  # dense bf16 matrix peak
-# The default form of the L2 modes multiplies 16-bit pieces on the bf16 matrix cores: six products for each of two
-# operands per term, a third operand (three products for each of two sums) where NaN inputs are ignored
-PIECES_FLOP, PIECES_MASKED_FLOP = 24, 36
+# The default form of the L2 modes multiplies 16-bit pieces on the matrix cores: three products of half-precision pieces
+# for each of two operands per term, a third operand (two products for each of two sums) where NaN inputs are ignored;
+# the parameter gradients six products of bf16 pieces for each of two.  Half precision has the rate of bf16.
+PIECES_FLOP, PIECES_MASKED_FLOP, PIECES_PARAMS_FLOP = 12, 20, 24
 # HBM bytes per launch of the dominant kernel of the headline workload, from rocprofv3 FETCH_SIZE / WRITE_SIZE runs
 # scaled by a copy kernel of known size; not measured inside this run: "traffic_source" names the committed summary.
 MEASURED_TRAFFIC = {
@@ -235,7 +236,7 @@ def main():
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": "config3: Similarity L2 fwd 256x64x32x32, 128 templates 64x3x3, s1 p1 "
                                "-> 256x128x32x32 (M=262144 N=128 K=576)",
-                   "algo": args.algo or "auto (16-bit pieces on the bf16 matrix cores, fp32 sums; tiles with an output "
+                   "algo": args.algo or "auto (16-bit pieces on the matrix cores, fp32 sums; tiles with an output "
                                         "near zero are recomputed term by term)",
                    "entry_point": "simnets_hip_similarity_fwd (packs the parameters in every step)",
                    "gmac_per_step": gmac3},
@@ -621,7 +622,7 @@ def main():
         _, ms = timed(lambda: pkg.similarity_parameters_grad(X3, T3, W3, G3, similarity_function="L2", **kw3),
                       args.steps, args.warmup)
         others["config5_similarity_params_grad_L2"] = entry(ms, gmac3, 67108864 + 3 * 589824 + 134217728, "pieces",
-                                                            flop=PIECES_FLOP)
+                                                            flop=PIECES_PARAMS_FLOP)
         Y2 = pkg.mex(X2, O2, n2, normalize_offsets=True, **kw2)
         G2 = to_dev(np.random.default_rng(6789).normal(size=(64, 64, 16, 16)).astype(np.float32))
         _, ms = timed(lambda: pkg.mex_input_grad(X2, O2, Y2, G2, n2, normalize_offsets=True, **kw2), args.steps,
