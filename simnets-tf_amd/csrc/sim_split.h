@@ -26,10 +26,9 @@ struct SplitPlan {
     int cg;       // channels of a staged chunk: 16 (a matrix step is one tap) or 8 (a step is two taps)
     int chunks;   // ceil(C / cg)
     int steps;    // matrix steps per chunk: taps, or ceil(taps / 2)
-    int pieces;   // 16-bit pieces of the packed parameters per step: 4, with missing values 8
+    int pieces;   // 16-bit pieces of the packed parameters per step: 4, with missing values 8 (input gradient: 6)
     int n_mtiles; // ceil(O / 32)
     int n_ptiles; // ceil(B oh ow / 128)
-    int parts;    // input gradient: shares of an image of g whose largest sizes are found apart
     int Wp, Hv;   // columns of a staged row; rows of one image's staged stack
     size_t packed, chan, rows, flags, exact, logs, total;   // workspace, from its own start
 };
@@ -41,9 +40,6 @@ SplitPlan sim_split_plan(const SimPlan &p);
 // parameters were multiplied by, and the line below which outputs are recomputed.  Behind those of the n_mtiles * 32
 // templates the constants of the normalized modes.
 enum SplitRow { SPLIT_BIAS, SPLIT_BIAS_LESSER, SPLIT_UNSCALE, SPLIT_THR, SPLIT_GUARD = SPLIT_BIAS };
-// Input gradient, per input channel: its centre, the exponents that take its two scales back (integers), and whether a
-// coefficient is infinite.
-enum SplitGradRow { SPLIT_CENTRE, SPLIT_EXP_A, SPLIT_EXP_B, SPLIT_INFINITE };
 // Per channel, [field][chunks * cg], zeros behind the last channel: the scale s, -c s, and m.
 enum SplitChannel { SPLIT_S, SPLIT_NCS, SPLIT_M, SPLIT_CHANNEL_FIELDS };
 
@@ -56,6 +52,8 @@ struct SplitPack {
     int O, C, taps, K, cg, chunks, steps, pieces, n_mtiles, mode;
     float fudge, norm_const;
     float line;   // outputs below `line` times sum w t'^2 are recomputed term by term
+    float *ctr;   // input gradient: centres of the rows
+    int pack_blocks;   // ... workgroups of its packing launch, chunks * n_mtiles * ceil(steps / 4)
     FastDiv d_taps, d_steps;
     int blocks;   // of the packing launch: each template of the n_mtiles * 32, one at a time
 };

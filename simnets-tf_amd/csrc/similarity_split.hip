@@ -67,35 +67,29 @@ typedef __attribute__((address_space(1))) float global_float;
 typedef __attribute__((address_space(1))) float2_t global_float2;
 
 constexpr int kThreads = 256;
-enum SplitKind {
-    SPLIT_FWD,
-    SPLIT_MASKED,   // forward, NaN inputs ignored
-    SPLIT_GRAD,     // input gradient
-    SPLIT_GRAD3     // ... in three bf16 pieces
-};
+enum SplitKind { SPLIT_FWD, SPLIT_MASKED /* forward, NaN inputs ignored */, SPLIT_GRAD /* input gradient */ };
 
 // staged pixels of a chunk of 16 channels (twice as many of 8): two workgroups' tiles fit the 160 KB of a compute unit
 constexpr int split_lds_pixels(int kind) { return kind == SPLIT_MASKED ? 360 : kind == SPLIT_FWD ? 408 : 816; }
-constexpr int split_operands(int kind) { return kind == SPLIT_MASKED ? 5 : kind == SPLIT_FWD ? 4 : kind == SPLIT_GRAD ? 2 : 3; }
+constexpr int split_operands(int kind) { return kind == SPLIT_MASKED ? 5 : kind == SPLIT_FWD ? 4 : 3; }
 constexpr int split_lds_bytes(int kind) { return split_lds_pixels(kind) * 32 * split_operands(kind); }
 // pixels of one staged plane [channel group][pixel]
 constexpr int split_plane_pixels(int kind, int cg) { return split_lds_pixels(kind) * (cg == 16 ? 1 : 2); }
-constexpr int split_pieces(int kind) { return kind == SPLIT_MASKED ? 8 : kind == SPLIT_GRAD3 ? 6 : 4; }
+constexpr int split_pieces(int kind) { return kind == SPLIT_MASKED ? 8 : kind == SPLIT_FWD ? 4 : 6; }
 
 struct SplitArgs {
     const float *in;
     float *out;
     const void *packed;
     const float *chan, *rows;   // see SplitPack
-    const float *peaks;         // input gradient: [image][parts] the largest size in a part of g, negative if it has infinities
-    int parts;
+    const float *ctr;           // input gradient: centres of the rows
     const float2 *exact;   // see SplitPack
     const float *logs;
     int *flags;      // [pixel tile][mtile]
     int C, H, W, O, ow, npix, total;   // npix = oh ow, total = B npix
     int bw, sh, sw, ph, pw, taps, chunks, steps, n_mtiles, Wp, Hv;
     int gmax;        // matrix tiles of templates per workgroup: 4, 2 or 1
-    int per_sum;     // matrix steps whose products share accumulators
+    int per_sum;     // chunks whose products share accumulators
     float oob;
     const float *x;  // input gradient: the forward's input, of the output's shape; templates and weights [C][O][taps]
     const float *templates, *weights;
@@ -300,12 +294,11 @@ __device__ __forceinline__ void split_recompute(lds_char *lds, int ptile, int mt
 }
 #endif
 
-// Input gradient of short contractions (split_grad_exact): three bf16 pieces, exact, and six products.  One workgroup: G
-// tiles of 32 input channels (from mtile0) x 128 pixels; a wave holds one of them x NI pixel tiles.
+// Input gradient.  One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
 template <int CG, int G>
-__device__ __forceinline__ void split_grad3_body(const SplitArgs &a, char *lds, int mtile0, int flag)
+__device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, int mtile0, int flag)
 {
-    constexpr int KIND = SPLIT_GRAD3;
+    constexpr int KIND = SPLIT_GRAD;
     constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND);
     constexpr int P = split_plane_pixels(KIND, CG);
     constexpr int kPlane = split_lds_pixels(KIND) * 32;
@@ -449,7 +442,7 @@ __device__ __forceinline__ void split_grad3_body(const SplitArgs &a, char *lds, 
     float ctr[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-        ctr[r] = a.chan[mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4];
+        ctr[r] = a.ctr[mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int n = n0 + (ntile0 + i) * 32 + col;
@@ -492,17 +485,6 @@ __device__ __forceinline__ void split_grad3_body(const SplitArgs &a, char *lds, 
     }
 }
 
-template <int CG>
-__global__ __launch_bounds__(kThreads, 2) void sim_split_grad3_kernel(const SplitArgs a, int flag)
-{
-    __shared__ __align__(16) char split_lds[split_lds_bytes(SPLIT_GRAD3)];
-    const int full = a.n_mtiles / a.gmax, y = blockIdx.y;
-    if (a.gmax == 2 && y < full)
-        split_grad3_body<CG, 2>(a, split_lds, y * 2, flag);
-    else
-        split_grad3_body<CG, 1>(a, split_lds, y < full ? y : full * a.gmax, flag);
-}
-
 // How a workgroup's pixels, 128 from n0 on, lie in the stack of padded images: the virtual row of the first, and what is
 // staged for them.
 __device__ __forceinline__ int split_virtual_row(const SplitArgs &a, int n, int &img, int &c)
@@ -516,12 +498,12 @@ __device__ __forceinline__ int split_virtual_row(const SplitArgs &a, int n, int 
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef const __attribute__((address_space(4))) float uniform_float;
 
-// One workgroup: G template tiles of 32 (from mtile0; input gradient: of input channels) x 128 pixels; a wave holds one
-// template tile x NI pixel tiles.  flag: forward, the normalized mode; input gradient, NaN inputs ignored.
+// Forward.  One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel
+// tiles.
 template <int KIND, int CG, int G>
-__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 &near, int ptile, int mtile0, int flag)
+__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 &near, int ptile, int mtile0, int norm)
 {
-    constexpr bool MASKED = KIND == SPLIT_MASKED, GRAD = KIND == SPLIT_GRAD;
+    constexpr bool MASKED = KIND == SPLIT_MASKED;
     constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND), kWaves = kThreads / 64;
     constexpr int P = split_plane_pixels(KIND, CG);
     constexpr int kPlane = split_lds_pixels(KIND) * 32;
@@ -539,23 +521,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
     const int rows = split_virtual_row(a, min(n0 + kSplitPixels, a.total) - 1, img1, c1) - v0 + a.taps / a.bw;
     const int staged = min(rows * a.Wp, P), per_half = (staged + 63) / 64;
 
-    // input gradient: every image of g has a scale, its largest value at 2^14 (exponents in LDS)
-    __attribute__((address_space(3))) int *image_exp = (__attribute__((address_space(3))) int *)(lds + split_lds_bytes(KIND));
-    if (GRAD) {
-        for (int i = tid; i <= img1 - img0; i += kThreads) {
-            const float *peak = a.peaks + (size_t)(img0 + i) * a.parts;
-            float most = 0.0f;
-            bool infinite = false;
-            for (int j = 0; j < a.parts; ++j) {
-                most = fmaxf(most, __builtin_fabsf(peak[j]));
-                infinite |= __builtin_signbit(peak[j]) != 0;
-            }
-            const int exp = most > 0.0f ? 14 - split_exponent(most) : 0;
-            image_exp[i] = min(150, max(-150, exp)) * 2 + infinite;
-        }
-        __syncthreads();
-    }
-
     // The images from this tile's first on, for loads that give zero outside of them (and wherever voffset is kOutside).
     const unsigned plane = (unsigned)a.H * a.W * 4u;
     constexpr unsigned kOutside = 0x80000000u;
@@ -565,7 +530,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
         __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)(behind < 0x7ffffffcu ? behind : 0x7ffffffcu), 0x00020000);
     // where this lane's staged elements come from (the same for every chunk)
     unsigned src[kItems];
-    int exps[GRAD ? kItems : 1];
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
         const int item = wave + kWaves * i, g = CG == 16 && item >= per_half, q = (item - (g ? per_half : 0)) * 64 + lane;
@@ -573,8 +537,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
         const int v = v0 + vr, img = (int)fast_div((unsigned)v, a.d_hv), r = v - img * a.Hv - a.ph;
         const bool in = q < staged && r >= 0 && r < a.H && c >= 0 && c < a.W;
         src[i] = in ? (unsigned)((((img - img0) * a.C + 8 * g) * a.H + r) * a.W + c) * 4u : kOutside;
-        if (GRAD)
-            exps[GRAD ? i : 0] = in ? image_exp[img - img0] >> 1 : 0;
     }
     // and this lane's operands: the LDS byte address of its pixel's first tap
     int at[NI];
@@ -586,17 +548,14 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
     }
 
     // sum: of the chunks before this one, whose own is acc; with missing values tm, the present -w (t'^2 + m / s^2), and lg
-    // (input gradient: of A, and su2, ac2 of B)
     constexpr bool TWO = !MASKED && NI <= 2;   // the two products' chunk sums apart: room for them
-    f32x16 sum[NI], acc[NI], su2[GRAD ? NI : 1], ac2[TWO ? NI : 1], tm[MASKED ? NI : 1], lg[MASKED ? NI : 1];
+    f32x16 sum[NI], acc[NI], ac2[TWO ? NI : 1], tm[MASKED ? NI : 1], lg[MASKED ? NI : 1];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         sum[i] = 0.0f;
         acc[i] = 0.0f;
         if (TWO)
             ac2[i] = 0.0f;
-        if (GRAD)
-            su2[i] = 0.0f;
         if (MASKED) {
             tm[i] = 0.0f;
             lg[i] = 0.0f;
@@ -610,35 +569,35 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
     for (int q = 0; q < NA; ++q)
         next[q] = pp[q * 64 + lane];
 
-    // (wide rows of the input gradient have more items than there are registers for)
-    constexpr int kRound = GRAD ? 4 : kItems;
-    float x[kRound][8];
-    auto request = [&](int chunk, int first) {   // a chunk's values of this lane's pixels, channels behind the last as the last
+    float x[kItems][8];
+    auto request = [&](int chunk) {   // a chunk's values of this lane's pixels, channels behind the last as the last
 #pragma unroll
-        for (int i = 0; i < kRound; ++i) {
-            const int item = wave + kWaves * (first + i);
-            if (first + i >= kItems || item >= kHalves * per_half)
+        for (int i = 0; i < kItems; ++i) {
+            const int item = wave + kWaves * i;
+            if (item >= kHalves * per_half)
                 continue;
             const int g = CG == 16 && item >= per_half, there = a.C - 1 - (chunk * CG + 8 * g);
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 x[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                    rsrc, src[(first + i) % kItems], (chunk * CG + max(-8 * g, min(j, there))) * plane, 0));
+                    rsrc, src[i], (chunk * CG + max(-8 * g, min(j, there))) * plane, 0));
         }
     };
-    auto convert = [&](int chunk, int first) {
+    request(0);
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < kRound; ++i) {
-            const int item = wave + kWaves * (first + i), at = (first + i) % kItems;
-            if (first + i >= kItems || item >= kHalves * per_half)
+        for (int i = 0; i < kItems; ++i) {
+            const int item = wave + kWaves * i;
+            if (item >= kHalves * per_half)
                 continue;
             const int g = CG == 16 && item >= per_half, q = (item - (g ? per_half : 0)) * 64 + lane;
             const int c0 = chunk * CG + 8 * g;
             uniform_float *chan = (uniform_float *)(a.chan + c0);
-            if (!GRAD && a.oob != 0.0f)   // (a NaN too)
+            if (a.oob != 0.0f)   // (a NaN too)
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    x[i][j] = src[at] == kOutside ? a.oob : x[i][j];
+                    x[i][j] = src[i] == kOutside ? a.oob : x[i][j];
             if (c0 + 8 > a.C)    // channels behind the last have zero parameters: any finite value will do
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
@@ -646,12 +605,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
             f16x8 v[5];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                _Float16 hi, lo;
-                if (GRAD) {
-                    split2(ldexpf(x[i][j], exps[GRAD ? at : 0]), hi, lo);
-                    v[0][j] = hi; v[1][j] = lo;
-                    continue;
-                }
                 const float s = chan[SPLIT_S * a.chunks * CG + j], ncs = chan[SPLIT_NCS * a.chunks * CG + j];
                 float d = __builtin_fmaf(x[i][j], s, ncs);
                 float d2 = __builtin_fmaf(d, d, -chan[SPLIT_M * a.chunks * CG + j]);
@@ -661,6 +614,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                     d2 = ok ? d2 : 0.0f;
                     v[4][j] = ok ? (_Float16)1.0f : (_Float16)0.0f;
                 }
+                _Float16 hi, lo;
                 split2(d2, hi, lo);
                 v[0][j] = hi; v[1][j] = lo;
                 split2(d, hi, lo);
@@ -672,28 +626,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                 for (int b = 0; b < NB; ++b)
                     *reinterpret_cast<f16x8 *>(dst + b * kPlane) = v[b];
             }
-        }
-    };
-    int since = 0;
-    auto add_up = [&]() {   // a sum of its own for every so many steps' products: see the head of the file
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            sum[i] += TWO && !GRAD ? acc[i] + ac2[TWO ? i : 0] : acc[i];
-            if (GRAD)
-                su2[GRAD ? i : 0] += ac2[TWO ? i : 0];
-            acc[i] = 0.0f;
-            if (TWO)
-                ac2[i] = 0.0f;
-        }
-        since = 0;
-    };
-    request(0, 0);
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
-        __syncthreads();
-        convert(chunk, 0);
-        if (kItems > kRound && wave + kWaves * kRound < kHalves * per_half) {
-            request(chunk, kRound);
-            convert(chunk, kRound);
         }
         __syncthreads();
         int dh = 0, dw = 0;
@@ -728,12 +660,12 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
             for (int q = 0; q < NA; ++q)
                 next[q] = pp[q * 64 + lane];
             if (step + 1 == a.steps && chunk + 1 < a.chunks)
-                request(chunk + 1, 0);
+                request(chunk + 1);
         };
         int off = next_offset();
         if (!active) {
             if (chunk + 1 < a.chunks)
-                request(chunk + 1, 0);
+                request(chunk + 1);
         } else if constexpr (NI == 4) {
             // An accumulator's products follow one another at 48 cycles, two accumulators' in turn at 32: two pixel tiles at
             // a time, their squares while their cross terms' operands are requested, then the other way round.
@@ -770,8 +702,6 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                     fetch_pair(Bq, 1 - pair, pair == 0 ? off : off_next, 0);
                     products(pair, A[2], A[3], Be);
                 }
-                if (++since == a.per_sum)
-                    add_up();
                 off = off_next;
             }
         } else {
@@ -797,21 +727,20 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                         fetch_all(B[0], at[i] + off);
                     const f16x8 (&b)[NB] = B[i & kAhead];
                     f32x16 &cross = TWO ? ac2[TWO ? i : 0] : acc[i];
-                    constexpr int c = GRAD ? 0 : 2;   // the second product's operand (input gradient: g for both)
                     mul(acc[i], A0, b[1]);
                     if (MASKED)
                         mul(lg[MASKED ? i : 0], A[NA - 1], b[NB - 1]);
-                    mul(cross, A2, b[c + 1]);
+                    mul(cross, A2, b[3]);
                     if (MASKED)
                         mul(tm[MASKED ? i : 0], A[NA - 4], b[NB - 1]);
                     mul(acc[i], A[1], b[0]);
                     if (MASKED)
                         mul(lg[MASKED ? i : 0], A[NA - 2], b[NB - 1]);
-                    mul(cross, A[3], b[c]);
+                    mul(cross, A[3], b[2]);
                     if (MASKED)   // (the lesser piece of what tm sums, where small sums are kept)
                         mul(acc[i], A[NA - 3], b[NB - 1]);
                     mul(acc[i], A[0], b[0]);
-                    mul(cross, A[2], b[c]);
+                    mul(cross, A[2], b[2]);
                     if (kAhead)
                         __builtin_amdgcn_sched_barrier(0);
                 }
@@ -819,26 +748,31 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
 #pragma unroll
                     for (int b = 0; b < NB; ++b)
                         B[0][b] = B[kAhead][b];
-                if (++since == a.per_sum)
-                    add_up();
                 off = off_next;
             }
         }
+        // a sum of its own for every so many products: see the head of the file
+        if ((chunk + 1) % a.per_sum == 0 || chunk + 1 == a.chunks)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                sum[i] += TWO ? acc[i] + ac2[TWO ? i : 0] : acc[i];
+                acc[i] = 0.0f;
+                if (TWO)
+                    ac2[i] = 0.0f;
+            }
     }
-    if (since > 0)
-        add_up();
 
     // lane: pixel col of each tile, templates 8 (r / 4) + 4 half + r % 4
     if (!active)
         return;
     const f32x4 *rows4 = reinterpret_cast<const f32x4 *>(a.rows) + mtile * kSplitRows + 4 * half;
-    const float *lgs = GRAD ? a.rows : a.rows + (size_t)4 * a.n_mtiles * kSplitRows + mtile * kSplitRows + 4 * half;
+    const float *lgs = a.rows + (size_t)4 * a.n_mtiles * kSplitRows + mtile * kSplitRows + 4 * half;
     f32x4 row[16];
     float lgm[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         row[r] = rows4[8 * (r / 4) + r % 4];
-        lgm[r] = KIND == SPLIT_FWD && flag ? lgs[8 * (r / 4) + r % 4] : 0.0f;
+        lgm[r] = !MASKED && norm ? lgs[8 * (r / 4) + r % 4] : 0.0f;
     }
     // stores by a pixel's offset and a row's; rows behind the last template go outside of the buffer
     const int left = a.O - mtile * kSplitRows;
@@ -847,45 +781,11 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
     const size_t room = ((size_t)(a.total / a.npix - img0) * a.O - mtile * kSplitRows) * image;
     const __amdgpu_buffer_rsrc_t to =
         __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)(room < 0x7ffffffcu ? room : 0x7ffffffcu), 0x00020000);
-    const __amdgpu_buffer_rsrc_t inputs = __builtin_amdgcn_make_buffer_rsrc(   // input gradient: the forward's, of the output's shape
-        (void *)((GRAD ? a.x : a.in) + (tile - a.out)), 0, (int)(room < 0x7ffffffcu ? room : 0x7ffffffcu), 0x00020000);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int n = n0 + (ntile0 + i) * 32 + col;
         const int img = (int)fast_div((unsigned)n, a.d_npix);
         const unsigned pixel = n < a.total ? ((unsigned)((img - img0) * a.O + 4 * half) * a.npix + (n - img * a.npix)) * 4u : kOutside;
-        if constexpr (GRAD) {
-            float xs[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                xs[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                    inputs, 8 * (r / 4) + r % 4 + 4 * half < left ? pixel : kOutside, (8 * (r / 4) + r % 4) * image, 0));
-            const int exp = n < a.total ? image_exp[img - img0] : 0;
-            float v[16], any = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float A = ldexpf(sum[i][r], __float_as_int(row[r][SPLIT_EXP_A]) - (exp >> 1));
-                const float B = ldexpf(su2[i][r], __float_as_int(row[r][SPLIT_EXP_B]) - (exp >> 1));
-                v[r] = __builtin_fmaf(-(xs[r] - row[r][SPLIT_CENTRE]), B, A);
-                any = __builtin_fmaf(v[r], 0.0f, any);   // NaN once a value is not finite
-            }
-            if (any != any && n < a.total) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int ml = 8 * (r / 4) + r % 4 + 4 * half;
-                    // an infinite factor leaves its sums NaN: only the terms tell
-                    if (v[r] != v[r] && ml < left && ((exp & 1) || row[r][SPLIT_INFINITE] != 0.0f))
-                        v[r] = split_grad_terms(img, mtile * kSplitRows + ml, n - img * a.npix, xs[r]);
-                    if (flag && xs[r] != xs[r])
-                        v[r] = 0.0f;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v[r]), to,
-                    8 * (r / 4) + r % 4 + 4 * half < left ? pixel : kOutside, (8 * (r / 4) + r % 4) * image, 0);
-            continue;
-        }
         unsigned flagged = 0;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -902,7 +802,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                 v = __builtin_fmaf(sum[i][r], row[r][SPLIT_UNSCALE], row[r][SPLIT_BIAS]) + row[r][SPLIT_BIAS_LESSER];
                 const float mag = __builtin_fabsf(v);
                 fine = mag >= row[r][SPLIT_THR] && mag < 1e37f;
-                if (flag)
+                if (norm)
                     v = __builtin_fmaf(0.5f, v, lgm[r]);
             }
             flagged |= fine ? 0u : 1u << r;
@@ -926,7 +826,7 @@ template <int KIND, int CG>
 __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs a, int flag)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-    __shared__ __align__(16) char split_lds[split_lds_bytes(KIND) + (KIND == SPLIT_GRAD ? kSplitPixels * sizeof(int) : 0)];
+    __shared__ __align__(16) char split_lds[split_lds_bytes(KIND)];
     __shared__ int any_near;   // of the workgroup's outputs, one below the guard's line
     if (KIND != SPLIT_GRAD && threadIdx.x == 0)
         any_near = 0;
@@ -945,13 +845,18 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
     // consecutive workgroups go to the eight XCDs in turn: a run of neighbouring pixel tiles, which share rows, to each
     const int run = gridDim.x / 8, x = blockIdx.x;
     const int ptile = x < run * 8 ? x % 8 * run + x / 8 : x;
-    if (KIND == SPLIT_FWD && g == 4)
-        split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, near, ptile, mtile0, flag);
-    else if (g == 2)
-        split_body<KIND, CG, 2>(a, split_lds, near, ptile, mtile0, flag);
-    else
-        split_body<KIND, CG, 1>(a, split_lds, near, ptile, mtile0, flag);
-    if constexpr (KIND != SPLIT_GRAD) {
+    if constexpr (KIND == SPLIT_GRAD) {
+        if (g == 2)
+            split_grad_body<CG, 2>(a, split_lds, mtile0, flag);
+        else
+            split_grad_body<CG, 1>(a, split_lds, mtile0, flag);
+    } else {
+        if (KIND == SPLIT_FWD && g == 4)
+            split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, near, ptile, mtile0, flag);
+        else if (g == 2)
+            split_body<KIND, CG, 2>(a, split_lds, near, ptile, mtile0, flag);
+        else
+            split_body<KIND, CG, 1>(a, split_lds, near, ptile, mtile0, flag);
         if (near[0] | near[1] | near[2] | near[3])
             any_near = 1;
         __syncthreads();
@@ -981,8 +886,8 @@ __device__ __forceinline__ float split_grad_centre(const SplitPack &a, float par
 }
 
 // Packs the input gradient's coefficients, rows = input channels, contraction = (template, flipped tap): three pieces
-// each of s w (t - c) and s w.  A workgroup: a tile of rows, a chunk and four of its steps.
-__global__ __launch_bounds__(kThreads) void sim_split_grad3_pack_kernel(const SplitPack a, float scale)
+// each of s w (t - c) and s w.  Same blocks as split_pack_block.
+__global__ __launch_bounds__(kThreads) void sim_split_grad_pack_kernel(const SplitPack a, float scale)
 {
     __shared__ float centre[kSplitRows];
     const int tid = threadIdx.x, parts = (a.steps + 3) / 4;
@@ -998,7 +903,7 @@ __global__ __launch_bounds__(kThreads) void sim_split_grad3_pack_kernel(const Sp
         if ((tid & 15) == 0) {
             centre[16 * i + (tid >> 4)] = c;
             if (chunk == 0 && part == 0)
-                a.chan[mtile * kSplitRows + 16 * i + (tid >> 4)] = c;
+                a.ctr[mtile * kSplitRows + 16 * i + (tid >> 4)] = c;
         }
     }
     __syncthreads();
@@ -1030,133 +935,6 @@ __global__ __launch_bounds__(kThreads) void sim_split_grad3_pack_kernel(const Sp
         dst[q * 64] = v[q];
 }
 
-// The input gradient's launch in front.  First its coefficients, an input channel (a row of the product, n_mtiles * 32 of
-// them) to a workgroup: two pieces each of s w (t - c) and s w, c the channel's mean, the largest at 2^13; contraction =
-// (template, flipped tap).  Then the largest sizes in g, a share of an image to a workgroup.
-__global__ __launch_bounds__(kThreads) void sim_split_grad_pack_kernel(const SplitPack a, float scale, const float *g,
-                                                                       long long image, float *peaks, int parts)
-{
-    __shared__ float2 row_tw[kSplitRowLds];
-    __shared__ float wave_sum[kThreads / 64];
-    __shared__ int ints[kThreads / 64][2];
-    const int tid = threadIdx.x, wave = tid >> 6, rows = a.n_mtiles * kSplitRows;
-    if ((int)blockIdx.x >= rows) {
-        const int part = ((int)blockIdx.x - rows) % parts, img = ((int)blockIdx.x - rows) / parts;
-        const long long from = image * part / parts, end = image * (part + 1) / parts;
-        const float *src = g + (size_t)img * image;
-        float most = 0.0f;
-        bool infinite = false;
-        long long i = from + tid;
-        for (; i + 7 * kThreads < end; i += 8 * kThreads) {
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                v[j] = __builtin_fabsf(src[i + j * kThreads]);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                infinite |= v[j] == INFINITY;
-                most = v[j] < INFINITY ? fmaxf(most, v[j]) : most;
-            }
-        }
-        for (; i < end; i += kThreads) {
-            const float v = __builtin_fabsf(src[i]);
-            infinite |= v == INFINITY;
-            most = v < INFINITY ? fmaxf(most, v) : most;
-        }
-        for (int d = 32; d > 0; d >>= 1)
-            most = fmaxf(most, __shfl_xor(most, d, 64));
-        if ((tid & 63) == 0)
-            wave_sum[wave] = most;
-        infinite = __syncthreads_or(infinite);
-        if (tid == 0) {
-            most = fmaxf(fmaxf(wave_sum[0], wave_sum[1]), fmaxf(wave_sum[2], wave_sum[3]));
-            peaks[(size_t)img * parts + part] = infinite ? -most : most;
-        }
-        return;
-    }
-    // (neighbouring channels to one XCD: see split_pack_block)
-    const int c = (int)blockIdx.x % 8 * (rows / 8) + (int)blockIdx.x / 8, n = a.O * a.taps;
-    const bool real = c < a.C;
-    auto load = [&](int k) {
-        const int o = (int)fast_div((unsigned)k, a.d_taps);
-        const size_t at = ((size_t)o * a.C + c) * a.taps + (k - o * a.taps);
-        return make_float2(a.templates[at], scale * a.weights[at]);
-    };
-    float sum = 0.0f;
-    if (real)
-#pragma unroll 4
-        for (int k = tid; k < n; k += kThreads) {
-            const float2 tw = load(k);
-            if (k < kSplitRowLds)
-                row_tw[k] = tw;
-            sum += tw.x;
-        }
-    for (int d = 32; d > 0; d >>= 1)
-        sum += __shfl_xor(sum, d, 64);
-    if ((tid & 63) == 0)
-        wave_sum[wave] = sum;
-    __syncthreads();
-    sum = ((wave_sum[0] + wave_sum[1]) + (wave_sum[2] + wave_sum[3])) / (float)n;
-    const float centre = real && __builtin_fabsf(sum) < 1e18f ? sum : 0.0f;
-    auto element = [&](int k) { return k < kSplitRowLds ? row_tw[k] : load(k); };
-    int top[2] = {kNoExponent, kNoExponent};
-    bool infinite = false;
-    if (real)
-#pragma unroll 1
-        for (int k = tid; k < n; k += kThreads) {
-            const float2 tw = element(k);
-            const float both = tw.y * (tw.x - centre);
-            infinite |= __builtin_isinf(both) || __builtin_isinf(tw.y);
-            top[0] = max(top[0], split_exponent(both));
-            top[1] = max(top[1], split_exponent(tw.y));
-        }
-    for (int d = 32; d > 0; d >>= 1) {
-        top[0] = max(top[0], __shfl_xor(top[0], d, 64));
-        top[1] = max(top[1], __shfl_xor(top[1], d, 64));
-    }
-    if ((tid & 63) == 0) {
-        ints[wave][0] = top[0];
-        ints[wave][1] = top[1];
-    }
-    infinite = __syncthreads_or(infinite);
-    int shift[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int most = max(max(ints[0][i], ints[1][i]), max(ints[2][i], ints[3][i]));
-        shift[i] = most > kNoExponent ? 13 - most : 0;
-    }
-    if (tid == 0) {
-        float4 row;
-        row.x = centre;
-        row.y = __builtin_bit_cast(float, -shift[0]);
-        row.z = __builtin_bit_cast(float, -shift[1]);
-        row.w = infinite ? 1.0f : 0.0f;
-        reinterpret_cast<float4 *>(a.rows)[c] = row;
-    }
-#pragma unroll 1
-    for (int i = tid; i < a.chunks * a.steps * 2; i += kThreads) {
-        const int half = i & 1, at = i >> 1, chunk = (int)fast_div((unsigned)at, a.d_steps), step = at - chunk * a.steps;
-        const int tap = a.cg == 16 ? step : 2 * step + half;
-        f16x8 v[4];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int o = chunk * a.cg + (a.cg == 16 ? 8 * half : 0) + j;
-            const bool there = real && o < a.O && tap < a.taps;
-            const float2 tw = element(there ? o * a.taps + (a.taps - 1 - tap) : 0);
-            _Float16 hi, lo;
-            split2_param(there ? ldexpf(tw.y * (tw.x - centre), shift[0]) : 0.0f, hi, lo);
-            v[0][j] = hi; v[1][j] = lo;
-            split2_param(there ? ldexpf(tw.y, shift[1]) : 0.0f, hi, lo);
-            v[2][j] = hi; v[3][j] = lo;
-        }
-        f16x8 *dst = reinterpret_cast<f16x8 *>(a.packed) +
-                     ((size_t)(c / kSplitRows) * a.chunks * a.steps + at) * a.pieces * 64 + 32 * half + c % kSplitRows;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            dst[q * 64] = v[q];
-    }
-}
-
 }  // namespace
 
 // The guard's line as a share of sum w t'^2: where this form's error (see the head of the file) is that of the sum it
@@ -1175,7 +953,7 @@ static SplitPlan split_geometry(const SimPlan &p, int kind)
         return s;
     // a workgroup addresses the images it touches by 31 bits
     const long long touched = (kSplitPixels - 1) / (1LL * p.oh * p.ow) + 2;
-    if (4 * touched * std::max(1LL * p.C * p.H * p.W, 1LL * p.O * p.oh * p.ow) >= (1LL << 31))
+    if (kind != SPLIT_GRAD && 4 * touched * std::max(1LL * p.C * p.H * p.W, 1LL * p.O * p.oh * p.ow) >= (1LL << 31))
         return s;
     s.Wp = (p.ow - 1) * p.sw + p.bw;
     s.Hv = (p.oh - 1) * p.sh + p.bh;
@@ -1210,12 +988,9 @@ static SplitPlan split_geometry(const SimPlan &p, int kind)
     s.chan = s.packed + (size_t)s.n_mtiles * s.chunks * s.steps * s.pieces * 1024;
     s.rows = s.chan + align_up((size_t)std::max(SPLIT_CHANNEL_FIELDS * s.chunks * s.cg, mpad) * sizeof(float), 256);
     s.flags = s.rows + align_up((size_t)5 * mpad * sizeof(float), 256);
-    // (input gradient: the largest sizes in shares of g's images)
-    s.parts = (int)std::max(1LL, std::min(16LL, 1LL * p.C * p.H * p.W / 16384));
-    s.exact = s.flags + align_up(kind == SPLIT_GRAD ? (size_t)p.B * s.parts * sizeof(float)
-                                                    : (size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
-    s.logs = s.exact + (kind >= SPLIT_GRAD ? 0 : align_up((size_t)p.O * p.K * sizeof(float2), 256));
-    s.total = s.logs + (kind >= SPLIT_GRAD || p.mode == SIM_MODE_L2 ? 0 : align_up((size_t)p.O * p.K * sizeof(float), 256));
+    s.exact = s.flags + align_up((size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
+    s.logs = s.exact + (kind == SPLIT_GRAD ? 0 : align_up((size_t)p.O * p.K * sizeof(float2), 256));
+    s.total = s.logs + (kind == SPLIT_GRAD || p.mode == SIM_MODE_L2 ? 0 : align_up((size_t)p.O * p.K * sizeof(float), 256));
     s.on = true;
     return s;
 }
@@ -1237,7 +1012,7 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     SplitPack a;
     a.templates = templates; a.weights = weights;
     a.packed = reinterpret_cast<unsigned short *>(ws + sp.packed);
-    a.chan = reinterpret_cast<float *>(ws + sp.chan);
+    a.chan = a.ctr = reinterpret_cast<float *>(ws + sp.chan);
     a.rows = reinterpret_cast<float *>(ws + sp.rows);
     a.exact = reinterpret_cast<float2 *>(ws + sp.exact);
     a.logs = reinterpret_cast<float *>(ws + sp.logs);
@@ -1247,6 +1022,7 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     a.d_taps = make_fast_div((unsigned)a.taps);
     a.d_steps = make_fast_div((unsigned)std::max(1, sp.steps));
     a.norm_const = p.mode == SIM_MODE_L2_NORM ? split_norm_const(p.K) : 0.0f;
+    a.pack_blocks = sp.on ? sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4) : 0;
     a.blocks = sp.on ? std::min(sp.n_mtiles * kSplitRows, 512) : 0;
     return a;
 }
@@ -1257,7 +1033,7 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
 {
     a.in = input; a.out = output;
     a.packed = ws + sp.packed;
-    a.chan = reinterpret_cast<const float *>(ws + sp.chan);
+    a.chan = a.ctr = reinterpret_cast<const float *>(ws + sp.chan);
     a.rows = reinterpret_cast<const float *>(ws + sp.rows);
     a.flags = reinterpret_cast<int *>(ws + sp.flags);
     a.exact = reinterpret_cast<const float2 *>(ws + sp.exact);
@@ -1268,7 +1044,7 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     a.bw = p.bw; a.sh = p.sh; a.sw = p.sw; a.ph = p.ph; a.pw = p.pw; a.taps = p.bh * p.bw;
     a.chunks = sp.chunks; a.steps = sp.steps; a.n_mtiles = sp.n_mtiles; a.Wp = sp.Wp; a.Hv = sp.Hv;
     a.oob = p.oob;
-    a.per_sum = KIND == SPLIT_GRAD ? 3 : std::max(2, sp.steps);
+    a.per_sum = std::max(1, 2 / sp.steps);
     a.d_npix = make_fast_div((unsigned)a.npix);
     a.d_ow = make_fast_div((unsigned)p.ow);
     a.d_wp = make_fast_div((unsigned)sp.Wp);
@@ -1281,12 +1057,7 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
         a.gmax /= 2;
     const int rest = sp.n_mtiles % a.gmax;
     const dim3 grid((unsigned)sp.n_ptiles, (unsigned)(sp.n_mtiles / a.gmax + (rest == 0 ? 0 : rest == 3 && KIND != SPLIT_FWD ? 2 : 1)));
-    if constexpr (KIND == SPLIT_GRAD3) {
-        if (sp.cg == 16)
-            hipLaunchKernelGGL(sim_split_grad3_kernel<16>, grid, dim3(kThreads), 0, s, a, flag);
-        else
-            hipLaunchKernelGGL(sim_split_grad3_kernel<8>, grid, dim3(kThreads), 0, s, a, flag);
-    } else if (sp.cg == 16)
+    if (sp.cg == 16)
         hipLaunchKernelGGL((sim_split_kernel<KIND, 16>), grid, dim3(kThreads), 0, s, a, flag);
     else
         hipLaunchKernelGGL((sim_split_kernel<KIND, 8>), grid, dim3(kThreads), 0, s, a, flag);
@@ -1303,13 +1074,9 @@ int sim_split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, 
 // ------------------------------------------------------------------------------------------------
 // Input gradient of the L2 modes at stride 1:  dX = A - (X - c) B,  A = sum g s w (t - c),  B = sum g s w  over (template,
 // tap) - the forward's contraction with g as the image (its channels are the templates, the taps flipped) and the input
-// channels as rows.  Two pieces each of g, every image of it scaled by its largest value, and of the coefficients, every
-// row by its largest; a sum of its own for every three steps (what the matrix unit cuts off its products grows with
-// the sum: 1.6e-7 with one for nine).  Scales by an image's largest value: a pixel whose values are 2^-30 of that and less
-// keeps fewer than 24 bits, 2^-50 of the largest absolutely.  32 x 128 x 28 x 28, 128 templates, 3 x 3, kernel: fp32 matrix
-// instructions 196 us, three bf16 pieces 103, this form 62 and 1 more to find the scales; error against 64 bits 6.0e-7,
-// 2.0e-7, 1.5e-7 of the gradient's 2-norm.  Short contractions keep the three pieces (split_grad_exact), small grids the
-// fp32 matrix instructions (sim_mfma_kernel), which split the contraction over workgroups.
+// channels as rows, g in three pieces against the three of each coefficient.  32 x 128 x 28 x 28, 128 templates, 3 x 3: 196 us
+// on the fp32 matrix instructions -> 101 us, error against 64 bits 6.0e-7 -> 2.0e-7 of the gradient's 2-norm.  Small grids
+// keep that kernel (sim_mfma_kernel), which splits the contraction over workgroups.
 // ------------------------------------------------------------------------------------------------
 static SimPlan grad_as_forward(const SimPlan &p)
 {
@@ -1321,18 +1088,12 @@ static SimPlan grad_as_forward(const SimPlan &p)
     return q;
 }
 
-// Whether the contraction is too short for two pieces.  Its terms have either sign, so that what the pieces leave out (6e-8
-// of a term) stays in the sum, where three pieces only have the sum's roundings, which grow with its length.  Error
-// against 64 bits, two pieces and three: 576 terms 1.3e-7 and 1.35e-7, 1152 1.5e-7 and 2.0e-7, 288 1.1e-7 and 0.9e-7,
-// 64 1.0e-7 and 0.5e-7.
-static bool split_grad_exact(const SimPlan &p) { return p.O * p.bh * p.bw < 576; }
-
 static SplitPlan split_grad_plan(const SimPlan &p)
 {
     if (!p.split || p.mode == SIM_MODE_L1 || p.B == 0 || p.sh != 1 || p.sw != 1 || p.ph > p.bh - 1 || p.pw > p.bw - 1)
         return SplitPlan();
     const SimPlan q = grad_as_forward(p);
-    const SplitPlan s = split_geometry(q, split_grad_exact(p) ? SPLIT_GRAD3 : SPLIT_GRAD);
+    const SplitPlan s = split_geometry(q, SPLIT_GRAD);
     // Fewer tiles than fill the chip twice: a workgroup walks the whole contraction, 1.6 us to stage a chunk and 0.49 a step,
     // where the fp32 form splits it over workgroups and takes some 45 us + 1 per tap + 38 per 10^9 terms.  Short
     // contractions are the faster ones here (8 x 128 x 16 x 16, 128 templates, 3 x 3, 64 tiles: 53 us, fp32 form 62; 64 templates 30
@@ -1363,21 +1124,10 @@ int sim_split_grad_input_launch(const SimPlan &p, const float *input, const floa
     SplitArgs g = {};
     g.x = input; g.templates = templates; g.weights = weights;
     g.scale = p.mode != SIM_MODE_L2 ? 1.0f : 2.0f;   // the normalized functor halves the plain one
-    const int ignore_nan = p.mode == SIM_MODE_L2_NORM_IGNORE_NAN;
-    if (split_grad_exact(p)) {
-        hipLaunchKernelGGL(sim_split_grad3_pack_kernel, dim3(sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4)), dim3(kThreads), 0, s,
-                           a, g.scale);
-        if (hipGetLastError() != hipSuccess)
-            return SIMNETS_ERR_HIP;
-        return split_launch<SPLIT_GRAD3>(q, sp, output_grad, input_grad, ws, ignore_nan, s, g);
-    }
-    float *peaks = reinterpret_cast<float *>(ws + sp.flags);
-    g.peaks = peaks; g.parts = sp.parts;
-    hipLaunchKernelGGL(sim_split_grad_pack_kernel, dim3(sp.n_mtiles * kSplitRows + p.B * sp.parts), dim3(kThreads), 0, s, a,
-                       g.scale, output_grad, 1LL * p.O * p.oh * p.ow, peaks, sp.parts);
+    hipLaunchKernelGGL(sim_split_grad_pack_kernel, dim3(a.pack_blocks), dim3(kThreads), 0, s, a, g.scale);
     if (hipGetLastError() != hipSuccess)
         return SIMNETS_ERR_HIP;
-    return split_launch<SPLIT_GRAD>(q, sp, output_grad, input_grad, ws, ignore_nan, s, g);
+    return split_launch<SPLIT_GRAD>(q, sp, output_grad, input_grad, ws, p.mode == SIM_MODE_L2_NORM_IGNORE_NAN, s, g);
 }
 
 }  // namespace simnets

@@ -478,3 +478,41 @@ def test_split_input_gradient_scales(pkg, O, block):
     assert not got[5].any()
     err = (got - want).flatten(2).norm(dim=2) / want.flatten(2).norm(dim=2).clamp_min(1e-300)
     assert float(err.max()) <= 4 * math.sqrt(O * block * block) * 2.0 ** -24, float(err.max())
+
+
+@pytest.mark.parametrize("kind", ["templates", "routed", "loud", "pixel"])
+@pytest.mark.parametrize("O, block", [(64, 3), (32, 3), (128, 3)])    # 576, 288, 1152 terms
+def test_split_input_gradient_over_templates_and_pixels_of_any_size(pkg, O, block, kind):
+    """Output gradients that reach templates whose weights are small beside others', and pixels whose output gradients are
+    small beside others': every element by itself has the error of a sum of its terms, whatever stands beside them."""
+    g = torch.Generator(device="cuda").manual_seed(71)
+    B, C, H, W = 36, 37, 23, 30
+    x = torch.randn((B, C, H, W), generator=g, device="cuda")
+    t = torch.randn((O, C, block, block), generator=g, device="cuda")
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    go = torch.randn((B, O, H - block + 1, W - block + 1), generator=g, device="cuda")
+    clear = torch.ones((B, 1, H, W), dtype=torch.bool)
+    if kind == "templates":    # ten orders of magnitude, the output gradient the larger the smaller the weights
+        f = 10.0 ** (torch.rand((O, 1, 1, 1), generator=g, device="cuda") * 10 - 6)
+        w, go = w * f, go / f[:, 0][None]
+    elif kind == "routed":     # to four templates of small weights alone
+        w[::O // 4] *= 1e-10
+        go[:, torch.arange(O, device="cuda") % (O // 4) != 0] = 0.0
+    elif kind == "loud":       # one template with large weights that nothing reaches
+        w[5] *= 1e8
+        go[:, 5] = 0.0
+    else:                      # one output pixel of an image beside the others
+        r, c = 7, 12
+        go[:, :, r, c] *= 1e14
+        clear[:, :, r:r + block, c:c + block] = False
+    kw = dict(blocks=[block, block], strides=[1, 1], padding=[0, 0])
+    assert pieces_used(pkg, (B, C, H, W), O, **kw)["input"]
+    got = pkg.similarity_input_grad(x, t, w, go, **kw).double().cpu()
+    xd, td, wd, gd = (v.double().cpu() for v in (x, t, w, go))
+    up = lambda a, k: torch.nn.functional.conv_transpose2d(a, k)
+    want = 2 * (up(gd, wd * td) - xd * up(gd, wd))
+    # A - (x - c) B, c of the templates' size at most: each of A and B rounds 6 K / 16 times, at no more than the sum of its
+    # terms' sizes
+    size = 2 * (up(gd.abs(), wd * (td.abs() + 1)) + (xd.abs() + 1) * up(gd.abs(), wd))
+    err = ((got - want).abs() / size.clamp_min(1e-300))[clear.expand_as(got)]
+    assert float(err.max()) <= 2 * (O * block * block / 16 + 8) * 2.0 ** -24, float(err.max())
