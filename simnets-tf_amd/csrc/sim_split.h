@@ -38,9 +38,9 @@ SplitPlan sim_split_plan(const SimPlan &p);
 // Per template four floats: what the sums of a row lack (bias, in two floats; with missing values the guard: outputs below
 // it times the sum of the present w (t'^2 + m / s^2) are recomputed), the power of two that takes back what the packed
 // parameters were multiplied by, and the line below which outputs are recomputed.  Behind those of the n_mtiles * 32
-// templates the constants of the normalized modes.
+// templates the constants of the normalized modes, and by what the line rises with the level.
 enum SplitRow { SPLIT_BIAS, SPLIT_BIAS_LESSER, SPLIT_UNSCALE, SPLIT_THR, SPLIT_GUARD = SPLIT_BIAS };
-// Per channel, [field][chunks * cg], zeros behind the last channel: the scale s, -c s, and m.
+// Per channel, [level][field][chunks * cg], zeros behind the last channel: the scale s, -c s, and m.
 enum SplitChannel { SPLIT_S, SPLIT_NCS, SPLIT_M, SPLIT_CHANNEL_FIELDS };
 
 struct SplitPack {
@@ -102,6 +102,10 @@ __device__ __forceinline__ float split_sum(float hi, float lo)
 // v = hi + lo / 2048, each the nearest half-precision value to what is left: 24 bits for |v| from 2^-14 to 65504, and to
 // 2^-36 absolutely below that.  A v beyond 65504 gives an infinity and a NaN.
 constexpr float kSplitLow = 2048.0f;
+// The forward's scales: levels of 2^-3 of the packed ones (a parameter times 2^-24 is still a half-precision value; with missing
+// values the lesser pieces meet twice as much).
+constexpr int kSplitLevels = 9, kSplitMaskedLevels = 5, kSplitLevelBits = 3;
+constexpr float kSplitMost = 181.0f;   // the largest staged value, its square below 2^15
 
 __device__ __forceinline__ void split2(float v, _Float16 &hi, _Float16 &lo)
 {
@@ -173,8 +177,9 @@ __device__ __forceinline__ int split_wave_max(int v)
 //
 // Scales, all powers of two.  A channel's s: w s^-2 of about one size for all channels, so that the terms of a sum are
 // as its values x'^2 s^2 are, and the largest of 256 sampled w (t - t2)^2 / 2 at 2^-3.  So a value is 24 bits while its
-// term is above 2^-14, is off by 2^-36 absolutely below, and overflows (a NaN, recomputed) some 700 times further from the
-// centre than the templates are from one another.  m: the sampled mean of t'^2 s^2, see similarity_split.hip.
+// term is above 2^-14, is off by 2^-36 absolutely below, and its square overflows 250 to 700 times further from the
+// centre than the templates are from one another; workgroups that meet many such inputs take smaller scales (levels).  m:
+// the sampled mean of t'^2 s^2, see similarity_split.hip.
 // A template's row: its largest parameter at 2^13.
 __device__ inline void split_pack_block(const SplitPack &a, int index, float *lds)
 {
@@ -262,11 +267,13 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
     if (block == 0)
         for (int c = tid; c < a.chunks * a.cg; c += 256) {
             const bool there = c < a.C;
-            const float s = there ? ldexpf(1.0f, le[c]) : 0.0f;
             float *dst = a.chan + c;
-            dst[SPLIT_S * a.chunks * a.cg] = s;
-            dst[SPLIT_NCS * a.chunks * a.cg] = there ? -(lc[c] * s) : 0.0f;
-            dst[SPLIT_M * a.chunks * a.cg] = there ? lm[c] : 0.0f;
+            for (int level = 0; level < kSplitLevels; ++level, dst += SPLIT_CHANNEL_FIELDS * a.chunks * a.cg) {
+                const float s = there ? ldexpf(1.0f, le[c] - kSplitLevelBits * level) : 0.0f;
+                dst[SPLIT_S * a.chunks * a.cg] = s;
+                dst[SPLIT_NCS * a.chunks * a.cg] = there ? -(lc[c] * s) : 0.0f;
+                dst[SPLIT_M * a.chunks * a.cg] = there ? ldexpf(lm[c], -2 * kSplitLevelBits * level) : 0.0f;
+            }
         }
     for (int m = block; m < a.n_mtiles * kSplitRows; m += a.blocks) {
         // The loops below run once or twice in a workgroup: unrolled, their code takes longer to fetch than to run.
@@ -281,7 +288,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
         for (int k = tid + (m == block ? 256 * kAhead : 0); k < in_lds; k += 256)
             row_tw[k] = make_float2(mt[k], mw[k]);
         double sum[3] = {};   // w t'^2, w m / s^2, logarithms
-        float size[2] = {};   // w / s^2, w t^2
+        float size[2] = {};   // w / s^2 or 2 w |t'| / s, w t^2
         bool bad = false, weighted = false;
         int top = kNoExponent;
 #pragma unroll 1
@@ -296,7 +303,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             weighted |= w != 0.0f;
             sum[0] += (double)w * tc * tc;
             sum[1] += (double)w * spread;
-            size[0] += ldexpf(w, -2 * es);
+            size[0] += fmaxf(ldexpf(w, -2 * es), ldexpf(2.0f * w * __builtin_fabsf(tc), -es));
             size[1] += w * t * t;
             const int ew = split_exponent(w);
             top = max(top, max(ew - 2 * es, ew + split_exponent(tc) + 2 - es));
@@ -341,8 +348,9 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             sum[2] = all[2];
             const double both = all[0] + all[1], line = a.line * fmax(all[0], 0.5 * both);
             double thr = weighted ? 0x1p-60 : 0.0;   // without weights zero is the exact sum
-            // the values' absolute error is below 2^-25 of such a sum
-            thr = fmax(thr, all[3] * 0x1p-13 / (double)sqrtf((float)a.K));
+            // The values' absolute error, 2^-36 each, stays below 2^-23 of such a sum; 2^6 times as much with each level.
+            const double values = all[3] * 0x1p-13 / (double)sqrtf((float)a.K);
+            thr = fmax(thr, values);
             if (!masked)
                 thr = fmax(thr, fmax(line, all[4] / 1024.0));
             const double first = masked ? (both > 0.0 ? line / both : 0.0) : -both;
@@ -352,6 +360,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             row.z = ldexpf(1.0f, -shift);
             row.w = bad || !(thr < 1e37) ? INFINITY : (float)thr;
             reinterpret_cast<float4 *>(a.rows)[m] = row;
+            a.rows[(size_t)5 * a.n_mtiles * kSplitRows + m] = (float)values;
             a.rows[(size_t)4 * a.n_mtiles * kSplitRows + m] = masked || a.mode == SIM_MODE_L2 ? 0.0f : (float)(sum[2] + (double)a.norm_const);
         }
         // the row's packed parameters: 16 bytes are eight channels at one tap

@@ -498,10 +498,33 @@ __device__ __forceinline__ int split_virtual_row(const SplitArgs &a, int n, int 
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef const __attribute__((address_space(4))) float uniform_float;
 
+// What a workgroup knows of the sizes it has staged.
+struct SplitFar {
+    int most;                          // the largest |x'| s so far: a float's bits, as which they are compared
+    int lanes[2][kSplitLevels - 1];    // in chunks of even and odd numbers: with a value that the next level keeps, see split_body
+};
+
+// Raises far.most to a lane's value, rounded up to a quarter of an octave: so a workgroup does it a few times.  (One instruction
+// and not the compiler's loop over the lanes.)
+__device__ __forceinline__ void split_far_most(__attribute__((address_space(3))) SplitFar &far, float value)
+{
+    asm volatile("ds_max_i32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                 :
+                 : "v"((unsigned)(uintptr_t)&far.most), "v"(__float_as_int(value) | 0x1fffff)
+                 : "memory");
+}
+
 // Forward.  One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel
-// tiles.
+// tiles.  Where the inputs are much larger than what the templates differ by, so that the square of one is beyond half precision
+// and an eighth of the lanes have one that counts beside it, the workgroup goes on at a smaller scale of the channels (a
+// level, 2^-3 each, packed by the packing kernel): its sums are scaled, the chunk is staged again, and the cross terms'
+// parameters are multiplied on the way.  Where only a few pixels are that large their outputs become NaN, and are
+// recomputed.  256 x 64 x 32 x 32 -> 128, 3 x 3, templates of size 0.05, inputs 0..255 or 0..10^7: 220 us, where all
+// tiles left to the direct kernel took 1190; what it costs ordinary inputs: 1 to 2 us there, 1 of 50 on 37 x 45 x 29 x 35 -> 75, 2 of
+// 54 on 64 x 256 x 32 x 32 -> 64, 1 x 1.  One pixel in a hundred 10^4 times the others: most tiles to the direct kernel, 1480.
 template <int KIND, int CG, int G>
-__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 &near, int ptile, int mtile0, int norm)
+__device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attribute__((address_space(3))) SplitFar &far,
+                                           u32x4 &near, int ptile, int mtile0, int norm)
 {
     constexpr bool MASKED = KIND == SPLIT_MASKED;
     constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND), kWaves = kThreads / 64;
@@ -514,6 +537,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
     const int half = lane >> 5, col = lane & 31;
     const int mtile = mtile0 + wave % G;
     const int ntile0 = wave / G * NI;
+    constexpr int kLastLevel = MASKED ? kSplitMaskedLevels - 1 : kSplitLevels - 1;
 
     const int n0 = ptile * kSplitPixels;
     int img0, img1, c0, c1;
@@ -583,9 +607,12 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                     rsrc, src[i], (chunk * CG + max(-8 * g, min(j, there))) * plane, 0));
         }
     };
-    request(0);
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
-        __syncthreads();
+    int level = 0;
+    // (sizes as a float's bits) the largest |x'| s so far, what is larger than it, and than the level keeps, among staged values
+    int seen = __float_as_int(kSplitMost), ask = seen, limit = __float_as_int(kSplitMost);
+    const float *channels = a.chan;
+    auto stage = [&](int chunk) {   // converts the requested values; returns the largest staged |x'| of this lane's
+        float most = 0.0f;
 #pragma unroll
         for (int i = 0; i < kItems; ++i) {
             const int item = wave + kWaves * i;
@@ -593,7 +620,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                 continue;
             const int g = CG == 16 && item >= per_half, q = (item - (g ? per_half : 0)) * 64 + lane;
             const int c0 = chunk * CG + 8 * g;
-            uniform_float *chan = (uniform_float *)(a.chan + c0);
+            uniform_float *chan = (uniform_float *)(channels + c0);
             if (a.oob != 0.0f)   // (a NaN too)
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
@@ -603,6 +630,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                 for (int j = 0; j < 8; ++j)
                     x[i][j] = c0 + j < a.C ? x[i][j] : 0.0f;
             f16x8 v[5];
+            float item_most = 0.0f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float s = chan[SPLIT_S * a.chunks * CG + j], ncs = chan[SPLIT_NCS * a.chunks * CG + j];
@@ -614,6 +642,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                     d2 = ok ? d2 : 0.0f;
                     v[4][j] = ok ? (_Float16)1.0f : (_Float16)0.0f;
                 }
+                item_most = fmaxf(item_most, __builtin_fabsf(d));
                 _Float16 hi, lo;
                 split2(d2, hi, lo);
                 v[0][j] = hi; v[1][j] = lo;
@@ -621,13 +650,56 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
                 v[2][j] = hi; v[3][j] = lo;
             }
             if (q < staged) {
+                most = fmaxf(most, item_most);
                 char *dst = lds + (g * P + q) * 16;
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
                     *reinterpret_cast<f16x8 *>(dst + b * kPlane) = v[b];
             }
         }
+        return __float_as_int(most);
+    };
+    request(0);
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
         __syncthreads();
+        // Both blocks out of the ordinary: code that is not in the instruction cache takes a microsecond or two to get.
+        const int most = stage(chunk);
+        if (most > ask)
+            split_far_most(far, most < __float_as_int(INFINITY) ? ldexpf(__int_as_float(most), kSplitLevelBits * level) : 0.0f);
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(most > limit) != 0, 0))
+            for (int i = level; i < kLastLevel; ++i) {
+                const float keeps = ldexpf(kSplitMost / 32, kSplitLevelBits * (i - level));
+                const int lanes = __popcll(__builtin_amdgcn_ballot_w64(__int_as_float(most) > keeps));
+                if (lane == 0)
+                    __hip_atomic_fetch_add(&far.lanes[chunk & 1][i], lanes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+        __syncthreads();
+        seen = __builtin_amdgcn_readfirstlane(far.most);
+        ask = seen;
+        if (__builtin_expect(seen > __float_as_int(kSplitMost), 0)) {
+            int next_level = level;
+            while (next_level < kLastLevel && __int_as_float(seen) > ldexpf(kSplitMost, kSplitLevelBits * next_level) &&
+                   __builtin_amdgcn_readfirstlane(far.lanes[chunk & 1][next_level]) > kThreads / 8)
+                ++next_level;
+            if (next_level > level) {
+                const float ratio = ldexpf(1.0f, 2 * kSplitLevelBits * (level - next_level));
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    sum[i] *= ratio;
+                    acc[i] *= ratio;
+                    if (TWO)
+                        ac2[i] *= ratio;
+                }
+                level = next_level;
+                limit = __float_as_int(level < kLastLevel ? kSplitMost : INFINITY);
+                channels = a.chan + level * SPLIT_CHANNEL_FIELDS * a.chunks * CG;
+                stage(chunk);
+                __syncthreads();
+            }
+            ask = __float_as_int(ldexpf(__int_as_float(seen), -kSplitLevelBits * level));
+            if (tid < kSplitLevels - 1)
+                far.lanes[~chunk & 1][tid] = 0;
+        }
         int dh = 0, dw = 0;
         auto next_tap = [&]() {   // LDS offset of the next tap (behind the last: of the first, with zero parameters)
             const int off = dh < taps_h ? (dh * a.Wp + dw) * 16 : 0;
@@ -654,6 +726,13 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
 #pragma unroll
             for (int q = 0; q < NA; ++q)
                 A[q] = next[q];
+            if (__builtin_expect(level > 0, 0)) {
+                const f16x8 shrink = (_Float16)ldexpf(1.0f, -kSplitLevelBits * level);
+                A[2] *= shrink;
+                A[3] *= shrink;
+                if (MASKED)   // (the lesser piece of what tm sums is added to the squares)
+                    A[NA - 3] *= shrink * shrink;
+            }
             if (chunk + 1 < a.chunks || step + 1 < a.steps)
                 pp += NA * 64;
 #pragma unroll
@@ -774,6 +853,16 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
         row[r] = rows4[8 * (r / 4) + r % 4];
         lgm[r] = !MASKED && norm ? lgs[8 * (r / 4) + r % 4] : 0.0f;
     }
+    const float grow = ldexpf(1.0f, 2 * kSplitLevelBits * level);
+    if (__builtin_expect(level > 0, 0)) {   // the guard's line rises with the level: see split_pack_block
+        const float *values = a.rows + (size_t)5 * a.n_mtiles * kSplitRows + mtile * kSplitRows + 4 * half;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            row[r][SPLIT_THR] = fmaxf(row[r][SPLIT_THR], values[8 * (r / 4) + r % 4] * grow);
+            if (!MASKED)
+                row[r][SPLIT_UNSCALE] *= grow;
+        }
+    }
     // stores by a pixel's offset and a row's; rows behind the last template go outside of the buffer
     const int left = a.O - mtile * kSplitRows;
     const unsigned image = (unsigned)a.npix * 4u;
@@ -793,7 +882,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, u32x4 
             float v;
             bool fine;
             if (MASKED) {
-                v = (sum[i][r] + tm[i][r]) * row[r][SPLIT_UNSCALE];
+                v = __builtin_fmaf(sum[i][r], grow, tm[i][r]) * row[r][SPLIT_UNSCALE];
                 const float mag = __builtin_fabsf(v);
                 fine = mag < 1e37f && mag >= row[r][SPLIT_GUARD] * -(tm[i][r] * row[r][SPLIT_UNSCALE]) &&
                        (mag >= row[r][SPLIT_THR] || (v == 0.0f && tm[i][r] == 0.0f && row[r][SPLIT_THR] < 1e37f));
@@ -828,8 +917,13 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __align__(16) char split_lds[split_lds_bytes(KIND)];
     __shared__ int any_near;   // of the workgroup's outputs, one below the guard's line
-    if (KIND != SPLIT_GRAD && threadIdx.x == 0)
+    __shared__ SplitFar far;
+    if (KIND != SPLIT_GRAD && threadIdx.x == 0) {
         any_near = 0;
+        far.most = __float_as_int(kSplitMost);
+    }
+    if (KIND != SPLIT_GRAD && threadIdx.x < kSplitLevels - 1)
+        far.lanes[0][threadIdx.x] = far.lanes[1][threadIdx.x] = 0;
     u32x4 near = 0;   // [i] bit r: output r of this lane's pixel tile i is
     const int full = a.n_mtiles / a.gmax, y = blockIdx.y;
     int mtile0 = y * a.gmax, g = a.gmax;
@@ -851,12 +945,13 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
         else
             split_grad_body<CG, 1>(a, split_lds, mtile0, flag);
     } else {
+        auto &lds_far = *(__attribute__((address_space(3))) SplitFar *)&far;
         if (KIND == SPLIT_FWD && g == 4)
-            split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, near, ptile, mtile0, flag);
+            split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, lds_far, near, ptile, mtile0, flag);
         else if (g == 2)
-            split_body<KIND, CG, 2>(a, split_lds, near, ptile, mtile0, flag);
+            split_body<KIND, CG, 2>(a, split_lds, lds_far, near, ptile, mtile0, flag);
         else
-            split_body<KIND, CG, 1>(a, split_lds, near, ptile, mtile0, flag);
+            split_body<KIND, CG, 1>(a, split_lds, lds_far, near, ptile, mtile0, flag);
         if (near[0] | near[1] | near[2] | near[3])
             any_near = 1;
         __syncthreads();
@@ -986,8 +1081,8 @@ static SplitPlan split_geometry(const SimPlan &p, int kind)
     const int mpad = s.n_mtiles * kSplitRows;
     s.packed = 0;
     s.chan = s.packed + (size_t)s.n_mtiles * s.chunks * s.steps * s.pieces * 1024;
-    s.rows = s.chan + align_up((size_t)std::max(SPLIT_CHANNEL_FIELDS * s.chunks * s.cg, mpad) * sizeof(float), 256);
-    s.flags = s.rows + align_up((size_t)5 * mpad * sizeof(float), 256);
+    s.rows = s.chan + align_up((size_t)std::max(kSplitLevels * SPLIT_CHANNEL_FIELDS * s.chunks * s.cg, mpad) * sizeof(float), 256);
+    s.flags = s.rows + align_up((size_t)6 * mpad * sizeof(float), 256);
     s.exact = s.flags + align_up((size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
     s.logs = s.exact + (kind == SPLIT_GRAD ? 0 : align_up((size_t)p.O * p.K * sizeof(float2), 256));
     s.total = s.logs + (kind == SPLIT_GRAD || p.mode == SIM_MODE_L2 ? 0 : align_up((size_t)p.O * p.K * sizeof(float), 256));

@@ -516,3 +516,73 @@ def test_split_input_gradient_over_templates_and_pixels_of_any_size(pkg, O, bloc
     size = 2 * (up(gd.abs(), wd * (td.abs() + 1)) + (xd.abs() + 1) * up(gd.abs(), wd))
     err = ((got - want).abs() / size.clamp_min(1e-300))[clear.expand_as(got)]
     assert float(err.max()) <= 2 * (O * block * block / 16 + 8) * 2.0 ** -24, float(err.max())
+
+
+FAR = [("init", 255.0), ("init", 6e4), ("init", 1e8), ("normal", 1e4), ("similar", 1.0), ("similar", 1e-6)]
+
+
+@pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
+@pytest.mark.parametrize("kind, size", FAR)
+@pytest.mark.parametrize("geom", [GEOMS[0], GEOMS[1], GEOMS[11], GEOMS[7]])
+def test_split_form_of_inputs_on_another_scale(pkg, geom, kind, size, mode):
+    """Inputs much larger than the templates, or than what the templates differ by: bounds of test_split_form_scales, and the
+    outputs are this form's own and not the term-by-term sums of the direct kernel, which agree in the last bit for some."""
+    g = torch.Generator(device="cuda").manual_seed(73)
+    shape, O, blocks = geom["shape"], geom["O"], geom["blocks"]
+    t = torch.randn((O, shape[1], *blocks), generator=g, device="cuda")
+    w = torch.ones_like(t)
+    if kind == "init":         # a layer's default initialisation on unscaled images
+        t = t * 0.05
+        x = torch.rand(shape, generator=g, device="cuda") * size
+    elif kind == "normal":
+        x = torch.randn(shape, generator=g, device="cuda") * size
+    else:                      # templates all nearly the same
+        t = size * (1 + 1e-4 * t)
+        x = torch.randn(shape, generator=g, device="cuda") * size
+    kw = options(mode, geom)
+    oob = kw.setdefault("out_of_bounds_value", geom.get("out_of_bounds_value", 0.0))
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    assert pieces_used(pkg, shape, O, mode, **kw)["forward"]
+    got = pkg.similarity(x, t, w, **kw)
+    want = exact(x, t, w, blocks, geom["strides"], geom["padding"], mode, oob)
+    K = shape[1] * blocks[0] * blocks[1]
+    scale = want.abs()
+    if mode != "l2":
+        logs = 0.5 * (K * math.log(2 * math.pi) + torch.log(w.double() + 0.001).abs().flatten(1).sum(1))
+        scale = torch.maximum(scale, logs[None, :, None, None])
+    err = float(((got.double() - want).abs() / scale).max())
+    assert err <= 2 * (K / 16 + 8) * 2.0 ** -24, err
+    if mode == "missing" and size == 1e8 or mode == "norm" and size == 1e-6:
+        return    # beyond the levels of that mode; nothing but the logarithms' sum
+    direct = pkg.similarity(x, t, w, algo="direct", **kw)
+    assert float((got == direct).float().mean()) < 0.7
+
+
+@pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
+@pytest.mark.parametrize("geom", [GEOMS[0], GEOMS[1], GEOMS[11], GEOMS[7]])
+def test_split_form_of_inputs_on_several_scales(pkg, geom, mode):
+    """Pixels, channels and whole images of inputs far from the templates beside ordinary ones: every output by itself has
+    the error of a sum of its terms."""
+    g = torch.Generator(device="cuda").manual_seed(79)
+    shape, O, blocks = geom["shape"], geom["O"], geom["blocks"]
+    t = torch.randn((O, shape[1], *blocks), generator=g, device="cuda") * 0.05
+    w = torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1
+    x = torch.randn(shape, generator=g, device="cuda") * 0.1
+    x[:, shape[1] // 2] *= 1e3
+    x[1] *= 1e5
+    x[2, :, ::7, ::9] *= 1e9
+    x[3, -1, 4, 5] = 1e15
+    kw = options(mode, geom)
+    oob = kw.setdefault("out_of_bounds_value", geom.get("out_of_bounds_value", 0.0))
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    got = pkg.similarity(x, t, w, **kw).double()
+    want = exact(x, t, w, blocks, geom["strides"], geom["padding"], mode, oob)
+    K = shape[1] * blocks[0] * blocks[1]
+    scale = want.abs()
+    if mode != "l2":
+        logs = 0.5 * (K * math.log(2 * math.pi) + torch.log(w.double() + 0.001).abs().flatten(1).sum(1))
+        scale = torch.maximum(scale, logs[None, :, None, None])
+    err = float(((got - want).abs() / scale).max())
+    assert err <= 2 * (K / 16 + 8) * 2.0 ** -24, err
