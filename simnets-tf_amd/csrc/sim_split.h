@@ -38,7 +38,7 @@ SplitPlan sim_split_plan(const SimPlan &p);
 // Per template four floats: what the sums of a row lack (bias, in two floats; with missing values the guard: outputs below
 // it times the sum of the present w (t'^2 + m / s^2) are recomputed), the power of two that takes back what the packed
 // parameters were multiplied by, and the line below which outputs are recomputed.  Behind those of the n_mtiles * 32
-// templates the constants of the normalized modes, and by what the line rises with the level.
+// templates the constants of the normalized modes, and pairs by which the line rises with the staged values.
 enum SplitRow { SPLIT_BIAS, SPLIT_BIAS_LESSER, SPLIT_UNSCALE, SPLIT_THR, SPLIT_GUARD = SPLIT_BIAS };
 // Per channel, [level][field][chunks * cg], zeros behind the last channel: the scale s, -c s, and m.
 enum SplitChannel { SPLIT_S, SPLIT_NCS, SPLIT_M, SPLIT_CHANNEL_FIELDS };
@@ -105,6 +105,8 @@ constexpr float kSplitLow = 2048.0f;
 // The forward's scales: levels of 2^-3 of the packed ones (a parameter times 2^-24 is still a half-precision value; with missing
 // values the lesser pieces meet twice as much).
 constexpr int kSplitLevels = 9, kSplitMaskedLevels = 5, kSplitLevelBits = 3;
+constexpr float kSplitParamShare = 0.07f;   // 2^-25.8 / 2^-22
+constexpr float kSplitSeen = 2.0f;     // staged values up to this need no attention
 constexpr float kSplitMost = 181.0f;   // the largest staged value, its square below 2^15
 
 __device__ __forceinline__ void split2(float v, _Float16 &hi, _Float16 &lo)
@@ -290,7 +292,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
         double sum[3] = {};   // w t'^2, w m / s^2, logarithms
         float size[2] = {};   // w / s^2 or 2 w |t'| / s, w t^2
         bool bad = false, weighted = false;
-        int top = kNoExponent;
+        int top = kNoExponent, bottom = kNoExponent;   // the largest of the parameters' exponents, and of -(those of w / s^2)
 #pragma unroll 1
         for (int k = tid; k < (m < a.O ? a.K : 0); k += 256) {   // (a thread's own elements of the row)
             const float2 own = k < in_lds ? row_tw[k] : make_float2(mt[k], mw[k]);
@@ -307,6 +309,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             size[1] += w * t * t;
             const int ew = split_exponent(w);
             top = max(top, max(ew - 2 * es, ew + split_exponent(tc) + 2 - es));
+            bottom = ew > kNoExponent ? max(bottom, 2 * es - ew) : bottom;
             // weights and templates outside this range: the pieces of their products may leave the range of
             // normal numbers, so such a template is left to the term-by-term kernel
             bad |= !(w == 0.0f || (w >= 0x1p-60f && w <= 0x1p20f)) || !(__builtin_fabsf(t) <= 0x1p60f);
@@ -326,6 +329,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             for (int i = 0; i < 2; ++i)
                 size[i] += __shfl_xor(size[i], d, 64);
             top = max(top, __shfl_xor(top, d, 64));
+            bottom = max(bottom, __shfl_xor(bottom, d, 64));
         }
         if ((tid & 63) == 0) {
 #pragma unroll
@@ -335,10 +339,12 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             for (int i = 0; i < 2; ++i)
                 sums[8 * wave + 3 + i] = size[i];
             ints[4 * wave] = top;
+            ints[4 * wave + 1] = bottom;
         }
         bad = __syncthreads_or(bad);
         weighted = __syncthreads_or(weighted);
         top = max(max(ints[0], ints[4]), max(ints[8], ints[12]));
+        bottom = max(max(ints[1], ints[5]), max(ints[9], ints[13]));
         const int shift = top > kNoExponent / 2 ? min(120, max(-120, 13 - top)) : 0;
         if (tid == 0) {
             double all[5];
@@ -349,8 +355,14 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             const double both = all[0] + all[1], line = a.line * fmax(all[0], 0.5 * both);
             double thr = weighted ? 0x1p-60 : 0.0;   // without weights zero is the exact sum
             // The values' absolute error, 2^-36 each, stays below 2^-23 of such a sum; 2^6 times as much with each level.
-            const double values = all[3] * 0x1p-13 / (double)sqrtf((float)a.K);
-            thr = fmax(thr, values);
+            const double root = (double)sqrtf((float)a.K), values = all[3] * 0x1p-13 / root;
+            // The parameters' is 2^-25 of the scaled ones, 2^-25.8 in the mean of its square: of a sum with d_k scaled values
+            // and weights a_k, 2^-25.8 sqrt(sum d_k^4), which is at most D^2 sqrt(K) and D sqrt(sum / min a_k), D the largest
+            // value.  It stays below 2^-22 of the sum.
+            const double params = fmin(kSplitParamShare * root, ldexp(1.0, min(100, bottom - shift - 6))) * ldexp(1.0, -shift);
+            thr = fmax(thr, fmax(values, params * (kSplitSeen * kSplitSeen)));
+            if (masked)   // (the third operand's parameters meet ones)
+                thr = fmax(thr, ldexp(kSplitParamShare * root, -shift));
             if (!masked)
                 thr = fmax(thr, fmax(line, all[4] / 1024.0));
             const double first = masked ? (both > 0.0 ? line / both : 0.0) : -both;
@@ -360,7 +372,7 @@ __device__ inline void split_pack_block(const SplitPack &a, int index, float *ld
             row.z = ldexpf(1.0f, -shift);
             row.w = bad || !(thr < 1e37) ? INFINITY : (float)thr;
             reinterpret_cast<float4 *>(a.rows)[m] = row;
-            a.rows[(size_t)5 * a.n_mtiles * kSplitRows + m] = (float)values;
+            reinterpret_cast<float2 *>(a.rows + (size_t)5 * a.n_mtiles * kSplitRows)[m] = make_float2((float)values, (float)params);
             a.rows[(size_t)4 * a.n_mtiles * kSplitRows + m] = masked || a.mode == SIM_MODE_L2 ? 0.0f : (float)(sum[2] + (double)a.norm_const);
         }
         // the row's packed parameters: 16 bytes are eight channels at one tap

@@ -609,7 +609,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
     };
     int level = 0;
     // (sizes as a float's bits) the largest |x'| s so far, what is larger than it, and than the level keeps, among staged values
-    int seen = __float_as_int(kSplitMost), ask = seen, limit = __float_as_int(kSplitMost);
+    int seen = __float_as_int(kSplitSeen), ask = seen, limit = __float_as_int(kSplitMost);
     const float *channels = a.chan;
     auto stage = [&](int chunk) {   // converts the requested values; returns the largest staged |x'| of this lane's
         float most = 0.0f;
@@ -854,11 +854,15 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
         lgm[r] = !MASKED && norm ? lgs[8 * (r / 4) + r % 4] : 0.0f;
     }
     const float grow = ldexpf(1.0f, 2 * kSplitLevelBits * level);
-    if (__builtin_expect(level > 0, 0)) {   // the guard's line rises with the level: see split_pack_block
-        const float *values = a.rows + (size_t)5 * a.n_mtiles * kSplitRows + mtile * kSplitRows + 4 * half;
+    if (__builtin_expect(seen > __float_as_int(kSplitSeen), 0)) {   // the guard's line rises with the staged values: see split_pack_block
+        const float2 *more = reinterpret_cast<const float2 *>(a.rows + (size_t)5 * a.n_mtiles * kSplitRows) + mtile * kSplitRows + 4 * half;
+        // (what is beyond 2^8 of the level's leaves its outputs NaN)
+        const float largest = fminf(__int_as_float(seen), ldexpf(256.0f, kSplitLevelBits * level)), square = largest * largest;
+        const float scaled = MASKED && level > 0 ? kSplitParamShare * sqrtf((float)a.K) * grow : 0.0f;   // (the scaled lesser pieces)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            row[r][SPLIT_THR] = fmaxf(row[r][SPLIT_THR], values[8 * (r / 4) + r % 4] * grow);
+            const float2 by = more[8 * (r / 4) + r % 4];
+            row[r][SPLIT_THR] = fmaxf(fmaxf(row[r][SPLIT_THR], by.x * grow), fmaxf(by.y * square, row[r][SPLIT_UNSCALE] * scaled));
             if (!MASKED)
                 row[r][SPLIT_UNSCALE] *= grow;
         }
@@ -920,7 +924,7 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
     __shared__ SplitFar far;
     if (KIND != SPLIT_GRAD && threadIdx.x == 0) {
         any_near = 0;
-        far.most = __float_as_int(kSplitMost);
+        far.most = __float_as_int(kSplitSeen);
     }
     if (KIND != SPLIT_GRAD && threadIdx.x < kSplitLevels - 1)
         far.lanes[0][threadIdx.x] = far.lanes[1][threadIdx.x] = 0;
@@ -1082,7 +1086,7 @@ static SplitPlan split_geometry(const SimPlan &p, int kind)
     s.packed = 0;
     s.chan = s.packed + (size_t)s.n_mtiles * s.chunks * s.steps * s.pieces * 1024;
     s.rows = s.chan + align_up((size_t)std::max(kSplitLevels * SPLIT_CHANNEL_FIELDS * s.chunks * s.cg, mpad) * sizeof(float), 256);
-    s.flags = s.rows + align_up((size_t)6 * mpad * sizeof(float), 256);
+    s.flags = s.rows + align_up((size_t)7 * mpad * sizeof(float), 256);
     s.exact = s.flags + align_up((size_t)s.n_ptiles * s.n_mtiles * sizeof(int), 256);
     s.logs = s.exact + (kind == SPLIT_GRAD ? 0 : align_up((size_t)p.O * p.K * sizeof(float2), 256));
     s.total = s.logs + (kind == SPLIT_GRAD || p.mode == SIM_MODE_L2 ? 0 : align_up((size_t)p.O * p.K * sizeof(float), 256));

@@ -586,3 +586,35 @@ def test_split_form_of_inputs_on_several_scales(pkg, geom, mode):
         scale = torch.maximum(scale, logs[None, :, None, None])
     err = float(((got - want).abs() / scale).max())
     assert err <= 2 * (K / 16 + 8) * 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
+@pytest.mark.parametrize("factor", [1e4, 1e6, 1e8])
+@pytest.mark.parametrize("geom", [GEOMS[0], GEOMS[1], GEOMS[11], GEOMS[7]])
+def test_split_form_of_weights_far_below_their_templates_largest(pkg, geom, factor, mode):
+    """One weight of a template is `factor` times the others', the input is on the template there and far from it
+    elsewhere: the small weights' terms are all there is of the sum, and it has the error of a sum of its terms.  (The
+    large weights lie where the packing kernel takes no samples.)"""
+    g = torch.Generator(device="cuda").manual_seed(83)
+    shape, O, (bh, bw) = geom["shape"], geom["O"], geom["blocks"]
+    t = torch.full((O, shape[1], bh, bw), 0.25, device="cuda")
+    w = (torch.rand(t.shape, generator=g, device="cuda") * 1.9 + 0.1) / factor
+    x = torch.randn(shape, generator=g, device="cuda").sign() * 20
+    rows = range(O) if bh * bw > 1 else range(32, O)
+    for m in rows:
+        c = 1 + m % 3 if bh * bw > 1 else m
+        w[m, c, bh // 2, bw // 2] *= factor
+        x[:, c] = 0.25
+    kw = options(mode, geom)
+    oob = kw.setdefault("out_of_bounds_value", 0.25)
+    if mode == "missing":
+        x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
+    got = pkg.similarity(x, t, w, **kw).double()
+    want = exact(x, t, w, geom["blocks"], geom["strides"], geom["padding"], mode, oob)
+    K = shape[1] * bh * bw
+    scale = want.abs()
+    if mode != "l2":
+        logs = 0.5 * (K * math.log(2 * math.pi) + torch.log(w.double() + 0.001).abs().flatten(1).sum(1))
+        scale = torch.maximum(scale, logs[None, :, None, None])
+    err = float(((got - want).abs() / scale.clamp_min(1e-30)).max())
+    assert err <= 2 * (K / 16 + 8) * 2.0 ** -24, err
