@@ -824,8 +824,9 @@ struct GradPArgs {
 // of the spread of the templates, which bounds the cancellation: the error is eps sqrt(N) |g| (xc^2 + tc^2),
 // the same order as that of the term-by-term sums unless every template and every patch sit in one point.
 // MOM (L1): scaled-sign form.  With d = x - t, 2^-64 sign(d) = med3(d, -2^-64, 2^-64): four instructions per term (sub,
-// med3, fma, fma) instead of seven with compares and selects; the sum of g sign(d) is scaled back where it leaves,
-// bit-identical to them unless 0 < |x - t| < 2^-64 or |g| < 2^-62.  32 x 64 x 32 x 32, 128 templates, 3 x 3: 267 -> 241 us
+// med3, fma, fma) instead of seven with compares and selects.  g is staged times 2^32, so that the sum of g sign(d) is
+// 2^-32 of itself and the sum of g |d| 2^32 times, and both are scaled back where they leave: bit-identical to the
+// seven unless 0 < |x - t| < 2^-64, |g| < 2^-94 or a sum of g |d| beyond 2^96.  32 x 64 x 32 x 32, 128 templates, 3 x 3: 267 -> 241 us
 // with two-source differences, stages of eight, the pairs (d, sign) and (sum, sum) across the parities, and staging
 // without branches (1030 -> 340 instructions a chunk); two waves to a SIMD issue one instruction per 3.3 cycles (instruction
 // streams of this kind without memory: 2.7).  A pixel chunk with a NaN input (found while staging, uniform for the
@@ -1048,7 +1049,10 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
     auto store_chunk = [&](int buf, const float4 (&gv)[GR], const float4 (&xv)[XR]) {
 #pragma unroll
         for (int r = 0; r < GR; ++r) {
-            reinterpret_cast<float4 *>(gs[buf])[(sg + NSG * r) * PCP + sp] = gv[r];
+            float4 v = gv[r];
+            if constexpr (SGN)
+                v = make_float4(v.x * 0x1p32f, v.y * 0x1p32f, v.z * 0x1p32f, v.w * 0x1p32f);
+            reinterpret_cast<float4 *>(gs[buf])[(sg + NSG * r) * PCP + sp] = v;
             if constexpr (MOM2 && !IGN) {
                 gacc[r].x += gv[r].x; gacc[r].y += gv[r].y; gacc[r].z += gv[r].z; gacc[r].w += gv[r].w;
             }
@@ -1363,9 +1367,9 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
 #pragma unroll
     for (int oo = 0; oo < LO && !MF; ++oo) {
         const size_t o = (size_t)lane_o(oo) * a.Kpad + k0;
-        constexpr float kBack = SGN ? 0x1p64f : 1.0f;
-        *reinterpret_cast<float4 *>(pt + o) = make_float4(at[oo][0] * kBack, at[oo][1] * kBack, at[oo][2] * kBack, at[oo][3] * kBack);
-        *reinterpret_cast<float4 *>(pw + o) = make_float4(aw[oo][0], aw[oo][1], aw[oo][2], aw[oo][3]);
+        constexpr float kT = SGN ? 0x1p32f : 1.0f, kW = SGN ? 0x1p-32f : 1.0f;
+        *reinterpret_cast<float4 *>(pt + o) = make_float4(at[oo][0] * kT, at[oo][1] * kT, at[oo][2] * kT, at[oo][3] * kT);
+        *reinterpret_cast<float4 *>(pw + o) = make_float4(aw[oo][0] * kW, aw[oo][1] * kW, aw[oo][2] * kW, aw[oo][3] * kW);
         if constexpr (IGN || (NORM && !MOM))
             *reinterpret_cast<float4 *>(pn + o) = make_float4(an[oo][0], an[oo][1], an[oo][2], an[oo][3]);
         if constexpr (MOM2) {

@@ -524,8 +524,8 @@ def test_similarity_l1_grads_at_ties_and_nan(pkg):
 
 @pytest.mark.parametrize("nan", [False, True])
 def test_similarity_l1_params_grad_scaled_sign_form_equals_the_term_by_term_form(pkg, nan):
-    """L1 parameter gradients by default take sign and magnitude from 2^64 (x - t) (fma, med3); with algo='direct'
-    they use compares and selects.  Same sums in the same order: bit-identical, ties and zero weights included;
+    """L1 parameter gradients by default take the sign as 2^-64 sign(x - t) (med3); with algo='direct' they use compares and
+    selects.  Same sums in the same order: bit-identical, ties and zero weights included;
     pixel chunks with a NaN input run the compare-and-select arithmetic in both."""
     x, t, w = sim_inputs(22, (3, 5, 17, 19), 37, (3, 3))
     t[0, 0, 1, 1] = x[0, 0, 4, 4]
@@ -548,6 +548,19 @@ def test_similarity_l1_params_grad_scaled_sign_form_equals_the_term_by_term_form
     ok = ~np.isnan(want_dw)
     assert_grad_close(fast[0], want_dt, true_dt, "templates grad")
     assert_grad_close(np.where(ok, fast[1], 0), np.where(ok, want_dw, 0), np.where(ok, true_dw, 0), "weights grad")
+
+
+@pytest.mark.parametrize("size", [1e-25, 1e-20, 1e25])
+def test_similarity_l1_params_grad_scaled_sign_form_of_small_and_large_output_gradients(pkg, size):
+    """Output gradients whose product with 2^-64, the size of a sign in the scaled-sign form, is no normal number, and large
+    ones: the sums of the term-by-term form, bit by bit."""
+    x, t, w = sim_inputs(24, (3, 5, 17, 19), 37, (3, 3))
+    kw = dict(similarity_function="L1", blocks=[3, 3], strides=[1, 1], padding=[1, 1])
+    og = (np.random.default_rng(10).normal(size=orc.similarity_fwd(x, t, w, **kw).shape) * size).astype(np.float32)
+    fast = pkg.similarity_parameters_grad(dev(x), dev(t), dev(w), dev(og), **kw)
+    exact = pkg.similarity_parameters_grad(dev(x), dev(t), dev(w), dev(og), algo="direct", **kw)
+    for a, b in zip(fast, exact):
+        assert torch.isfinite(b).all() and b.any() and torch.equal(a, b)
 
 
 @pytest.mark.parametrize("shape,O,block,stride", [
