@@ -192,11 +192,23 @@ class _PreparedCache:
 
 
 def _plain(v):
-    """An attribute as part of a prepared call's key: what is compared must not change with the layer's lists, and a NaN
-    (an out-of-bounds value) must equal itself."""
-    if type(v) is list:
+    """An attribute as part of a prepared call's key: a copy where it can be changed in place, and a NaN (an out-of-bounds
+    value) equal to itself."""
+    kind = type(v)
+    if kind is list:
         return tuple(v)
-    return v if v == v else "nan"
+    if kind is int or kind is float or kind is str:
+        return v if v == v else "nan"
+    if isinstance(v, np.ndarray):
+        v = v.tolist()
+    if isinstance(v, dict):
+        return tuple((k, _plain(e)) for k, e in v.items())
+    return tuple(map(_plain, v)) if isinstance(v, (list, tuple)) else v
+
+
+def _inherits(layer, cls):
+    """Whether the layer's attributes are those of `cls` itself, and not of an attrs() put in its place."""
+    return getattr(layer.attrs, "__func__", None) is cls.attrs
 
 
 def _uninitialized(parameter):
@@ -273,11 +285,12 @@ class Similarity(torch.nn.Module):
             x = x.permute(0, 3, 1, 2).contiguous()
         if not torch.is_grad_enabled() and x.is_cuda:
             # inference: the parameters are packed once per (input shape, parameter identity and version, layer
-            # attributes, stream); calls run the forward kernels on the prepared buffer.  (The key is made on every call:
-            # 1.2 us; from the attributes' dict, made hashable, 3.7.)
+            # attributes, stream); calls run the forward kernels on the prepared buffer.  (The key is made on every call,
+            # from the attributes themselves: 0.5 us; from the dict, made hashable, 2.8.)
             key = (x.shape, x.device, self.similarity_function, _plain(self.blocks), _plain(self.strides), _plain(self.padding),
                    self.normalization_term, self.normalization_term_fudge, self.ignore_nan_input,
-                   _plain(self.out_of_bounds_value))
+                   _plain(self.out_of_bounds_value)) if _inherits(self, Similarity) else (
+                       x.shape, x.device, _plain(self.attrs()))
             out = self._prepared.get(
                 ops._current_stream(x.device), (templates, sweights), key, lambda: ops.similarity_prepare(
                     x.shape, templates.detach(), sweights.detach().abs(), **self.attrs()))(x)
@@ -376,7 +389,8 @@ class Mex(torch.nn.Module):
             key = (x.shape, x.device, self.num_instances, self.softmax_mode, _plain(self.padding), _plain(self.strides),
                    _plain(self.blocks), self.epsilon, _plain(self.blocks_out_of_bounds_value), self.blocks_round_down,
                    self.use_unshared_regions, _plain(self.shared_offset_region), _plain(self.unshared_offset_region),
-                   self.normalize_offsets)
+                   self.normalize_offsets) if _inherits(self, Mex) else (
+                       x.shape, x.device, self.num_instances, _plain(self.attrs()))
             out = self._prepared.get(ops._current_stream(x.device), (offsets,), key, lambda: ops.mex_prepare(
                 x.shape, offsets.detach(), self.num_instances, **self.attrs()))(x)
         else:

@@ -500,6 +500,57 @@ def test_modules_notice_rebound_parameters_changed_attributes_and_other_streams(
     assert sim._prepared.last(pkg.ops._current_stream(x.device)) is main
 
 
+def test_modules_notice_attributes_changed_in_place(pkg):
+    """A prepared buffer belongs to the attributes' values: lists of any kind changed in place, arrays, an attrs() of a
+    subclass or of one layer, and a NaN that stays one."""
+    class Strides(list):
+        pass
+
+    class Fudged(pkg.Similarity):
+        fudge = 0.001
+
+        def attrs(self):
+            return dict(super().attrs(), normalization_term=True, normalization_term_fudge=self.fudge)
+
+    x = torch.randn((2, 4, 9, 9), device="cuda", generator=torch.Generator(device="cuda").manual_seed(12))
+    sim = pkg.Similarity(9, blocks=[3, 3], strides=[1, 1], padding=[1, 1]).cuda()
+    mexl = pkg.Mex(5, blocks=[-1, 1, 1], strides=[9, 1, 1], softmax_mode=True, unshared_offset_region=[2]).cuda()
+    fudged = Fudged(9, blocks=[3, 3], strides=[1, 1], padding=[1, 1]).cuda()
+
+    def both(layer, x):
+        with torch.no_grad():
+            fast = layer(x)
+        assert torch.equal(fast, layer(x).detach())
+        return fast
+
+    y = both(sim, x)
+    sim.strides = Strides([1, 1])
+    mexl.strides = Strides([9, 1, 1])
+    z = both(mexl, both(sim, x))
+    sim.strides[0] = 2
+    mexl.strides[2] = 2
+    assert both(sim, x).shape[2] == 5 and both(mexl, y).shape[3] == 5 and z.shape[2:] == (9, 9)
+    sim.strides = np.array([1, 1])
+    assert torch.equal(both(sim, x), y)
+    sim.strides[1] = 3
+    assert both(sim, x).shape[3] == 3
+    first = both(fudged, x)
+    fudged.fudge = 0.5
+    assert not torch.equal(both(fudged, x), first)
+    plain = dict(sim.attrs(), strides=[1, 1])
+    sim.attrs = lambda: plain
+    assert torch.equal(both(sim, x), y)
+    plain["strides"][0] = 2
+    assert both(sim, x).shape[2] == 5
+    fudged.out_of_bounds_value = float("nan")
+    with torch.no_grad():
+        fudged(x)
+        kept = fudged._prepared.last()
+        fudged.out_of_bounds_value = -float("nan")
+        fudged(x)
+    assert fudged._prepared.last() is kept
+
+
 @pytest.mark.parametrize("im,n", [((64, 32, 16, 16), 64),      # panel form, one chunk
                                   ((16, 64, 8, 8), 128),       # panel form, two halves
                                   ((40, 16, 8, 8), 20)])       # fused kernel
