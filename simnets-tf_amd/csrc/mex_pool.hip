@@ -160,7 +160,7 @@ __device__ __forceinline__ void max_chunk(float (&best)[4][4], const float *xs, 
 // the short dependent phases; one half only when there are no slots for a second one.  With the Similarity inside two such
 // workgroups fit a compute unit's registers, and their phases overlap: against one of four halves (a copy of the offsets
 // tiles and a fetch of taps and parameters per 256 columns) the missing-data network takes 185 us instead of 191 at 2048
-// images, 221 instead of 232 at 700 with 64 templates and 96 instances, 68.0 instead of 68.6 at 512.
+// images, 221 instead of 232 at 700 with 64 templates and 96 instances, and the same (65 us) at 512.
 // SIMF: the input of the MEX layer is a Similarity layer's output whose channels are exactly the MEX patch (blocks
 // [O, 1, 1], no padding): the staging evaluates Similarity channel k of its pixel from the layer's input (the patch
 // taps of the pixel sit in LDS, the packed parameters of channel k come through scalar loads) with the Similarity
@@ -656,7 +656,7 @@ __device__ __forceinline__ void pack_row32(const float (&x)[32], int normalize, 
 // the scaled offsets; nothing of the product form (column maxima, packed exponentials, row ranges) is touched.
 // Two halves and one chunk, not pooled: three workgroups on a compute unit instead of two, whose load, exponential and
 // store phases overlap.  For their LDS the partial maxima use the panel tile's place (a barrier more), for their registers
-// the offsets tiles go to LDS as they arrive.  1024 x 32 x 16 x 16 -> 64 instances: 33.2 -> 31.4 us (3.2 TB/s of input and
+// the offsets tiles go to LDS as they arrive.  1024 x 32 x 16 x 16 -> 64 instances: 33.3 -> 30.2 us (3.3 TB/s of input and
 // output); 256 x 32 x 16 x 16 -> 200 31.4 -> 29.0.  Holding the offsets in registers spills and loses 20 %.
 constexpr bool panel_three(int nh, int nch, bool pool, bool inf) { return nh == 2 && nch == 1 && !pool && !inf; }
 

@@ -5,28 +5,30 @@
 // bits, hi + lo (split2), and three products of pieces are formed on v_mfma_f32_32x32x16_f16; the one left out, lo lo, is
 // below 2^-22 of the whole with either sign.  Half precision has a narrow exponent: the packing kernel scales channels and
 // templates by powers of two (split_pack_block), the lesser piece of a value is kept times 2048 and meets a copy of hi
-// divided by as much, and a value that overflows makes its outputs NaN, which the guard below hands on.  Input gradient:
-// three bf16 pieces and six products (see the end of the file).
+// divided by as much, workgroups whose inputs are on another scale than the templates take smaller ones (split_body), and a
+// value that overflows all the same makes its outputs NaN, which the guard below hands on.  Input gradient: three bf16
+// pieces and six products (see the end of the file).
 //
 // Precision.  The matrix unit cuts what lies below 2^-26 of a sum off each of its products, and these have 22 bits: of
 // terms of one sign that is a bias (4.4e-7 at 576 elements).  So the squares are those about their channel's sampled mean,
 // x'^2 - m, whose sums stay small and have no bias, and a chunk's products (144 elements of 3 x 3) have a sum of their own
-// that is added in fp32.  Error against 64 bits (2-norm, relative): 256 x 64 x 32 x 32 -> 128, 3 x 3, inputs unrelated to the
-// templates 0.4e-7 (three bf16 pieces: 0.8e-7, term by term 3.6e-7), 256 channels 0.4e-7 (1.3e-7); inputs all zero
-// 1.0e-7 (0.6e-7), without their negative values 0.4e-7, ten times as large 0.8e-7 (1.7e-7).
+// that is added in fp32.  Error against 64 bits (2-norm, relative; weights 0.1 to 2): 64 channels, 3 x 3, inputs unrelated to
+// the templates 0.45e-7 (three bf16 pieces 0.8e-7, term by term 3.6e-7), all zero 0.65e-7 (0.6e-7, 4.1e-7), without their
+// negative values 0.4e-7, ten to 10^7 times the templates 0.7e-7 (1.7e-7, 3.5e-7); 256 channels, 1 x 1, 0.4e-7 to 0.6e-7 (2.3e-7).
 // Inputs near a template lose to cancellation, as T / out, T = sum w t'^2.  A patch at out / T = 2, 1 and 0.5 from its
-// template, 576 elements: 0.5e-7, 0.9e-7 and 2.3e-7 (root mean square; term by term 3.6e-7), 2304: 0.4e-7, 0.8e-7, 2.1e-7
-// (7.7e-7), 64: 0.6e-7, 0.9e-7, 1.0e-7 (1.3e-7).  The guard's line lies at 0.43 T (half for the shortest patches,
-// split_line).
+// template, 576 elements: 0.9e-7, 1.4e-7 and 2.4e-7 (root mean square; term by term 3.6e-7), 2304: 0.6e-7, 0.9e-7, 2.1e-7
+// (7.2e-7), 64: 0.8e-7, 1.1e-7, 1.2e-7 (1.2e-7).  The guard's line lies at 0.43 T (half for the shortest patches,
+// split_line).  It also lies where the pieces' own limits would show: parameters far below their template's largest,
+// values far below what the tile holds (split_pack_block).
 // An output below the line (or below 1/1024 of the uncentred sum w t^2, the guard of the sqrt-weight form; or not finite) is
-// computed again term by term by its workgroup (split_recompute): the others keep their value, so it does not matter
-// what shares a tile.  A tile with more of them than that is worth, or with a template whose parameters are negative,
-// huge or tiny, is flagged and left whole to the direct kernel's launch behind this one, which otherwise returns at once.
-// Templates fitted to the inputs (k-means of 1/f images with three factors over the channels, 256 x 64 x 32 x 32 -> 128, 3 x 3):
-// 0.15 % of the outputs in 84 % of the tiles, 0.46 ms; with every such tile left to the direct kernel 1.39, the sqrt-weight
-// form 0.81.  64 x 16 x 32 x 32 -> 64: 46 us, 83 and 55; 64 x 8 x 32 x 32 -> 32, 72 elements, 0.9 % of the outputs: 31, 47 and 30,
-// and with 1.3 %, where some tiles have too many: 53.  Several templates near every output are the worst that can be: 256
-// x 576 x 14 x 14 -> 128, 1 x 1, 6 % of the outputs, 643 us where the sqrt-weight form takes 420.
+// computed again term by term by its workgroup (split_recompute), and the others keep their value.  A tile with more of
+// them than that is worth, or with a template whose parameters are negative, huge or tiny, is flagged and left whole to
+// the direct kernel's launch behind this one, which otherwise returns at once.
+// Templates fitted to the inputs (k-means of 1/f images with three factors over the channels): 256 x 64 x 32 x 32 -> 128, 3 x 3,
+// 0.3 % of the outputs below the line: 319 us (unrelated templates 228, sqrt-weight form 764, direct kernel 1017); 64 x
+// 16 x 32 x 32 -> 64, 0.3 %: 36 (28, 49, 49); 64 x 8 x 32 x 32 -> 32, 72 elements, 1.5 % and 2.1 %: 28 and 30 (22, 25, 26).  Where many
+// tiles are left: 64 x 32 x 32 x 32 -> 64 of two factors, 1.2 %: 136 (35, 85, 86); 256 x 8 x 32 x 32 -> 32, 3 %: 109 (42, 49, 50); 256 x 576 x
+// 14 x 14 -> 128, 1 x 1, 7 %: 585 (132, 864, 455).
 //
 // Missing values (NaN inputs ignored): both operands 0 and a third, the 0/1 mask of present values, which contracts with
 // -w (t'^2 + m) and with the logarithm term, two pieces each; T is that of the present values.
@@ -40,9 +42,9 @@
 // offset per pixel, one per channel, zeros outside of the image: no 64-bit address per value).  256 registers: two
 // workgroups per compute unit, so that one stages while the other multiplies.
 //
-// Measured (whole call, vector form, three bf16 pieces, this form): 256 x 64 x 32 x 32 -> 128, 3 x 3: 0.80, 0.372, 0.228 ms.
-// The kernel's 210 us are 1.1 PFLOP/s of matrix products at 1.55 GHz: the clock sinks with them (products of random
-// numbers alone run at 1.57 PFLOP/s and 1.65 GHz, of zeros at 2.35), 155 us would be that rate.  37 x 45 x 29 x 35 -> 75: 172, 66,
+// Measured (whole call, vector form, three bf16 pieces, this form): 256 x 64 x 32 x 32 -> 128, 3 x 3: 0.80, 0.372, 0.229 ms.
+// The kernel's 211 us are 1.1 PFLOP/s of matrix products at 1.55 GHz, matrix units busy 56 %: the clock sinks with them
+// (products of random numbers alone run at 1.57 PFLOP/s and 1.65 GHz, of zeros at 2.35), 155 us would be that rate.  37 x 45 x 29 x 35 -> 75: 172, 66,
 // 50 us, where half of the products are padding (96 templates, 48 channels, 37632 pixels).  64 images of the first with a
 // quarter missing: 427, 160, 108 us.
 // Tried: 2 x 2 tiles a wave (half of the LDS reads, twice the parameter loads): 250 us for 228.
@@ -1173,7 +1175,8 @@ int sim_split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, 
 // ------------------------------------------------------------------------------------------------
 // Input gradient of the L2 modes at stride 1:  dX = A - (X - c) B,  A = sum g s w (t - c),  B = sum g s w  over (template,
 // tap) - the forward's contraction with g as the image (its channels are the templates, the taps flipped) and the input
-// channels as rows, g in three pieces against the three of each coefficient.  32 x 128 x 28 x 28, 128 templates, 3 x 3: 196 us
+// channels as rows, g in three pieces against the three of each coefficient: eight bits each, but with the exponents of fp32,
+// which g and the weights use (gradients of one template, or of one pixel, may be many orders below others').  32 x 128 x 28 x 28, 128 templates, 3 x 3: 196 us
 // on the fp32 matrix instructions -> 101 us, error against 64 bits 6.0e-7 -> 2.0e-7 of the gradient's 2-norm.  Small grids
 // keep that kernel (sim_mfma_kernel), which splits the contraction over workgroups.
 // ------------------------------------------------------------------------------------------------
