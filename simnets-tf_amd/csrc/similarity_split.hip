@@ -44,9 +44,9 @@
 //
 // Measured (whole call, vector form, three bf16 pieces, this form): 256 x 64 x 32 x 32 -> 128, 3 x 3: 0.80, 0.372, 0.229 ms.
 // The kernel's 211 us are 1.1 PFLOP/s of matrix products at 1.55 GHz, matrix units busy 56 %: the clock sinks with them
-// (products of random numbers alone run at 1.57 PFLOP/s and 1.65 GHz, of zeros at 2.35), 155 us would be that rate.  37 x 45 x 29 x 35 -> 75: 172, 66,
-// 50 us, where half of the products are padding (96 templates, 48 channels, 37632 pixels).  64 images of the first with a
-// quarter missing: 427, 160, 108 us.
+// (products of random numbers alone run at 1.57 PFLOP/s and 1.65 GHz, of zeros at 2.35), 155 us would be that rate.  37 x 45 x
+// 29 x 35 -> 75: 172, 66, 50 us, where half of the products are padding (96 templates, 48 channels, 37632 pixels).  64 images of
+// the first with a quarter missing: 427, 160, 110 us.
 // Tried: 2 x 2 tiles a wave (half of the LDS reads, twice the parameter loads): 250 us for 228.
 #include <hip/hip_runtime.h>
 
