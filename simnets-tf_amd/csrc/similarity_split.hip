@@ -517,13 +517,15 @@ __device__ __forceinline__ void split_far_most(__attribute__((address_space(3)))
 }
 
 // Forward.  One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel
-// tiles.  Where the inputs are much larger than what the templates differ by, so that the square of one is beyond half precision
-// and an eighth of the lanes have one that counts beside it, the workgroup goes on at a smaller scale of the channels (a
-// level, 2^-3 each, packed by the packing kernel): its sums are scaled, the chunk is staged again, and the cross terms'
-// parameters are multiplied on the way.  Where only a few pixels are that large their outputs become NaN, and are
-// recomputed.  256 x 64 x 32 x 32 -> 128, 3 x 3, templates of size 0.05, inputs 0..255 or 0..10^7: 220 us, where all
-// tiles left to the direct kernel took 1190; what it costs ordinary inputs: 1 to 2 us there, 1 of 50 on 37 x 45 x 29 x 35 -> 75, 2 of
-// 54 on 64 x 256 x 32 x 32 -> 64, 1 x 1.  One pixel in a hundred 10^4 times the others: most tiles to the direct kernel, 1480.
+// tiles.  Where the inputs are much larger than what the templates differ by, so that the square of one is beyond half
+// precision, the workgroup goes on at a smaller scale of the channels (a level, 2^-3 each, packed by the packing kernel): its
+// sums are scaled, the chunk is staged again, and the cross terms' parameters are multiplied on the way.  Ordinary values
+// keep their bits at the first level (what it may lose, 2^-7 / sqrt(K) of the weights' sum, is below the guard's line);
+// for the higher ones an eighth of the lanes need values that count there, and where only a few pixels are that large
+// their outputs become NaN and are recomputed.  256 x 64 x 32 x 32 -> 128, 3 x 3, templates of size 0.05, inputs 0..255 or 0..10^7:
+// 220 us, where all tiles left to the direct kernel took 1190; inputs 0.05 and a border of 100: 222 and 1222; one pixel in a
+// hundred 10^3 times the others: 225 and 1440, 10^4 times: 1490 and 1470.  What it costs ordinary inputs: 1 to 2 us there,
+// 1 of 50 on 37 x 45 x 29 x 35 -> 75, 2 of 54 on 64 x 256 x 32 x 32 -> 64, 1 x 1.
 template <int KIND, int CG, int G>
 __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attribute__((address_space(3))) SplitFar &far,
                                            u32x4 &near, int ptile, int mtile0, int norm)
@@ -681,7 +683,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
         if (__builtin_expect(seen > __float_as_int(kSplitMost), 0)) {
             int next_level = level;
             while (next_level < kLastLevel && __int_as_float(seen) > ldexpf(kSplitMost, kSplitLevelBits * next_level) &&
-                   __builtin_amdgcn_readfirstlane(far.lanes[chunk & 1][next_level]) > kThreads / 8)
+                   (next_level == 0 || __builtin_amdgcn_readfirstlane(far.lanes[chunk & 1][next_level]) > kThreads / 8))
                 ++next_level;
             if (next_level > level) {
                 const float ratio = ldexpf(1.0f, 2 * kSplitLevelBits * (level - next_level));

@@ -518,7 +518,7 @@ def test_split_input_gradient_over_templates_and_pixels_of_any_size(pkg, O, bloc
     assert float(err.max()) <= 2 * (O * block * block / 16 + 8) * 2.0 ** -24, float(err.max())
 
 
-FAR = [("init", 255.0), ("init", 6e4), ("init", 1e8), ("normal", 1e4), ("similar", 1.0), ("similar", 1e-6)]
+FAR = [("init", 255.0), ("init", 6e4), ("init", 1e8), ("normal", 1e4), ("similar", 1.0), ("similar", 1e-6), ("pixels", 1e3), ("border", 100.0)]
 
 
 @pytest.mark.parametrize("mode", ["l2", "norm", "missing"])
@@ -536,11 +536,17 @@ def test_split_form_of_inputs_on_another_scale(pkg, geom, kind, size, mode):
         x = torch.rand(shape, generator=g, device="cuda") * size
     elif kind == "normal":
         x = torch.randn(shape, generator=g, device="cuda") * size
+    elif kind == "pixels":     # one in a hundred
+        x = torch.randn(shape, generator=g, device="cuda")
+        x *= 1 + size * (torch.rand((shape[0], 1, *shape[2:]), generator=g, device="cuda") < 0.01)
+    elif kind == "border":
+        t = t * 0.05
+        x = torch.randn(shape, generator=g, device="cuda") * 0.05
     else:                      # templates all nearly the same
         t = size * (1 + 1e-4 * t)
         x = torch.randn(shape, generator=g, device="cuda") * size
     kw = options(mode, geom)
-    oob = kw.setdefault("out_of_bounds_value", geom.get("out_of_bounds_value", 0.0))
+    oob = kw.setdefault("out_of_bounds_value", size if kind == "border" else geom.get("out_of_bounds_value", 0.0))
     if mode == "missing":
         x[torch.rand(shape, generator=g, device="cuda") < 0.25] = float("nan")
     assert pieces_used(pkg, shape, O, mode, **kw)["forward"]
@@ -553,8 +559,8 @@ def test_split_form_of_inputs_on_another_scale(pkg, geom, kind, size, mode):
         scale = torch.maximum(scale, logs[None, :, None, None])
     err = float(((got.double() - want).abs() / scale).max())
     assert err <= 2 * (K / 16 + 8) * 2.0 ** -24, err
-    if mode == "missing" and size == 1e8 or mode == "norm" and size == 1e-6:
-        return    # beyond the levels of that mode; nothing but the logarithms' sum
+    if mode == "missing" and size == 1e8 or mode == "norm" and (size == 1e-6 or kind == "border"):
+        return    # beyond the levels of that mode; away from the border nothing but the logarithms' sum
     direct = pkg.similarity(x, t, w, algo="direct", **kw)
     assert float((got == direct).float().mean()) < 0.7
 
