@@ -17,7 +17,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
+#include "fast_div.h"
 #include "internal.h"
 #include "mex_common.h"
 #include "valu_tile.h"
@@ -505,10 +507,9 @@ __global__ __launch_bounds__(256) void mex_sum_splits_kernel(const float *__rest
 
 // ... four elements per thread with all the splits' loads (at most 8) in flight together: n a multiple of 4, 16-byte
 // aligned pointers.  The same additions in the same order.
-__global__ __launch_bounds__(256) void mex_sum_splits4_kernel(const float4 *__restrict__ parts, long long n4, int splits,
-                                                             float4 *__restrict__ dx)
+__device__ __forceinline__ void sum_splits4(const float4 *__restrict__ parts, long long n4, int splits, float4 *__restrict__ dx,
+                                            long long i)
 {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4)
         return;
     float4 v[8];
@@ -522,6 +523,12 @@ __global__ __launch_bounds__(256) void mex_sum_splits4_kernel(const float4 *__re
             s.x += v[z].x; s.y += v[z].y; s.z += v[z].z; s.w += v[z].w;
         }
     dx[i] = s;
+}
+
+__global__ __launch_bounds__(256) void mex_sum_splits4_kernel(const float4 *__restrict__ parts, long long n4, int splits,
+                                                             float4 *__restrict__ dx)
+{
+    sum_splits4(parts, n4, splits, dx, (long long)blockIdx.x * 256 + threadIdx.x);
 }
 
 void launch_sum_splits(const float *parts, long long n, int splits, float *dx, hipStream_t s)
@@ -875,590 +882,559 @@ __global__ __launch_bounds__(256, PIPE ? 2 : 3) void mex_grad_offsets_mfma_kerne
 // of the input or of its gradient) is read and written as one run of 1 KB, or runs of whole images, with 16-byte
 // accesses.  The values pass through LDS tiles [plane][column] with column = region * 64 + slot, and wave r does
 // the matrix steps of region r on its 64 columns.
+// Everything the kernel reads outside of its term-by-term path, in one block: fetched at once, and not piece by piece where
+// it is first needed (a round trip to memory each).
 struct RowsArgs {
+    const float *in, *out, *g;
+    const float *offe, *omax, *orng;   // the packed offsets
+    float *dx, *partial;               // (of split 0; null: not wanted)
+    long long dx_split;                // floats from one split's input gradient to the next's
+    float c0, c1;
+    int B, M, K, n_mg, mg_per_split;
     int lgW, Ws, RS;   // log2(width), windows per row, windows per image
     int lgHW, HW;      // pixels of an image
-    int nx, ty, tz;    // workgroup numbering (rows_block): pixel groups, tiles along the two other grid dimensions
+    int chunks, pxl;   // of 256 pixels: in all, per workgroup
+    int nx, ty, tz;    // workgroup numbering (rows_block): pixel groups, tiles along the two other grid dimensions,
+    int per_die;       // ... an eighth of them all
+    FastDiv d_tiles, d_ty;   // ty * tz; ty
 };
 
-// Workgroups that read the same rows - the tiles (y, z) of one pixel group x - get consecutive turns on ONE
-// accelerator die (linear workgroup id mod 8), so that the rows come from memory once and from that die's L2 for the
-// other tiles.  The launch is one-dimensional with 8 * ceil(nx / 8) * ty * tz workgroups; false: no such group.
+// Workgroups that read the same rows - the tiles (y, z) of one pixel group x - get turns on ONE accelerator die (linear
+// workgroup id mod 8), so that the rows come from memory once and from that die's L2 for the other tiles: each die takes an
+// eighth of all tiles, in order.  (Whole groups to a die, x mod 8, leave dies idle where there are few: the 2 x 2
+// maps of 32 images, one group, 35.5 -> 16.0 us.)  The launch is one-dimensional with 8 g.per_die workgroups; false:
+// nothing is left for this one.
 __device__ __forceinline__ bool rows_block(const RowsArgs &g, int *x, int *y, int *z)
 {
-    const int l = blockIdx.x, tiles = g.ty * g.tz;
-    const int j = l >> 3, tile = j % tiles;
-    *x = (j / tiles) * 8 + (l & 7);
-    *y = tile % g.ty;
-    *z = tile / g.ty;
-    return *x < g.nx;
+    const int l = blockIdx.x, tiles = g.ty * g.tz, i = (l & 7) * g.per_die + (l >> 3);
+    if (i >= g.nx * tiles)
+        return false;
+    *x = (int)fast_div((unsigned)i, g.d_tiles);
+    const int tile = i - *x * tiles;
+    *z = (int)fast_div((unsigned)tile, g.d_ty);
+    *y = tile - *z * g.ty;
+    return true;
 }
 
-// A thread's four neighbouring pixels (a 16-byte piece of a row; width >= 4, so they share the row) of the chunk's
-// 256: image, first pixel, tile columns.  Pixels 0 and 2 belong to region rbase, 1 and 3 to rbase + 1.  A chunk
-// starts on an even row (or a whole image), so the columns and rbase depend on the quad alone, not on the chunk.
+// A thread's four neighbouring pixels (16 bytes) of the chunk's 256: image, first pixel, tile columns.  They share a row, and
+// pixels 0 and 2 belong to region rbase, 1 and 3 to rbase + 1; on maps of two columns (W2) they are a window and belong to
+// the four regions in turn.  A chunk starts on an even row (or a whole image), so columns and regions depend on the quad
+// alone, not on the chunk.
+template <bool W2>
 struct RowsQuad {
-    int img, pix0, rbase;
-    bool img_ok;
-    int col[4];
+    int img, pix0, rbase, col0;
+    __device__ __forceinline__ RowsQuad(const RowsArgs &g, int chunk, int quad)
+    {
+        const int gpix = chunk * 256 + 4 * quad;
+        img = gpix >> g.lgHW;
+        pix0 = gpix & (g.HW - 1);
+        const int h = pix0 >> g.lgW, w0 = pix0 & ((1 << g.lgW) - 1);
+        rbase = W2 ? 0 : (h & 1) * 2;
+        col0 = (rbase << 6) + img * g.RS + (h >> 1) * g.Ws + (w0 >> 1) - chunk * 64;
+    }
+    __device__ __forceinline__ int region(int e) const { return W2 ? e : rbase + (e & 1); }
+    __device__ __forceinline__ int col(int e) const { return W2 ? col0 + (e << 6) : col0 + ((e & 1) << 6) + (e >> 1); }
+    // of the pooled map: the quad's first window
+    __device__ __forceinline__ int window(const RowsArgs &g) const
+    {
+        const int h = pix0 >> g.lgW, w0 = pix0 & ((1 << g.lgW) - 1);
+        return (h >> 1) * g.Ws + (w0 >> 1);
+    }
 };
 
-__device__ __forceinline__ RowsQuad rows_quad(const MexKernelArgs &a, const RowsArgs &g, int chunk, int quad)
+// The output gradients of a thread's pixel quad as they come from memory: 16 bytes of g, or - POOLED, g is that of the
+// windows' sums - the gradients of the windows the quad lies in (x, y; each belongs to two pixels; W2: one, x).
+// rows_quad_g expands them where they are used: expanding here would wait for the load where it is issued.
+template <bool W2, bool POOLED>
+struct RowsGrad {
+    typedef std::conditional_t<!POOLED, float4, std::conditional_t<W2, float, float2>> type;
+};
+
+__device__ __forceinline__ void rows_quad_g(const float4 &v, float (&gg)[4])
 {
-    RowsQuad q;
-    const int gpix = chunk * 256 + 4 * quad;
-    q.img = gpix >> g.lgHW;
-    q.pix0 = gpix & (g.HW - 1);
-    q.img_ok = q.img < a.B;
-    const int h = q.pix0 >> g.lgW, w0 = q.pix0 & ((1 << g.lgW) - 1);
-    q.rbase = (h & 1) * 2;
-    const int sl = q.img * g.RS + (h >> 1) * g.Ws + (w0 >> 1) - chunk * 64;
-    q.col[0] = (q.rbase << 6) + sl;
-    q.col[1] = q.col[0] + 64;
-    q.col[2] = q.col[0] + 1;
-    q.col[3] = q.col[1] + 1;
-    return q;
+    gg[0] = v.x; gg[1] = v.y; gg[2] = v.z; gg[3] = v.w;
 }
 
-// The output gradients of a thread's pixel quad for plane (img, m) as they come from memory: 16 bytes of g, or - g
-// pooled - the two window gradients the quad's row lies in (x, y; each belongs to two pixels).  rows_quad_g expands
-// them where they are used: expanding here would wait for the load where it is issued.
-__device__ __forceinline__ float4 rows_load_g(const MexGradArgs &ga, const RowsArgs &g, const RowsQuad &q, size_t img,
-                                              int m)
+__device__ __forceinline__ void rows_quad_g(const float2 &v, float (&gg)[4])
 {
-    if (!ga.gpool)
-        return *reinterpret_cast<const float4 *>(ga.g + (img * ga.k.M + m) * (size_t)g.HW + q.pix0);
-    const int h = q.pix0 >> g.lgW, w0 = q.pix0 & ((1 << g.lgW) - 1);
-    const float2 v = *reinterpret_cast<const float2 *>(ga.g + (img * ga.k.M + m) * (size_t)(g.HW >> 2) +
-                                                       (size_t)(h >> 1) * g.Ws + (w0 >> 1));
-    return make_float4(v.x, v.y, 0.0f, 0.0f);
+    gg[0] = gg[1] = v.x;
+    gg[2] = gg[3] = v.y;
 }
 
-__device__ __forceinline__ void rows_quad_g(const MexGradArgs &ga, const float4 &v, float (&gg)[4])
+__device__ __forceinline__ void rows_quad_g(float v, float (&gg)[4])
 {
-    gg[0] = v.x;
-    gg[1] = ga.gpool ? v.x : v.y;
-    gg[2] = ga.gpool ? v.y : v.z;
-    gg[3] = ga.gpool ? v.y : v.w;
+    gg[0] = gg[1] = gg[2] = gg[3] = v;
+}
+
+// A uniform address and a lane's offset in elements (less than 2^31 bytes: rows_geometry)
+template <typename T>
+__device__ __forceinline__ T rows_load(const float *base, unsigned at)
+{
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + 4 * at);
 }
 
 // per region: is some instance's offsets range beyond kGradRowsRange or not finite (flags[r]: term by term); flags[4]:
-// does some range exceed kLooseBoundRange; flags[5]: does some range exceed kGradProductRange.  All threads of the
-// workgroup call it; the flags (six) are in place behind its last barrier.
-// (All loads go out before the first is looked at.)
-__device__ __forceinline__ void rows_ranges(const MexKernelArgs &a, int tid, int *flags)
-{
-    if (tid < 6)
-        flags[tid] = 0;
-    const int per = a.n_mgroups * GM_TM;
-    int big = 0, mid = 0, wide[4] = {0, 0, 0, 0};
-    for (int mb = 0; mb < a.M; mb += 1024) {
-        float v[4][4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                v[u][r] = a.orng[r * per + min(mb + 256 * u + tid, a.M - 1)];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (mb + 256 * u + tid < a.M) {
-                    big |= !(v[u][r] <= kLooseBoundRange);
-                    mid |= !(v[u][r] <= kGradProductRange);
-                    wide[r] |= !(v[u][r] <= kGradRowsRange);
-                }
+// does some range exceed kLooseBoundRange.  All threads of the workgroup call flag(); the flags (five, zero before a
+// barrier) are in place behind the next one.  The constructor requests the first 256 instances' ranges.
+struct RowsRanges {
+    float v[4];
+    __device__ __forceinline__ RowsRanges(const RowsArgs &g, int tid)
+    {
+        load(g, min(tid, g.M - 1));
     }
-    __syncthreads();
-    const bool first = (tid & 63) == 0;
+    __device__ __forceinline__ void load(const RowsArgs &g, int m)
+    {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-        if (__any(wide[r]) && first)
-            flags[r] = 1;   // (every writer writes the same value)
-    if (__any(mid) && first)
-        flags[5] = 1;
-    if (__any(big) && first)
-        flags[4] = 1;
-    __syncthreads();
+        for (int r = 0; r < 4; ++r)
+            v[r] = g.orng[r * g.n_mg * GM_TM + m];
+    }
+    __device__ __forceinline__ void flag(const RowsArgs &g, int tid, int *flags)
+    {
+        for (int m = tid;;) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (m < g.M && !(v[r] <= kLooseBoundRange)) {
+                    flags[4] = 1;      // (every writer writes the same value)
+                    if (!(v[r] <= kGradRowsRange))
+                        flags[r] = 1;
+                }
+            m += 256;
+            if (m >= g.M)
+                break;
+            load(g, m);
+        }
+    }
+};
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// The term-by-term path of the kernel below reads its arguments from the kernel's argument segment (they are the last, in front
+// of the implicit ones) and is a call: inlined, what it keeps in scalar registers is fetched, and spilled, at the kernel's start.
+static_assert(sizeof(MexGradArgs) % 8 == 0, "the explicit arguments end with the block");
+__device__ __forceinline__ const MexGradArgs &rows_term_args()
+{
+    return *reinterpret_cast<const MexGradArgs *>(reinterpret_cast<const char *>(__builtin_amdgcn_implicitarg_ptr()) -
+                                                  sizeof(MexGradArgs));
 }
 
-// Input gradient.  Workgroup (rows_block) x: chunk of 256 pixels; y: tile of 16 * KSUB patch elements; z: split of the
-// instance groups.  Per instance group the pixel factors W [32][256] are formed from rows of `out` and `g`, the four
-// regions' offset exponentials [16 * KSUB][32] come from the packed offsets, and wave r accumulates region r's
-// 16 * KSUB x 64 gradients; these leave through a tile [patch element][column], times 2^(xs - a) from rows of the
-// input, as rows of the gradient.  A region with a wide offsets range is done term by term (the other three are not
-// held up by it).
-template <int KSUB>
-__global__ __launch_bounds__(256, KSUB == 1 ? 3 : KSUB == 2 ? 2 : 1) void mex_grad_input_rows_kernel(const MexGradArgs ga, const RowsArgs g)
+// The regions with a wide offsets range, or with a chunk's wide pixels: late holds a bit per chunk for each.  GX_KT patch elements of
+// a region per wave and turn for the input gradient; for the offsets the tile of KT patch elements as GO_MT x GO_KT wave
+// tiles over all chunks.
+// (Arguments of a call are in vector registers: all are uniform.)
+template <int KT>
+__device__ __noinline__ void rows_terms(int bx_v, int n_chunks_v, int k0_v, int mg_begin_v, int mg_end_v, float *dx_v, int offsets_v,
+                                        int4 late_v)
 {
-    const MexKernelArgs &a = ga.k;
-    constexpr int KT = 16 * KSUB;
-    constexpr int WP = 272, EP = 36, OP = 260;   // row pitches: the matrix steps' and the tile's accesses hit 64 banks
-    constexpr int kWt = 32 * WP, kEo = 4 * KT * EP, kOt = KT * OP;
-    constexpr int kTile = kWt + kEo > kOt ? kWt + kEo : kOt;
-    __shared__ __attribute__((aligned(16))) float smem[kTile];
-    __shared__ float ap[256];          // per column: the pixel's bound (0 for an empty slot)
+    const MexGradArgs &ga = rows_term_args();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int bx = uniform(bx_v), n_chunks = uniform(n_chunks_v), k0 = uniform(k0_v), mg_begin = uniform(mg_begin_v),
+              mg_end = uniform(mg_end_v), offsets = uniform(offsets_v);
+    const int late[4] = {uniform(late_v.x), uniform(late_v.y), uniform(late_v.z), uniform(late_v.w)};
+    const unsigned long long dx_bits = (unsigned long long)(uintptr_t)dx_v;
+    float *dx = reinterpret_cast<float *>((unsigned long long)(unsigned)uniform((int)(dx_bits >> 32)) << 32 | (unsigned)uniform((int)dx_bits));
+    const int M = ga.k.M, K = ga.k.K, m_begin = min(M, mg_begin * GM_TM), m_end = min(M, mg_end * GM_TM);
+    constexpr int NX = KT / GX_KT, NO = KT / GO_KT, NM = 32 / GO_MT;
+    if (dx != nullptr)
+        for (int s = 0; s < n_chunks; ++s)
+            for (int u = wave; u < 4 * NX; u += 4) {
+                const int r = u / NX, kk0 = k0 + u % NX * GX_KT;
+                if ((late[r] >> s & 1) && kk0 < K)
+                    mex_grad_input_wave(ga, r, bx * ga.pxl + s, kk0, lane, m_begin, m_end, dx);
+            }
+    if (offsets)
+        for (int m0 = m_begin; m0 < m_end; m0 += 32)
+            for (int u = wave; u < 4 * NM * NO; u += 4) {
+                const int r = u / (NM * NO), i = u % (NM * NO), mm0 = m0 + i / NO * GO_MT, kk0 = k0 + i % NO * GO_KT;
+                if (late[r] && mm0 < M && kk0 < K)
+                    mex_grad_offsets_wave(ga, r, bx, mm0, kk0, lane);
+            }
+}
+#endif
+
+// Both gradients, or either.  Workgroup (rows_block) x: group of ga.pxl chunks of 256 pixels; y: tile of 16 * KSUB patch
+// elements; z: split of the instance groups.  A thread's pixels are one quad of the chunk, its planes pl0, pl0 + 4, ... of
+// every block of 32: a wave's load is four planes of sixteen quads, whole runs of memory on maps of any size (2 x 2 ones
+// included: neighbouring planes of an image are neighbours in memory), and what concerns one pixel - its bound a - needs
+// no LDS.  Per instance group the pixel factors W [32][256] are formed once, from rows of `out` and `g`, and serve both
+// products: wave r multiplies region r's W with the offset exponentials (input gradient, added up over the groups) and
+// with the tile's patch exponentials 2^(xs - a) of its 64 columns, which it holds as matrix operands in registers
+// (offsets gradient, to the partial sums at once; with several chunks the workgroup adds to what it has stored).  The input gradient
+// leaves through a tile [patch element][column], times 2^(xs - a), as rows.  A region with a wide offsets range is done
+// term by term (the other three are not held up by it).
+//
+// Bound by the latency of a workgroup's phases, two workgroups to a compute unit, of which the matrix steps are a third.
+// The two gradients were a kernel each: both read `out` and `g` and formed W, the one for the offsets once more for every 32 patch
+// elements.  512 images, whole call, 32 channels of 16 x 16 -> 64
+// instances, 64 of 8 x 8 -> 128, 128 of 4 x 4 -> 256, 256 of 2 x 2 -> 512: both gradients 57, 54, 59, 72 -> 44, 39, 41, 52 us, the
+// input's alone 27.5, 27.5, 34, 48 -> 29, 26, 29, 40, the offsets' alone, with twice the partial sums, 34, 30, 32.5, 46 -> 38, 34, 33,
+// 42.  32 images, both, the kernels of four such layers and their sums: 118 -> 75.  The bound is taken over the first group's
+// instances: errors against 64 bits as before, and a third to a half of it for offsets that span 24 to 48 exponents on 2 x 2 maps.
+// W2: the map has two columns, a quad is a window and its pixels belong to the four regions.
+//
+// The tile's pitch, 20 modulo 64: sixteen lanes' 16-byte operands of a column of rows, or of a row, lie in different banks.
+template <int KSUB, bool W2, bool POOLED>
+__global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(const RowsArgs g, const MexGradArgs ga)
+{
+    constexpr int KT = 16 * KSUB, NJ = KT / 4;
+    constexpr int TP = 276, EP = 36;
+    __shared__ __attribute__((aligned(16))) float wt[32 * TP];        // W, and before and behind it the patch elements' tile
+    __shared__ __attribute__((aligned(16))) float eo[4 * KT * EP];    // [region][patch element][instance]
     __shared__ float tab[2][128];      // per (region, instance of the group): omax + c0, for this group and the next
-    __shared__ int wide_sh[6];         // per region: term by term; [4]: some range beyond the loose bound's
-    float *wt = smem, *eo = smem + kWt, *ot = smem;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lr = lane & 15, lq = lane >> 4;
-    int chunk, by, bz;
-    if (!rows_block(g, &chunk, &by, &bz))
-        return;
-    const int k0 = by * KT;
-    const int n_mg = a.n_mgroups, per = n_mg * GM_TM;
-    const int mg_begin = bz * ga.mg_per_split, mg_end = min(n_mg, mg_begin + ga.mg_per_split);
-    float *dxo = ga.msplit > 1 ? ga.dx_splits + (size_t)bz * a.B * a.C * a.H * a.W : ga.dx;
-    const RowsQuad q = rows_quad(a, g, chunk, lane);
-    const int pl0 = wave;              // this thread's planes of a block of 32: pl0, pl0 + 4, ...
-    const size_t HW = (size_t)g.HW;
-    const size_t img = q.img_ok ? q.img : 0;
-    // operands of an instance group: this thread's eight rows pieces of `out` and `g`, its share of the four regions'
-    // offset exponentials, the next group's instance constants - requested a group ahead (the first before the bound
-    // is worked out, the others while the matrix steps run)
-    float4 ov[8], gv[8], en[2 * KSUB];
-    float tn = 0.0f;
-    auto request = [&](int mg) {
-        // (those past the last instance, image or patch element on a clamped address or skipped)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int m = min(mg * GM_TM + pl0 + 4 * j, a.M - 1);
-            ov[j] = *reinterpret_cast<const float4 *>(ga.out + (img * a.M + m) * HW + q.pix0);
-            gv[j] = rows_load_g(ga, g, q, img, m);
-        }
-#pragma unroll
-        for (int j = 0; j < 2 * KSUB; ++j) {
-            const int i = tid + 256 * j;
-            const int r = i / (KT * 8), row = (i % (KT * 8)) >> 3, c4 = i & 7;
-            en[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (k0 + row < a.K)
-                en[j] = *reinterpret_cast<const float4 *>(a.offe + (((size_t)r * n_mg + mg) * a.K + k0 + row) * GM_TM + 4 * c4);
-        }
-        if (tid < 128 && mg + 1 < mg_end)
-            tn = a.omax[(tid >> 5) * per + (mg + 1) * GM_TM + (tid & 31)] + a.c0;
-    };
-    if (mg_begin < mg_end)
-        request(mg_begin);
-    // ---- the bound of every pixel: a = min over (a few) instances of outs_m - c0 - lo_m, see
-    //      mex_grad_input_mfma_kernel.  The rows of the first four instances, which give it unless some offsets
-    //      range is large, are requested before the ranges are looked at ----
-    float4 bo[8];
-    float lo_n = 0.0f;
-    auto request_bound = [&](int mb, int m_scan) {
-        if (tid < 128) {
-            const int m = min(mb + (tid & 31), a.M - 1);
-            lo_n = a.omax[(tid >> 5) * per + m] - a.orng[(tid >> 5) * per + m];
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int m = mb + pl0 + 4 * j;
-            bo[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (q.img_ok && m < m_scan)
-                bo[j] = *reinterpret_cast<const float4 *>(ga.out + (img * a.M + m) * HW + q.pix0);
-        }
-    };
-    request_bound(0, min(a.M, 4));
-    rows_ranges(a, tid, wide_sh);
-    const int roomy = wide_sh[4];
-    const bool slot_ok = chunk * 64 + (tid & 63) < a.slots;
-    // Large offsets ranges: the bound from `out` and the offsets' minima is loose by up to the range, which costs the
-    // factors their precision (and, beyond kGradProductRange, the product form).  The pixel's own maximum over all of
-    // K - one sweep over the rows of the input - is tight: the exponents then stay within the pixel's patch range, and
-    // a region keeps the product form while those ranges are at most kGradPixelRange and its offsets span at most
-    // kGradRowsRange.
-    float amin = INFINITY;             // the bound of column tid
-    if (roomy) {
-        float amax = -INFINITY, alo = INFINITY;
-        for (int kb = 0; kb < a.K; kb += 32) {
-            float4 xr[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                xr[j] = *reinterpret_cast<const float4 *>(a.in + (img * a.K + min(kb + pl0 + 4 * j, a.K - 1)) * HW + q.pix0);
-            __syncthreads();           // the previous block's readers are done with the tile
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int pl = pl0 + 4 * j;
-                const bool use = q.img_ok && kb + pl < a.K;
-                const float v[4] = {xr[j].x, xr[j].y, xr[j].z, xr[j].w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    wt[pl * WP + q.col[e]] = use ? v[e] * a.c1 : __builtin_nanf("");   // (fmax / fmin skip NaN)
-            }
-            __syncthreads();
-#pragma unroll 8
-            for (int pl = 0; pl < 32; ++pl) {
-                const float t = wt[pl * WP + tid];
-                amax = fmaxf(amax, t);
-                alo = fminf(alo, t);
-            }
-        }
-        // a pixel with an infinite value, nothing finite, or a patch range beyond the bound sends its region term by term
-        const bool px_ok = !slot_ok || (fabsf(amax) < INFINITY && amax - alo <= kGradPixelRange);
-        const int bad = __any(!px_ok) ? 1 : 0;
-        if (lane == 0)
-            wide_sh[wave] |= bad;      // (columns of wave w belong to region w)
-        amin = amax;
-    }
-    const int m_scan = roomy ? 0 : min(a.M, 4);
-    for (int mb = 0; mb < m_scan; mb += 32) {
-        if (tid < 128)
-            tab[0][tid] = lo_n;
-        __syncthreads();               // tab in place; the previous block's readers are done with the tile
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int pl = pl0 + 4 * j;
-            const bool use = q.img_ok && mb + pl < m_scan;
-            const float v[4] = {bo[j].x, bo[j].y, bo[j].z, bo[j].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                wt[pl * WP + q.col[e]] =
-                    use ? __builtin_fmaf(v[e], a.c1, -(a.c0 + tab[0][(q.rbase + (e & 1)) * 32 + pl])) : INFINITY;
-        }
-        __syncthreads();
-#pragma unroll 8
-        for (int pl = 0; pl < 32; ++pl)
-            amin = fminf(amin, wt[pl * WP + tid]);
-    }
-    ap[tid] = slot_ok ? amin : 0.0f;
-    if (tid < 128 && mg_begin < mg_end)   // (the loop above is done with the table: its last readers passed the
-        tab[mg_begin & 1][tid] = a.omax[(tid >> 5) * per + mg_begin * GM_TM + (tid & 31)] + a.c0;   // barrier in front of the reduction)
-    __syncthreads();
-    const bool my_wide = wide_sh[wave] != 0;
-    const bool any_wide = (wide_sh[0] | wide_sh[1] | wide_sh[2] | wide_sh[3]) != 0;
-    float bound[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        bound[e] = ap[q.col[e]];
-
-    floatx4 acc[KSUB][4];
-#pragma unroll
-    for (int ks = 0; ks < KSUB; ++ks)
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            acc[ks][t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int NJ = KT / 4;
-    float4 xv[NJ];                     // the epilogue's rows of the input, requested during the last matrix steps
-    for (int mg = mg_begin; mg < mg_end; ++mg) {
-        __syncthreads();               // the previous group's matrix steps are done with wt / eo
-        const float *tb = tab[mg & 1];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int pl = pl0 + 4 * j;
-            const bool use = q.img_ok && mg * GM_TM + pl < a.M;
-            const float o[4] = {ov[j].x, ov[j].y, ov[j].z, ov[j].w};
-            float gg[4];
-            rows_quad_g(ga, gv[j], gg);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                // (a - outs) first: a small, once-rounded difference; the instance constant is added to that (forming
-                // a + mo first, about the size of outs, was tried for the tight bound: worse on half of the data)
-                const float ex = __builtin_fmaf(-o[e], a.c1, bound[e]) + tb[(q.rbase + (e & 1)) * 32 + pl];
-                wt[pl * WP + q.col[e]] = use ? gg[e] * __builtin_amdgcn_exp2f(ex) : 0.0f;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2 * KSUB; ++j) {
-            const int i = tid + 256 * j;
-            const int r = i / (KT * 8), row = (i % (KT * 8)) >> 3, c4 = i & 7;
-            *reinterpret_cast<float4 *>(eo + (r * KT + row) * EP + 4 * c4) = en[j];
-        }
-        if (tid < 128)
-            tab[(mg + 1) & 1][tid] = tn;
-        if (mg + 1 < mg_end) {
-            request(mg + 1);
-        } else {
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const int k = min(k0 + pl0 + 4 * j, a.K - 1);
-                xv[j] = *reinterpret_cast<const float4 *>(a.in + (img * a.K + k) * HW + q.pix0);
-            }
-        }
-        __syncthreads();
-        if (!my_wide) {
-#pragma unroll
-            for (int ms = 0; ms < GM_TM; ms += 4) {
-                float bv[4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    bv[t] = wt[(ms + lq) * WP + wave * 64 + t * 16 + lr];
-#pragma unroll
-                for (int ks = 0; ks < KSUB; ++ks) {
-                    const float av = eo[(wave * KT + ks * 16 + lr) * EP + ms + lq];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                        acc[ks][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[t], acc[ks][t], 0, 0, 0);
-                }
-            }
-        }
-    }
-    // ---- d patch_k = 2^(xs_k - a) * acc: through the tile [patch element][column] to rows of the gradient ----
-    if (mg_begin >= mg_end) {
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-            xv[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-    __syncthreads();                   // the last matrix steps are done with wt / eo, which the tile overlies
-#pragma unroll
-    for (int ks = 0; ks < KSUB; ++ks)
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                ot[(ks * 16 + 4 * lq + v) * OP + wave * 64 + t * 16 + lr] = acc[ks][t][v];
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int kl = pl0 + 4 * j, k = k0 + kl;
-        if (!q.img_ok || k >= a.K)
-            continue;
-        const float x[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
-        float d[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            d[e] = ot[kl * OP + q.col[e]] * __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], a.c1, -bound[e]));
-        float *dst = dxo + (img * a.K + k) * HW + q.pix0;
-        if (!any_wide) {
-            *reinterpret_cast<float4 *>(dst) = make_float4(d[0], d[1], d[2], d[3]);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (!wide_sh[q.rbase + (e & 1)])
-                    dst[e] = d[e];
-        }
-    }
-    if (any_wide) {
-        // the regions with a wide offsets range, term by term: GX_KT patch elements of a region per wave and turn
-        constexpr int NSUB = KT / GX_KT;
-        for (int u = wave; u < 4 * NSUB; u += 4) {
-            const int r = u / NSUB, kk0 = k0 + (u % NSUB) * GX_KT;
-            if (wide_sh[r] && kk0 < a.K)
-                mex_grad_input_wave(ga, r, chunk, kk0, lane, min(a.M, mg_begin * GM_TM), min(a.M, mg_end * GM_TM), dxo);
-        }
-    }
-}
-
-// Offsets gradient.  Workgroup (rows_block) x: group of ga.pxl chunks of 256 pixels; y: tile of 32 instances; z: tile
-// of 32 patch elements.  Per chunk the tile's pixel factors W [32][256] and patch exponentials [32][256] are formed from
-// rows of `out`, `g` and the input - relative to the bound over the tile's own instances, which the rows just read
-// give - and wave r adds region r's 32 x 32 products over its 64 columns.  Partial sums [chunk group][region][M][K]
-// like mex_grad_offsets_mfma_kernel's.
-__global__ __launch_bounds__(256, 2) void mex_grad_offsets_rows_kernel(const MexGradArgs ga, const RowsArgs g)
-{
-    const MexKernelArgs &a = ga.k;
-    constexpr int TP = 260;
-    __shared__ float wt[32 * TP];      // [instance][column]
-    __shared__ float ex[32 * TP];      // [patch element][column]
-    __shared__ float pm[4 * 256];      // per column: the four waves' minima
-    __shared__ int wide_sh[6];
+    __shared__ float lo_tab[128];      // ... and c0 + the offsets' minimum, of the first group
+    __shared__ int wide_sh[5];         // see RowsRanges
+    __shared__ int late[4];            // per region: the chunks (bits) that are left to the term-by-term waves
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lq = lane >> 4;
     int bx, by, bz;
     if (!rows_block(g, &bx, &by, &bz))
         return;
-    const int m0 = by * 32, k0 = bz * 32;
-    const int n_mg = a.n_mgroups, per = n_mg * GM_TM;
-    const int pl0 = wave;
-    const size_t HW = (size_t)g.HW;
-    // the constants of this thread's planes for its two regions (the same in every chunk)
-    const RowsQuad q0 = rows_quad(a, g, 0, lane);   // (the columns and regions are the same in every chunk)
-    const int rbase = q0.rbase;
-    float lo[8][2], omc[8][2];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int par = 0; par < 2; ++par) {
-            const int idx = (rbase + par) * per + min(m0 + pl0 + 4 * j, a.M - 1);
-            const float om = a.omax[idx];
-            lo[j][par] = a.c0 + (om - a.orng[idx]);
-            omc[j][par] = om + a.c0;
-        }
-    floatx4 acc[2][2];
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-            acc[mt][kt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    // the rows of a chunk: this thread's pieces of eight instances of `out` and `g` and of eight channels of the
-    // input; those of chunk s + 1 are requested as soon as chunk s has gone to LDS, in front of its matrix steps
-    float4 ov[8], gv[8], xv[8];
-    bool img_ok = false;
-    auto request = [&](int s) {
-        const RowsQuad q = rows_quad(a, g, bx * ga.pxl + s, lane);
-        img_ok = q.img_ok;
-        const size_t img = q.img_ok ? q.img : 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int m = min(m0 + pl0 + 4 * j, a.M - 1), k = min(k0 + pl0 + 4 * j, a.K - 1);
-            ov[j] = *reinterpret_cast<const float4 *>(ga.out + (img * a.M + m) * HW + q.pix0);
-            gv[j] = rows_load_g(ga, g, q, img, m);
-            xv[j] = *reinterpret_cast<const float4 *>(a.in + (img * a.K + k) * HW + q.pix0);
-        }
+    const bool want_input = g.dx != nullptr, want_offsets = g.partial != nullptr;
+    const int k0 = by * KT;
+    const int n_mg = g.n_mg, per = n_mg * GM_TM;
+    const int mg_begin = bz * g.mg_per_split, mg_end = min(n_mg, mg_begin + g.mg_per_split);
+    float *dxo = g.dx + bz * g.dx_split;
+    int pl0 = lane >> 4;
+    const RowsQuad<W2> q0(g, 0, wave * 16 + (lane & 15));   // (its columns and regions are the same in every chunk)
+    // where pixel e of the quad lies in row pl0 + 4 j
+    const int tile0 = pl0 * TP + q0.col(0);
+    auto tile_index = [&](int j, int e) { return tile0 + 4 * j * TP + (W2 ? e * 64 : (e & 1) * 64 + (e >> 1)); };
+    // Matrix operands, 16 bytes to a read: the terms of a product are added in any order both operands agree on, so lane (lr,
+    // lq) takes four columns 16 lq + 4 i ... of row lr (four steps of a contraction over columns); and a product's columns
+    // may stand for any pixels: column lr of product t is pixel 4 lr + t (the four products' operands of one row).
+    auto read4 = [&](const float *at, float (&v)[4]) {
+        const float4 f = *reinterpret_cast<const float4 *>(at);
+        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
     };
-    // chunks of this workgroup that hold pixels (uniform)
-    const int n_steps = min(ga.pxl, ga.slots_pad / 64 - bx * ga.pxl);
-    if (n_steps > 0)
-        request(0);
-    rows_ranges(a, tid, wide_sh);      // (behind the requests above: one wait for everything)
-    // Some range beyond kGradProductRange: the bound of every pixel is its own maximum over all of K (a sweep over the
-    // rows of the input per chunk, see mex_grad_input_rows_kernel); a region then keeps the product form unless a range
-    // of its offsets is beyond kGradRowsRange (or not finite) or one of its pixels spans more than kGradPixelRange
-    // (found while sweeping: `bad`, which discards the region's sums at the end).
-    const bool sweep = wide_sh[5] != 0;
-    const bool unbounded = wide_sh[wave] != 0;   // (or beyond kGradRowsRange: term by term whatever the pixels)
-    int bad = unbounded ? 1 : 0;
-    // the offset exponentials of the epilogue: requested in front of the last matrix steps
-    float eov[2][2][4];
-    for (int s = 0; s < n_steps; ++s) {
-        const bool cur_ok = img_ok;
-        float cand[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+    const float *const by_row = wt + lr * TP + wave * 64 + 16 * lq;
+    float *const by_col = wt + wave * 64 + 4 * lr;
+
+    // operands of an instance group: this thread's eight pieces of rows of `out` and `g`, its share of the four regions'
+    // offset exponentials, the next group's instance constants - requested a group ahead, while the matrix steps run
+    typedef typename RowsGrad<W2, POOLED>::type Grad;
+    float4 ov[8], en[2 * KSUB];
+    Grad gv[8];
+    float tn = 0.0f;
+    // a chunk's first image, and this lane's pixels from there on
+    const int gplane = POOLED ? g.HW >> 2 : g.HW;
+    const float *out_c, *g_c, *x_c;
+    unsigned out_at, g_at, x_at;
+    size_t first;
+    bool img_ok;
+    auto locate_chunk = [&](int chunk) {
+        const RowsQuad<W2> q(g, chunk, wave * 16 + (lane & 15));
+        const int img0 = chunk * 256 >> g.lgHW;
+        img_ok = q.img < g.B;
+        const unsigned img = img_ok ? q.img - img0 : 0;
+        first = (size_t)img0 * g.K * g.HW;
+        out_c = g.out + (size_t)img0 * g.M * g.HW;
+        g_c = g.g + (size_t)img0 * g.M * gplane;
+        x_c = g.in + first;
+        out_at = img * g.M * g.HW + q.pix0;
+        g_at = img * g.M * gplane + (POOLED ? q.window(g) : q.pix0);
+        x_at = img * g.K * g.HW + q.pix0;
+    };
+    auto request = [&](int mg) {
+        // (those past the last instance, image or patch element on a clamped address)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            if (m0 + pl0 + 4 * j >= a.M)
-                continue;
-            const float o[4] = {ov[j].x, ov[j].y, ov[j].z, ov[j].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                cand[e] = fminf(cand[e], __builtin_fmaf(o[e], a.c1, -lo[j][e & 1]));
+            const unsigned m = min(mg * GM_TM + pl0 + 4 * j, g.M - 1);
+            ov[j] = rows_load<float4>(out_c, out_at + m * g.HW);
+            gv[j] = rows_load<Grad>(g_c, g_at + m * gplane);
         }
+#pragma unroll
+        for (int j = 0; j < 2 * KSUB; ++j) {
+            const int i = tid + 256 * j;
+            const int r = i / (KT * 8), row = (i % (KT * 8)) >> 3, c4 = i & 7;
+            en[j] = rows_load<float4>(g.offe, ((r * n_mg + mg) * g.K + min(k0 + row, g.K - 1)) * GM_TM + 4 * c4);
+        }
+        tn = g.omax[(tid >> 5 & 3) * per + min(mg + 1, n_mg - 1) * GM_TM + (tid & 31)];
+    };
+    float4 xv[NJ];                     // rows of the input's tile, for 2^(xs - a)
+    auto request_input = [&]() {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            xv[j] = rows_load<float4>(x_c, x_at + (unsigned)min(k0 + pl0 + 4 * j, g.K - 1) * g.HW);
+    };
+
+    const int n_chunks = min(g.pxl, g.chunks - bx * g.pxl);
+    // (loads return in order: the small ones, which the flags wait for, in front of the rows)
+    RowsRanges ranges(g, tid);
+    const int own = (tid >> 5 & 3) * per + mg_begin * GM_TM + (tid & 31);   // (the packed arrays are padded to whole groups)
+    const float om = g.omax[own], rng = g.orng[own];
+    if (tid < 5)
+        wide_sh[tid] = 0;
+    if (tid < 4)
+        late[tid] = 0;
+    locate_chunk(bx * g.pxl);
+    request(mg_begin);
+    if (want_offsets)
+        request_input();
+    __syncthreads();
+    if (tid < 128) {
+        tab[mg_begin & 1][tid] = om + g.c0;
+        lo_tab[tid] = g.c0 + (om - rng);
+    }
+    ranges.flag(g, tid, wide_sh);
+    __syncthreads();
+    const bool roomy = wide_sh[4] != 0;
+    const int unbounded = __builtin_amdgcn_readfirstlane(wide_sh[wave]);   // this wave's region: term by term whatever its pixels
+
+    const bool nothing = (wide_sh[0] & wide_sh[1] & wide_sh[2] & wide_sh[3]) != 0;   // all four regions
+    if (nothing && tid < 4)
+        late[tid] = (1 << n_chunks) - 1;
+    for (int s = nothing ? n_chunks : 0; s < n_chunks; ++s) {
+        asm volatile("" : "+v"(pl0));   // (what follows from it is cheap to form again, and too much to keep across the chunks)
+        if (s > 0) {
+            locate_chunk(bx * g.pxl + s);
+            request(mg_begin);
+            if (want_offsets)
+                request_input();
+            if (tid < 128)
+                tab[mg_begin & 1][tid] = g.omax[(tid >> 5) * per + mg_begin * GM_TM + (tid & 31)] + g.c0;
+        }
+        // ---- the bound of every pixel: a >= every xs_k of its patch ----
+        // The minimum over a group of instances of outs_m - c0 - lo_m, see mex_grad_input_mfma_kernel.  Where some offsets
+        // range is large that is loose by up to the range, which costs the factors their precision (and, beyond
+        // kGradProductRange, the product form): there it is the pixel's own maximum over all of K, from one sweep over
+        // the rows of the input.  The exponents then stay within the pixel's patch range, and a region keeps the
+        // product form while those ranges are at most kGradPixelRange and its offsets span at most kGradRowsRange.
         float bound[4];
-        if (sweep) {
-            const RowsQuad q = rows_quad(a, g, bx * ga.pxl + s, lane);
-            const size_t img = q.img_ok ? q.img : 0;
-            float amax = -INFINITY, alo = INFINITY;
-            for (int kb = 0; kb < a.K; kb += 32) {
-                __syncthreads();       // the previous matrix steps / the previous block's readers are done with the tile
-                // (two rows at a time: the chunk's own operands stay in their registers meanwhile)
+        if (roomy) {
+            float alo[4];
 #pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    float4 xr[2];
+            for (int e = 0; e < 4; ++e) {
+                bound[e] = -INFINITY;
+                alo[e] = INFINITY;
+            }
+            for (int k = pl0; k < g.K; k += 32) {
+                float4 xr[8];
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        xr[j] = *reinterpret_cast<const float4 *>(
-                            a.in + (img * a.K + min(kb + pl0 + 4 * (2 * h + j), a.K - 1)) * HW + q.pix0);
+                for (int j = 0; j < 8; ++j)   // (behind the last: the last)
+                    xr[j] = rows_load<float4>(x_c, x_at + (unsigned)min(k + 4 * j, g.K - 1) * g.HW);
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int pl = pl0 + 4 * (2 * h + j);
-                        const bool use = q.img_ok && kb + pl < a.K;
-                        const float v[4] = {xr[j].x, xr[j].y, xr[j].z, xr[j].w};
+                for (int j = 0; j < 8; ++j) {
+                    const float v[4] = {xr[j].x, xr[j].y, xr[j].z, xr[j].w};
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            wt[pl * TP + q0.col[e]] = use ? v[e] * a.c1 : __builtin_nanf("");   // (fmax / fmin skip NaN)
+                    for (int e = 0; e < 4; ++e) {   // (fmax / fmin skip NaN)
+                        bound[e] = fmaxf(bound[e], v[e] * g.c1);
+                        alo[e] = fminf(alo[e], v[e] * g.c1);
                     }
                 }
+            }
+            if (s > 0) {               // (each chunk decides for itself; its last readers are behind a barrier)
+                if (lane == 0)
+                    wide_sh[wave] = unbounded;
                 __syncthreads();
-#pragma unroll 8
-                for (int pl = 0; pl < 32; ++pl) {
-                    const float t = wt[pl * TP + tid];
-                    amax = fmaxf(amax, t);
-                    alo = fminf(alo, t);
-                }
             }
-            const bool slot_ok = (bx * ga.pxl + s) * 64 + (tid & 63) < a.slots;
-            const bool px_ok = !slot_ok || (fabsf(amax) < INFINITY && amax - alo <= kGradPixelRange);
-            bad |= __any(!px_ok) ? 1 : 0;          // (columns of wave w belong to region w)
-            pm[tid] = slot_ok ? amax : 0.0f;
-            __syncthreads();
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                bound[e] = cur_ok ? pm[q0.col[e]] : 0.0f;
-        } else {
-            __syncthreads();           // the previous chunk's matrix steps are done with wt / ex, its readers with pm
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                pm[pl0 * 256 + q0.col[e]] = cand[e];
-            __syncthreads();
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int c = q0.col[e];
-                bound[e] = cur_ok ? fminf(fminf(pm[c], pm[256 + c]), fminf(pm[512 + c], pm[768 + c])) : 0.0f;
+                for (int d = 16; d < 64; d <<= 1) {
+                    bound[e] = fmaxf(bound[e], __shfl_xor(bound[e], d, 64));
+                    alo[e] = fminf(alo[e], __shfl_xor(alo[e], d, 64));
+                }
+                // a pixel with an infinite value, nothing finite, or a patch range beyond the bound sends its region term by term
+                if (img_ok && !(fabsf(bound[e]) < INFINITY && bound[e] - alo[e] <= kGradPixelRange))
+                    wide_sh[q0.region(e)] = 1;
             }
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int pl = pl0 + 4 * j;
-            const bool use_m = cur_ok && m0 + pl < a.M, use_k = cur_ok && k0 + pl < a.K;
-            const float o[4] = {ov[j].x, ov[j].y, ov[j].z, ov[j].w};
-            float gg[4];
-            rows_quad_g(ga, gv[j], gg);
-            const float x[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float we = __builtin_fmaf(-o[e], a.c1, bound[e]) + omc[j][e & 1];
-                wt[pl * TP + q0.col[e]] = use_m ? gg[e] * __builtin_amdgcn_exp2f(we) : 0.0f;
-                ex[pl * TP + q0.col[e]] = use_k ? __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], a.c1, -bound[e])) : 0.0f;
-            }
-        }
-        if (s + 1 < n_steps) {
-            request(s + 1);
         } else {
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int e = 0; e < 4; ++e)
+                bound[e] = INFINITY;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int m = min(m0 + mt * 16 + 4 * lq + v, a.M - 1);
-                    const float *eo = a.offe + (((size_t)wave * n_mg + m / GM_TM) * a.K) * GM_TM + m % GM_TM;
+            for (int j = 0; j < 8; ++j) {
+                const float o[4] = {ov[j].x, ov[j].y, ov[j].z, ov[j].w};
+                const bool there = mg_begin * GM_TM + pl0 + 4 * j < g.M;
 #pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-                        eov[mt][kt][v] = eo[(size_t)min(k0 + kt * 16 + lr, a.K - 1) * GM_TM];
+                for (int e = 0; e < 4; ++e) {
+                    const float b = __builtin_fmaf(o[e], g.c1, -lo_tab[q0.region(e) * 32 + pl0 + 4 * j]);
+                    bound[e] = fminf(bound[e], there ? b : INFINITY);
                 }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                for (int d = 16; d < 64; d <<= 1)
+                    bound[e] = fminf(bound[e], __shfl_xor(bound[e], d, 64));
         }
-        __syncthreads();
-        if (!unbounded) {
-#pragma unroll 4
-            for (int ps = 0; ps < 64; ps += 4) {
-                float wa[2], xb[2];
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    wa[i] = wt[(i * 16 + lr) * TP + wave * 64 + ps + lq];
-                    xb[i] = ex[(i * 16 + lr) * TP + wave * 64 + ps + lq];
+        for (int e = 0; e < 4; ++e)
+            bound[e] = img_ok ? bound[e] : 0.0f;
+
+        // ---- the patch exponentials as matrix operands: patch element 16 kt + lr, columns 16 lq + 4 i + ... of this wave's ----
+        float exr[KSUB][4][4];
+        if (want_offsets) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float x[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+                const bool use = img_ok && k0 + pl0 + 4 * j < g.K;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v = __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], g.c1, -bound[e]));
+                    wt[tile_index(j, e)] = use ? v : 0.0f;
                 }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int kt = 0; kt < KSUB; ++kt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    read4(by_row + kt * 16 * TP + 4 * i, exr[kt][i]);
+        }
+
+        floatx4 acc[KSUB][4];
+#pragma unroll
+        for (int ks = 0; ks < KSUB; ++ks)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                acc[ks][t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        int my_wide = unbounded;
+        for (int mg = mg_begin; mg < mg_end; ++mg) {
+            __syncthreads();           // everyone is done with the tile, the offset exponentials and the flags
+            const float *tb = tab[mg & 1];
+            my_wide = __builtin_amdgcn_readfirstlane(wide_sh[wave]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int pl = pl0 + 4 * j;
+                const bool use = img_ok && mg * GM_TM + pl < g.M;
+                const float o[4] = {ov[j].x, ov[j].y, ov[j].z, ov[j].w};
+                float gg[4];
+                rows_quad_g(gv[j], gg);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    // (a - outs) first: a small, once-rounded difference; the instance constant is added to that (forming
+                    // a + mo first, about the size of outs, was tried for the tight bound: worse on half of the data)
+                    const float ex = __builtin_fmaf(-o[e], g.c1, bound[e]) + tb[q0.region(e) * 32 + pl];
+                    const float w = gg[e] * __builtin_amdgcn_exp2f(ex);
+                    wt[tile_index(j, e)] = use ? w : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2 * KSUB; ++j) {
+                const int i = tid + 256 * j;
+                const int r = i / (KT * 8), row = (i % (KT * 8)) >> 3, c4 = i & 7;
+                const bool use = k0 + row < g.K;
+                *reinterpret_cast<float4 *>(eo + (r * KT + row) * EP + 4 * c4) = use ? en[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+            if (tid < 128)
+                tab[(mg + 1) & 1][tid] = tn + g.c0;
+            if (mg + 1 < mg_end)
+                request(mg + 1);
+            else if (want_input)
+                request_input();
+            __syncthreads();
+            if (want_input && !my_wide) {
+                // (lane lq: instances 8 lq + i)
+                float av[KSUB][2][4];
+#pragma unroll
+                for (int ks = 0; ks < KSUB; ++ks)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        read4(eo + (wave * KT + ks * 16 + lr) * EP + 8 * lq + 4 * h, av[ks][h]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    float bv[4];
+                    read4(by_col + (8 * lq + i) * TP, bv);
+#pragma unroll
+                    for (int ks = 0; ks < KSUB; ++ks)
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            acc[ks][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[ks][i / 4][i % 4], bv[t], acc[ks][t], 0, 0, 0);
+                }
+            }
+            if (want_offsets && !my_wide) {
+                floatx4 sum[2][KSUB];
 #pragma unroll
                 for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-                        acc[mt][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[mt], xb[kt], acc[mt][kt], 0, 0, 0);
+                    for (int kt = 0; kt < KSUB; ++kt)
+                        sum[mt][kt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float wa[2][4];
+#pragma unroll
+                    for (int mt = 0; mt < 2; ++mt)
+                        read4(by_row + mt * 16 * TP + 4 * i, wa[mt]);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+#pragma unroll
+                        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                            for (int kt = 0; kt < KSUB; ++kt)
+                                sum[mt][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(exr[kt][i][c], wa[mt][c], sum[mt][kt], 0, 0, 0);
+                }
+                // partial sums, times 2^(os_mk - mo_m): a lane's are four neighbouring patch elements of an instance
+                float *dst = g.partial + ((size_t)bx * 4 + wave) * g.M * g.K;
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                    for (int kt = 0; kt < KSUB; ++kt) {
+                        const int m = mg * GM_TM + mt * 16 + lr, k = k0 + kt * 16 + 4 * lq;
+                        const float *e = eo + (wave * KT + kt * 16 + 4 * lq) * EP + mt * 16 + lr;
+                        float add[4];
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            add[v] = sum[mt][kt][v] * e[v * EP];
+                        if (m >= g.M || k >= g.K)
+                            continue;
+                        float *at = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + 4 * ((unsigned)m * g.K + k));
+                        if ((g.K & 3) == 0) {
+                            float4 old = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                            if (s > 0)
+                                old = *reinterpret_cast<const float4 *>(at);
+                            *reinterpret_cast<float4 *>(at) = make_float4(old.x + add[0], old.y + add[1], old.z + add[2], old.w + add[3]);
+                        } else {
+#pragma unroll
+                            for (int v = 0; v < 4; ++v)
+                                if (k + v < g.K)
+                                    at[v] = s > 0 ? at[v] + add[v] : add[v];
+                        }
+                    }
             }
         }
-    }
-    // ---- partial sums of this chunk group: acc * 2^(os_mk - mo_m) ----
-    if (sweep) {
-        __syncthreads();               // (everyone has read the flags)
-        if (lane == 0)
-            wide_sh[wave] = bad;
-        __syncthreads();
-    }
-    const bool my_wide = wide_sh[wave] != 0;
-    const bool any_wide = (wide_sh[0] | wide_sh[1] | wide_sh[2] | wide_sh[3]) != 0;
-    if (!my_wide) {
-        float *dst = ga.partial + ((size_t)bx * a.R + wave) * a.M * a.K;
+        if (my_wide && lane == 0)
+            late[wave] |= 1 << s;
+
+        // ---- d patch_k = 2^(xs_k - a) * acc: through the tile [patch element][column] to rows of the gradient ----
+        __syncthreads();               // the last matrix steps are done with the tile and the tables
+        if (want_input) {
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+            for (int ks = 0; ks < KSUB; ++ks)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = m0 + mt * 16 + 4 * lq + v;
-                if (m >= a.M)
+                for (int v = 0; v < 4; ++v)
+                    *reinterpret_cast<float4 *>(by_col + (ks * 16 + 4 * lq + v) * TP) =
+                        make_float4(acc[ks][0][v], acc[ks][1][v], acc[ks][2][v], acc[ks][3][v]);
+            __syncthreads();
+            const bool any_wide = (wide_sh[0] | wide_sh[1] | wide_sh[2] | wide_sh[3]) != 0;
+            float *dst = dxo + first;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int k = k0 + pl0 + 4 * j;
+                if (!img_ok || k >= g.K)
                     continue;
+                const float x[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+                float d[4];
 #pragma unroll
-                for (int kt = 0; kt < 2; ++kt) {
-                    const int k = k0 + kt * 16 + lr;
-                    if (k < a.K)
-                        dst[(size_t)m * a.K + k] = acc[mt][kt][v] * eov[mt][kt][v];
+                for (int e = 0; e < 4; ++e)
+                    d[e] = wt[tile_index(j, e)] * __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], g.c1, -bound[e]));
+                float *to = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + 4 * (x_at + (unsigned)k * g.HW));
+                if (!any_wide) {
+                    *reinterpret_cast<float4 *>(to) = make_float4(d[0], d[1], d[2], d[3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (!wide_sh[q0.region(e)])
+                            to[e] = d[e];
                 }
             }
-    }
-    if (any_wide) {
-        // the regions with a wide offsets range, term by term: this workgroup's tile as GO_MT x GO_KT wave tiles
-        constexpr int NU = (32 / GO_MT) * (32 / GO_KT);
-        for (int u = wave; u < 4 * NU; u += 4) {
-            const int r = u / NU, i = u % NU;
-            const int mm0 = m0 + (i / (32 / GO_KT)) * GO_MT, kk0 = k0 + (i % (32 / GO_KT)) * GO_KT;
-            if (wide_sh[r] && mm0 < a.M && kk0 < a.K)
-                mex_grad_offsets_wave(ga, r, bx, mm0, kk0, lane);
+            __syncthreads();           // everyone is done with the tile and the flags
         }
     }
+    __syncthreads();
+#if defined(__HIP_DEVICE_COMPILE__)
+    if ((late[0] | late[1] | late[2] | late[3]) != 0)
+        rows_terms<KT>(bx, n_chunks, k0, mg_begin, mg_end, want_input ? dxo : nullptr, want_offsets,
+                       make_int4(late[0], late[1], late[2], late[3]));
+#endif
 }
 
 // dOff[r,m,k] = sum over pixel chunks, in a fixed order (reproducible): a workgroup takes 32 consecutive elements,
@@ -1796,6 +1772,77 @@ __global__ __launch_bounds__(256) void mex_grad_offsets_finish_wide_rows_kernel(
         gr[k] -= expf(nr[k]) * sum;   // reads back what this thread stored above
 }
 
+// What is left after mex_grads_rows_kernel, in one launch: the first `rows` workgroups take a row of the offsets gradient each
+// (K a multiple of 4, at most kFinishRowsMaxK), the others the sums of the input gradient's splits (mex_sum_splits4_kernel).
+// K / 4 threads hold four elements of the row each, 1024 / K groups of them every so many chunks; the groups' sums are
+// added in order, then the chain rule through the normalisation, if `normalized` is given.  Eight chunks are requested at
+// a time.  512 images, 64 channels of 8 x 8, 128 instances, two splits: 10.4 us in two launches, 8.2 in one; 32 channels of 16 x
+// 16, 512 partial sums of 256 rows: 9.4 us with a wave to a row, 5.6.
+__global__ __launch_bounds__(256) void mex_grads_finish_kernel(const float *__restrict__ partial, long long n, int chunks,
+                                                              int rows, int K, const float *__restrict__ normalized,
+                                                              float *__restrict__ doff, const float4 *__restrict__ parts,
+                                                              long long n4, int splits, float4 *__restrict__ dx)
+{
+    __shared__ __attribute__((aligned(16))) float4 sm[256];
+    __shared__ float wave_sum[4];
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= rows) {
+        sum_splits4(parts, n4, splits, dx, (long long)(blockIdx.x - rows) * 256 + tid);
+        return;
+    }
+    const int row = blockIdx.x, Kq = K >> 2, G = 256 / Kq;
+    const int grp = tid / Kq, q = tid - grp * Kq;
+    const bool first = grp == 0;
+    float nv[4];
+    if (normalized != nullptr)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            nv[e] = normalized[(size_t)row * K + 4 * q + e];
+    float4 t = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (grp < G) {
+        const float4 *src = reinterpret_cast<const float4 *>(partial + (size_t)row * K) + q;
+        for (int c0 = grp; c0 < chunks; c0 += 8 * G) {
+            float4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)   // (behind the last: this group's first)
+                v[u] = src[(size_t)(c0 + u * G < chunks ? c0 + u * G : grp) * (n >> 2)];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (c0 + u * G < chunks) {
+                    t.x += v[u].x; t.y += v[u].y; t.z += v[u].z; t.w += v[u].w;
+                }
+        }
+    }
+    sm[tid] = t;
+    __syncthreads();
+    float sum = 0.0f;
+    if (first) {
+        for (int j = 1; j < min(G, chunks); ++j) {
+            const float4 v = sm[j * Kq + q];
+            t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+        }
+        sum = (t.x + t.y) + (t.z + t.w);
+    }
+    float v[4] = {t.x, t.y, t.z, t.w};
+    if (normalized != nullptr) {
+        for (int d = 32; d > 0; d >>= 1)
+            sum += __shfl_xor(sum, d, 64);
+        if ((tid & 63) == 0)
+            wave_sum[tid >> 6] = sum;
+        __syncthreads();
+        sum = (wave_sum[0] + wave_sum[1]) + (wave_sum[2] + wave_sum[3]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] -= expf(nv[e]) * sum;
+    }
+    if (!first)
+        return;
+    float *dst = doff + (size_t)row * K + 4 * q;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        dst[e] = v[e];
+}
+
 // Few instances over long patches on few pixels (a network's classifier head: 10 instances x 512 channels on one
 // pixel per image): the tiled kernels above would run a handful of workgroups in long serial chains, in three
 // launches.  Here a thread owns one patch element k (a workgroup spans K) and keeps the region's offsets for that
@@ -1907,10 +1954,10 @@ struct MexGradTiling {
     bool factors_input, factors_offsets;
     int slots_pad, Mp, Kp;
     size_t factor_bytes;
-    // the row-wise kernels (mex_grad_input_rows_kernel, mex_grad_offsets_rows_kernel): the layer qualifies (the
-    // pointers are checked at the launch), and their tiling
+    // the row-wise kernel (mex_grads_rows_kernel): the layer qualifies (the pointers are checked at the launch), and its
+    // tiling
     bool rows;
-    int rows_ksub;                        // input gradient: 16 * ksub patch elements per workgroup
+    int rows_ksub;                        // 16 * ksub patch elements per workgroup
     int rows_msplit, rows_mg_per_split;   // ... and the split of its instance groups
     int rows_pxl, rows_cpr;               // offsets gradient: chunks per workgroup, workgroups along the pixels
 };
@@ -1933,8 +1980,11 @@ bool rows_geometry(const MexPlan &p)
     return std::isfinite(p.epsilon) && p.use_unshared && d.offsets_c == 1 && d.offsets_h == 2 && d.offsets_w == 2 &&
            d.channels_out == 1 && d.block_c == p.C && d.block_h == 1 && d.block_w == 1 && d.stride_h == 1 &&
            d.stride_w == 1 && d.pad_c == 0 && d.pad_h == 0 && d.pad_w == 0 && d.height_out == p.H &&
-           d.width_out == p.W && log2_exact(p.H) >= 1 && log2_exact(p.W) >= 2 && p.W <= 128 &&
-           d.region_size == (p.H / 2) * (p.W / 2) && (long long)p.B * p.H * p.W <= 0x3fffffffLL;
+           d.width_out == p.W && log2_exact(p.H) >= 1 && log2_exact(p.W) >= 1 && p.W <= 128 &&
+           d.region_size == (p.H / 2) * (p.W / 2) && (long long)p.B * p.H * p.W <= 0x3fffffffLL &&
+           // (32-bit offsets in bytes: of an image or a chunk's images, and of the packed offsets)
+           std::max<long long>(256, 1LL * p.H * p.W) * std::max<long long>(d.M, d.K) < (1LL << 29) &&
+           4LL * (d.M + GM_TM - 1) / GM_TM * GM_TM * d.K < (1LL << 29);
 }
 
 MexGradTiling mex_grad_tiling(const MexPlan &p)
@@ -1996,20 +2046,21 @@ MexGradTiling mex_grad_tiling(const MexPlan &p)
     t.rows_ksub = 1; t.rows_msplit = 1; t.rows_mg_per_split = n_mg; t.rows_pxl = 1; t.rows_cpr = 0;
     if (t.rows) {
         const long long chunks = t.slots_pad / 64;
-        auto ktiles = [&](int ksub) { return (long long)((d.K + 16 * ksub - 1) / (16 * ksub)); };
-        t.rows_ksub = std::min(4, (d.K + 15) / 16);
-        if (t.rows_ksub == 3)
-            t.rows_ksub = 4;
-        while (t.rows_ksub > 1 && chunks * ktiles(t.rows_ksub) < 512)
-            t.rows_ksub >>= 1;
-        const long long wgs_in = chunks * ktiles(t.rows_ksub);
-        if (wgs_in < 512 && n_mg >= 4)
-            t.rows_msplit = (int)std::max<long long>(1, std::min<long long>(std::min(8, n_mg / 2), 512 / std::max<long long>(wgs_in, 1)));
+        // 32 patch elements to a workgroup, or 16 if 32 leave the chip short of two workgroups to a compute unit and 16 leave
+        // it less so, whatever the split of the instance groups, or if 32 need a split where 16 do not (512 images, 64 channels of 8 x 8, 128
+        // instances: 27.4 + 8.2 us with two splits and their sums, 28.0 + 5.1 without)
+        auto split_of = [&](long long wgs) {
+            return wgs >= 512 || n_mg < 4 ? 1LL : std::max<long long>(1, std::min<long long>(std::min(8, n_mg / 2), 512 / std::max<long long>(wgs, 1)));
+        };
+        const long long wide = chunks * ((d.K + 31) / 32), narrow = chunks * ((d.K + 15) / 16);
+        const long long wide_wgs = wide * split_of(wide);
+        t.rows_ksub = d.K <= 16 || (wide_wgs < 512 && narrow * split_of(narrow) > wide_wgs) || (wide < 512 && narrow >= 512) ? 1 : 2;
+        const long long tiles = (d.K + 16 * t.rows_ksub - 1) / (16 * t.rows_ksub);
+        t.rows_msplit = (int)split_of(chunks * tiles);
         t.rows_mg_per_split = (n_mg + t.rows_msplit - 1) / t.rows_msplit;
         t.rows_msplit = (n_mg + t.rows_mg_per_split - 1) / t.rows_mg_per_split;
         if (t.rows_msplit > 1)
             t.split_bytes = std::max(t.split_bytes, align_up((size_t)t.rows_msplit * p.B * p.C * p.H * p.W * sizeof(float), 256));
-        const long long tiles = (long long)((d.M + 31) / 32) * ((d.K + 31) / 32);
         t.rows_pxl = 16;
         while (t.rows_pxl > 1 && (chunks + t.rows_pxl - 1) / t.rows_pxl * tiles < 512)
             t.rows_pxl >>= 1;
@@ -2247,12 +2298,63 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
                 return rc;
         }
     }
-    RowsArgs rg;
-    rg.lgW = log2_exact(p.W); rg.Ws = p.W / 2; rg.RS = d.region_size; rg.HW = p.H * p.W; rg.lgHW = log2_exact(rg.HW);
-    if (use_rows)
-        ga.slots_pad = t.slots_pad;
+    if (use_rows) {
+        RowsArgs rg;
+        rg.in = input; rg.out = output; rg.g = output_grad;
+        rg.offe = ga.k.offe; rg.omax = ga.k.omax; rg.orng = ga.k.orng;
+        rg.dx = !want_input ? nullptr : t.rows_msplit > 1 ? ga.dx_splits : input_grad;
+        rg.dx_split = n_in;
+        rg.partial = want_offsets ? ga.partial : nullptr;
+        rg.c0 = ga.k.c0; rg.c1 = ga.k.c1;
+        rg.B = p.B; rg.M = d.M; rg.K = d.K; rg.n_mg = (d.M + GM_TM - 1) / GM_TM; rg.mg_per_split = t.rows_mg_per_split;
+        rg.lgW = log2_exact(p.W); rg.Ws = p.W / 2; rg.RS = d.region_size; rg.HW = p.H * p.W; rg.lgHW = log2_exact(rg.HW);
+        rg.chunks = t.slots_pad / 64; rg.pxl = t.rows_pxl;
+        rg.nx = t.rows_cpr; rg.ty = (d.K + 16 * t.rows_ksub - 1) / (16 * t.rows_ksub); rg.tz = t.rows_msplit;
+        rg.d_tiles = make_fast_div((unsigned)(rg.ty * rg.tz)); rg.d_ty = make_fast_div((unsigned)rg.ty);
+        MexGradArgs gr = ga;   // for the term-by-term path
+        gr.wbuf = gr.exbuf = nullptr;
+        gr.pxl = t.rows_pxl; gr.cpr = t.rows_cpr; gr.slots_pad = t.slots_pad;
+        const long long per_die = (1LL * rg.nx * rg.ty * rg.tz + 7) / 8, wgs = 8 * per_die;
+        if (wgs > 0x7fffffffLL)
+            return SIMNETS_ERR_TOO_LARGE;
+        rg.per_die = (int)per_die;
+        const dim3 grid((unsigned)wgs);
+#define SIMNETS_ROWS_LAUNCH(KSUB, W2)                                                                            \
+    if (grad_is_pooled)                                                                                          \
+        hipLaunchKernelGGL((mex_grads_rows_kernel<KSUB, W2, true>), grid, dim3(256), 0, s, rg, gr);              \
+    else                                                                                                         \
+        hipLaunchKernelGGL((mex_grads_rows_kernel<KSUB, W2, false>), grid, dim3(256), 0, s, rg, gr)
+        if (t.rows_ksub == 2 && p.W > 2) {
+            SIMNETS_ROWS_LAUNCH(2, false);
+        } else if (t.rows_ksub == 2) {
+            SIMNETS_ROWS_LAUNCH(2, true);
+        } else if (p.W > 2) {
+            SIMNETS_ROWS_LAUNCH(1, false);
+        } else {
+            SIMNETS_ROWS_LAUNCH(1, true);
+        }
+#undef SIMNETS_ROWS_LAUNCH
+        if (hipGetLastError() != hipSuccess)
+            return SIMNETS_ERR_HIP;
+        // sums of the splits and of the chunks, in one launch if both are there to do (n_in is a multiple of 4: whole planes
+        // of at least four pixels)
+        const long long rows = (long long)d.num_regions * d.M, n4 = want_input && t.rows_msplit > 1 ? n_in / 4 : 0;
+        const long long wgs_sum = (n4 + 255) / 256;
+        if (want_offsets && d.K % 4 == 0 && d.K <= kFinishRowsMaxK && rows + wgs_sum <= 0x7fffffffLL) {
+            hipLaunchKernelGGL(mex_grads_finish_kernel, dim3((unsigned)(rows + wgs_sum)), dim3(256), 0, s, ga.partial, n_off,
+                               t.rows_cpr, (int)rows, d.K, p.normalize_offsets ? ga.off : nullptr, offsets_grad,
+                               reinterpret_cast<const float4 *>(ga.dx_splits), n4, t.rows_msplit,
+                               reinterpret_cast<float4 *>(input_grad));
+            return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
+        }
+        if (n4 > 0) {
+            launch_sum_splits(ga.dx_splits, n_in, t.rows_msplit, input_grad, s);
+            if (hipGetLastError() != hipSuccess)
+                return SIMNETS_ERR_HIP;
+        }
+    }
 
-    if (want_input) {
+    if (want_input && !use_rows) {
         MexGradArgs gi = ga;
         gi.overlap = t.overlap ? 1 : 0;
         gi.msplit = t.msplit; gi.mg_per_split = t.mg_per_split;
@@ -2269,29 +2371,7 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
                 return SIMNETS_ERR_HIP;
         }
         const long long gx = (long long)d.num_regions * gi.cpr;
-        if (use_rows) {
-            gi.wbuf = gi.exbuf = nullptr;
-            gi.msplit = t.rows_msplit; gi.mg_per_split = t.rows_mg_per_split;
-            const int kt = 16 * t.rows_ksub, gy = (d.K + kt - 1) / kt;
-            if (gy > 65535)
-                return SIMNETS_ERR_TOO_LARGE;
-            rg.nx = t.slots_pad / 64; rg.ty = gy; rg.tz = t.rows_msplit;
-            const long long wgs = (long long)((rg.nx + 7) / 8 * 8) * gy * t.rows_msplit;
-            if (wgs > 0x7fffffffLL)
-                return SIMNETS_ERR_TOO_LARGE;
-            const dim3 grid((unsigned)wgs);
-            if (t.rows_ksub == 4)
-                hipLaunchKernelGGL(mex_grad_input_rows_kernel<4>, grid, dim3(256), 0, s, gi, rg);
-            else if (t.rows_ksub == 2)
-                hipLaunchKernelGGL(mex_grad_input_rows_kernel<2>, grid, dim3(256), 0, s, gi, rg);
-            else
-                hipLaunchKernelGGL(mex_grad_input_rows_kernel<1>, grid, dim3(256), 0, s, gi, rg);
-            if (t.rows_msplit > 1) {
-                if (hipGetLastError() != hipSuccess)
-                    return SIMNETS_ERR_HIP;
-                launch_sum_splits(gi.dx_splits, n_in, t.rows_msplit, input_grad, s);
-            }
-        } else if (t.mfma) {
+        if (t.mfma) {
             const int gy = (d.K + GM_KT - 1) / GM_KT;
             if (gx > 0x7fffffffLL || gy > 65535)
                 return SIMNETS_ERR_TOO_LARGE;
@@ -2330,17 +2410,7 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
             go.wbuf = go.exbuf = nullptr;
         const long long gx = (long long)d.num_regions * go.cpr;
         if (use_rows) {
-            go.wbuf = go.exbuf = nullptr;
-            go.pxl = t.rows_pxl;
-            go.cpr = t.rows_cpr;
-            const int gy = (d.M + 31) / 32, gz = (d.K + 31) / 32;
-            if (gy > 65535 || gz > 65535)
-                return SIMNETS_ERR_TOO_LARGE;
-            rg.nx = t.rows_cpr; rg.ty = gy; rg.tz = gz;
-            const long long wgs = (long long)((rg.nx + 7) / 8 * 8) * gy * gz;
-            if (wgs > 0x7fffffffLL)
-                return SIMNETS_ERR_TOO_LARGE;
-            hipLaunchKernelGGL(mex_grad_offsets_rows_kernel, dim3((unsigned)wgs), dim3(256), 0, s, go, rg);
+            go.cpr = t.rows_cpr;   // (launched above)
         } else if (t.mfma) {
             const int gy = (d.M + GOM_MT - 1) / GOM_MT, gz = (d.K + GOM_KT - 1) / GOM_KT;
             if (gx > 0x7fffffffLL || gy > 65535 || gz > 65535)
