@@ -11,8 +11,8 @@
 // A workgroup takes 64 patch elements x up to 128 templates over a share of the pixels; its partial sums go to the
 // workspace and are added in order by the finish kernel.
 //
-// Measured (32 x 128 x 28 x 28, 128 templates, 3 x 3): 207 us on the fp32 matrix instructions -> 86 us + 16 us of packing,
-// 1.04 PFLOP/s of matrix products; the finish kernel 20 -> 13 us with 28 shares of the pixels for 170.  Error against 64
+// Measured (32 x 128 x 28 x 28, 128 templates, 3 x 3): 207 us on the fp32 matrix instructions -> 86 us + 10 us of packing,
+// 1.04 PFLOP/s of matrix products; the finish kernel 20 -> 9 us with 28 shares of the pixels for 170.  Error against 64
 // bits 2.5e-7 -> 2.0e-7 (templates) and 1.9e-7 (weights) of the gradient's 2-norm; with one set of accumulators 2.9e-7.
 //
 // LDS pitches are chosen so that slot = patch element modulo 8: the eight lanes that read together hit different banks.
@@ -34,6 +34,7 @@ constexpr int kThreads = 256;
 constexpr int kSlots = 816;          // 16-byte slots of one piece; the last holds zeros
 constexpr int kColumns = 64;         // patch elements of a workgroup
 constexpr int kImages = 8;           // images of a matrix operand
+constexpr int kPackRows = 8, kPackGroups = kSplitRows / kPackRows;   // templates of a workgroup that packs g
 
 struct ParamsArgs {
     const float *g, *x, *templates;
@@ -117,21 +118,24 @@ __device__ __forceinline__ void params_channel_block(const ParamsArgs &a, int c)
     }
 }
 
-// The first C blocks: params_channel_block.  The S n_mtiles behind: g of one share of the pixels and one template tile, a
-// thread one template's pairs of pixels (eight neighbouring threads read 64 contiguous bytes), and the share's sums G.
+// The first C blocks: params_channel_block.  The 4 S n_mtiles behind: g of one share of the pixels and eight templates, a
+// thread one template's pairs of pixels (eight neighbouring lanes read 64 contiguous bytes, a wave writes whole lines of
+// 128), and the share's sums G.  32 x 128 x 28 x 28, 128 templates, 3 x 3 (32 MB to move): with 32 templates to a workgroup, 112
+// of them, 17.7 us, so 10.5.
 __global__ __launch_bounds__(kThreads) void sim_split_params_pack_kernel(const ParamsArgs a)
 {
     if ((int)blockIdx.x < a.C) {
         params_channel_block(a, blockIdx.x);
         return;
     }
-    const int tid = threadIdx.x, block = blockIdx.x - a.C;
+    __shared__ float wave_sum[kThreads / 64][kPackRows];
+    const int tid = threadIdx.x, lane = tid & 63, block = (blockIdx.x - a.C) / kPackGroups;
     const int mtile = block / a.S, s = block - mtile * a.S;
-    const int row = tid >> 3, o = mtile * kSplitRows + row;
+    const int row = (blockIdx.x - a.C) % kPackGroups * kPackRows + (lane >> 3), o = mtile * kSplitRows + row;
     const int q0 = first_unit(a, s) * a.pairs, q1 = first_unit(a, s + 1) * a.pairs;
     const size_t npix = (size_t)a.oh * a.ow;
     float sum = 0.0f;
-    for (int q = q0 + (tid & 7); q < q1; q += 8) {
+    for (int q = q0 + (tid >> 6) * 8 + (lane & 7); q < q1; q += kThreads / 8) {
         const int u = (int)fast_div((unsigned)q, a.d_pairs), pp = q - u * a.pairs;
         const Unit un = unit_of(a, u);
         const int py = (int)fast_div((unsigned)pp, a.d_tw2);
@@ -167,8 +171,12 @@ __global__ __launch_bounds__(kThreads) void sim_split_params_pack_kernel(const P
     }
     for (int d = 4; d > 0; d >>= 1)
         sum += __shfl_xor(sum, d, 8);
-    if ((tid & 7) == 0 && o < a.O)
-        a.partial[((size_t)2 * a.S + s) * a.Opad * a.Kpad + (size_t)o * a.Kpad] = sum;
+    if ((lane & 7) == 0)
+        wave_sum[tid >> 6][lane >> 3] = sum;
+    __syncthreads();
+    if (tid < 64 && (lane & 7) == 0 && o < a.O)
+        a.partial[((size_t)2 * a.S + s) * a.Opad * a.Kpad + (size_t)o * a.Kpad] =
+            (wave_sum[0][lane >> 3] + wave_sum[1][lane >> 3]) + (wave_sum[2][lane >> 3] + wave_sum[3][lane >> 3]);
 }
 
 // This share's sums of one patch element k and a lane's sixteen templates; with the first share what was subtracted.
@@ -563,7 +571,7 @@ int sim_split_params_launch(const SimPlan &p, const SplitParamsPlan &sp, const f
     a.d_chan = make_fast_div((unsigned)sp.chan);
     a.d_pitch = make_fast_div((unsigned)sp.pitch);
     a.d_taps = make_fast_div((unsigned)a.taps);
-    hipLaunchKernelGGL(sim_split_params_pack_kernel, dim3(p.C + sp.S * sp.n_mtiles), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL(sim_split_params_pack_kernel, dim3(p.C + sp.S * sp.n_mtiles * kPackGroups), dim3(kThreads), 0, s, a);
     hipLaunchKernelGGL(sim_split_params_kernel, dim3(sp.S, sp.k_groups, sp.m_groups), dim3(kThreads), 0, s, a);
     return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
 }
