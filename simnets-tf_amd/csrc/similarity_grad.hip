@@ -809,6 +809,7 @@ struct GradPArgs {
     int n_ktiles, n_tiles;
     long long npix;    // B*oh*ow
     int nchunks, cps;  // pixel chunks in total, and per split
+    int seg;           // chunks whose terms are added up in one go (vector forms)
     int S;
     float oob;
     FastDiv d_ow, d_ohow;
@@ -1201,6 +1202,48 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
         nan_chunk = __syncthreads_or(nan_chunk);
     else
         __syncthreads();
+    // partial sums of this split
+    const size_t slab = (size_t)a.Opad * a.Kpad;
+    float *pt = a.partial + (size_t)split * slab;
+    float *pw = a.partial + ((size_t)a.S + split) * slab;
+    float *pn = a.partial + ((size_t)2 * a.S + split) * slab;
+    // Vector forms: a segment's chunks one after the other, whose sums are added to those of the segments before it.  (A sum of
+    // all the chunks' terms in turn loses more: 32 x 64 x 32 x 32, 128 templates, L1, 19 chunks of 32 pixels 4.6e-7 of the
+    // gradient, 10 and 9 3.3e-7.)
+    bool first = true;
+    auto store_sums = [&]() {
+        auto add = [&](float *to, float (&v)[LK], float scale) {
+            float4 sum = make_float4(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
+            if (!first) {
+                const float4 before = *reinterpret_cast<const float4 *>(to);
+                sum.x += before.x; sum.y += before.y; sum.z += before.z; sum.w += before.w;
+            }
+            *reinterpret_cast<float4 *>(to) = sum;
+#pragma unroll
+            for (int i = 0; i < LK; ++i)
+                v[i] = 0.0f;
+        };
+        unsigned at0 = (unsigned)lane_o(0) * a.Kpad + k0;
+        asm volatile("" : "+v"(at0));        // (the addresses are formed here, and not kept across the loop)
+#pragma unroll
+        for (int oo = 0; oo < LO; ++oo) {
+            const size_t o = (size_t)at0 + (size_t)(lane_o(oo) - lane_o(0)) * a.Kpad;
+            constexpr float kT = SGN ? 0x1p32f : 1.0f, kW = SGN ? 0x1p-32f : 1.0f;
+            add(pt + o, at[oo], kT);
+            add(pw + o, aw[oo], kW);
+            if constexpr (IGN || (NORM && !MOM))
+                add(pn + o, an[oo], 1.0f);
+            if constexpr (MOM2) {
+                if (split == 0)
+                    *reinterpret_cast<float4 *>(a.partial + (size_t)3 * a.S * slab + o) =
+                        make_float4(ctr[0], ctr[1], ctr[2], ctr[3]);
+            }
+        }
+        first = false;
+    };
+    int seg_end = min(chunk_begin + a.seg, chunk_end);
+    if (!MF && chunk_begin >= chunk_end)
+        store_sums();   // (zeros)
     for (int chunk = chunk_begin; chunk < chunk_end && !ROW; ++chunk) {
         const int buf = (chunk - chunk_begin) & 1;
         const bool more = chunk + 1 < chunk_end;
@@ -1339,13 +1382,12 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
             nan_chunk = __syncthreads_or(more && has_nan(xv));
         else
             __syncthreads();
+        if (!MF && chunk + 1 == seg_end) {
+            store_sums();
+            seg_end = min(seg_end + a.seg, chunk_end);
+        }
     }
 
-    // partial sums of this split
-    const size_t slab = (size_t)a.Opad * a.Kpad;
-    float *pt = a.partial + (size_t)split * slab;
-    float *pw = a.partial + ((size_t)a.S + split) * slab;
-    float *pn = a.partial + ((size_t)2 * a.S + split) * slab;
     if constexpr (MF) {
         // tile i, register v: template row 8 (v / 4) + 4 * parity + v % 4, column mcol
 #pragma unroll
@@ -1363,20 +1405,6 @@ __global__ __launch_bounds__(kThreads, 2) void sim_grad_params_kernel(const Grad
                 if (split == 0)
                     a.partial[(size_t)3 * a.S * slab + o] = mctr;
             }
-    }
-#pragma unroll
-    for (int oo = 0; oo < LO && !MF; ++oo) {
-        const size_t o = (size_t)lane_o(oo) * a.Kpad + k0;
-        constexpr float kT = SGN ? 0x1p32f : 1.0f, kW = SGN ? 0x1p-32f : 1.0f;
-        *reinterpret_cast<float4 *>(pt + o) = make_float4(at[oo][0] * kT, at[oo][1] * kT, at[oo][2] * kT, at[oo][3] * kT);
-        *reinterpret_cast<float4 *>(pw + o) = make_float4(aw[oo][0] * kW, aw[oo][1] * kW, aw[oo][2] * kW, aw[oo][3] * kW);
-        if constexpr (IGN || (NORM && !MOM))
-            *reinterpret_cast<float4 *>(pn + o) = make_float4(an[oo][0], an[oo][1], an[oo][2], an[oo][3]);
-        if constexpr (MOM2) {
-            if (split == 0)
-                *reinterpret_cast<float4 *>(a.partial + (size_t)3 * a.S * slab + o) =
-                    make_float4(ctr[0], ctr[1], ctr[2], ctr[3]);
-        }
     }
     if constexpr (MOM2 && !IGN && !ROW) {
         // pixel slots -> one sum per template, in slot order; the finish kernel reads patch-element tile 0's copy
@@ -1677,7 +1705,7 @@ __global__ __launch_bounds__(256) void sim_grad_params_finish_kernel(
 }
 
 struct GpTiling {
-    int WO, OWG, KWG, n_otiles, n_ktiles, Opad, Kpad, nchunks, cps, S, nacc;
+    int WO, OWG, KWG, n_otiles, n_ktiles, Opad, Kpad, nchunks, cps, seg, S, nacc;
     bool small;   // few templates over short patches: sim_grad_params_small_kernel (cps: pixels per split)
     bool fast;    // unless the caller asked for the term-by-term arithmetic (algo DIRECT): moment form (L2 modes),
                   // scaled-sign form (L1)
@@ -1710,6 +1738,28 @@ GpTiling gp_tiling(const SimPlan &p)
     if (t.nchunks >= 8 && t.nchunks / 8 >= 512 / tiles)
         S = std::min(S, t.nchunks / 8);
     S = std::max(S, 1);
+    t.seg = std::max(1, (t.nchunks + S - 1) / S);
+    if (!t.moment && t.nchunks >= 64) {
+        // Vector forms: a split's tiles run on one of the eight dies, 64 workgroups to a die at a time, and the last round of
+        // them takes as long as a full one: of one to four rounds the number that costs least, in chunks of some 10
+        // us.  A workgroup's prologue and epilogue take 0.6, storing and adding up 10^6 floats of a moment 0.33, and a
+        // segment more 0.7: the sums are no longer than above (seg).  Forward and gradients, L1, 3 x 3, before and with
+        // the choice: 32 x 64 x 32 x 32 -> 128 580, 566 us, 64 x 16 x 40 x 40 -> 32 341, 310; 5 x 5: 32 x 64 x 32 x 32 -> 64
+        // 1007, 907, 200 x 48 x 9 x 9 -> 48 478, 406.
+        double best = 0;
+        for (int rounds = 1; rounds <= 4; ++rounds) {
+            const int most = std::min(8 * (64 * rounds / tiles), t.nchunks);
+            if (most < 8)
+                continue;
+            const int cps = (t.nchunks + most - 1) / most, splits = (t.nchunks + cps - 1) / cps;
+            const int used = ((splits + 7) / 8 * tiles + 63) / 64, segments = (cps + t.seg - 1) / t.seg;
+            const double cost = used * (cps + 0.6 + 0.7 * (segments - 1)) + 0.33e-6 * splits * t.Opad * t.Kpad;
+            if (best == 0 || cost < best) {
+                best = cost;
+                S = splits;
+            }
+        }
+    }
     t.cps = (t.nchunks + S - 1) / S;
     t.S = t.cps > 0 ? (t.nchunks + t.cps - 1) / t.cps : 1;
     if (t.S < 8) {
@@ -1721,6 +1771,8 @@ GpTiling gp_tiling(const SimPlan &p)
         t.S = s2;
         t.cps = (std::max(t.nchunks, 1) + s2 - 1) / s2;
     }
+    const int segments = std::max(1, (t.cps + t.seg - 1) / t.seg);
+    t.seg = std::max(1, (t.cps + segments - 1) / segments);
     t.nacc = (t.moment || p.mode == SIM_MODE_L2_NORM || p.mode == SIM_MODE_L2_NORM_IGNORE_NAN) ? 3 : 2;
     t.small = t.moment && p.K >= 1 && p.K <= 9 && p.O <= 4 * (32 / p.K) && npix < 0x7fffffffLL;
     if (t.small) {
@@ -1853,7 +1905,7 @@ int sim_grad_params(const SimPlan &p, const float *input, const float *templates
     a.bh = p.bh; a.bw = p.bw; a.sh = p.sh; a.sw = p.sw; a.ph = p.ph; a.pw = p.pw; a.K = p.K;
     a.Opad = t.Opad; a.Kpad = t.Kpad; a.n_ktiles = t.n_ktiles; a.n_tiles = t.n_otiles * t.n_ktiles;
     a.npix = (long long)p.B * p.oh * p.ow;
-    a.nchunks = t.nchunks; a.cps = t.cps; a.S = t.S;
+    a.nchunks = t.nchunks; a.cps = t.cps; a.seg = t.seg; a.S = t.S;
     a.oob = p.oob;
     a.d_ow = make_fast_div((unsigned)p.ow);
     a.d_ohow = make_fast_div((unsigned)(p.oh * p.ow));
