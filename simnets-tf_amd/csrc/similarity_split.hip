@@ -1123,6 +1123,7 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     a.pieces = sp.pieces; a.n_mtiles = sp.n_mtiles; a.mode = p.mode; a.fudge = p.fudge;
     a.line = split_line(p.K);
     a.d_taps = make_fast_div((unsigned)a.taps);
+    a.d_K = make_fast_div((unsigned)a.K);
     a.d_steps = make_fast_div((unsigned)std::max(1, sp.steps));
     a.norm_const = p.mode == SIM_MODE_L2_NORM ? split_norm_const(p.K) : 0.0f;
     a.pack_blocks = sp.on ? sp.chunks * sp.n_mtiles * ((sp.steps + 3) / 4) : 0;
