@@ -296,146 +296,218 @@ __device__ __forceinline__ void split_recompute(lds_char *lds, int ptile, int mt
 }
 #endif
 
-// Input gradient.  One workgroup: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template tile x NI pixel tiles.
-template <int CG, int G>
-__device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, int mtile0, int flag)
+// How a workgroup's pixels, 128 from n0 on, lie in the stack of padded images: the virtual row of the first, and what is
+// staged for them.
+__device__ __forceinline__ int split_virtual_row(const SplitArgs &a, int n, int &img, int &c)
+{
+    img = (int)fast_div((unsigned)n, a.d_npix);
+    const int rem = n - img * a.npix, r = (int)fast_div((unsigned)rem, a.d_ow);
+    c = rem - r * a.ow;
+    return img * a.Hv + r * a.sh;
+}
+
+// Input gradient.  One workgroup of WAVES waves: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template
+// tile x NI pixel tiles.  Four waves, two workgroups to a compute unit: each stages a chunk between two barriers while the other
+// multiplies.  Eight waves (G = 4), one to a compute unit: twice the rows from what is staged; the next chunk's values are
+// requested two steps ahead and converted into a second buffer, so that a wave does so while another one multiplies.
+template <int CG, int G, int WAVES>
+__device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, int ptile, int mtile0, int flag)
 {
     constexpr int KIND = SPLIT_GRAD;
-    constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND);
+    constexpr bool WIDE = WAVES == 8;
+    constexpr int NI = 4 * G / WAVES, NB = split_operands(KIND), NA = split_pieces(KIND);
     constexpr int P = split_plane_pixels(KIND, CG);
     constexpr int kPlane = split_lds_pixels(KIND) * 32;
-    constexpr int kItems = (split_lds_pixels(KIND) * 2 + kThreads - 1) / kThreads;
+    constexpr int kHalves = CG / 8;                               // groups of eight channels
+    constexpr int kItems = (kHalves * ((P + 63) / 64) + WAVES - 1) / WAVES;   // of 64 pixels and eight channels
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5, col = lane & 31;
     const int mtile = mtile0 + wave % G;
     const int ntile0 = (wave / G) * NI;
 
-    const int n0 = blockIdx.x * kSplitPixels;
-    auto virtual_row = [&](int n, int &img, int &rem, int &c) {   // of the stack of padded images; pixel n's first
-        img = (int)fast_div((unsigned)n, a.d_npix);
-        rem = n - img * a.npix;
-        const int r = (int)fast_div((unsigned)rem, a.d_ow);
-        c = rem - r * a.ow;
-        return img * a.Hv + r * a.sh;
-    };
-    int img0, rem0, c0, i1, i2, i3;
-    const int v0 = virtual_row(n0, img0, rem0, c0);
-    const int rows = virtual_row(min(n0 + kSplitPixels, a.total) - 1, i1, i2, i3) - v0 + a.taps / a.bw;
-    const int staged = min(rows * a.Wp, P);
+    const int n0 = ptile * kSplitPixels;
+    int img0, img1, c0, c1;
+    const int v0 = split_virtual_row(a, n0, img0, c0);
+    const int rows = split_virtual_row(a, min(n0 + kSplitPixels, a.total) - 1, img1, c1) - v0 + a.taps / a.bw;
+    const int staged = min(rows * a.Wp, P), per_half = (staged + 63) / 64;
 
-    // where this thread's staged elements come from (the same for every chunk)
+    // where this lane's staged elements come from (the same for every chunk): bytes from the tile's first image for the loads
+    // of eight waves, which give zero outside of it; elements of the whole tensor, which may be larger, for those of four
+    constexpr unsigned kOutside = WIDE ? 0x80000000u : 0xffffffffu;
+    const unsigned plane = (unsigned)a.H * a.W;
+    const int first = WIDE ? img0 : 0;
+    const float *base = a.in + (size_t)first * a.C * plane;
+    const size_t behind = (size_t)(a.total / a.npix - first) * a.C * plane * 4u;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)(behind < 0x7ffffffcu ? behind : 0x7ffffffcu), 0x00020000);
     unsigned src[kItems];
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
-        const int e = tid + i * kThreads;
-        const int g = CG == 16 && e >= staged, q = e - (g ? staged : 0);
+        const int item = wave + WAVES * i, g = CG == 16 && item >= per_half, q = (item - (g ? per_half : 0)) * 64 + lane;
         const int vr = (int)fast_div((unsigned)q, a.d_wp), c = q - vr * a.Wp - a.pw;
         const int v = v0 + vr, img = (int)fast_div((unsigned)v, a.d_hv), r = v - img * a.Hv - a.ph;
-        const bool in = r >= 0 && r < a.H && c >= 0 && c < a.W;
-        src[i] = in ? (unsigned)(((img * a.C + 8 * g) * a.H + r) * a.W + c) : 0xffffffffu;
+        const bool in = q < staged && r >= 0 && r < a.H && c >= 0 && c < a.W;
+        src[i] = in ? (unsigned)((((img - first) * a.C + 8 * g) * a.H + r) * a.W + c) * (WIDE ? 4u : 1u) : kOutside;
     }
     // and this lane's operands: the LDS byte address of its pixel's first tap
     int at[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-        const int n = min(n0 + (ntile0 + i) * 32 + col, a.total - 1);
-        int img, rem, c;
-        const int v = virtual_row(n, img, rem, c);
+        int img, c;
+        const int v = split_virtual_row(a, min(n0 + (ntile0 + i) * 32 + col, a.total - 1), img, c);
         at[i] = ((CG == 16 ? half * P : 0) + (v - v0) * a.Wp + c * a.sw) * 16;
     }
 
-    // (input gradient: hi + lo = A, tm + lg = B)
-    f32x16 hi[NI], lo[NI], tm[NI], lg[NI];
+    // hi[0] + lo[0] = A, hi[1] + lo[1] = B
+    f32x16 hi[2][NI], lo[2][NI];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        hi[i] = 0.0f;
-        lo[i] = 0.0f;
-        tm[i] = 0.0f;
-        lg[i] = 0.0f;
-    }
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            hi[f][i] = 0.0f;
+            lo[f][i] = 0.0f;
+        }
     const bool active = mtile < a.n_mtiles;
-    const bf16x8 *pp = (const bf16x8 *)a.packed + (size_t)(active ? mtile : 0) * a.chunks * a.steps * NA * 64 + lane;
+    const bf16x8 *pp = (const bf16x8 *)a.packed + (size_t)(active ? mtile : 0) * a.chunks * a.steps * NA * 64;
     bf16x8 next[NA];
 #pragma unroll
     for (int q = 0; q < NA; ++q)
-        next[q] = pp[q * 64];
+        next[q] = pp[q * 64 + lane];
 
-    const unsigned plane = (unsigned)a.H * a.W;
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
-        __syncthreads();
+    constexpr int kAhead = WIDE ? 2 : 0;   // items requested ahead: up to 512 pixels' of sixteen channels
+    float x[kItems][8];
+    auto request_item = [&](int i, int chunk) {   // channels behind the last as the last
+        const int item = wave + WAVES * i;
+        if (item >= kHalves * per_half)
+            return;
+        const int g = CG == 16 && item >= per_half, there = a.C - 1 - (chunk * CG + 8 * g);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const unsigned channel = chunk * CG + max(-8 * g, min(j, there));
+            if (WIDE)
+                x[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, src[i], channel * plane * 4u, 0));
+            else
+                x[i][j] = src[i] != kOutside ? base[(size_t)src[i] + (size_t)channel * plane] : 0.0f;
+        }
+    };
+    auto stage_item = [&](int i, int chunk, char *to) {
+        const int item = wave + WAVES * i;
+        if (item >= kHalves * per_half)
+            return;
+        const int g = CG == 16 && item >= per_half, q = (item - (g ? per_half : 0)) * 64 + lane;
+        const int c0 = chunk * CG + 8 * g;
+        if (c0 + 8 > a.C)   // channels behind the last have zero parameters: any finite value will do
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                x[i][j] = c0 + j < a.C ? x[i][j] : 0.0f;
+        bf16x8 v[3];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            __bf16 p0, p1, p2;
+            split3_any(x[i][j], p0, p1, p2);
+            v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
+        }
+        if (q < staged) {
+            char *dst = to + (g * P + q) * 16;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                *reinterpret_cast<bf16x8 *>(dst + b * kPlane) = v[b];
+        }
+    };
+    auto request = [&](int chunk) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+            request_item(i, chunk);
+    };
+    auto stage = [&](int chunk, char *to) {
 #pragma unroll
         for (int i = 0; i < kItems; ++i) {
-            const int e = tid + i * kThreads;
-            if (e < (CG == 16 ? 2 : 1) * staged) {
-                const int g = CG == 16 && e >= staged;
-                const int q = e - (g ? staged : 0);
-                const int cbase = chunk * CG + 8 * g;
-                float x[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const bool in = src[i] != 0xffffffffu && cbase + j < a.C;
-                    x[j] = in ? a.in[(size_t)src[i] + (size_t)(chunk * CG + j) * plane] : a.oob;
-                }
-                bf16x8 v[3];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    __bf16 p0, p1, p2;   // (channels behind the last have zero parameters: any finite value will do)
-                    split3_any(cbase + j >= a.C ? 0.0f : x[j], p0, p1, p2);
-                    v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
-                }
-                char *dst = lds + (g * P + q) * 16;
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    *reinterpret_cast<bf16x8 *>(dst + b * kPlane) = v[b];
-            }
+            if (i >= kAhead)
+                request_item(i, chunk);
+            stage_item(i, chunk, to);
         }
+    };
+    if (WIDE) {
+        request(0);
+        stage(0, lds);
+    }
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+        const char *from = lds + (WIDE && (chunk & 1) ? split_lds_bytes(KIND) : 0);
+        const bool more = chunk + 1 < a.chunks;
         __syncthreads();
+        if (!WIDE) {
+            stage(chunk, lds);
+            __syncthreads();
+        }
         int dh = 0, dw = 0;
-        auto next_tap = [&]() {   // LDS offset of the tap (behind the last: of the first, with zero parameters)
-            const int off = (dh * a.Wp + dw) * 16;
+        const int taps_h = a.taps / a.bw;
+        auto next_tap = [&]() {   // LDS offset of the next tap (behind the last: of the first, with zero parameters)
+            const int off = dh < taps_h ? (dh * a.Wp + dw) * 16 : 0;
             if (++dw == a.bw) {
                 dw = 0;
                 ++dh;
             }
             return off;
         };
-        for (int step = 0; step < a.steps; ++step) {
+        auto next_offset = [&]() {   // of a step's operands
+            const int off = next_tap();
+            if (CG == 16)
+                return off;
+            const int off2 = next_tap();
+            return half ? off2 : off;
+        };
+        constexpr int kNext = WIDE ? 1 : 0;   // (of a pixel tile and of the one behind it; no registers left for it with four waves)
+        bf16x8 B[1 + kNext][NB];
+        auto fetch = [&](bf16x8 (&to)[NB], int off) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                to[b] = *reinterpret_cast<const bf16x8 *>(from + off + b * kPlane);
+        };
+        int off = next_offset();
+        if (WIDE)
+            fetch(B[0], at[0] + off);
+        auto multiply = [&](int step, bool ask) {   // ask: for the next chunk's values, behind the next step's parameters
             bf16x8 A[NA];
 #pragma unroll
             for (int q = 0; q < NA; ++q)
                 A[q] = next[q];
-            if (chunk + 1 < a.chunks || step + 1 < a.steps)
+            if (more || step + 1 < a.steps)
                 pp += NA * 64;
 #pragma unroll
             for (int q = 0; q < NA; ++q)
-                next[q] = pp[q * 64];
-            int off = next_tap();
-            if (CG == 8) {
-                const int off2 = 2 * step + 1 < a.taps ? next_tap() : 0;
-                off = half ? off2 : off;
-            }
+                next[q] = pp[q * 64 + lane];
+            if (ask)
+                request(chunk + 1);
+            const int off_next = next_offset();
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
-                bf16x8 B[NB];
+                if (WIDE) {
+                    fetch(B[(i + 1) & kNext], i + 1 < NI ? at[(i + 1) % NI] + off : at[0] + off_next);
+                    __builtin_amdgcn_sched_barrier(0);
+                } else
+                    fetch(B[0], at[i] + off);
+                // an accumulator's products follow one another at 48 cycles, two accumulators' in turn at 32
+                auto products = [&](f32x16 (&to)[2][NI], int p, int v) {
 #pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    B[b] = *reinterpret_cast<const bf16x8 *>(lds + at[i] + off + b * kPlane);
-                auto mul = [](f32x16 &acc, const bf16x8 &x, const bf16x8 &y) {
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc, 0, 0, 0);
+                    for (int f = 0; f < 2; ++f)
+                        to[f][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[3 * f + p], B[i & kNext][v], to[f][i], 0, 0, 0);
                 };
-#pragma unroll
-                for (int f = 0; f < 6; f += 3) {
-                    f32x16 &h = f == 0 ? hi[i] : tm[i], &l = f == 0 ? lo[i] : lg[i];
-                    mul(l, A[f + 2], B[0]);
-                    mul(l, A[f], B[2]);
-                    mul(h, A[f], B[0]);
-                    mul(l, A[f + 1], B[1]);
-                    mul(l, A[f + 1], B[0]);
-                    mul(l, A[f], B[1]);
-                }
+                products(lo, 2, 0);
+                products(lo, 0, 2);
+                products(hi, 0, 0);
+                products(lo, 1, 1);
+                products(lo, 1, 0);
+                products(lo, 0, 1);
+                if (WIDE)
+                    __builtin_amdgcn_sched_barrier(0);
             }
-        }
+            off = off_next;
+        };
+        for (int step = 0; step < a.steps; ++step)
+            multiply(step, WIDE && more && step == max(0, a.steps - 2));
+        if (WIDE && more)
+            stage(chunk + 1, lds + (chunk & 1 ? 0 : split_lds_bytes(KIND)));
     }
 
     // lane: pixel col of each tile, templates (input gradient: channels) 8 (r / 4) + 4 half + r % 4
@@ -461,14 +533,14 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
         float v[16], any = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            v[r] = __builtin_fmaf(-(x[r] - ctr[r]), tm[i][r] + lg[i][r], hi[i][r] + lo[i][r]);
+            v[r] = __builtin_fmaf(-(x[r] - ctr[r]), hi[1][i][r] + lo[1][i][r], hi[0][i][r] + lo[0][i][r]);
             any = __builtin_fmaf(v[r], 0.0f, any);   // NaN once a value is not finite
         }
         if (any != any) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float A = split_sum(hi[i][r], lo[i][r]);
-                v[r] = __builtin_fmaf(-(x[r] - ctr[r]), split_sum(tm[i][r], lg[i][r]), A);
+                const float A = split_sum(hi[0][i][r], lo[0][i][r]);
+                v[r] = __builtin_fmaf(-(x[r] - ctr[r]), split_sum(hi[1][i][r], lo[1][i][r]), A);
 #if defined(__HIP_DEVICE_COMPILE__)
                 if (v[r] != v[r] && __builtin_isinf(A))
                     v[r] = split_grad_terms(img, min(mtile * kSplitRows + 8 * (r / 4) + 4 * half + r % 4, a.O - 1),
@@ -485,16 +557,6 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
                 a.out[base + (size_t)ml * a.npix] = v[r];
         }
     }
-}
-
-// How a workgroup's pixels, 128 from n0 on, lie in the stack of padded images: the virtual row of the first, and what is
-// staged for them.
-__device__ __forceinline__ int split_virtual_row(const SplitArgs &a, int n, int &img, int &c)
-{
-    img = (int)fast_div((unsigned)n, a.d_npix);
-    const int rem = n - img * a.npix, r = (int)fast_div((unsigned)rem, a.d_ow);
-    c = rem - r * a.ow;
-    return img * a.Hv + r * a.sh;
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -949,9 +1011,9 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
     const int ptile = x < run * 8 ? x % 8 * run + x / 8 : x;
     if constexpr (KIND == SPLIT_GRAD) {
         if (g == 2)
-            split_grad_body<CG, 2>(a, split_lds, mtile0, flag);
+            split_grad_body<CG, 2, 4>(a, split_lds, ptile, mtile0, flag);
         else
-            split_grad_body<CG, 1>(a, split_lds, mtile0, flag);
+            split_grad_body<CG, 1, 4>(a, split_lds, ptile, mtile0, flag);
     } else {
         auto &lds_far = *(__attribute__((address_space(3))) SplitFar *)&far;
         if (KIND == SPLIT_FWD && g == 4)
@@ -972,6 +1034,17 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
         } else if ((int)threadIdx.x < g && mtile0 + (int)threadIdx.x < a.n_mtiles)
             a.flags[(size_t)ptile * a.n_mtiles + mtile0 + threadIdx.x] = 0;
     }
+#endif
+}
+
+// Input gradient, four template tiles to a workgroup of eight waves.
+template <int CG>
+__global__ __launch_bounds__(2 * kThreads, 2) void sim_split_grad_wide_kernel(const SplitArgs a, int flag)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __shared__ __align__(16) char split_lds[2 * split_lds_bytes(SPLIT_GRAD)];
+    const int run = gridDim.x / 8, x = blockIdx.x;
+    split_grad_body<CG, 4, 8>(a, split_lds, x < run * 8 ? x % 8 * run + x / 8 : x, blockIdx.y * 4, flag);
 #endif
 }
 
@@ -1131,6 +1204,21 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     return a;
 }
 
+// Workgroups of eight waves and four template tiles, one to a compute unit, instead of four waves and two, two to a unit: 0.93 of
+// the time of a chip that either kind fills.  A compute unit that gets a single one of the lesser takes 0.55.  All template
+// tiles in fours (96 channels, the last of three tiles' two waves idle: 32 x 96 x 28 x 28 -> 128 76 -> 81 us), and 31 bits for
+// the images of a tile.  Measured, 128 channels, 28 x 28 -> 128, 3 x 3, by the number of tiles (us, before and after):
+// 135 97 -> 83, 172 97 -> 84, 196 93 -> 82, 252 100 -> 92, 392 176 -> 162, 503 189 -> 178; 258 148 -> 159, 343 149 -> 162, left to the others.
+// 1 x 1, 196: 29 -> 22; 5 x 5, 196: 216 -> 204.
+static bool split_grad_wide(const SimPlan &p, const SplitPlan &s)
+{
+    const long long touched = (kSplitPixels - 1) / (1LL * p.oh * p.ow) + 2, groups = 1LL * s.n_ptiles * (s.n_mtiles / 4);
+    if (s.n_mtiles % 4 != 0 || 4 * touched * p.C * p.H * p.W >= (1LL << 31))
+        return false;
+    const long long full = groups / 256, rest = groups % 256;
+    return 0.93 * (full + (rest != 0)) < full + (rest == 0 ? 0.0 : rest <= 128 ? 0.55 : 1.0);
+}
+
 template <int KIND>
 static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, float *output, char *ws, int flag,
                         hipStream_t s, SplitArgs a = {})
@@ -1155,6 +1243,14 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     a.d_hv = make_fast_div((unsigned)sp.Hv);
     a.d_taps = make_fast_div((unsigned)a.taps);
     a.d_bw = make_fast_div((unsigned)p.bw);
+    if (KIND == SPLIT_GRAD && split_grad_wide(p, sp)) {
+        const dim3 grid((unsigned)sp.n_ptiles, (unsigned)(sp.n_mtiles / 4));
+        if (sp.cg == 16)
+            hipLaunchKernelGGL(sim_split_grad_wide_kernel<16>, grid, dim3(2 * kThreads), 0, s, a, flag);
+        else
+            hipLaunchKernelGGL(sim_split_grad_wide_kernel<8>, grid, dim3(2 * kThreads), 0, s, a, flag);
+        return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
+    }
     // as many template tiles per staged pixel tile as leave a workgroup for every compute unit
     a.gmax = KIND == SPLIT_FWD ? 4 : 2;
     while (a.gmax > 1 && (a.gmax / 2 >= sp.n_mtiles || (long long)sp.n_ptiles * ((sp.n_mtiles + a.gmax - 1) / a.gmax) < 256))
@@ -1180,7 +1276,7 @@ int sim_split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, 
 // tap) - the forward's contraction with g as the image (its channels are the templates, the taps flipped) and the input
 // channels as rows, g in three pieces against the three of each coefficient: eight bits each, but with the exponents of fp32,
 // which g and the weights use (gradients of one template, or of one pixel, may be many orders below others').  32 x 128 x 28 x 28, 128 templates, 3 x 3: 196 us
-// on the fp32 matrix instructions -> 101 us, error against 64 bits 6.0e-7 -> 2.0e-7 of the gradient's 2-norm.  Small grids
+// on the fp32 matrix instructions -> 93 us, 82 with workgroups of eight waves (split_grad_wide), error against 64 bits 6.0e-7 -> 2.0e-7 of the gradient's 2-norm.  Small grids
 // keep that kernel (sim_mfma_kernel), which splits the contraction over workgroups.
 // ------------------------------------------------------------------------------------------------
 static SimPlan grad_as_forward(const SimPlan &p)
