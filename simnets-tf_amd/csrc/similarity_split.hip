@@ -41,6 +41,8 @@
 // into registers, one step ahead; the next chunk's input is requested during a chunk's last step, by buffer loads (an
 // offset per pixel, one per channel, zeros outside of the image: no 64-bit address per value).  256 registers: two
 // workgroups per compute unit, so that one stages while the other multiplies.
+// Where tiles are few for that, or the input gradient's rows many, a workgroup of eight waves to a compute unit, with two buffers:
+// split_forward_wide, split_grad_wide.
 //
 // Measured (whole call, vector form, three bf16 pieces, this form): 256 x 64 x 32 x 32 -> 128, 3 x 3: 0.80, 0.372, 0.229 ms.
 // The kernel's 211 us are 1.1 PFLOP/s of matrix products at 1.55 GHz, matrix units busy 56 %: the clock sinks with them
@@ -152,10 +154,10 @@ struct NearOutputs {
 // parameters are out of range, is flagged for the direct kernel instead.  G: the workgroup's template tiles, 4, 2 or 1.
 // LOGS: the mode has logarithm terms.  Inlined once, at the kernel's end: a call, or a copy in each split_body, spills SGPRs of
 // the bodies (37 x 45 x 29 x 35 -> 75 62 -> 65 to 72 us).
-template <int KIND, int CG, bool LOGS>
+template <int KIND, int CG, bool LOGS, int WAVES>
 __device__ __forceinline__ void split_recompute(lds_char *lds, int ptile, int mtile0, int G, u32x4 near)
 {
-    constexpr int kLanes = 8, kTerms = 12, kOutputs = kThreads / kLanes;
+    constexpr int kThreads = 64 * WAVES, kLanes = 8, kTerms = 12, kOutputs = kThreads / kLanes;
     typedef NearOutputs<KIND, CG> Near;
     static_assert(sizeof(Near) <= split_lds_bytes(KIND), "in the memory of the staged pieces");
     const SplitArgs a = split_kernel_args();
@@ -187,7 +189,7 @@ __device__ __forceinline__ void split_recompute(lds_char *lds, int ptile, int mt
         for (int i = 0; i < 4; ++i)
             for (unsigned rest = near[i]; rest; rest &= rest - 1, ++slot) {
                 const int r = __builtin_ctz(rest), ml = g * kSplitRows + 8 * (r / 4) + 4 * (tid >> 5 & 1) + r % 4;
-                q.list[slot] = (unsigned short)((((wave / G) * G + i) * 32 + (tid & 31)) << 7 | ml);
+                q.list[slot] = (unsigned short)((((wave / G) * (4 * G / WAVES) + i) * 32 + (tid & 31)) << 7 | ml);
             }
     }
     __syncthreads();
@@ -564,17 +566,17 @@ typedef const __attribute__((address_space(4))) float uniform_float;
 
 // What a workgroup knows of the sizes it has staged.
 struct SplitFar {
-    int most;                          // the largest |x'| s so far: a float's bits, as which they are compared
-    int lanes[2][kSplitLevels - 1];    // in chunks of even and odd numbers: with a value that the next level keeps, see split_body
+    int most[2];                       // the largest |x'| s so far: a float's bits, as which they are compared; chunks of even and odd numbers
+    int lanes[3][kSplitLevels - 1];    // of three chunks in turn: with a value that the next level keeps, see split_body
 };
 
 // Raises far.most to a lane's value, rounded up to a quarter of an octave: so a workgroup does it a few times.  (One instruction
 // and not the compiler's loop over the lanes.)
-__device__ __forceinline__ void split_far_most(__attribute__((address_space(3))) SplitFar &far, float value)
+__device__ __forceinline__ void split_far_most(__attribute__((address_space(3))) int &most, float value)
 {
     asm volatile("ds_max_i32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
                  :
-                 : "v"((unsigned)(uintptr_t)&far.most), "v"(__float_as_int(value) | 0x1fffff)
+                 : "v"((unsigned)(uintptr_t)&most), "v"(__float_as_int(value) | 0x1fffff)
                  : "memory");
 }
 
@@ -588,12 +590,18 @@ __device__ __forceinline__ void split_far_most(__attribute__((address_space(3)))
 // 220 us, where all tiles left to the direct kernel took 1190; inputs 0.05 and a border of 100: 222 and 1222; one pixel in a
 // hundred 10^3 times the others: 225 and 1440, 10^4 times: 1490 and 1470.  What it costs ordinary inputs: 1 to 2 us there,
 // 1 of 50 on 37 x 45 x 29 x 35 -> 75, 2 of 54 on 64 x 256 x 32 x 32 -> 64, 1 x 1.
-template <int KIND, int CG, int G>
+//
+// WAVES: four, two workgroups to a compute unit, each of which stages a chunk between two barriers while the other multiplies;
+// or eight, one to a unit, all rows from what is staged once: the next chunk's values are requested two steps ahead and
+// converted into a second buffer.  A barrier a chunk then: a wave may be a chunk ahead of another that has yet to read far, so
+// that consecutive chunks have places of their own there.
+template <int KIND, int CG, int G, int WAVES>
 __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attribute__((address_space(3))) SplitFar &far,
                                            u32x4 &near, int ptile, int mtile0, int norm)
 {
     constexpr bool MASKED = KIND == SPLIT_MASKED;
-    constexpr int NI = G, NB = split_operands(KIND), NA = split_pieces(KIND), kWaves = kThreads / 64;
+    constexpr bool WIDE = WAVES == 8;
+    constexpr int NI = 4 * G / WAVES, NB = split_operands(KIND), NA = split_pieces(KIND), kWaves = WAVES;
     constexpr int P = split_plane_pixels(KIND, CG);
     constexpr int kPlane = split_lds_pixels(KIND) * 32;
     constexpr int kHalves = CG / 8;                               // groups of eight channels
@@ -677,6 +685,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
     // (sizes as a float's bits) the largest |x'| s so far, what is larger than it, and than the level keeps, among staged values
     int seen = __float_as_int(kSplitSeen), ask = seen, limit = __float_as_int(kSplitMost);
     const float *channels = a.chan;
+    auto buffer = [&](int chunk) { return lds + (WIDE && (chunk & 1) ? split_lds_bytes(KIND) : 0); };
     auto stage = [&](int chunk) {   // converts the requested values; returns the largest staged |x'| of this lane's
         float most = 0.0f;
 #pragma unroll
@@ -717,7 +726,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
             }
             if (q < staged) {
                 most = fmaxf(most, item_most);
-                char *dst = lds + (g * P + q) * 16;
+                char *dst = buffer(chunk) + (g * P + q) * 16;
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
                     *reinterpret_cast<f16x8 *>(dst + b * kPlane) = v[b];
@@ -725,27 +734,34 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
         }
         return __float_as_int(most);
     };
-    request(0);
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
-        __syncthreads();
+    auto stage_and_tell = [&](int chunk) {
         // Both blocks out of the ordinary: code that is not in the instruction cache takes a microsecond or two to get.
         const int most = stage(chunk);
         if (most > ask)
-            split_far_most(far, most < __float_as_int(INFINITY) ? ldexpf(__int_as_float(most), kSplitLevelBits * level) : 0.0f);
+            split_far_most(far.most[chunk & 1], most < __float_as_int(INFINITY) ? ldexpf(__int_as_float(most), kSplitLevelBits * level) : 0.0f);
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(most > limit) != 0, 0))
             for (int i = level; i < kLastLevel; ++i) {
                 const float keeps = ldexpf(kSplitMost / 32, kSplitLevelBits * (i - level));
                 const int lanes = __popcll(__builtin_amdgcn_ballot_w64(__int_as_float(most) > keeps));
                 if (lane == 0)
-                    __hip_atomic_fetch_add(&far.lanes[chunk & 1][i], lanes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(&far.lanes[chunk % 3][i], lanes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
+    };
+    request(0);
+    if (WIDE)
+        stage_and_tell(0);
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
         __syncthreads();
-        seen = __builtin_amdgcn_readfirstlane(far.most);
+        if (!WIDE) {
+            stage_and_tell(chunk);
+            __syncthreads();
+        }
+        seen = max(seen, __builtin_amdgcn_readfirstlane(far.most[chunk & 1]));
         ask = seen;
         if (__builtin_expect(seen > __float_as_int(kSplitMost), 0)) {
             int next_level = level;
             while (next_level < kLastLevel && __int_as_float(seen) > ldexpf(kSplitMost, kSplitLevelBits * next_level) &&
-                   (next_level == 0 || __builtin_amdgcn_readfirstlane(far.lanes[chunk & 1][next_level]) > kThreads / 8))
+                   (next_level == 0 || __builtin_amdgcn_readfirstlane(far.lanes[chunk % 3][next_level]) > 64 * WAVES / 8))
                 ++next_level;
             if (next_level > level) {
                 const float ratio = ldexpf(1.0f, 2 * kSplitLevelBits * (level - next_level));
@@ -764,7 +780,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
             }
             ask = __float_as_int(ldexpf(__int_as_float(seen), -kSplitLevelBits * level));
             if (tid < kSplitLevels - 1)
-                far.lanes[~chunk & 1][tid] = 0;
+                far.lanes[(chunk + 2) % 3][tid] = 0;
         }
         int dh = 0, dw = 0;
         auto next_tap = [&]() {   // LDS offset of the next tap (behind the last: of the first, with zero parameters)
@@ -782,7 +798,8 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
             const int off2 = next_tap();
             return half ? off2 : off;
         };
-        auto fetch = [&](f16x8 &to, int from, int b) { to = *reinterpret_cast<const f16x8 *>(lds + from + b * kPlane); };
+        const char *staged_here = buffer(chunk);
+        auto fetch = [&](f16x8 &to, int from, int b) { to = *reinterpret_cast<const f16x8 *>(staged_here + from + b * kPlane); };
         auto mul = [](f32x16 &to, const f16x8 &p, const f16x8 &v) {
             to = __builtin_amdgcn_mfma_f32_32x32x16_f16(p, v, to, 0, 0, 0);
         };
@@ -804,7 +821,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
 #pragma unroll
             for (int q = 0; q < NA; ++q)
                 next[q] = pp[q * 64 + lane];
-            if (step + 1 == a.steps && chunk + 1 < a.chunks)
+            if (step == (WIDE ? max(0, a.steps - 2) : a.steps - 1) && chunk + 1 < a.chunks)
                 request(chunk + 1);
         };
         int off = next_offset();
@@ -905,6 +922,8 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
                 if (TWO)
                     ac2[i] = 0.0f;
             }
+        if (WIDE && chunk + 1 < a.chunks)
+            stage_and_tell(chunk + 1);
     }
 
     // lane: pixel col of each tile, templates 8 (r / 4) + 4 half + r % 4
@@ -977,7 +996,43 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
         near[i] = n < a.total ? flagged : 0u;
     }
 }
+
+// What a forward workgroup does around its body: body(far, near).
+template <int KIND, int CG, int WAVES, class Body>
+__device__ __forceinline__ void split_forward(const SplitArgs &a, char *lds, int ptile, int mtile0, int g, int norm, Body &&body)
+{
+    __shared__ int any_near;   // of the workgroup's outputs, one below the guard's line
+    __shared__ SplitFar far;
+    if (threadIdx.x == 0)
+        any_near = 0;
+    if (threadIdx.x < 2)
+        far.most[threadIdx.x] = __float_as_int(kSplitSeen);
+    if (threadIdx.x < kSplitLevels - 1)
+        far.lanes[0][threadIdx.x] = far.lanes[1][threadIdx.x] = far.lanes[2][threadIdx.x] = 0;
+    if (WAVES == 8)   // (its first chunk is staged, and told of, in front of the first barrier)
+        __syncthreads();
+    u32x4 near = 0;   // [i] bit r: output r of this lane's pixel tile i is
+    body(*(__attribute__((address_space(3))) SplitFar *)&far, near);
+    if (near[0] | near[1] | near[2] | near[3])
+        any_near = 1;
+    __syncthreads();
+    // (unlikely: the code behind everything else; between the bodies it costs 37 x 45 x 29 x 35 -> 75 4 us of 62)
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(any_near), 0)) {
+        if (KIND == SPLIT_MASKED || norm)
+            split_recompute<KIND, CG, true, WAVES>((lds_char *)lds, ptile, mtile0, g, near);
+        else
+            split_recompute<KIND, CG, KIND == SPLIT_MASKED, WAVES>((lds_char *)lds, ptile, mtile0, g, near);
+    } else if ((int)threadIdx.x < g && mtile0 + (int)threadIdx.x < a.n_mtiles)
+        a.flags[(size_t)ptile * a.n_mtiles + mtile0 + threadIdx.x] = 0;
+}
 #endif
+
+// Consecutive workgroups go to the eight XCDs in turn: a run of neighbouring pixel tiles, which share rows, to each.
+__device__ __forceinline__ int split_ptile()
+{
+    const int run = gridDim.x / 8, x = blockIdx.x;
+    return x < run * 8 ? x % 8 * run + x / 8 : x;
+}
 
 // The template tiles of a pixel tile are dealt out as groups of gmax and, of the rest, 2 and 1 (forward, of four: the rest
 // as one).  flag: forward, the normalized mode; input gradient, NaN inputs ignored.
@@ -986,15 +1041,6 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __align__(16) char split_lds[split_lds_bytes(KIND)];
-    __shared__ int any_near;   // of the workgroup's outputs, one below the guard's line
-    __shared__ SplitFar far;
-    if (KIND != SPLIT_GRAD && threadIdx.x == 0) {
-        any_near = 0;
-        far.most = __float_as_int(kSplitSeen);
-    }
-    if (KIND != SPLIT_GRAD && threadIdx.x < kSplitLevels - 1)
-        far.lanes[0][threadIdx.x] = far.lanes[1][threadIdx.x] = 0;
-    u32x4 near = 0;   // [i] bit r: output r of this lane's pixel tile i is
     const int full = a.n_mtiles / a.gmax, y = blockIdx.y;
     int mtile0 = y * a.gmax, g = a.gmax;
     if (y >= full) {
@@ -1006,34 +1052,35 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
             g = 1;
         }
     }
-    // consecutive workgroups go to the eight XCDs in turn: a run of neighbouring pixel tiles, which share rows, to each
-    const int run = gridDim.x / 8, x = blockIdx.x;
-    const int ptile = x < run * 8 ? x % 8 * run + x / 8 : x;
+    const int ptile = split_ptile();
     if constexpr (KIND == SPLIT_GRAD) {
         if (g == 2)
             split_grad_body<CG, 2, 4>(a, split_lds, ptile, mtile0, flag);
         else
             split_grad_body<CG, 1, 4>(a, split_lds, ptile, mtile0, flag);
-    } else {
-        auto &lds_far = *(__attribute__((address_space(3))) SplitFar *)&far;
-        if (KIND == SPLIT_FWD && g == 4)
-            split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2>(a, split_lds, lds_far, near, ptile, mtile0, flag);
-        else if (g == 2)
-            split_body<KIND, CG, 2>(a, split_lds, lds_far, near, ptile, mtile0, flag);
-        else
-            split_body<KIND, CG, 1>(a, split_lds, lds_far, near, ptile, mtile0, flag);
-        if (near[0] | near[1] | near[2] | near[3])
-            any_near = 1;
-        __syncthreads();
-        // (unlikely: the code behind everything else; between the bodies it costs 37 x 45 x 29 x 35 -> 75 4 us of 62)
-        if (__builtin_expect(__builtin_amdgcn_readfirstlane(any_near), 0)) {
-            if (KIND == SPLIT_MASKED || flag)
-                split_recompute<KIND, CG, true>((lds_char *)split_lds, ptile, mtile0, g, near);
+    } else
+        split_forward<KIND, CG, 4>(a, split_lds, ptile, mtile0, g, flag, [&](auto &far, u32x4 &near) __attribute__((always_inline)) {
+            if (KIND == SPLIT_FWD && g == 4)
+                split_body<KIND, CG, KIND == SPLIT_FWD ? 4 : 2, 4>(a, split_lds, far, near, ptile, mtile0, flag);
+            else if (g == 2)
+                split_body<KIND, CG, 2, 4>(a, split_lds, far, near, ptile, mtile0, flag);
             else
-                split_recompute<KIND, CG, KIND == SPLIT_MASKED>((lds_char *)split_lds, ptile, mtile0, g, near);
-        } else if ((int)threadIdx.x < g && mtile0 + (int)threadIdx.x < a.n_mtiles)
-            a.flags[(size_t)ptile * a.n_mtiles + mtile0 + threadIdx.x] = 0;
-    }
+                split_body<KIND, CG, 1, 4>(a, split_lds, far, near, ptile, mtile0, flag);
+        });
+#endif
+}
+
+// Forward without missing values, four template tiles to a workgroup of eight waves.
+template <int CG>
+__global__ __launch_bounds__(2 * kThreads, 2) void sim_split_forward_wide_kernel(const SplitArgs a, int flag)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int KIND = SPLIT_FWD;
+    __shared__ __align__(16) char split_lds[2 * split_lds_bytes(KIND)];
+    const int ptile = split_ptile(), mtile0 = blockIdx.y * 4;
+    split_forward<KIND, CG, 8>(a, split_lds, ptile, mtile0, 4, flag, [&](auto &far, u32x4 &near) __attribute__((always_inline)) {
+        split_body<KIND, CG, 4, 8>(a, split_lds, far, near, ptile, mtile0, flag);
+    });
 #endif
 }
 
@@ -1043,8 +1090,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void sim_split_grad_wide_kernel(co
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __align__(16) char split_lds[2 * split_lds_bytes(SPLIT_GRAD)];
-    const int run = gridDim.x / 8, x = blockIdx.x;
-    split_grad_body<CG, 4, 8>(a, split_lds, x < run * 8 ? x % 8 * run + x / 8 : x, blockIdx.y * 4, flag);
+    split_grad_body<CG, 4, 8>(a, split_lds, split_ptile(), blockIdx.y * 4, flag);
 #endif
 }
 
@@ -1219,6 +1265,18 @@ static bool split_grad_wide(const SimPlan &p, const SplitPlan &s)
     return 0.93 * (full + (rest != 0)) < full + (rest == 0 ? 0.0 : rest <= 128 ? 0.55 : 1.0);
 }
 
+// The forward's: where the workgroups of four waves and two template tiles are more than one and at most two to a compute
+// unit.  Fewer leave compute units to share; more run as four tiles to four waves, two workgroups to a unit, which is the faster
+// form of a full chip (256 x 64 x 32 x 32 -> 128, 3 x 3: 219 us, this form 267).  Measured, 128 channels, 28 x 28 -> 128, 3 x 3, by the
+// number of tiles (us, before and after): 135 64 -> 58, 196 68 -> 62, 252 72 -> 67; 1 x 1, 196: 28 -> 23; 5 x 5, 196: 143 -> 143;
+// three tiles of 75 templates, 30 x 45 x 29 x 35, 238: 32 -> 28.  With missing values no gain (22 x 128 x 28 x 28: 95 -> 95; 64 x 64 x 32 x
+// 32: 103 -> 107).
+static bool split_forward_wide(const SplitPlan &s)
+{
+    const long long groups = 1LL * s.n_ptiles * ((s.n_mtiles + 3) / 4);
+    return (s.n_mtiles % 4 == 0 || s.n_mtiles % 4 == 3) && groups > 128 && groups <= 256;
+}
+
 template <int KIND>
 static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *input, float *output, char *ws, int flag,
                         hipStream_t s, SplitArgs a = {})
@@ -1249,6 +1307,14 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
             hipLaunchKernelGGL(sim_split_grad_wide_kernel<16>, grid, dim3(2 * kThreads), 0, s, a, flag);
         else
             hipLaunchKernelGGL(sim_split_grad_wide_kernel<8>, grid, dim3(2 * kThreads), 0, s, a, flag);
+        return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
+    }
+    if (KIND == SPLIT_FWD && split_forward_wide(sp)) {
+        const dim3 grid((unsigned)sp.n_ptiles, (unsigned)((sp.n_mtiles + 3) / 4));
+        if (sp.cg == 16)
+            hipLaunchKernelGGL(sim_split_forward_wide_kernel<16>, grid, dim3(2 * kThreads), 0, s, a, flag);
+        else
+            hipLaunchKernelGGL(sim_split_forward_wide_kernel<8>, grid, dim3(2 * kThreads), 0, s, a, flag);
         return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
     }
     // as many template tiles per staged pixel tile as leave a workgroup for every compute unit
