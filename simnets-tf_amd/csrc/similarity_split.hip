@@ -1115,39 +1115,45 @@ __global__ __launch_bounds__(kThreads) void sim_split_grad_pack_kernel(const Spl
     const int tid = threadIdx.x, parts = (a.steps + 3) / 4;
     const int mtile = blockIdx.x / (a.chunks * parts), rest = blockIdx.x - mtile * a.chunks * parts;
     const int chunk = rest / parts, part = rest - chunk * parts;
+    // this lane's elements first: they arrive while the centres are formed (7.6 -> 4.9 us, 128 channels, 128 templates, 3 x 3)
+    const int step = 4 * part + (tid >> 6);
+    const int lane = tid & 63, half = lane >> 5, row = lane & 31, c = mtile * kSplitRows + row;
+    const int tap = a.cg == 16 ? step : 2 * step + half;
+    float t[8], w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {   // (any value outside)
+        const int o = chunk * a.cg + (a.cg == 16 ? 8 * half : 0) + j;
+        const size_t at = ((size_t)min(o, a.O - 1) * a.C + min(c, a.C - 1)) * a.taps + (a.taps - 1 - min(tap, a.taps - 1));
+        t[j] = a.templates[at];
+        w[j] = a.weights[at];
+    }
     float sum[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
         sum[i] = split_grad_centre_part(a, mtile * kSplitRows + 16 * i + (tid >> 4));
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const float c = split_grad_centre(a, sum[i]);
+        const float centred = split_grad_centre(a, sum[i]);
         if ((tid & 15) == 0) {
-            centre[16 * i + (tid >> 4)] = c;
+            centre[16 * i + (tid >> 4)] = centred;
             if (chunk == 0 && part == 0)
-                a.ctr[mtile * kSplitRows + 16 * i + (tid >> 4)] = c;
+                a.ctr[mtile * kSplitRows + 16 * i + (tid >> 4)] = centred;
         }
     }
     __syncthreads();
-    const int step = 4 * part + (tid >> 6);
     if (step >= a.steps)
         return;
-    const int lane = tid & 63, half = lane >> 5, row = lane & 31, c = mtile * kSplitRows + row;
-    const int tap = a.cg == 16 ? step : 2 * step + half;
+    const float middle = centre[row];
     bf16x8 v[6];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int o = chunk * a.cg + (a.cg == 16 ? 8 * half : 0) + j;
-        float t = 0.0f, w = 0.0f;
-        if (c < a.C && o < a.O && tap < a.taps) {
-            const size_t at = ((size_t)o * a.C + c) * a.taps + (a.taps - 1 - tap);
-            w = scale * a.weights[at];
-            t = a.templates[at] - centre[row];
-        }
+        const bool there = c < a.C && o < a.O && tap < a.taps;
+        const float ws = there ? scale * w[j] : 0.0f, td = there ? t[j] - middle : 0.0f;
         __bf16 p0, p1, p2;
-        split3_any(w * t, p0, p1, p2);
+        split3_any(ws * td, p0, p1, p2);
         v[0][j] = p0; v[1][j] = p1; v[2][j] = p2;
-        split3_any(w, p0, p1, p2);
+        split3_any(ws, p0, p1, p2);
         v[3][j] = p0; v[4][j] = p1; v[5][j] = p2;
     }
     bf16x8 *dst = reinterpret_cast<bf16x8 *>(a.packed) +
