@@ -604,6 +604,19 @@ __device__ __forceinline__ float pack_over_wave(float v, Op &&op)
     return v;
 }
 
+// Patch element k = (dc*bh + dh)*bw + dw -> where it lies relative to the patch origin.
+__device__ __forceinline__ void pack_patch_table(int4 *ktab, const MexPackTwin &tw, int K, int H, int W, int bh, int bw)
+{
+    for (int k = threadIdx.x; k < K; k += 256) {
+        const int dc = k / (bh * bw);
+        const int rem = k - dc * bh * bw;
+        const int dh = rem / bw, dw = rem - dh * bw;
+        ktab[k] = make_int4((dc * H + dh) * W + dw, dc, dh, dw);
+        if (tw.offp != nullptr)
+            tw.ktab[k] = ktab[k];
+    }
+}
+
 // One wave per (region, instance) row of the offsets: optional logsumexp normalisation
 // (python/simnets/keras.py:155-160) and the scaling, then the row is scattered into the k-major packed layout
 // [r][mgroup][k][tm]; for finite epsilon also its exponentials relative to the row maximum, the maximum and the
@@ -636,17 +649,8 @@ __global__ __launch_bounds__(256) void mex_pack_offsets_kernel(const float *__re
         }
         return;
     }
-    if (blockIdx.x == 0) {
-        // patch element k = (dc*bh + dh)*bw + dw -> where it lies relative to the patch origin
-        for (int k = threadIdx.x; k < K; k += 256) {
-            const int dc = k / (bh * bw);
-            const int rem = k - dc * bh * bw;
-            const int dh = rem / bw, dw = rem - dh * bw;
-            ktab[k] = make_int4((dc * H + dh) * W + dw, dc, dh, dw);
-            if (tw.offp != nullptr)
-                tw.ktab[k] = ktab[k];
-        }
-    }
+    if (blockIdx.x == 0)
+        pack_patch_table(ktab, tw, K, H, W, bh, bw);
     // a wave per (region, instance) with the instances padded to the groups of the layout (of the wider of the two
     // layouts when the launch writes a second one)
     const int lane = threadIdx.x & 63;
@@ -756,6 +760,144 @@ __global__ __launch_bounds__(256) void mex_pack_offsets_kernel(const float *__re
             tw.orng[row2] = grng;
         }
     }
+}
+
+// The same values with a wave to four rows, four instances of a region whose places in the layout are neighbours: their
+// reductions overlap, and 16 bytes leave a lane where four waves stored 4 bytes each into the same lines.  Instances and groups
+// in fours, 64 * KL elements at most.  Launch, one layout, rows x elements (us; the form above before and after its reductions in
+// registers, this one): 1024 x 128 5.2, -, 4.6; 1024 x 192 5.9, -, 4.8; 1024 x 256 6.6, -, 5.6; 2048 x 128 6.7, -, 5.2; 2048 x 256 10.3, -, 6.7;
+// 4096 x 256 17.3, -, 9.7.  Two layouts and the normalized rows: 1024 x 128 6.7, 6.1, 6.5; 2048 x 256 12.9, 12.2, 8.6.
+template <int KL>
+__global__ __launch_bounds__(256) void mex_pack_offsets4_kernel(const float *__restrict__ offsets, int R, int M, int K,
+                                                               int n_mgroups, int tm, int normalize, float scale,
+                                                               int finite_eps, float *__restrict__ offp,
+                                                               float *__restrict__ offe, float *__restrict__ omax,
+                                                               float *__restrict__ orng, int4 *__restrict__ ktab, int H,
+                                                               int W, int bh, int bw, float *__restrict__ normalized_out,
+                                                               MexPackTwin tw, int for_gradients)
+{
+    if (blockIdx.x == 0)
+        pack_patch_table(ktab, tw, K, H, W, bh, bw);
+    const int lane = threadIdx.x & 63;
+    // (the four workgroups of 64 rows numbered 8 apart, see above)
+    unsigned wg = blockIdx.x;
+    if (wg < (gridDim.x & ~31u))
+        wg = (((wg >> 5) * 8 + (wg & 7)) << 2) + ((wg >> 3) & 3);
+    const long long wave = (long long)wg * 4 + (threadIdx.x >> 6);
+    const int Mp = n_mgroups * tm, Mp2 = tw.offp != nullptr ? tw.n_mgroups * tw.tm : 0, fours = max(Mp, Mp2) / 4;
+    if (wave >= (long long)R * fours)
+        return;
+    const int r = (int)(wave / fours), m = 4 * (int)(wave - (long long)r * fours);
+    const bool first = m < Mp, second = m < Mp2;
+    float *dst = offp + ((size_t)r * n_mgroups + m / tm) * K * tm + m % tm;
+    float *dste = offe + (dst - offp);
+    float *dste2 = second ? tw.offe + ((size_t)r * tw.n_mgroups + m / tw.tm) * K * tw.tm + m % tw.tm : nullptr;
+    auto store = [&](float *to, int k, int pitch, const float4 &v) { *reinterpret_cast<float4 *>(to + (size_t)k * pitch) = v; };
+    const size_t row = (size_t)r * Mp + m, row2 = (size_t)r * Mp2 + m;
+    if (m >= M) {
+        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int k = lane; k < K; k += 64) {
+            if (first) {
+                store(dst, k, tm, zero);
+                if (finite_eps)
+                    store(dste, k, tm, zero);
+            }
+            if (second)
+                store(dste2, k, tw.tm, zero);
+        }
+        if (finite_eps && lane < 4) {
+            if (first)
+                omax[row + lane] = orng[row + lane] = 0.0f;
+            if (second)
+                tw.omax[row2 + lane] = tw.orng[row2 + lane] = 0.0f;
+        }
+        return;
+    }
+    const float *src = offsets + ((size_t)r * M + m) * K;
+    float rv[4][KL];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < KL; ++j)
+            rv[i][j] = src[(size_t)i * K + min(lane + 64 * j, K - 1)];   // (behind the last: the last)
+    auto there = [&](int j) { return lane + 64 * j < K; };
+    float xmx[4], xmn[4], lse[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        xmx[i] = -INFINITY;
+        xmn[i] = INFINITY;
+#pragma unroll
+        for (int j = 0; j < KL; ++j) {
+            xmx[i] = fmaxf(xmx[i], rv[i][j]);
+            xmn[i] = fminf(xmn[i], rv[i][j]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        xmx[i] = pack_over_wave(xmx[i], [](float p, float q) { return fmaxf(p, q); });
+        xmn[i] = pack_over_wave(xmn[i], [](float p, float q) { return fminf(p, q); });
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        lse[i] = 0.0f;
+        if (normalize) {
+            const float mxv = fabsf(xmx[i]) < INFINITY ? xmx[i] : 0.0f;
+            float sum = 0.0f;
+#pragma unroll
+            for (int j = 0; j < KL; ++j)
+                sum = there(j) ? sum + mex_exp_term(rv[i][j] - mxv) : sum;
+            lse[i] = mex_lse_of(pack_over_wave(sum, [](float p, float q) { return p + q; }), mxv);
+        }
+    }
+    if (normalized_out != nullptr)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < KL; ++j)
+                if (there(j))
+                    normalized_out[((size_t)r * M + m + i) * K + lane + 64 * j] = rv[i][j] - lse[i];
+    float xh[4], hi[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        xh[i] = scale >= 0.0f ? xmx[i] : xmn[i];
+        hi[i] = mex_scaled_offset(xh[i], lse[i], scale);
+        lo[i] = mex_scaled_offset(scale >= 0.0f ? xmn[i] : xmx[i], lse[i], scale);
+    }
+#pragma unroll
+    for (int j = 0; j < KL; ++j) {
+        if (!there(j))
+            continue;
+        const int k = lane + 64 * j;
+        float v[4], e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = mex_scaled_offset(rv[i][j], lse[i], scale);
+            e[i] = __builtin_amdgcn_exp2f(mex_offset_exponent(rv[i][j], xh[i], lse[i], scale));
+        }
+        if (first)
+            store(dst, k, tm, make_float4(v[0], v[1], v[2], v[3]));
+        if (!finite_eps)
+            continue;
+        if (first)
+            store(dste, k, tm, make_float4(e[0], e[1], e[2], e[3]));
+        if (second)
+            store(dste2, k, tw.tm, make_float4(e[0], e[1], e[2], e[3]));
+    }
+    if (!finite_eps)
+        return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (lane == i) {
+            const float grng = fabsf(hi[i]) > kGradOffsetsSize || fabsf(lo[i]) > kGradOffsetsSize ? INFINITY : hi[i] - lo[i];
+            if (first) {
+                omax[row + i] = hi[i];
+                orng[row + i] = for_gradients ? grng : hi[i] - lo[i];
+            }
+            if (second) {
+                tw.omax[row2 + i] = hi[i];
+                tw.orng[row2 + i] = grng;
+            }
+        }
 }
 
 template <int PX, int KS, int KC>
@@ -1142,7 +1284,13 @@ int mex_pack_offsets(const MexPlan &p, const float *offsets, int tm, int n_mgrou
     hipLaunchKernelGGL(mex_pack_offsets_kernel<KL>, grid, dim3(256), 0, hs, offsets, d.num_regions, d.M, d.K, n_mgroups, \
                        tm, p.normalize_offsets, a->scale, a->finite_eps, offp, offe, omax, orng, ktab, p.H, p.W,         \
                        d.block_h, d.block_w, row_blocks, pj, normalized_out, tw, for_gradients ? 1 : 0)
-    if (d.K <= 64)
+    const bool fours = d.M % 4 == 0 && tm % 4 == 0 && (tw.offp == nullptr || tw.tm % 4 == 0) && extra == 0;
+    // (few elements: more and shorter waves; the line is 1024 rows of 192, see the kernel)
+    if (fours && d.K > 64 && d.K <= 256 && waves * d.K >= 3 << 16)
+        hipLaunchKernelGGL(mex_pack_offsets4_kernel<4>, dim3((unsigned)((waves / 4 + 3) / 4)), dim3(256), 0, hs, offsets, d.num_regions,
+                           d.M, d.K, n_mgroups, tm, p.normalize_offsets, a->scale, a->finite_eps, offp, offe, omax, orng, ktab,
+                           p.H, p.W, d.block_h, d.block_w, normalized_out, tw, for_gradients ? 1 : 0);
+    else if (d.K <= 64)
         SIMNETS_PACK_LAUNCH(1);
     else if (d.K <= 256)
         SIMNETS_PACK_LAUNCH(4);

@@ -38,3 +38,30 @@ def check(got, want, terms):
     assert bool((got[~finite] == want[~finite]).all())
     scale = float(terms[terms.isfinite()].abs().max())
     assert float((got - want)[finite].abs().max()) <= 1e-5 * max(1.0, scale)
+
+
+@pytest.mark.parametrize("normalize", [False, True])
+@pytest.mark.parametrize("eps", [1.0, math.inf])
+@pytest.mark.parametrize("K", [65, 128, 191, 256])
+def test_four_rows_to_a_wave_are_the_same_bits(pkg, K, eps, normalize):
+    """Many rows in fours (mex_pack_offsets4_kernel) and, two instances fewer, not in fours: what both have, padding rows
+    included, is equal.  Rows with infinite entries, of one value, of NaN."""
+    gen = torch.Generator(device="cuda").manual_seed(67)
+    x = torch.randn(8, K, 4, 4, generator=gen, device="cuda")
+    off = torch.randn(4, 732, K, 1, 1, generator=gen, device="cuda") * 2
+    off[0, 3, 2] = -math.inf
+    off[1, 5] = 0.25
+    off[2, 7] = -math.inf
+    off[3, 9, 1] = math.inf
+    off[3, 11] = math.nan
+    go = torch.randn(8, 732, 4, 4, generator=gen, device="cuda")
+    go[:, 730:] = 0
+    results = []
+    for n in (732, 730):
+        leaves = [v.clone().requires_grad_() for v in (x, off[:, :n])]
+        out = pkg.layers.mex(*leaves, n, blocks=[K, 1, 1], strides=[K, 1, 1], unshared_offset_region=[2], epsilon=eps,
+                             softmax_mode=math.isfinite(eps), normalize_offsets=normalize)
+        grads = torch.autograd.grad(out, leaves, go[:, :n])
+        results.append((out.detach()[:, :730], grads[1][:, :730]))
+    for a, b in zip(*results):
+        assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b)) and torch.equal(a.isnan(), b.isnan())
