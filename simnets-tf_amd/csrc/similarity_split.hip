@@ -459,7 +459,7 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
             const int off2 = next_tap();
             return half ? off2 : off;
         };
-        constexpr int kNext = WIDE ? 1 : 0;   // (of a pixel tile and of the one behind it; no registers left for it with four waves)
+        constexpr int kNext = WIDE && NI > 1 ? 1 : 0;   // (of a pixel tile and of the one behind it; no registers left for it with four waves)
         bf16x8 B[1 + kNext][NB];
         auto fetch = [&](bf16x8 (&to)[NB], int off) {
 #pragma unroll
@@ -467,7 +467,7 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
                 to[b] = *reinterpret_cast<const bf16x8 *>(from + off + b * kPlane);
         };
         int off = next_offset();
-        if (WIDE)
+        if (kNext)
             fetch(B[0], at[0] + off);
         auto multiply = [&](int step, bool ask) {   // ask: for the next chunk's values, behind the next step's parameters
             bf16x8 A[NA];
@@ -484,7 +484,7 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
             const int off_next = next_offset();
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
-                if (WIDE) {
+                if (kNext) {
                     fetch(B[(i + 1) & kNext], i + 1 < NI ? at[(i + 1) % NI] + off : at[0] + off_next);
                     __builtin_amdgcn_sched_barrier(0);
                 } else
@@ -501,9 +501,10 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
                 products(lo, 1, 1);
                 products(lo, 1, 0);
                 products(lo, 0, 1);
-                if (WIDE)
+                if (kNext)
                     __builtin_amdgcn_sched_barrier(0);
             }
+            static_assert(!kNext || NI % 2 == 0, "the last of a step fetches the next one's first into place 0");
             off = off_next;
         };
         for (int step = 0; step < a.steps; ++step)
@@ -1077,27 +1078,27 @@ __global__ __launch_bounds__(kThreads, 2) void sim_split_kernel(const SplitArgs 
 #endif
 }
 
-// Forward without missing values, four template tiles to a workgroup of eight waves.
-template <int CG>
+// Forward without missing values, G template tiles, four or two, to a workgroup of eight waves.
+template <int CG, int G>
 __global__ __launch_bounds__(2 * kThreads, 2) void sim_split_forward_wide_kernel(const SplitArgs a, int flag)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int KIND = SPLIT_FWD;
     __shared__ __align__(16) char split_lds[2 * split_lds_bytes(KIND)];
-    const int ptile = split_ptile(), mtile0 = blockIdx.y * 4;
-    split_forward<KIND, CG, 8>(a, split_lds, ptile, mtile0, 4, flag, [&](auto &far, u32x4 &near) __attribute__((always_inline)) {
-        split_body<KIND, CG, 4, 8>(a, split_lds, far, near, ptile, mtile0, flag);
+    const int ptile = split_ptile(), mtile0 = blockIdx.y * G;
+    split_forward<KIND, CG, 8>(a, split_lds, ptile, mtile0, G, flag, [&](auto &far, u32x4 &near) __attribute__((always_inline)) {
+        split_body<KIND, CG, G, 8>(a, split_lds, far, near, ptile, mtile0, flag);
     });
 #endif
 }
 
-// Input gradient, four template tiles to a workgroup of eight waves.
-template <int CG>
+// Input gradient, G template tiles, four or two, to a workgroup of eight waves.
+template <int CG, int G>
 __global__ __launch_bounds__(2 * kThreads, 2) void sim_split_grad_wide_kernel(const SplitArgs a, int flag)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __align__(16) char split_lds[2 * split_lds_bytes(SPLIT_GRAD)];
-    split_grad_body<CG, 4, 8>(a, split_lds, split_ptile(), blockIdx.y * 4, flag);
+    split_grad_body<CG, G, 8>(a, split_lds, split_ptile(), blockIdx.y * G, flag);
 #endif
 }
 
@@ -1263,31 +1264,41 @@ SplitPack sim_split_pack_args(const SimPlan &p, const SplitPlan &sp, const float
     return a;
 }
 
+// Workgroups that are more than half and at most one to a compute unit: eight waves take four template tiles then, or two where
+// four leave fewer, instead of half as many tiles to four waves, two workgroups to a unit, which stage the same pixels twice.
+static bool split_wide_round(long long groups) { return groups > 128 && groups <= 256; }
+
 // Workgroups of eight waves and four template tiles, one to a compute unit, instead of four waves and two, two to a unit: 0.93 of
 // the time of a chip that either kind fills.  A compute unit that gets a single one of the lesser takes 0.55.  All template
 // tiles in fours (96 channels, the last of three tiles' two waves idle: 32 x 96 x 28 x 28 -> 128 76 -> 81 us), and 31 bits for
 // the images of a tile.  Measured, 128 channels, 28 x 28 -> 128, 3 x 3, by the number of tiles (us, before and after):
 // 135 97 -> 83, 172 97 -> 84, 196 93 -> 82, 252 100 -> 92, 392 176 -> 162, 503 189 -> 178; 258 148 -> 159, 343 149 -> 162, left to the others.
 // 1 x 1, 196: 29 -> 22; 5 x 5, 196: 216 -> 204.
-static bool split_grad_wide(const SimPlan &p, const SplitPlan &s)
+// Two tiles of rows, instead of one to four waves: 64 channels, 32 images -> 50, 32.3 -> 29.1; 128 channels, 20 images, 59 -> 55, 12 55 ->
+// 51; 48 x 14 x 14, 192 templates, 72 -> 70; not in chunks of eight channels (5 x 5, 64 -> 64: 62.6 -> 63.6).
+static int split_grad_wide(const SimPlan &p, const SplitPlan &s)
 {
-    const long long touched = (kSplitPixels - 1) / (1LL * p.oh * p.ow) + 2, groups = 1LL * s.n_ptiles * (s.n_mtiles / 4);
-    if (s.n_mtiles % 4 != 0 || 4 * touched * p.C * p.H * p.W >= (1LL << 31))
-        return false;
-    const long long full = groups / 256, rest = groups % 256;
-    return 0.93 * (full + (rest != 0)) < full + (rest == 0 ? 0.0 : rest <= 128 ? 0.55 : 1.0);
+    const long long touched = (kSplitPixels - 1) / (1LL * p.oh * p.ow) + 2;
+    if (4 * touched * p.C * p.H * p.W >= (1LL << 31))
+        return 0;
+    const long long groups = 1LL * s.n_ptiles * (s.n_mtiles / 4), full = groups / 256, rest = groups % 256;
+    if (s.n_mtiles % 4 == 0 && 0.93 * (full + (rest != 0)) < full + (rest == 0 ? 0.0 : rest <= 128 ? 0.55 : 1.0))
+        return 4;
+    return s.cg == 16 && s.n_mtiles % 2 == 0 && split_wide_round(1LL * s.n_ptiles * (s.n_mtiles / 2)) ? 2 : 0;
 }
 
 // The forward's: where the workgroups of four waves and two template tiles are more than one and at most two to a compute
 // unit.  Fewer leave compute units to share; more run as four tiles to four waves, two workgroups to a unit, which is the faster
 // form of a full chip (256 x 64 x 32 x 32 -> 128, 3 x 3: 219 us, this form 267).  Measured, 128 channels, 28 x 28 -> 128, 3 x 3, by the
 // number of tiles (us, before and after): 135 64 -> 58, 196 68 -> 62, 252 72 -> 67; 1 x 1, 196: 28 -> 23; 5 x 5, 196: 143 -> 143;
+// two tiles to a workgroup, 64 templates 51.6 -> 46.0, 1 x 1 24 -> 21, 128 templates, 20 images, 52 -> 46, 12 images 48 -> 43;
 // three tiles of 75 templates, 30 x 45 x 29 x 35, 238: 32 -> 28.  With missing values no gain (22 x 128 x 28 x 28: 95 -> 95; 64 x 64 x 32 x
 // 32: 103 -> 107).
-static bool split_forward_wide(const SplitPlan &s)
+static int split_forward_wide(const SplitPlan &s)
 {
-    const long long groups = 1LL * s.n_ptiles * ((s.n_mtiles + 3) / 4);
-    return (s.n_mtiles % 4 == 0 || s.n_mtiles % 4 == 3) && groups > 128 && groups <= 256;
+    if ((s.n_mtiles % 4 == 0 || s.n_mtiles % 4 == 3) && split_wide_round(1LL * s.n_ptiles * ((s.n_mtiles + 3) / 4)))
+        return 4;
+    return s.n_mtiles % 2 == 0 && split_wide_round(1LL * s.n_ptiles * (s.n_mtiles / 2)) ? 2 : 0;
 }
 
 template <int KIND>
@@ -1314,20 +1325,15 @@ static int split_launch(const SimPlan &p, const SplitPlan &sp, const float *inpu
     a.d_hv = make_fast_div((unsigned)sp.Hv);
     a.d_taps = make_fast_div((unsigned)a.taps);
     a.d_bw = make_fast_div((unsigned)p.bw);
-    if (KIND == SPLIT_GRAD && split_grad_wide(p, sp)) {
-        const dim3 grid((unsigned)sp.n_ptiles, (unsigned)(sp.n_mtiles / 4));
-        if (sp.cg == 16)
-            hipLaunchKernelGGL(sim_split_grad_wide_kernel<16>, grid, dim3(2 * kThreads), 0, s, a, flag);
-        else
-            hipLaunchKernelGGL(sim_split_grad_wide_kernel<8>, grid, dim3(2 * kThreads), 0, s, a, flag);
-        return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
-    }
-    if (KIND == SPLIT_FWD && split_forward_wide(sp)) {
-        const dim3 grid((unsigned)sp.n_ptiles, (unsigned)((sp.n_mtiles + 3) / 4));
-        if (sp.cg == 16)
-            hipLaunchKernelGGL(sim_split_forward_wide_kernel<16>, grid, dim3(2 * kThreads), 0, s, a, flag);
-        else
-            hipLaunchKernelGGL(sim_split_forward_wide_kernel<8>, grid, dim3(2 * kThreads), 0, s, a, flag);
+    const int wide = KIND == SPLIT_FWD ? split_forward_wide(sp) : KIND == SPLIT_GRAD ? split_grad_wide(p, sp) : 0;
+    if (wide) {
+        const dim3 grid((unsigned)sp.n_ptiles, (unsigned)((sp.n_mtiles + wide - 1) / wide));
+        void (*const kernels[2][2][2])(SplitArgs, int) = {
+            {{sim_split_forward_wide_kernel<8, 2>, sim_split_forward_wide_kernel<8, 4>},
+             {sim_split_forward_wide_kernel<16, 2>, sim_split_forward_wide_kernel<16, 4>}},
+            {{nullptr /* see split_grad_wide */, sim_split_grad_wide_kernel<8, 4>},
+             {sim_split_grad_wide_kernel<16, 2>, sim_split_grad_wide_kernel<16, 4>}}};
+        hipLaunchKernelGGL(kernels[KIND == SPLIT_GRAD][sp.cg == 16][wide == 4], grid, dim3(2 * kThreads), 0, s, a, flag);
         return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
     }
     // as many template tiles per staged pixel tile as leave a workgroup for every compute unit

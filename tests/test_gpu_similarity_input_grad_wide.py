@@ -22,6 +22,10 @@ TOL = 8e-7
     ((4, 128, 20, 250), 33, 3),        # wide rows
     ((3, 128, 80, 100), 33, 5),        # chunks of eight
     ((400, 112, 7, 7), 64, 3),         # three images to a tile
+    ((32, 64, 28, 28), 40, 3),         # two tiles of rows to a workgroup
+    ((12, 100, 28, 28), 33, 3),        # ... two groups of them
+    ((32, 50, 28, 28), 33, 5),         # chunks of eight: four waves
+    ((25, 48, 32, 32), 64, 1),         # ... a step a chunk
     ((44, 128, 28, 28), 30, 3),        # 270 tiles: four waves
     ((32, 96, 28, 28), 30, 3),         # three tiles of rows: four waves
 ])

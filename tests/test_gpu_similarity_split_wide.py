@@ -20,6 +20,9 @@ GEOMS = [
     ((40, 70, 24, 24), 128, 1),    # a step a chunk
     ((22, 24, 28, 28), 128, 5),    # chunks of eight channels
     ((18, 32, 28, 28), 256, 3),    # two groups of templates
+    ((32, 40, 28, 28), 50, 3),     # two tiles to a workgroup
+    ((12, 24, 28, 28), 100, 3),    # ... and two groups of them
+    ((22, 24, 28, 28), 64, 5),     # ... chunks of eight channels
 ]
 
 
@@ -77,9 +80,10 @@ def test_inputs_on_another_scale(pkg, geom, kind):
     check(pkg, x, t, w, geom[2], tol=2 * TOL)
 
 
+@pytest.mark.parametrize("templates", [128, 64])
 @pytest.mark.parametrize("pixels, copies", [(3, 1), (50, 1), (100, 1), (64, 2), (100, 4)])
-def test_outputs_near_a_template(pkg, pixels, copies):
-    x, t, w = tensors(GEOMS[3])
+def test_outputs_near_a_template(pkg, pixels, copies, templates):
+    x, t, w = tensors((GEOMS[3][0], templates, 1))
     t[:copies] = t[40]
     t[40:40 + copies] = t[40].clone()
     flat = x.view(x.shape[0], x.shape[1], -1)
