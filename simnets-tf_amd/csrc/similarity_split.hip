@@ -58,6 +58,7 @@
 #include "fast_div.h"
 #include "internal.h"
 #include "sim_split.h"
+#include "split_channel.h"
 
 namespace simnets {
 
@@ -350,7 +351,7 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
         const int vr = (int)fast_div((unsigned)q, a.d_wp), c = q - vr * a.Wp - a.pw;
         const int v = v0 + vr, img = (int)fast_div((unsigned)v, a.d_hv), r = v - img * a.Hv - a.ph;
         const bool in = q < staged && r >= 0 && r < a.H && c >= 0 && c < a.W;
-        src[i] = in ? (unsigned)((((img - first) * a.C + 8 * g) * a.H + r) * a.W + c) * (WIDE ? 4u : 1u) : kOutside;
+        src[i] = in ? (unsigned)((((img - first) * a.C + split_group_start(a.C, g)) * a.H + r) * a.W + c) * (WIDE ? 4u : 1u) : kOutside;
     }
     // and this lane's operands: the LDS byte address of its pixel's first tap
     int at[NI];
@@ -383,10 +384,10 @@ __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, i
         const int item = wave + WAVES * i;
         if (item >= kHalves * per_half)
             return;
-        const int g = CG == 16 && item >= per_half, there = a.C - 1 - (chunk * CG + 8 * g);
+        const int g = CG == 16 && item >= per_half, start = split_group_start(a.C, g);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const unsigned channel = chunk * CG + max(-8 * g, min(j, there));
+            const unsigned channel = split_channel_offset(a.C, start, chunk * CG, j);
             if (WIDE)
                 x[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, src[i], channel * plane * 4u, 0));
             else
@@ -669,17 +670,19 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
         next[q] = pp[q * 64 + lane];
 
     float x[kItems][8];
-    auto request = [&](int chunk) {   // a chunk's values of this lane's pixels, channels behind the last as the last
+    // a chunk's values of this lane's pixels (patches of 64 elements at least: eight channels or fewer come in chunks of eight, so
+    // that a group's start has a channel)
+    auto request = [&](int chunk) {
 #pragma unroll
         for (int i = 0; i < kItems; ++i) {
             const int item = wave + kWaves * i;
             if (item >= kHalves * per_half)
                 continue;
-            const int g = CG == 16 && item >= per_half, there = a.C - 1 - (chunk * CG + 8 * g);
+            const int g = CG == 16 && item >= per_half;
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 x[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                    rsrc, src[i], (chunk * CG + max(-8 * g, min(j, there))) * plane, 0));
+                    rsrc, src[i], split_channel_offset(a.C, 8 * g, chunk * CG, j) * plane, 0));
         }
     };
     int level = 0;

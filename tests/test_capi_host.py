@@ -308,6 +308,35 @@ int main() {
     assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.strip() == "0"
 
 
+def test_channels_of_split_kernels_lie_in_the_tensor(tmp_path):
+    # csrc/split_channel.h (where the split matrix kernels read a chunk's channels): the offset from a group's start is
+    # unsigned on the device, and what it leads to is a channel - the wanted one, or the last behind the last
+    src = tmp_path / "sc.cpp"
+    src.write_text(r"""
+#include <cstdio>
+#include "split_channel.h"
+using namespace simnets;
+int main() {
+    long bad = 0;
+    for (int C = 1; C <= 100; ++C)
+        for (int cg = 8; cg <= 16; cg += 8)
+            for (int first = 0; first < C; first += cg)
+                for (int g = 0; g < cg / 8; ++g)
+                    for (int j = 0; j < 8; ++j) {
+                        const int start = split_group_start(C, g), offset = split_channel_offset(C, start, first, j);
+                        const int wanted = first + 8 * g + j;
+                        bad += offset < 0 || start + offset >= C || (wanted < C && start + offset != wanted);
+                    }
+    printf("%ld\n", bad);
+    return 0;
+}
+""")
+    exe = tmp_path / "sc"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I" + os.path.join(ROOT, "simnets-tf_amd", "csrc"), str(src), "-o",
+                    str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.strip() == "0"
+
+
 def test_sum_pool_input_grad_validates_like_the_forward_call(pkg):
     l = pkg._lib.lib()
     I4 = C.c_int * 4

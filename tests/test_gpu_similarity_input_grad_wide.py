@@ -28,6 +28,9 @@ TOL = 8e-7
     ((25, 48, 32, 32), 64, 1),         # ... a step a chunk
     ((44, 128, 28, 28), 30, 3),        # 270 tiles: four waves
     ((32, 96, 28, 28), 30, 3),         # three tiles of rows: four waves
+    ((32, 32, 28, 28), 7, 1),          # eight templates or fewer, in a chunk of sixteen: four waves
+    ((32, 64, 28, 28), 8, 1),          # ... eight
+    ((32, 64, 28, 28), 9, 1),
 ])
 def test_input_gradient(pkg, shape, templates, block):
     gen = torch.Generator(device="cuda").manual_seed(43)
