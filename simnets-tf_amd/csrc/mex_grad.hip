@@ -1222,11 +1222,10 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                     }
                 }
             }
-            if (s > 0) {               // (each chunk decides for itself; its last readers are behind a barrier)
-                if (lane == 0)
-                    wide_sh[wave] = unbounded;
-                __syncthreads();
-            }
+            // each chunk decides for itself: behind the readers of the ranges' flags above, or of the chunk's before
+            if (s > 0 && lane == 0)
+                wide_sh[wave] = unbounded;
+            __syncthreads();
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 for (int d = 16; d < 64; d <<= 1) {

@@ -73,3 +73,26 @@ def test_row_wise_gradients(pkg, shape, n, spread, outlier, normalize):
     want = pkg.mex_grads(x, raw, full, pkg.sum_pooling_input_grad(gp, full.shape, (2, 2)), n, **kw)
     got = pkg.mex_sum_pool_grads(x, raw, full, gp, n, (2, 2), **kw)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("shape", [(65930, 6, 2, 2), (1030, 6, 16, 16)])   # two chunks to a workgroup
+def test_pixels_of_one_chunk_leave_the_next_ones_alone(pkg, shape):
+    """Offsets that span 29 exponents, so that each chunk's pixels decide; those of the first chunk send all four regions
+    term by term.  The input's gradient of the other chunks is the same bits as without them."""
+    gen = torch.Generator(device="cuda").manual_seed(101)
+    b, c, h, w = shape
+    n, chunk = 5, 256 // (h * w)   # (images)
+    off = torch.rand(4, n, c, 1, 1, generator=gen, device="cuda") * 20
+    off[:, 0, 0], off[:, 0, 1] = 0, 20
+    g = torch.randn(b, n, h, w, generator=gen, device="cuda")
+    kw = dict(blocks=[c, 1, 1], strides=[c, 1, 1], unshared_offset_region=[2], softmax_mode=True)
+    results = []
+    for outlier in (False, True):
+        x = torch.randn(shape, generator=torch.Generator(device="cuda").manual_seed(103), device="cuda")
+        if outlier:
+            x[0, 0, :2, :2], x[0, 1, :2, :2] = 70, -70
+        out, want_x, want_off = reference(x, off, g)
+        dx, doff = pkg.mex_grads(x, off, out, g, n, **kw)
+        assert max(err(dx, want_x), err(doff, want_off)) <= TOL
+        results.append(dx)
+    assert torch.equal(results[0][chunk:], results[1][chunk:])
