@@ -973,8 +973,11 @@ __device__ __forceinline__ T rows_load(const float *base, unsigned at)
     return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + 4 * at);
 }
 
-// per region: is some instance's offsets range beyond kGradRowsRange or not finite (flags[r]: term by term); flags[4]:
-// does some range exceed kLooseBoundRange.  All threads of the workgroup call flag(); the flags (five, zero before a
+// What a region does term by term: bits of the flags below.
+enum { kRowsInput = 1, kRowsOffsets = 2 };
+
+// per region: is some instance's offsets range beyond kGradRowsRange or not finite (flags[r]: both gradients term by term);
+// flags[4]: does some range exceed kLooseBoundRange.  All threads of the workgroup call flag(); the flags (five, zero before a
 // barrier) are in place behind the next one.  The constructor requests the first 256 instances' ranges.
 struct RowsRanges {
     float v[4];
@@ -996,7 +999,7 @@ struct RowsRanges {
                 if (m < g.M && !(v[r] <= kLooseBoundRange)) {
                     flags[4] = 1;      // (every writer writes the same value)
                     if (!(v[r] <= kGradRowsRange))
-                        flags[r] = 1;
+                        flags[r] = kRowsInput | kRowsOffsets;
                 }
             m += 256;
             if (m >= g.M)
@@ -1005,6 +1008,8 @@ struct RowsRanges {
         }
     }
 };
+
+constexpr int kLateOffsets = 1 << 16;
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // The term-by-term path of the kernel below reads its arguments from the kernel's argument segment (they are the last, in front
@@ -1016,9 +1021,9 @@ __device__ __forceinline__ const MexGradArgs &rows_term_args()
                                                   sizeof(MexGradArgs));
 }
 
-// The regions with a wide offsets range, or with a chunk's wide pixels: late holds a bit per chunk for each.  GX_KT patch elements of
-// a region per wave and turn for the input gradient; for the offsets the tile of KT patch elements as GO_MT x GO_KT wave
-// tiles over all chunks.
+// The regions with a wide offsets range, or with a chunk's wide pixels: late holds a bit per chunk (sixteen at most) for the input
+// gradient of each, and kLateOffsets.  GX_KT patch elements of a region per wave and turn for the input gradient; for the offsets
+// the tile of KT patch elements as GO_MT x GO_KT wave tiles over all chunks.
 // (Arguments of a call are in vector registers: all are uniform.)
 template <int KT>
 __device__ __noinline__ void rows_terms(int bx_v, int n_chunks_v, int k0_v, int mg_begin_v, int mg_end_v, float *dx_v, int offsets_v,
@@ -1045,7 +1050,7 @@ __device__ __noinline__ void rows_terms(int bx_v, int n_chunks_v, int k0_v, int 
         for (int m0 = m_begin; m0 < m_end; m0 += 32)
             for (int u = wave; u < 4 * NM * NO; u += 4) {
                 const int r = u / (NM * NO), i = u % (NM * NO), mm0 = m0 + i / NO * GO_MT, kk0 = k0 + i % NO * GO_KT;
-                if (late[r] && mm0 < M && kk0 < K)
+                if ((late[r] & kLateOffsets) && mm0 < M && kk0 < K)
                     mex_grad_offsets_wave(ga, r, bx, mm0, kk0, lane);
             }
 }
@@ -1182,7 +1187,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
 
     const bool nothing = (wide_sh[0] & wide_sh[1] & wide_sh[2] & wide_sh[3]) != 0;   // all four regions
     if (nothing && tid < 4)
-        late[tid] = (1 << n_chunks) - 1;
+        late[tid] = (1 << n_chunks) - 1 | kLateOffsets;
     for (int s = nothing ? n_chunks : 0; s < n_chunks; ++s) {
         asm volatile("" : "+v"(pl0));   // (what follows from it is cheap to form again, and too much to keep across the chunks)
         if (s > 0) {
@@ -1232,9 +1237,13 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                     bound[e] = fmaxf(bound[e], __shfl_xor(bound[e], d, 64));
                     alo[e] = fminf(alo[e], __shfl_xor(alo[e], d, 64));
                 }
-                // a pixel with an infinite value, nothing finite, or a patch range beyond the bound sends its region term by term
-                if (img_ok && !(fabsf(bound[e]) < INFINITY && bound[e] - alo[e] <= kGradPixelRange))
-                    wide_sh[q0.region(e)] = 1;
+                // A pixel with an infinite value or nothing finite sends its region term by term, one with a patch range
+                // beyond the bound the region's input gradient.  (To the offsets' gradient a patch element far below the pixel's
+                // largest adds next to nothing: W is 2^kGradRowsRange of g at most.  512 x 32 x 16 x 16 -> 64, such a
+                // pixel in each image: 45 us where the offsets' gradient took 192 term by term, both 105 and 255.)
+                const bool finite = fabsf(bound[e]) < INFINITY;
+                if (img_ok && !(finite && bound[e] - alo[e] <= kGradPixelRange))
+                    atomicOr(&wide_sh[q0.region(e)], finite ? kRowsInput : kRowsInput | kRowsOffsets);
             }
         } else {
 #pragma unroll
@@ -1321,7 +1330,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
             else if (want_input)
                 request_input();
             __syncthreads();
-            if (want_input && !my_wide) {
+            if (want_input && !(my_wide & kRowsInput)) {
                 // (lane lq: instances 8 lq + i)
                 float av[KSUB][2][4];
 #pragma unroll
@@ -1340,7 +1349,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                             acc[ks][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[ks][i / 4][i % 4], bv[t], acc[ks][t], 0, 0, 0);
                 }
             }
-            if (want_offsets && !my_wide) {
+            if (want_offsets && !(my_wide & kRowsOffsets)) {
                 floatx4 sum[2][KSUB];
 #pragma unroll
                 for (int mt = 0; mt < 2; ++mt)
@@ -1391,7 +1400,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
             }
         }
         if (my_wide && lane == 0)
-            late[wave] |= 1 << s;
+            late[wave] |= ((my_wide & kRowsInput) != 0 ? 1 << s : 0) | ((my_wide & kRowsOffsets) != 0 ? kLateOffsets : 0);
 
         // ---- d patch_k = 2^(xs_k - a) * acc: through the tile [patch element][column] to rows of the gradient ----
         __syncthreads();               // the last matrix steps are done with the tile and the tables
@@ -1403,7 +1412,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                     *reinterpret_cast<float4 *>(by_col + (ks * 16 + 4 * lq + v) * TP) =
                         make_float4(acc[ks][0][v], acc[ks][1][v], acc[ks][2][v], acc[ks][3][v]);
             __syncthreads();
-            const bool any_wide = (wide_sh[0] | wide_sh[1] | wide_sh[2] | wide_sh[3]) != 0;
+            const bool any_wide = ((wide_sh[0] | wide_sh[1] | wide_sh[2] | wide_sh[3]) & kRowsInput) != 0;
             float *dst = dxo + first;
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
@@ -1421,7 +1430,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (!wide_sh[q0.region(e)])
+                        if (!(wide_sh[q0.region(e)] & kRowsInput))
                             to[e] = d[e];
                 }
             }

@@ -96,3 +96,29 @@ def test_pixels_of_one_chunk_leave_the_next_ones_alone(pkg, shape):
         assert max(err(dx, want_x), err(doff, want_off)) <= TOL
         results.append(dx)
     assert torch.equal(results[0][chunk:], results[1][chunk:])
+
+
+@pytest.mark.parametrize("value", [-70, -float("inf")])
+@pytest.mark.parametrize("shape", [(65930, 6, 2, 2), (1030, 6, 16, 16), (70, 24, 8, 4)])
+def test_offsets_gradient_keeps_its_form_for_wide_pixels(pkg, shape, value):
+    """Offsets that span 29 exponents and pixels that span more than 64: the input's gradient is formed term by term, the
+    offsets' as without them - the same bits where those pixels' output gradients are zero."""
+    gen = torch.Generator(device="cuda").manual_seed(107)
+    b, c, h, w = shape
+    n = 5
+    off = torch.rand(4, n, c, 1, 1, generator=gen, device="cuda") * 20
+    off[:, 0, 0], off[:, 0, 1] = 0, 20
+    g = torch.randn(b, n, h, w, generator=gen, device="cuda")
+    kw = dict(blocks=[c, 1, 1], strides=[c, 1, 1], unshared_offset_region=[2], softmax_mode=True)
+    results = []
+    for outlier in (False, True):
+        x = torch.randn(shape, generator=torch.Generator(device="cuda").manual_seed(103), device="cuda")
+        if outlier:
+            x[::7, 0, :2, :2], x[::7, 1, :2, :2] = 70, value
+        out, want_x, want_off = reference(x, off, g)
+        dx, doff = pkg.mex_grads(x, off, out, g, n, **kw)
+        assert max(err(dx, want_x), err(doff, want_off)) <= TOL
+        quiet = g.clone()
+        quiet[::7, :, :2, :2] = 0
+        results.append(pkg.mex_offsets_grad(x, off, out, quiet, n, **kw))
+    assert torch.equal(*results)
