@@ -1011,6 +1011,19 @@ struct RowsRanges {
 
 constexpr int kLateOffsets = 1 << 16;
 
+// A product and a sum with a rounding each, whatever else is fused: two kernels add up the same partial sums, bit for bit.
+__device__ __forceinline__ float rows_product(float a, float b)
+{
+#pragma clang fp contract(off)
+    return a * b;
+}
+
+__device__ __forceinline__ float rows_sum(float a, float b)
+{
+#pragma clang fp contract(off)
+    return a + b;
+}
+
 #if defined(__HIP_DEVICE_COMPILE__)
 // The term-by-term path of the kernel below reads its arguments from the kernel's argument segment (they are the last, in front
 // of the implicit ones) and is a call: inlined, what it keeps in scalar registers is fetched, and spilled, at the kernel's start.
@@ -1071,17 +1084,24 @@ __device__ __noinline__ void rows_terms(int bx_v, int n_chunks_v, int k0_v, int 
 // The two gradients were a kernel each: both read `out` and `g` and formed W, the one for the offsets once more for every 32 patch
 // elements.  512 images, whole call, 32 channels of 16 x 16 -> 64
 // instances, 64 of 8 x 8 -> 128, 128 of 4 x 4 -> 256, 256 of 2 x 2 -> 512: both gradients 57, 54, 59, 72 -> 44, 39, 41, 52 us, the
-// input's alone 27.5, 27.5, 34, 48 -> 29, 26, 29, 40, the offsets' alone, with twice the partial sums, 34, 30, 32.5, 46 -> 38, 34, 33,
-// 42.  32 images, both, the kernels of four such layers and their sums: 118 -> 75.  The bound is taken over the first group's
+// input's alone 27, 27, 33, 47 -> 24.5, 21, 27, 34, the offsets' alone 34, 30, 32, 45 -> 31.5 (mex_grad_offsets_rows_kernel), 30, 29, 37.
+// 32 images, both, the kernels of four such layers and their sums: 118 -> 75.  The bound is taken over the first group's
 // instances: errors against 64 bits as before, and a third to a half of it for offsets that span 24 to 48 exponents on 2 x 2 maps.
 // W2: the map has two columns, a quad is a window and its pixels belong to the four regions.
+// WANT: the only gradient wanted, or 0.  Compiled for one alone the kernel needs 20 to 30 registers less, none of them in memory: 28.5, 25,
+// 28.5, 37.5 and 37.5, 33.5, 32.5, 40.5 us where both are decided at run time.  (Compiled for both: 44 -> 46.5, 39 -> 41 on the
+// first and third.)
 //
 // The tile's pitch, 20 modulo 64: sixteen lanes' 16-byte operands of a column of rows, or of a row, lie in different banks.
-template <int KSUB, bool W2, bool POOLED>
+template <int KSUB, bool W2, bool POOLED, int WANT>
 __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(const RowsArgs g, const MexGradArgs ga)
 {
     constexpr int KT = 16 * KSUB, NJ = KT / 4;
     constexpr int TP = 276, EP = 36;
+    // The pixel's own maximum as the bound where the tile holds all of K: at hand for the offsets, one pass more over those rows for
+    // the input alone.  Both 44 -> 42.6 us (512 x 32 x 16 x 16 -> 64), input 22.8 -> 24.5, errors of offsets that span 20 exponents 3.8e-7
+    // -> 2.7e-7.  (KSUB 1: no registers left for it, 512 x 64 x 8 x 8 -> 128 37.8 -> 38.7.)
+    constexpr bool kTight = KSUB == 2;
     __shared__ __attribute__((aligned(16))) float wt[32 * TP];        // W, and before and behind it the patch elements' tile
     __shared__ __attribute__((aligned(16))) float eo[4 * KT * EP];    // [region][patch element][instance]
     __shared__ float tab[2][128];      // per (region, instance of the group): omax + c0, for this group and the next
@@ -1094,7 +1114,8 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
     int bx, by, bz;
     if (!rows_block(g, &bx, &by, &bz))
         return;
-    const bool want_input = g.dx != nullptr, want_offsets = g.partial != nullptr;
+    const bool want_input = WANT == kRowsInput || (WANT == 0 && g.dx != nullptr);
+    const bool want_offsets = WANT == kRowsOffsets || (WANT == 0 && g.partial != nullptr);
     const int k0 = by * KT;
     const int n_mg = g.n_mg, per = n_mg * GM_TM;
     const int mg_begin = bz * g.mg_per_split, mg_end = min(n_mg, mg_begin + g.mg_per_split);
@@ -1204,14 +1225,14 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
         // kGradProductRange, the product form): there it is the pixel's own maximum over all of K, from one sweep over
         // the rows of the input.  The exponents then stay within the pixel's patch range, and a region keeps the
         // product form while those ranges are at most kGradPixelRange and its offsets span at most kGradRowsRange.
-        float bound[4];
-        if (roomy) {
-            float alo[4];
+        // (Where the tile holds all of K the maximum is at hand, whatever the ranges.)
+        float bound[4], alo[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                bound[e] = -INFINITY;
-                alo[e] = INFINITY;
-            }
+        for (int e = 0; e < 4; ++e) {
+            bound[e] = -INFINITY;
+            alo[e] = INFINITY;
+        }
+        if (roomy || (kTight && g.K <= KT && !want_offsets)) {
             for (int k = pl0; k < g.K; k += 32) {
                 float4 xr[8];
 #pragma unroll
@@ -1227,6 +1248,16 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                     }
                 }
             }
+        } else if (kTight && g.K <= KT) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float v[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    bound[e] = fmaxf(bound[e], v[e] * g.c1);
+            }
+        }
+        if (roomy) {
             // each chunk decides for itself: behind the readers of the ranges' flags above, or of the chunk's before
             if (s > 0 && lane == 0)
                 wide_sh[wave] = unbounded;
@@ -1245,6 +1276,11 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                 if (img_ok && !(finite && bound[e] - alo[e] <= kGradPixelRange))
                     atomicOr(&wide_sh[q0.region(e)], finite ? kRowsInput : kRowsInput | kRowsOffsets);
             }
+        } else if (kTight && g.K <= KT) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                for (int d = 16; d < 64; d <<= 1)
+                    bound[e] = fmaxf(bound[e], __shfl_xor(bound[e], d, 64));
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -1295,11 +1331,9 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
 #pragma unroll
             for (int t = 0; t < 4; ++t)
                 acc[ks][t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-        int my_wide = unbounded;
         for (int mg = mg_begin; mg < mg_end; ++mg) {
             __syncthreads();           // everyone is done with the tile, the offset exponentials and the flags
             const float *tb = tab[mg & 1];
-            my_wide = __builtin_amdgcn_readfirstlane(wide_sh[wave]);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int pl = pl0 + 4 * j;
@@ -1330,7 +1364,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
             else if (want_input)
                 request_input();
             __syncthreads();
-            if (want_input && !(my_wide & kRowsInput)) {
+            if (want_input) {
                 // (lane lq: instances 8 lq + i)
                 float av[KSUB][2][4];
 #pragma unroll
@@ -1349,7 +1383,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                             acc[ks][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[ks][i / 4][i % 4], bv[t], acc[ks][t], 0, 0, 0);
                 }
             }
-            if (want_offsets && !(my_wide & kRowsOffsets)) {
+            if (want_offsets) {
                 floatx4 sum[2][KSUB];
 #pragma unroll
                 for (int mt = 0; mt < 2; ++mt)
@@ -1381,7 +1415,7 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                         float add[4];
 #pragma unroll
                         for (int v = 0; v < 4; ++v)
-                            add[v] = sum[mt][kt][v] * e[v * EP];
+                            add[v] = rows_product(sum[mt][kt][v], e[v * EP]);
                         if (m >= g.M || k >= g.K)
                             continue;
                         float *at = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + 4 * ((unsigned)m * g.K + k));
@@ -1389,16 +1423,18 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
                             float4 old = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                             if (s > 0)
                                 old = *reinterpret_cast<const float4 *>(at);
-                            *reinterpret_cast<float4 *>(at) = make_float4(old.x + add[0], old.y + add[1], old.z + add[2], old.w + add[3]);
+                            *reinterpret_cast<float4 *>(at) = make_float4(rows_sum(old.x, add[0]), rows_sum(old.y, add[1]),
+                                                                          rows_sum(old.z, add[2]), rows_sum(old.w, add[3]));
                         } else {
 #pragma unroll
                             for (int v = 0; v < 4; ++v)
                                 if (k + v < g.K)
-                                    at[v] = s > 0 ? at[v] + add[v] : add[v];
+                                    at[v] = s > 0 ? rows_sum(at[v], add[v]) : add[v];
                         }
                     }
             }
         }
+        const int my_wide = __builtin_amdgcn_readfirstlane(wide_sh[wave]);   // (its products are left unused)
         if (my_wide && lane == 0)
             late[wave] |= ((my_wide & kRowsInput) != 0 ? 1 << s : 0) | ((my_wide & kRowsOffsets) != 0 ? kLateOffsets : 0);
 
@@ -1442,6 +1478,243 @@ __global__ __launch_bounds__(256, KSUB == 1 ? 3 : 2) void mex_grads_rows_kernel(
     if ((late[0] | late[1] | late[2] | late[3]) != 0)
         rows_terms<KT>(bx, n_chunks, k0, mg_begin, mg_end, want_input ? dxo : nullptr, want_offsets,
                        make_int4(late[0], late[1], late[2], late[3]));
+#endif
+}
+
+// The offsets gradient by itself, on maps of four columns and more: of layers whose two gradients are a kernel each
+// (MexGradTiling::rows_apart), and wanted alone where the tile holds all of K, bit for bit as mex_grads_rows_kernel gives it.
+// Workgroup (rows_block) x: group of ga.pxl chunks; y: tile of 32 patch elements; z: group of instances.  Per chunk the group's
+// pixel factors W and the tile's patch exponentials are formed side by side, and wave r takes region r's 32 x 32 products over
+// its 64 columns: the sums stay in registers over the chunks, and the next chunk's rows are requested in front of the matrix
+// steps.  (In the other kernel a workgroup's sums, of all instance groups, are too many for that: each chunk's are added to
+// what is stored.)  The bound is the pixel's maximum where the tile holds all of K or some offsets range is large, as there, and
+// over the group's own instances otherwise.
+// Bound by the exponentials and their way through LDS, two workgroups to a compute unit.  Offsets alone, this kernel and the
+// other: 512 x 32 x 16 x 16 -> 64 31.5, 32.8 us, 2048 x 32 x 16 x 16 -> 64 82, 103; 512 x 96 x 16 x 16 -> 192 134, 177.
+template <bool POOLED>
+__global__ __launch_bounds__(256, 2) void mex_grad_offsets_rows_kernel(const RowsArgs g, const MexGradArgs ga)
+{
+    constexpr int TP = 276;            // (see mex_grads_rows_kernel)
+    __shared__ __attribute__((aligned(16))) float wt[32 * TP];   // [instance][column]
+    __shared__ __attribute__((aligned(16))) float et[32 * TP];   // [patch element][column]
+    __shared__ int wide_sh[5];         // see RowsRanges
+    __shared__ int odd_sh[4];          // per region: met a pixel that only the term-by-term path can take
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lq = lane >> 4;
+    int bx, by, mg;
+    if (!rows_block(g, &bx, &by, &mg))
+        return;
+    const int k0 = by * 32, per = g.n_mg * GM_TM;
+    const RowsQuad<false> q0(g, 0, wave * 16 + (lane & 15));
+    const int tile0 = lq * TP + q0.col(0);   // of row lq + 4 j
+    auto tile_index = [&](int j, int e) { return tile0 + 4 * j * TP + (e & 1) * 64 + (e >> 1); };
+
+    typedef typename RowsGrad<false, POOLED>::type Grad;
+    float4 ov[8], xv[8];
+    Grad gv[8];
+    const int gplane = POOLED ? g.HW >> 2 : g.HW;
+    const float *x_c;
+    unsigned x_at;
+    bool img_ok;
+    auto request = [&](int chunk) {    // (those past the last instance, image or patch element on a clamped address)
+        const RowsQuad<false> q(g, chunk, wave * 16 + (lane & 15));
+        const int img0 = chunk * 256 >> g.lgHW;
+        img_ok = q.img < g.B;
+        const unsigned img = img_ok ? q.img - img0 : 0;
+        const float *out_c = g.out + (size_t)img0 * g.M * g.HW, *g_c = g.g + (size_t)img0 * g.M * gplane;
+        const unsigned out_at = img * g.M * g.HW + q.pix0, g_at = img * g.M * gplane + (POOLED ? q.window(g) : q.pix0);
+        x_c = g.in + (size_t)img0 * g.K * g.HW;
+        x_at = img * g.K * g.HW + q.pix0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const unsigned m = min(mg * GM_TM + lq + 4 * j, g.M - 1);
+            ov[j] = rows_load<float4>(out_c, out_at + m * g.HW);
+            gv[j] = rows_load<Grad>(g_c, g_at + m * gplane);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            xv[j] = rows_load<float4>(x_c, x_at + (unsigned)min(k0 + lq + 4 * j, g.K - 1) * g.HW);
+    };
+    const int n_chunks = min(g.pxl, g.chunks - bx * g.pxl);
+    RowsRanges ranges(g, tid);
+    // this thread's instances in its two regions: c0 + the offsets' largest, and smallest
+    float hi[8][2], lo[8][2];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int at = q0.region(e) * per + mg * GM_TM + lq + 4 * j;   // (the packed arrays are padded to whole groups)
+            hi[j][e] = g.omax[at];
+            lo[j][e] = g.orng[at];
+        }
+    if (tid < 5)
+        wide_sh[tid] = 0;
+    if (tid < 4)
+        odd_sh[tid] = 0;
+    request(bx * g.pxl);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            lo[j][e] = g.c0 + (hi[j][e] - lo[j][e]);
+            hi[j][e] += g.c0;
+        }
+    __syncthreads();
+    ranges.flag(g, tid, wide_sh);
+    __syncthreads();
+    const bool roomy = wide_sh[4] != 0;
+    const bool nothing = (wide_sh[0] & wide_sh[1] & wide_sh[2] & wide_sh[3]) != 0;   // all four regions term by term
+
+    floatx4 total[2][2];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+            total[mt][kt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    float eov[2][2][4];                // the offset exponentials of the sums
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                eov[mt][kt][v] = g.offe[(((size_t)wave * g.n_mg + mg) * g.K + min(k0 + kt * 16 + 4 * lq + v, g.K - 1)) * GM_TM +
+                                        mt * 16 + lr];
+    for (int s = nothing ? n_chunks : 0; s < n_chunks; ++s) {
+        // the bound of every pixel, see mex_grads_rows_kernel
+        float bound[4];
+        if (g.K <= 32 || roomy) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                bound[e] = -INFINITY;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float v[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    bound[e] = fmaxf(bound[e], v[e] * g.c1);
+            }
+            for (int k = lq; k < g.K && g.K > 32; k += 32) {
+                float4 xr[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)   // (behind the last: the last)
+                    xr[j] = rows_load<float4>(x_c, x_at + (unsigned)min(k + 4 * j, g.K - 1) * g.HW);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float v[4] = {xr[j].x, xr[j].y, xr[j].z, xr[j].w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        bound[e] = fmaxf(bound[e], v[e] * g.c1);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                for (int d = 16; d < 64; d <<= 1)
+                    bound[e] = fmaxf(bound[e], __shfl_xor(bound[e], d, 64));
+                if (roomy && img_ok && !(fabsf(bound[e]) < INFINITY))
+                    odd_sh[q0.region(e)] = 1;   // (every writer writes the same value)
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                bound[e] = INFINITY;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float o[4] = {ov[j].x, ov[j].y, ov[j].z, ov[j].w};
+                const bool there = mg * GM_TM + lq + 4 * j < g.M;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    bound[e] = fminf(bound[e], there ? __builtin_fmaf(o[e], g.c1, -lo[j][e & 1]) : INFINITY);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                for (int d = 16; d < 64; d <<= 1)
+                    bound[e] = fminf(bound[e], __shfl_xor(bound[e], d, 64));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            bound[e] = img_ok ? bound[e] : 0.0f;
+        __syncthreads();               // everyone is done with the tiles
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const bool use_m = img_ok && mg * GM_TM + lq + 4 * j < g.M, use_k = img_ok && k0 + lq + 4 * j < g.K;
+            const float o[4] = {ov[j].x, ov[j].y, ov[j].z, ov[j].w}, x[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+            float gg[4];
+            rows_quad_g(gv[j], gg);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float w = gg[e] * __builtin_amdgcn_exp2f(__builtin_fmaf(-o[e], g.c1, bound[e]) + hi[j][e & 1]);
+                const float v = __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], g.c1, -bound[e]));
+                wt[tile_index(j, e)] = use_m ? w : 0.0f;
+                et[tile_index(j, e)] = use_k ? v : 0.0f;
+            }
+        }
+        if (s + 1 < n_chunks)
+            request(bx * g.pxl + s + 1);
+        __syncthreads();
+        floatx4 sum[2][2];
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+                sum[mt][kt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float wa[2][4], xa[2][4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int at = (h * 16 + lr) * TP + wave * 64 + 16 * lq + 4 * i;
+                const float4 w = *reinterpret_cast<const float4 *>(wt + at), x = *reinterpret_cast<const float4 *>(et + at);
+                wa[h][0] = w.x; wa[h][1] = w.y; wa[h][2] = w.z; wa[h][3] = w.w;
+                xa[h][0] = x.x; xa[h][1] = x.y; xa[h][2] = x.z; xa[h][3] = x.w;
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                    for (int kt = 0; kt < 2; ++kt)
+                        sum[mt][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[kt][c], wa[mt][c], sum[mt][kt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)   // times 2^(os_mk - mo_m), as mex_grads_rows_kernel adds them
+                    total[mt][kt][v] = rows_sum(total[mt][kt][v], rows_product(sum[mt][kt][v], eov[mt][kt][v]));
+    }
+    __syncthreads();                   // (odd_sh is in place)
+    int late[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        late[r] = __builtin_amdgcn_readfirstlane(wide_sh[r] | odd_sh[r]) != 0 ? kLateOffsets : 0;
+    if (!__builtin_amdgcn_readfirstlane(wide_sh[wave] | odd_sh[wave])) {
+        // partial sums: a lane's are four neighbouring patch elements of an instance
+        float *dst = g.partial + ((size_t)bx * 4 + wave) * g.M * g.K;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                const int m = mg * GM_TM + mt * 16 + lr, k = k0 + kt * 16 + 4 * lq;
+                if (m >= g.M || k >= g.K)
+                    continue;
+                const floatx4 &t = total[mt][kt];
+                float *at = reinterpret_cast<float *>(reinterpret_cast<char *>(dst) + 4 * ((unsigned)m * g.K + k));
+                if ((g.K & 3) == 0) {
+                    *reinterpret_cast<float4 *>(at) = make_float4(t[0], t[1], t[2], t[3]);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (k + v < g.K)
+                            at[v] = t[v];
+                }
+            }
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    if ((late[0] | late[1] | late[2] | late[3]) != 0)
+        rows_terms<32>(bx, n_chunks, k0, mg, mg + 1, nullptr, 1, make_int4(late[0], late[1], late[2], late[3]));
 #endif
 }
 
@@ -1969,7 +2242,9 @@ struct MexGradTiling {
     bool rows;
     int rows_ksub;                        // 16 * ksub patch elements per workgroup
     int rows_msplit, rows_mg_per_split;   // ... and the split of its instance groups
-    int rows_pxl, rows_cpr;               // offsets gradient: chunks per workgroup, workgroups along the pixels
+    int rows_pxl, rows_cpr;               // chunks per workgroup, workgroups along the pixels
+    bool rows_apart;                      // the offsets gradient in a kernel of its own: mex_grad_offsets_rows_kernel
+    int offsets_pxl, offsets_cpr;         // chunks per workgroup and workgroups along the pixels of either's partial sums
 };
 
 inline int log2_exact(int v)   // log2 of a power of two, -1 otherwise
@@ -1983,7 +2258,7 @@ inline int log2_exact(int v)   // log2 of a power of two, -1 otherwise
 // 2 x 2 unshared offsets over whole-channel patches on a map with power-of-two sides: see the row-wise kernels.
 // A chunk of 256 pixels must be whole images or an even number of whole rows (width <= 128), so that it holds
 // exactly the 64 slots [64 chunk, 64 chunk + 64) of each of the four regions; a 16-byte piece lies in one row
-// (width >= 4).
+// (width 4 and more) or is a window (width 2).
 bool rows_geometry(const MexPlan &p)
 {
     const simnets_mex_dims &d = p.d;
@@ -2054,6 +2329,7 @@ MexGradTiling mex_grad_tiling(const MexPlan &p)
         t.partial_bytes = std::max(t.partial_bytes, align_up(rmk * t.head_wgs, 256));
     t.rows = rows_geometry(p);
     t.rows_ksub = 1; t.rows_msplit = 1; t.rows_mg_per_split = n_mg; t.rows_pxl = 1; t.rows_cpr = 0;
+    t.rows_apart = false; t.offsets_pxl = 1; t.offsets_cpr = 0;
     if (t.rows) {
         const long long chunks = t.slots_pad / 64;
         // 32 patch elements to a workgroup, or 16 if 32 leave the chip short of two workgroups to a compute unit and 16 leave
@@ -2075,7 +2351,22 @@ MexGradTiling mex_grad_tiling(const MexPlan &p)
         while (t.rows_pxl > 1 && (chunks + t.rows_pxl - 1) / t.rows_pxl * tiles < 512)
             t.rows_pxl >>= 1;
         t.rows_cpr = (int)((chunks + t.rows_pxl - 1) / t.rows_pxl);
-        t.partial_bytes = std::max(t.partial_bytes, align_up(rmk * t.rows_cpr, 256));
+        t.offsets_pxl = t.rows_pxl;
+        // The two gradients in a kernel each: W is formed twice, but the offsets' sums stay in registers and partial sums are fewer.
+        // Several tiles of patch elements, so that `out` and `g` are read several times either way, and either several chunks to a
+        // workgroup or many terms.  Both gradients, in one kernel and in two, and the offsets' alone (us): 512 x 96 x 16 x 16 -> 192 262,
+        // 242; 177, 134.  256 x 128 x 16 x 16 -> 256 190, 162; 123, 87.  1024 x 64 x 16 x 16 -> 64 130, 110; 76, 53.  2048 x 128 x 4 x 4 -> 512 181, 162;
+        // 135, 90.  Left in one: 512 x 48 x 16 x 16 -> 96 79, 83 (half of the second tile empty), 256 x 128 x 8 x 8 -> 512 106, 109.  A single tile
+        // and many groups, whose partial sums are many: 2048 x 32 x 8 x 8 -> 256 118, 117; 94, 65; with fewer groups
+        // 512 x 32 x 32 x 32 -> 128 243, 300.  16 elements fill half a tile: left in one.
+        t.rows_apart = p.W > 2 && (d.K > 48 ? t.rows_pxl > 1 || 256.0 * chunks * d.M * d.K >= 0x1p31 : d.K > 16 && d.K <= 32 && n_mg >= 8);
+        if (t.rows_apart) {
+            t.offsets_pxl = 16;
+            while (t.offsets_pxl > 1 && (chunks + t.offsets_pxl - 1) / t.offsets_pxl * ((d.K + 31) / 32) * n_mg < 512)
+                t.offsets_pxl >>= 1;
+        }
+        t.offsets_cpr = (int)((chunks + t.offsets_pxl - 1) / t.offsets_pxl);
+        t.partial_bytes = std::max(t.partial_bytes, align_up(rmk * t.offsets_cpr, 256));
     }
     return t;
 }
@@ -2312,47 +2603,62 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
         RowsArgs rg;
         rg.in = input; rg.out = output; rg.g = output_grad;
         rg.offe = ga.k.offe; rg.omax = ga.k.omax; rg.orng = ga.k.orng;
-        rg.dx = !want_input ? nullptr : t.rows_msplit > 1 ? ga.dx_splits : input_grad;
         rg.dx_split = n_in;
-        rg.partial = want_offsets ? ga.partial : nullptr;
         rg.c0 = ga.k.c0; rg.c1 = ga.k.c1;
         rg.B = p.B; rg.M = d.M; rg.K = d.K; rg.n_mg = (d.M + GM_TM - 1) / GM_TM; rg.mg_per_split = t.rows_mg_per_split;
         rg.lgW = log2_exact(p.W); rg.Ws = p.W / 2; rg.RS = d.region_size; rg.HW = p.H * p.W; rg.lgHW = log2_exact(rg.HW);
-        rg.chunks = t.slots_pad / 64; rg.pxl = t.rows_pxl;
-        rg.nx = t.rows_cpr; rg.ty = (d.K + 16 * t.rows_ksub - 1) / (16 * t.rows_ksub); rg.tz = t.rows_msplit;
-        rg.d_tiles = make_fast_div((unsigned)(rg.ty * rg.tz)); rg.d_ty = make_fast_div((unsigned)rg.ty);
+        rg.chunks = t.slots_pad / 64;
         MexGradArgs gr = ga;   // for the term-by-term path
         gr.wbuf = gr.exbuf = nullptr;
-        gr.pxl = t.rows_pxl; gr.cpr = t.rows_cpr; gr.slots_pad = t.slots_pad;
-        const long long per_die = (1LL * rg.nx * rg.ty * rg.tz + 7) / 8, wgs = 8 * per_die;
-        if (wgs > 0x7fffffffLL)
-            return SIMNETS_ERR_TOO_LARGE;
-        rg.per_die = (int)per_die;
-        const dim3 grid((unsigned)wgs);
-#define SIMNETS_ROWS_LAUNCH(KSUB, W2)                                                                            \
-    if (grad_is_pooled)                                                                                          \
-        hipLaunchKernelGGL((mex_grads_rows_kernel<KSUB, W2, true>), grid, dim3(256), 0, s, rg, gr);              \
-    else                                                                                                         \
-        hipLaunchKernelGGL((mex_grads_rows_kernel<KSUB, W2, false>), grid, dim3(256), 0, s, rg, gr)
-        if (t.rows_ksub == 2 && p.W > 2) {
-            SIMNETS_ROWS_LAUNCH(2, false);
-        } else if (t.rows_ksub == 2) {
-            SIMNETS_ROWS_LAUNCH(2, true);
-        } else if (p.W > 2) {
-            SIMNETS_ROWS_LAUNCH(1, false);
-        } else {
-            SIMNETS_ROWS_LAUNCH(1, true);
+        gr.slots_pad = t.slots_pad;
+        typedef void (*RowsKernel)(RowsArgs, MexGradArgs);
+        auto launch = [&](RowsKernel kernel, bool input, bool offsets, int ksub, int tz, int pxl, int cpr) {
+            rg.dx = !input ? nullptr : t.rows_msplit > 1 ? ga.dx_splits : input_grad;
+            rg.partial = offsets ? ga.partial : nullptr;
+            rg.pxl = gr.pxl = pxl;
+            rg.nx = gr.cpr = cpr; rg.ty = (d.K + 16 * ksub - 1) / (16 * ksub); rg.tz = tz;
+            rg.d_tiles = make_fast_div((unsigned)(rg.ty * rg.tz)); rg.d_ty = make_fast_div((unsigned)rg.ty);
+            const long long per_die = (1LL * rg.nx * rg.ty * rg.tz + 7) / 8, wgs = 8 * per_die;
+            if (wgs > 0x7fffffffLL)
+                return SIMNETS_ERR_TOO_LARGE;
+            rg.per_die = (int)per_die;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, s, rg, gr);
+            return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
+        };
+        auto kernel_of = [&](auto ksub, auto w2) -> RowsKernel {
+            constexpr int k = decltype(ksub)::value;
+            constexpr bool w = decltype(w2)::value;
+            if (!want_offsets || t.rows_apart)
+                return grad_is_pooled ? mex_grads_rows_kernel<k, w, true, kRowsInput> : mex_grads_rows_kernel<k, w, false, kRowsInput>;
+            if (!want_input)
+                return grad_is_pooled ? mex_grads_rows_kernel<k, w, true, kRowsOffsets> : mex_grads_rows_kernel<k, w, false, kRowsOffsets>;
+            return grad_is_pooled ? mex_grads_rows_kernel<k, w, true, 0> : mex_grads_rows_kernel<k, w, false, 0>;
+        };
+        // (alone, in a tile that holds all of K: 16 elements would fill half of it, 1024 x 16 x 16 x 16 -> 64 44 us, 41 in the other kernel)
+        const bool offsets_apart = want_offsets && (t.rows_apart || (!want_input && p.W > 2 && d.K > 16 && d.K <= 16 * t.rows_ksub));
+        const std::integral_constant<int, 1> one;
+        const std::integral_constant<int, 2> two;
+        if (want_input || !offsets_apart) {
+            rc = launch(t.rows_ksub == 2 ? p.W > 2 ? kernel_of(two, std::false_type()) : kernel_of(two, std::true_type())
+                        : p.W > 2        ? kernel_of(one, std::false_type())
+                                         : kernel_of(one, std::true_type()),
+                        want_input, want_offsets && !offsets_apart, t.rows_ksub, t.rows_msplit, t.rows_pxl, t.rows_cpr);
+            if (rc)
+                return rc;
         }
-#undef SIMNETS_ROWS_LAUNCH
-        if (hipGetLastError() != hipSuccess)
-            return SIMNETS_ERR_HIP;
+        if (offsets_apart) {
+            rc = launch(grad_is_pooled ? mex_grad_offsets_rows_kernel<true> : mex_grad_offsets_rows_kernel<false>, false, true, 2, rg.n_mg,
+                        t.offsets_pxl, t.offsets_cpr);
+            if (rc)
+                return rc;
+        }
         // sums of the splits and of the chunks, in one launch if both are there to do (n_in is a multiple of 4: whole planes
         // of at least four pixels)
         const long long rows = (long long)d.num_regions * d.M, n4 = want_input && t.rows_msplit > 1 ? n_in / 4 : 0;
         const long long wgs_sum = (n4 + 255) / 256;
         if (want_offsets && d.K % 4 == 0 && d.K <= kFinishRowsMaxK && rows + wgs_sum <= 0x7fffffffLL) {
             hipLaunchKernelGGL(mex_grads_finish_kernel, dim3((unsigned)(rows + wgs_sum)), dim3(256), 0, s, ga.partial, n_off,
-                               t.rows_cpr, (int)rows, d.K, p.normalize_offsets ? ga.off : nullptr, offsets_grad,
+                               t.offsets_cpr, (int)rows, d.K, p.normalize_offsets ? ga.off : nullptr, offsets_grad,
                                reinterpret_cast<const float4 *>(ga.dx_splits), n4, t.rows_msplit,
                                reinterpret_cast<float4 *>(input_grad));
             return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
@@ -2420,7 +2726,7 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
             go.wbuf = go.exbuf = nullptr;
         const long long gx = (long long)d.num_regions * go.cpr;
         if (use_rows) {
-            go.cpr = t.rows_cpr;   // (launched above)
+            go.cpr = t.offsets_cpr;   // (launched above)
         } else if (t.mfma) {
             const int gy = (d.M + GOM_MT - 1) / GOM_MT, gz = (d.K + GOM_KT - 1) / GOM_KT;
             if (gx > 0x7fffffffLL || gy > 65535 || gz > 65535)

@@ -1,5 +1,5 @@
 """Both MEX gradients of layers with 2 x 2 unshared offsets over whole-channel patches on maps with power-of-two sides
-(mex_grads_rows_kernel, csrc/mex_grad.hip): maps of two columns, several chunks of pixels to a workgroup (its partial sums are
+(mex_grads_rows_kernel and mex_grad_offsets_rows_kernel, csrc/mex_grad.hip): maps of two columns, several chunks of pixels to a workgroup (its partial sums are
 added to), 16 and 32 patch elements to a workgroup, instance groups split, rows that are no whole 16-byte pieces, few chunks on
 eight dies, and regions that a wide offsets range, or one chunk's wide pixels, send to the term-by-term path.
 Reference: torch in 64 bits."""
@@ -43,6 +43,14 @@ def err(got, want):
     ((1026, 8, 16, 16), 3, 4.5, True),       # ... one chunk's pixels term by term, the other's not
     ((520, 33, 8, 8), 40, 0.5, False),       # 16 elements to a workgroup, the last of 33
     ((70, 48, 4, 4), 70, 3.0, False),
+    # the offsets' gradient in a kernel of its own
+    ((1030, 24, 16, 16), 40, 0.5, False),    # a single tile of patch elements, two groups, two chunks to a workgroup
+    ((1030, 17, 16, 16), 9, 3.0, True),      # ... one group, rows that are no whole 16-byte pieces, infinite pixels' flags
+    ((515, 50, 16, 16), 20, 0.5, False),     # two tiles, the last of 18; the input's gradient beside it
+    ((2100, 70, 4, 8), 40, 3.0, True),       # three, tight bounds
+    ((515, 64, 16, 16), 8, 12.0, False),     # ... term by term
+    ((33, 20, 8, 8), 230, 0.5, False),       # eight groups
+    ((130, 256, 8, 8), 1030, 0.5, False),    # many terms
 ])
 @pytest.mark.parametrize("normalize", [False, True])
 def test_row_wise_gradients(pkg, shape, n, spread, outlier, normalize):
@@ -122,3 +130,26 @@ def test_offsets_gradient_keeps_its_form_for_wide_pixels(pkg, shape, value):
         quiet[::7, :, :2, :2] = 0
         results.append(pkg.mex_offsets_grad(x, off, out, quiet, n, **kw))
     assert torch.equal(*results)
+
+
+def test_offsets_gradient_of_an_infinite_pixel(pkg):
+    """Offsets that span 29 exponents: an infinite value makes its own element's gradient NaN and leaves the others to the
+    other pixels."""
+    gen = torch.Generator(device="cuda").manual_seed(109)
+    shape, n = (520, 64, 16, 16), 6
+    x = torch.randn(shape, generator=gen, device="cuda")
+    off = torch.rand(4, n, 64, 1, 1, generator=gen, device="cuda") * 20
+    off[:, 0, 0], off[:, 0, 1] = 0, 20
+    g = torch.randn(shape[0], n, 16, 16, generator=gen, device="cuda")
+    kw = dict(blocks=[64, 1, 1], strides=[64, 1, 1], unshared_offset_region=[2], softmax_mode=True)
+    plain = pkg.mex_offsets_grad(x, off, reference(x, off, g)[0], g, n, **kw)
+    x[3, 7, 4, 6] = float("inf")   # region 0
+    out = reference(x, off, g)[0]
+    assert out[3, :, 4, 6].isinf().all()
+    doff = pkg.mex_grads(x, off, out, g, n, **kw)[1]
+    assert torch.equal(doff[0].isnan().nonzero()[:, 1].unique().cpu(), torch.tensor([7]))
+    assert err(doff[1:], plain[1:].double()) <= TOL
+    g[3, :, 4, 6] = 0
+    want = reference(torch.where(x.isinf(), torch.zeros_like(x), x), off, g)[2]
+    keep = [k for k in range(64) if k != 7]
+    assert err(doff[:, :, keep], want[:, :, keep]) <= TOL
