@@ -2570,8 +2570,15 @@ int mex_grads(const MexPlan &p, const float *input, const float *offsets, const 
         }
         if (want_offsets) {
             const long long rows = (long long)d.num_regions * d.M;
-            hipLaunchKernelGGL(mex_grad_offsets_finish_tall_rows_kernel, dim3((unsigned)rows), dim3(1024), 0, s, ga.partial,
-                               n_off, t.head_wgs, d.K, p.normalize_offsets ? ga.off : nullptr, offsets_grad);
+            // (1024 threads to a row pay from some 48 partial sums on: 512 elements, 10 instances, the offsets' gradient alone, 8 of them
+            // 14.9 us with 256 threads and 16.4 with 1024, 32 16.0 and 16.6, 60 17.9 and 16.7, 128 21.9 and 19.3; 256 regions of 64
+            // elements, one 49.0 and 52.3)
+            if (t.head_wgs >= 48)
+                hipLaunchKernelGGL(mex_grad_offsets_finish_tall_rows_kernel, dim3((unsigned)rows), dim3(1024), 0, s, ga.partial,
+                                   n_off, t.head_wgs, d.K, p.normalize_offsets ? ga.off : nullptr, offsets_grad);
+            else
+                hipLaunchKernelGGL(mex_grad_offsets_finish_wide_rows_kernel, dim3((unsigned)rows), dim3(256), 0, s, ga.partial,
+                                   n_off, t.head_wgs, d.K, p.normalize_offsets ? ga.off : nullptr, offsets_grad);
             if (hipGetLastError() != hipSuccess)
                 return SIMNETS_ERR_HIP;
         }
