@@ -1617,8 +1617,9 @@ __global__ __launch_bounds__(256) void sim_grad_params_small_kernel(const GradPA
 // neighbours in rows of whole 16-byte pieces) x 256 / E groups (E = 32, or 8 when there are few elements): group j adds the
 // splits j, j + G, ..., the group sums are added in group order through LDS.
 // moment != 0: the partial sums are the moments S1, S2, G of sim_grad_params_kernel<.., MOM = true>.
-// Bound by reading them: 28 splits of 128 x 1152, 33 MB, 14.7 us with an element to a thread (a 64-bit division and eight
-// requests for four splits each), 9.3 with four.
+// Bound by reading them: 28 splits of 128 x 1152, 33 MB, 14.7 us with an element to a thread and a 64-bit division, 9.3 with
+// four.  The whole call (us) with one and with four: 147456 elements 97.1, 95.5, 589824 194, 176; 50000 58.8, 58.7, 40000 50.5,
+// 51.5, 9156 40.3, 53.3, 8192, 208 splits, 32.5, 45.3.
 template <int V>
 __global__ __launch_bounds__(256) void sim_grad_params_finish_kernel(
     const float *__restrict__ partial, const float *__restrict__ templates, const float *__restrict__ weights, int O,
@@ -1634,7 +1635,7 @@ __global__ __launch_bounds__(256) void sim_grad_params_finish_kernel(
     const bool ign = mode == SIM_MODE_L2_NORM_IGNORE_NAN;
     const int G = 256 / E;
     const int e = threadIdx.x % E, grp = threadIdx.x / E;
-    const unsigned idx = blockIdx.x * E + e;   // V elements of a row of the slabs
+    const unsigned idx = blockIdx.x * E + e;   // V elements of a row
     const int o = (int)fast_div(idx, d_row), k = V * (int)(idx - o * d_row.d);
     const bool live = o < O && k < K;
     const size_t src = live ? (size_t)o * Kpad + k : 0;
@@ -1870,16 +1871,17 @@ static int gp_finish(const SimPlan &p, const GpTiling &t, const float *templates
 {
     if ((long long)p.O * p.K == 0)
         return SIMNETS_OK;
-    // rows of whole 16-byte pieces (all but the small form's): four elements to a thread
-    const int V = t.Kpad % 4 == 0 ? 4 : 1;
-    const long long total = (long long)p.O * (t.Kpad / V);
-    const int E = (long long)p.O * p.K <= 4096 ? 8 : 32;  // few elements: more threads per element
+    // Four elements to a thread where that leaves two workgroups to a compute unit, rows of whole 16-byte pieces (all but the small
+    // form's) provided; few elements: more threads per element.
+    const int V = t.Kpad % 4 == 0 && (long long)p.O * p.K >= 65536 ? 4 : 1, pieces = (p.K + V - 1) / V;
+    const long long total = (long long)p.O * pieces;
+    const int E = (long long)p.O * p.K <= 4096 ? 8 : 32;
     if (total + E > 0xffffffffLL)
         return SIMNETS_ERR_TOO_LARGE;
     const unsigned blocks = (unsigned)((total + E - 1) / E);
     auto *kernel = V == 4 ? sim_grad_params_finish_kernel<4> : sim_grad_params_finish_kernel<1>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, reinterpret_cast<const float *>(workspace), templates, weights,
-                       p.O, p.K, t.Opad, t.Kpad, t.S, p.mode, t.moment ? 1 : 0, p.fudge, E, make_fast_div((unsigned)(t.Kpad / V)),
+                       p.O, p.K, t.Opad, t.Kpad, t.S, p.mode, t.moment ? 1 : 0, p.fudge, E, make_fast_div((unsigned)pieces),
                        templates_grad, weights_grad);
     return hipGetLastError() == hipSuccess ? SIMNETS_OK : SIMNETS_ERR_HIP;
 }

@@ -20,6 +20,8 @@ TOL = 1.5e-6
     ((16, 64, 14, 14), 64, 3, 1),      # two chunks to a split
     ((24, 40, 33, 31), 200, 3, 2),
     ((7, 16, 20, 21), 130, 1, 1),
+    ((9, 75, 15, 14), 97, 3, 1),       # 65475 elements, one to a thread of the finish
+    ((9, 75, 15, 14), 98, 3, 1),       # 66150, four; rows of 675
 ])
 def test_parameter_gradients_of_split_pixels(pkg, shape, templates, block, stride, function):
     gen = torch.Generator(device="cuda").manual_seed(41)
@@ -47,3 +49,29 @@ def test_parameter_gradients_of_split_pixels(pkg, shape, templates, block, strid
         error = float((a.double() - b).norm() / b.norm())
         print("%s %.2g" % (name, error))
         assert error <= TOL
+
+
+@pytest.mark.parametrize("missing", [0.0, 0.25])
+@pytest.mark.parametrize("templates", [14, 98])   # one element to a thread of the finish, and four
+def test_parameter_gradients_with_normalization(pkg, templates, missing):
+    gen = torch.Generator(device="cuda").manual_seed(47)
+    x = torch.randn(9, 75, 15, 14, generator=gen, device="cuda")
+    t = torch.randn(templates, 75, 3, 3, generator=gen, device="cuda")
+    w = torch.rand(t.shape, generator=gen, device="cuda") * 1.9 + 0.1
+    kw = dict(blocks=[3, 3], strides=[1, 1], padding=[1, 1], normalization_term=True)
+    if missing:
+        x = x.masked_fill_(torch.rand(x.shape, generator=gen, device="cuda") < missing, float("nan"))
+        kw.update(ignore_nan_input=True, out_of_bounds_value=float("nan"))
+    out = pkg.similarity(x, t, w, **kw)
+    go = torch.randn(out.shape, generator=gen, device="cuda")
+    got = pkg.similarity_parameters_grad(x, t, w, go, **kw)
+    pad = torch.nn.functional.pad(x.double(), (1, 1, 1, 1), value=float("nan") if missing else 0.0)
+    there = (pad == pad).double()
+    x0, keep = (torch.nn.functional.unfold(v, 3) for v in (torch.nan_to_num(pad), there))
+    g = go.double().flatten(2)
+    s0, s1, s2 = (torch.einsum("bmp,bkp->mk", g, v) for v in (keep, x0, x0 * x0))
+    t64, w64 = t.double().flatten(1), w.double().flatten(1)
+    want_t = w64 * (s1 - t64 * s0)
+    want_w = 0.5 * (s0 / (w64 + 0.001) - (s2 - 2 * t64 * s1 + t64 * t64 * s0))
+    for a, b in zip(got, (want_t, want_w)):
+        assert float((a.double().flatten(1) - b).norm() / b.norm()) <= TOL
