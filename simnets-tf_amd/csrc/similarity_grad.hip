@@ -1750,16 +1750,23 @@ GpTiling gp_tiling(const SimPlan &p)
         // us.  A workgroup's prologue and epilogue take 0.6, storing and adding up 10^6 floats of a moment 0.33, and a
         // segment more 0.7: the sums are no longer than above (seg).  Forward and gradients, L1, 3 x 3, before and with
         // the choice: 32 x 64 x 32 x 32 -> 128 580, 566 us, 64 x 16 x 40 x 40 -> 32 341, 310; 5 x 5: 32 x 64 x 32 x 32 -> 64
-        // 1007, 907, 200 x 48 x 9 x 9 -> 48 478, 406.
-        double best = 0;
+        // 1007, 907, 200 x 48 x 9 x 9 -> 48 478, 406.  Of 59 sizes none was the slower for it but the one where this says the same of both
+        // numbers (19 x 47 x 21 x 22 -> 160, 3 x 3, stride 2: 72 splits 53.4 us, 24 57.5): the number above unless another is better
+        // by a hundredth.
+        auto cost_of = [&](int most, int *splits) {
+            const int cps = (t.nchunks + most - 1) / most;
+            *splits = (t.nchunks + cps - 1) / cps;
+            const int used = ((*splits + 7) / 8 * tiles + 63) / 64, segments = (cps + t.seg - 1) / t.seg;
+            return used * (cps + 0.6 + 0.7 * (segments - 1)) + 0.33e-6 * *splits * t.Opad * t.Kpad;
+        };
+        int splits;
+        double best = 0.99 * cost_of(S, &splits);
         for (int rounds = 1; rounds <= 4; ++rounds) {
             const int most = std::min(8 * (64 * rounds / tiles), t.nchunks);
             if (most < 8)
                 continue;
-            const int cps = (t.nchunks + most - 1) / most, splits = (t.nchunks + cps - 1) / cps;
-            const int used = ((splits + 7) / 8 * tiles + 63) / 64, segments = (cps + t.seg - 1) / t.seg;
-            const double cost = used * (cps + 0.6 + 0.7 * (segments - 1)) + 0.33e-6 * splits * t.Opad * t.Kpad;
-            if (best == 0 || cost < best) {
+            const double cost = cost_of(most, &splits);
+            if (cost < best) {
                 best = cost;
                 S = splits;
             }
