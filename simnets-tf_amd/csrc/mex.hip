@@ -581,7 +581,7 @@ __global__ __launch_bounds__(256, PX == 2 ? 4 : 1) void mex_fwd_kernel(const Mex
 // op over the lanes of a wave, every lane's: lanes 32 and 16 apart, then 8, 4, 2 and 1 by turns within rows of sixteen, whose
 // lanes that far apart are equal by then.  The order of an exchange with the lane whose number differs in each bit, highest
 // first (which mex_pool.hip's packing by one thread follows), without its six passes through LDS: with the extremes' pass
-// no longer made twice the launch takes 4.4 us where it took 5.3 (32 rows of 144), 6.1 for 6.7 (1024 of 128), 4.8 for 5.7 (10 of
+// no longer made twice the launch takes 3.8 us where it took 4.2 (32 rows of 144), 4.7 for 5.6 (1024 of 128), 4.7 for 5.2 (10 of
 // 512).
 template <class Op>
 __device__ __forceinline__ float pack_over_wave(float v, Op &&op)

@@ -2316,10 +2316,6 @@ MexGradTiling mex_grad_tiling(const MexPlan &p)
     t.factors_input = t.mfma && k_tiles >= 4 && d.M >= 128;
     t.factors_offsets = t.mfma && m_tiles * ((d.K + GOM_KT - 1) / GOM_KT) >= 16;
     t.factor_bytes = align_up((size_t)d.num_regions * t.slots_pad * ((size_t)t.Mp + t.Kp) * sizeof(float), 256);
-    // Row-wise kernels: about two workgroups per compute unit at least.  The input gradient takes as many patch
-    // elements per workgroup as that allows (each tile of them reads all of `out` and `g`), then splits the instance
-    // groups; the offsets gradient walks as many chunks per workgroup as that allows (each workgroup writes a
-    // partial sum of its tile).
     // The head kernel: terms few enough for one exponential each (a classifier head has 512 x 10 x 512 of them)
     t.head = d.M <= kHeadMaxM && d.K >= 64 && d.K <= 1024 && slots >= 1 &&
              (long long)d.num_regions * slots * d.M * d.K <= (16LL << 20) && (long long)p.C * p.H * p.W <= 0x7fffffffLL;
@@ -2332,6 +2328,9 @@ MexGradTiling mex_grad_tiling(const MexPlan &p)
     t.rows_apart = false; t.offsets_pxl = 1; t.offsets_cpr = 0;
     if (t.rows) {
         const long long chunks = t.slots_pad / 64;
+        // Row-wise kernels, about two workgroups per compute unit at least: tiles of patch elements (each reads all of `out` and `g`), the
+        // split of the instance groups (of the input gradient's sums), and as many chunks to a workgroup as that allows (each
+        // writes a partial sum of its tile).
         // 32 patch elements to a workgroup, or 16 if 32 leave the chip short of two workgroups to a compute unit and 16 leave
         // it less so, whatever the split of the instance groups, or if 32 need a split where 16 do not (512 images, 64 channels of 8 x 8, 128
         // instances: 27.4 + 8.2 us with two splits and their sums, 28.0 + 5.1 without)

@@ -311,7 +311,7 @@ __device__ __forceinline__ int split_virtual_row(const SplitArgs &a, int n, int 
 
 // Input gradient.  One workgroup of WAVES waves: G template tiles of 32 (from mtile0) x 128 pixels; a wave holds one template
 // tile x NI pixel tiles.  Four waves, two workgroups to a compute unit: each stages a chunk between two barriers while the other
-// multiplies.  Eight waves (G = 4), one to a compute unit: twice the rows from what is staged; the next chunk's values are
+// multiplies.  Eight waves (G = 4 or 2), one to a compute unit: twice the rows from what is staged; the next chunk's values are
 // requested two steps ahead and converted into a second buffer, so that a wave does so while another one multiplies.
 template <int CG, int G, int WAVES>
 __device__ __forceinline__ void split_grad_body(const SplitArgs &a, char *lds, int ptile, int mtile0, int flag)
