@@ -1618,8 +1618,9 @@ __global__ __launch_bounds__(256) void sim_grad_params_small_kernel(const GradPA
 // splits j, j + G, ..., the group sums are added in group order through LDS.
 // moment != 0: the partial sums are the moments S1, S2, G of sim_grad_params_kernel<.., MOM = true>.
 // Bound by reading them: 28 splits of 128 x 1152, 33 MB, 14.7 us with an element to a thread and a 64-bit division, 9.3 with
-// four.  The whole call (us) with one and with four: 147456 elements 97.1, 95.5, 589824 194, 176; 50000 58.8, 58.7, 40000 50.5,
-// 51.5, 9156 40.3, 53.3, 8192, 208 splits, 32.5, 45.3.
+// four.  The whole call (us) with one and with four, L2: 589824 elements 192, 174, 147456 95.9, 94.6, 50000 88.1, 87.4, 40000 51.5,
+// 51.8, 23040 37.6, 40.5, 8192, 208 splits, 32.5, 45.3; L1: 67680 52.5, 49.6, 21888 232.4, 229.7, 10440 27.3, 26.8, 9000 49.1, 50.0, 4608
+// 182.5, 184.7.
 template <int V>
 __global__ __launch_bounds__(256) void sim_grad_params_finish_kernel(
     const float *__restrict__ partial, const float *__restrict__ templates, const float *__restrict__ weights, int O,
@@ -1878,9 +1879,11 @@ static int gp_finish(const SimPlan &p, const GpTiling &t, const float *templates
 {
     if ((long long)p.O * p.K == 0)
         return SIMNETS_OK;
-    // Four elements to a thread where that leaves two workgroups to a compute unit, rows of whole 16-byte pieces (all but the small
-    // form's) provided; few elements: more threads per element.
-    const int V = t.Kpad % 4 == 0 && (long long)p.O * p.K >= 65536 ? 4 : 1, pieces = (p.K + V - 1) / V;
+    // Four elements to a thread where there are enough of them, with two sums to add up fewer than with three, rows of whole
+    // 16-byte pieces (all but the small form's) provided; few elements: more threads per element.
+    const int V = t.Kpad % 4 == 0 && (long long)p.O * p.K >= (p.mode == SIM_MODE_L1 ? 10000 : 40000) ? 4 : 1;
+    // Pieces of a row; in fours up to whole workgroups of 32, so that one reads whole lines of one row (0.5 to 1 us less).
+    const int pieces = V == 4 ? std::min(t.Kpad / 4, (p.K + 127) / 128 * 32) : p.K;
     const long long total = (long long)p.O * pieces;
     const int E = (long long)p.O * p.K <= 4096 ? 8 : 32;
     if (total + E > 0xffffffffLL)

@@ -20,8 +20,9 @@ TOL = 1.5e-6
     ((16, 64, 14, 14), 64, 3, 1),      # two chunks to a split
     ((24, 40, 33, 31), 200, 3, 2),
     ((7, 16, 20, 21), 130, 1, 1),
-    ((9, 75, 15, 14), 97, 3, 1),       # 65475 elements, one to a thread of the finish
-    ((9, 75, 15, 14), 98, 3, 1),       # 66150, four; rows of 675
+    ((9, 75, 15, 14), 59, 3, 1),       # 39825 elements, one to a thread of the finish (L2)
+    ((9, 75, 15, 14), 60, 3, 1),       # 40500, four; rows of 675
+    ((9, 75, 15, 14), 14, 3, 1),       # 9450, one (L1)
 ])
 def test_parameter_gradients_of_split_pixels(pkg, shape, templates, block, stride, function):
     gen = torch.Generator(device="cuda").manual_seed(41)
@@ -52,7 +53,7 @@ def test_parameter_gradients_of_split_pixels(pkg, shape, templates, block, strid
 
 
 @pytest.mark.parametrize("missing", [0.0, 0.25])
-@pytest.mark.parametrize("templates", [14, 98])   # one element to a thread of the finish, and four
+@pytest.mark.parametrize("templates", [14, 61])   # one element to a thread of the finish, and four
 def test_parameter_gradients_with_normalization(pkg, templates, missing):
     gen = torch.Generator(device="cuda").manual_seed(47)
     x = torch.randn(9, 75, 15, 14, generator=gen, device="cuda")
