@@ -678,11 +678,11 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, char *lds, __attr
             const int item = wave + kWaves * i;
             if (item >= kHalves * per_half)
                 continue;
-            const int g = CG == 16 && item >= per_half;
+            const int g = CG == 16 && item >= per_half, there = a.C - 1 - (chunk * CG + 8 * g);
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 x[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                    rsrc, src[i], split_channel_offset(a.C, 8 * g, chunk * CG, j) * plane, 0));
+                    rsrc, src[i], (chunk * CG + max(-8 * g, min(j, there))) * plane, 0));
         }
     };
     int level = 0;

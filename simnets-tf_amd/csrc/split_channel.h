@@ -1,4 +1,4 @@
-// Which channel a staging lane of the split matrix kernels reads (similarity_split.hip): plain C++, also compiled by the
+// Which channel a staging lane of the input gradient's split kernel reads (similarity_split.hip): plain C++, also compiled by the
 // host-side tests.  A chunk holds one or two groups of eight channels; a lane's address starts at its group's first channel in
 // chunk 0 and a uniform offset, unsigned, leads from there.  Channels behind the last are read as the last.
 #pragma once

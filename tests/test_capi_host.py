@@ -309,7 +309,7 @@ int main() {
 
 
 def test_channels_of_split_kernels_lie_in_the_tensor(tmp_path):
-    # csrc/split_channel.h (where the split matrix kernels read a chunk's channels): the offset from a group's start is
+    # csrc/split_channel.h (where the input gradient's split kernel reads a chunk's channels): the offset from a group's start is
     # unsigned on the device, and what it leads to is a channel - the wanted one, or the last behind the last
     src = tmp_path / "sc.cpp"
     src.write_text(r"""
